@@ -59,6 +59,16 @@ SIGNATURES: dict[str, tuple[list, type]] = {
                          _I, _I, _P], _I),
     "ddpm_gen_bwd": ([_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _L, _P, _L, _P, _L, _L, _L, _L, _L, _I,
                       _I, _I, _I, _I, _P], _I),
+    "ddpm_flat_cat_elems": ([_L, _L, _L, _L, _I, _I], _L),
+    "ddpm_flat_gen_fwd_pack": ([_P, _P, _P, _P, _P, _P, _P, _L, _L, _L, _L, _L, _I, _I, _I, _I, _I,
+                                _I, _P], _I),
+    "ddpm_flat_fuse_conv_workspace_bytes": ([_L, _L, _L, _L, _I, _I], _L),
+    "ddpm_flat_fuse_conv_fwd_packed": ([_P, _P, _P, _P, _L, _L, _L, _L, _L, _I, _I, _P], _I),
+    "ddpm_flat_fuse_conv_bwd_workspace_bytes": ([_L, _L, _L, _L, _I, _I], _L),
+    "ddpm_flat_fuse_conv_bwd": ([_P, _P, _P, _P, _P, _P, _P, _L, _L, _L, _L, _L, _I, _I, _P], _I),
+    "ddpm_flat_gen_bwd_workspace_bytes": ([_L, _L, _L, _L, _I, _I, _I, _I, _I, _I], _L),
+    "ddpm_flat_gen_bwd": ([_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _L, _L, _L, _L, _L, _I, _I, _I,
+                           _I, _I, _I, _P], _I),
 }
 
 

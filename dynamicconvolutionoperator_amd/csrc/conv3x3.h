@@ -6,6 +6,7 @@
 // the weight gradient's reduction inside the input-gradient launch.
 #pragma once
 
+#include "flat.h"
 #include "gen_common.h"
 
 namespace ddpm {
@@ -22,6 +23,11 @@ struct ConvGeom {
   int cc_per;         // 32-plane chunks per K split
   int seg;            // staged elements per segment row (sw + 2 * kCvPad)
   int x4;             // input rows copied in 16-byte lanes (W % 8 == 0, aligned base)
+  int flat;           // the input is a flat tensor (FlatLay) of `kp` planes per image: tiles of
+                      // 256 positions (tiles_h = f.ft, tiles_w = 1), H and W the image's
+  int kp;
+  int oflat;          // the output is flat too (layout f, M planes per image)
+  FlatLay f;
 };
 
 template <typename T>
@@ -186,16 +192,29 @@ __device__ __forceinline__ void cw_reduce_share(const CwReduce& r, int wg, int w
 // launching.  pack (optional): a packing for its workgroups to run.  defer
 // (optional): describe the split reduction there (items 0 with one split)
 // instead of launching it.
+// f (optional): cat and grad_out are flat tensors of layout f with 4C and gp
+// planes per image.
 int cw_run(const void* cat, const void* grad_out, void* grad_weight, void* grad_bias,
            void* workspace, int64_t workspace_bytes, int64_t n, int64_t c, int64_t h, int64_t w,
-           int dtype, hipStream_t stream, bool check_only, const CvPack* pack, CwReduce* defer);
+           int dtype, hipStream_t stream, bool check_only, const CvPack* pack, CwReduce* defer,
+           const FlatLay* f = nullptr, int64_t gp = 0);
+// Whether tensors that the caller holds as NCHW are copied flat (layout f)
+// rather than staged as they lie: see conv3x3.hip.
+bool cv_flat_rule(FlatLay& f, int64_t n, int64_t k, int64_t h, int64_t w, int esz);
+// The same for grad_out (c planes) and the concat (4c, whole 16-plane blocks)
+// of the weight gradient together.
+bool cv_flat_both(FlatLay& f, int64_t n, int64_t c, int64_t h, int64_t w, int esz);
+// Bytes of its split partials on flat tensors (c <= 128).
+int64_t cw_flat_partial_bytes(const FlatLay& f, int64_t n, int64_t c, int esz);
 
 // The fuse convolution's forward weight packing as a descriptor for another
 // launch (defined in conv3x3.hip): validates the forward's shape (n, 4c -> c,
 // h, w; `dtype` the concat's code) and workspace (as for ddpm_fuse_conv_fwd),
 // and describes packing `weight` into the start of `workspace` in the layout
-// the forward over `cat` reads; total 0 for an empty shape.
+// the forward over `cat` reads; total 0 for an empty shape.  f (optional):
+// `cat` is a flat tensor of that layout.
 int cv_fwd_pack(CvPack& p, const void* cat, const void* weight, void* workspace,
-                int64_t workspace_bytes, int64_t n, int64_t c, int64_t h, int64_t w, int dtype);
+                int64_t workspace_bytes, int64_t n, int64_t c, int64_t h, int64_t w, int dtype,
+                const FlatLay* f = nullptr);
 
 }  // namespace ddpm

@@ -53,12 +53,19 @@ constexpr int kCvPad = 8;                  // staged column halo (one chunk of 2
 constexpr int kCvMaxMB = 4;                // 16-plane blocks of m per workgroup, at most
 constexpr int kCvFillWGs = 256;            // workgroups to aim for (the CU count of an MI355X)
 
-// The weight packing as its own kernel (cv_pack_item per thread).
+// The weight packing as its own kernel (cv_pack_item per thread); the
+// workgroups past it run the flat copy of the input, where there is one.
 template <typename T, int MB>
 __global__ __launch_bounds__(256) void conv3x3_pack_kernel(const T* __restrict__ wt,
                                                            uint32_t* __restrict__ pk, ConvGeom g,
-                                                           int rot, int pairs, int nat) {
+                                                           int rot, int pairs, int nat, FlatCopy fc) {
   const int total = g.mgroups * g.nc32 * 9 * MB * 64;
+  const uint32_t blocks = (uint32_t)(total + 255) / 256;
+  if (blockIdx.x >= blocks) {
+    const uint32_t c = (blockIdx.x - blocks) * 256u + threadIdx.x;
+    if (c < fc.chunks) flat_copy_chunk<T>(fc, g.f, c);
+    return;
+  }
   const int idx = (int)(blockIdx.x * blockDim.x + threadIdx.x);
   if (idx < total) cv_pack_item<T, MB>(wt, pk, g, rot, pairs, nat, idx);
 }
@@ -120,18 +127,65 @@ __device__ __forceinline__ void cv_store(const f32x4 (&acc)[2][MB], int mg, cons
   }
 }
 
+// cv_store of a flat tile: positions pos and pos + 16 of a plane.  A flat
+// output holds zero at the positions outside the image; the K splits' partial
+// sums are [ks][n][M][ft * 256].
+template <typename T, bool BIAS, int MB>
+__device__ __forceinline__ void cv_store_flat(const f32x4 (&acc)[2][MB], int mg, const ConvGeom& g,
+                                              const T* __restrict__ bias, T* __restrict__ out,
+                                              float* __restrict__ part, int ksplit, int n, int pos,
+                                              int quad) {
+  const uint32_t FS = (uint32_t)g.f.ft * kFlatTile;
+#pragma unroll
+  for (int blk = 0; blk < 2; ++blk) {
+    const int p = pos + 16 * blk;
+    const int row = p / g.f.P, col = p - row * g.f.P;
+    const bool in = row < g.H && col < g.W;
+    if (g.ks > 1) {
+      float* __restrict__ po = part + ((size_t)ksplit * g.N + n) * g.M * FS + p;
+#pragma unroll
+      for (int ib = 0; ib < MB; ++ib)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int m = (mg * MB + ib) * 16 + 4 * quad + e;
+          if (m < g.M) po[(size_t)m * FS] = acc[blk][ib][e];
+        }
+    } else {
+      const size_t os = g.oflat ? g.f.S : (size_t)g.H * g.W;
+      T* __restrict__ po = g.oflat ? out + g.f.lead + (size_t)n * g.M * os + p
+                                   : out + (size_t)n * g.M * os + (size_t)row * g.W + col;
+      if (!g.oflat && !in) continue;
+#pragma unroll
+      for (int ib = 0; ib < MB; ++ib)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int m = (mg * MB + ib) * 16 + 4 * quad + e;
+          if (m < g.M) {
+            float v = acc[blk][ib][e];
+            if constexpr (BIAS) v += to_f(bias[m]);
+            po[(size_t)m * os] = from_f<T>(in ? v : 0.f);
+          }
+        }
+    }
+  }
+}
+
 // out: the result in T (ks = 1), or with K split (ks > 1) the fp32 partial
 // sums part[ksplit][n][M][H*W] (no bias) that conv3x3_reduce_kernel adds up.
 // CH: 32-plane chunks per stage (2 for 2-byte types when a K split's chunk
 // count is even: twice the MFMA work per stage and per barrier).
-// AL: aligned layout -- one-row segments of 256 columns on an image whose
+// LAY kCvAl: aligned layout -- one-row segments of 256 columns on an image whose
 // width is a multiple of 256, 16-byte input rows, whole 32-plane chunks: the
 // copies take their offsets from per-lane parts formed once and scalar parts
 // formed per stage, without per-copy tests.
+// LAY kCvFlat: a flat input (FlatLay): the copies are the aligned layout's
+// without its column and row tests (a neighbour outside the image is a zero
+// of the layout).
 // MGL: the workgroup runs g.mgl m groups one after another in one staging
 // pipeline (g.mgl = 1 otherwise).
-template <typename T, bool BIAS, int MB, bool WIDE, bool PAIR = false, int CH = 1, bool AL = false,
-          bool MGL = false>
+enum CvLayout : int { kCvGeneric = 0, kCvAl = 1, kCvFlat = 2 };
+template <typename T, bool BIAS, int MB, bool WIDE, bool PAIR = false, int CH = 1,
+          int LAY = kCvGeneric, bool MGL = false>
 __global__ __launch_bounds__(kCvThreads) void conv3x3_kernel(const T* __restrict__ in,
                                                              const uint32_t* __restrict__ pk,
                                                              const T* __restrict__ bias,
@@ -142,6 +196,8 @@ __global__ __launch_bounds__(kCvThreads) void conv3x3_kernel(const T* __restrict
   typedef typename M::V V;
   typedef CvLds<T, MB, WIDE, CH> L;
   static_assert(!PAIR || CH == 1, "pair planes: one chunk per stage");
+  constexpr bool FL = LAY == kCvFlat, AL = LAY != kCvGeneric;
+  static_assert(!AL || WIDE, "aligned and flat layouts: one-row segments");
   constexpr int P = M::P;
   constexpr int E = (int)sizeof(T);
   extern __shared__ __attribute__((aligned(16))) uint32_t csm[];
@@ -178,7 +234,10 @@ __global__ __launch_bounds__(kCvThreads) void conv3x3_kernel(const T* __restrict
   const int wseg = (32 * wave) / g.sw;
   const int pcol0 = 32 * wave - wseg * g.sw;
 
-  const BufRes xres = make_buf(in + (int64_t)n * g.K * HW, (uint32_t)(g.K * HW * (int64_t)E));
+  // (flat: the resource starts at the zeros ahead of the image's first plane)
+  const BufRes xres =
+      FL ? make_buf(in + (int64_t)n * g.kp * g.f.S, (g.f.lead + (uint32_t)g.kp * g.f.S) * (uint32_t)E)
+         : make_buf(in + (int64_t)n * g.K * HW, (uint32_t)(g.K * HW * (int64_t)E));
   // 16-byte copies of a staged plane: chunk ci = pc + lane of copy `part`
   // (the last copy ends at the plane's end and may overlap the previous one)
   // is column chunk cw of segment row sgr; both are stage-invariant
@@ -202,7 +261,10 @@ __global__ __launch_bounds__(kCvThreads) void conv3x3_kernel(const T* __restrict
 #pragma unroll
     for (int part = 0; part < kParts; ++part) {
       const int gw = w0 + ccol[part];
-      alcol[part] = (unsigned)gw < (unsigned)W ? (uint32_t)gw * (uint32_t)E : kOob;
+      if constexpr (FL)
+        alcol[part] = (uint32_t)(ccol[part] + kCvPad) * (uint32_t)E;  // from the window's start
+      else
+        alcol[part] = (unsigned)gw < (unsigned)W ? (uint32_t)gw * (uint32_t)E : kOob;
     }
   }
   const BufRes xnul = make_buf(in, 0u);
@@ -218,9 +280,14 @@ __global__ __launch_bounds__(kCvThreads) void conv3x3_kernel(const T* __restrict
       // one image row per stage (a row outside the image copies through a
       // resource with no records); plane offset and row offset are scalar
       const int hh = h0 + ki - 1;
-      const bool rok = (unsigned)hh < (unsigned)H;
+      const bool rok = FL || (unsigned)hh < (unsigned)H;
       const BufRes rs = rok ? xres : xnul;
-      const uint32_t roff = rok ? (uint32_t)(hh * W) * (uint32_t)E : 0u;
+      // flat: the window of tile h0 starts kCvPad elements before its first
+      // position, one row pitch per kernel row away (lead >= P + 8: positive)
+      const uint32_t roff =
+          FL ? (uint32_t)((int)g.f.lead - kCvPad + h0 * kFlatTile + (ki - 1) * g.f.P) * (uint32_t)E
+             : (rok ? (uint32_t)(hh * W) * (uint32_t)E : 0u);
+      const uint32_t pstride = FL ? g.f.S : (uint32_t)HW;  // plane stride, elements
       // 16-byte chunks of a staged row: 68 (fp32, two overlapping copies) or
       // 34 (2-byte types, one copy of 34 lanes)
       constexpr int kCpp = (kCvPix + 2 * kCvPad) * E / 16;
@@ -229,7 +296,7 @@ __global__ __launch_bounds__(kCvThreads) void conv3x3_kernel(const T* __restrict
 #pragma unroll
         for (int j = 0; j < 32 * CH / kCvWaves; ++j) {
           const int cr = wave + kCvWaves * j;
-          const uint32_t so = (uint32_t)(ccb * 32 + cr) * (uint32_t)HW * (uint32_t)E + roff;
+          const uint32_t so = (uint32_t)(ccb * 32 + cr) * pstride * (uint32_t)E + roff;
 #pragma unroll
           for (int part = 0; part < kNp; ++part)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(
@@ -299,7 +366,11 @@ __global__ __launch_bounds__(kCvThreads) void conv3x3_kernel(const T* __restrict
   // ---- store of m group mg: lane holds out[m = (mg*MB + ib)*16 + 4*quad +
   //      e][pixel col16 of block]
   auto store_mg = [&](int mg) {
-    cv_store<T, BIAS, MB>(acc, mg, g, bias, out, part, ksplit, n, h0 + wseg, w0 + pcol0 + col16,
+    if constexpr (FL)
+      cv_store_flat<T, BIAS, MB>(acc, mg, g, bias, out, part, ksplit, n,
+                                 h0 * kFlatTile + pcol0 + col16, quad);
+    else
+      cv_store<T, BIAS, MB>(acc, mg, g, bias, out, part, ksplit, n, h0 + wseg, w0 + pcol0 + col16,
                           quad);
   };
 
@@ -464,6 +535,43 @@ __global__ __launch_bounds__(256) void conv3x3_reduce_kernel(const float* __rest
   VecIO<T, VEC>::store(out + i0, v);
 }
 
+// The same sum over the partials of a flat launch, [ks][n*M][FS]: four
+// positions of a plane per thread (P % 4 == 0: of one row), written to a flat
+// output (zero outside the image) or to the image.
+template <typename T, bool BIAS>
+__global__ __launch_bounds__(256) void conv3x3_reduce_flat_kernel(const float* __restrict__ part,
+                                                                  const T* __restrict__ bias,
+                                                                  T* __restrict__ out, ConvGeom g,
+                                                                  uint32_t items) {
+  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+  if (i >= items) return;
+  const uint32_t FS = (uint32_t)g.f.ft * kFlatTile;
+  const uint32_t plane = i / (FS / 4);
+  const int p = (int)(i - plane * (FS / 4)) * 4;
+  const int row = p / g.f.P, col = p - row * g.f.P;
+  const bool in = row < g.H && col < g.W;
+  if (!g.oflat && !in) return;
+  const float b = BIAS ? to_f(bias[plane % (uint32_t)g.M]) : 0.f;
+  float v[4] = {b, b, b, b};
+  const size_t step = (size_t)g.N * g.M * FS;
+  const float* __restrict__ src = part + (size_t)plane * FS + p;
+  for (int s = 0; s < g.ks; ++s) {
+    const f32x4 a = *reinterpret_cast<const f32x4*>(src + s * step);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] += a[e];
+  }
+  if (g.oflat) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = in && col + e < g.W ? v[e] : 0.f;
+    VecIO<T, 4>::store(out + g.f.lead + (size_t)plane * g.f.S + p, v);
+  } else {
+    T* __restrict__ o = out + ((size_t)plane * g.H + row) * g.W + col;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (col + e < g.W) o[e] = from_f<T>(v[e]);
+  }
+}
+
 namespace {
 
 template <typename F>
@@ -486,10 +594,41 @@ int cv_pow2ceil(int64_t v) {
   return p;
 }
 
+// Input-plane splits and m blocks of flat tiles.  A flat grid is any number of
+// workgroups, and one past a multiple of the CUs costs a whole round of them
+// (fp32 forward at 1x64x128x128: 68 tiles x 4 splits = 272 workgroups 30.0 us,
+// x 3 = 204 workgroups of half again the stages 24 us): the choice minimizes
+// rounds x stages by the measured cost of a stage (us, of one or more m
+// blocks) and of the partials' second pass.
+void cv_split_flat(ConvGeom& g, int64_t tiles, int64_t m, int esz) {
+  const double base = esz == 4 ? 0.65 : 0.45, per = esz == 4 ? 0.36 : 0.14;
+  double best = 1e30;
+  for (int mb = kCvMaxMB; mb >= 1; mb /= 2) {
+    const int64_t groups = (m + mb * 16 - 1) / (mb * 16);
+    if (mb > 1 && groups * mb * 16 - m >= mb * 8 && m < mb * 16) continue;  // idle m blocks
+    for (int ks = 1; ks <= g.nc32; ++ks) {
+      const int cc = (g.nc32 + ks - 1) / ks;
+      if ((g.nc32 + cc - 1) / cc != ks) continue;
+      const int64_t wgs = tiles * groups * ks;
+      const double rounds = (double)((wgs + kCvFillWGs - 1) / kCvFillWGs);
+      double t = rounds * (2.5 + 3 * cc * (base + per * mb));
+      if (ks > 1) t += 3.5 + 4e-6 * (double)tiles * kFlatTile * (double)m * (ks + 1) / 4.0;
+      if (t < best) {
+        best = t;
+        g.mb = mb;
+        g.ks = ks;
+        g.cc_per = cc;
+      }
+    }
+  }
+}
+
 // Segment shape and m-block count for a shape: SW = the image width rounded
 // up to a power of two within [32, 256]; MB = 4, halved while the grid has
 // fewer than kCvFillWGs workgroups.  `esz` sizes the LDS staging buffers.
-void cv_geom(ConvGeom& g, int64_t n, int64_t k, int64_t m, int64_t h, int64_t w, int esz) {
+// f: flat tiles of layout f instead of segments.
+void cv_geom(ConvGeom& g, int64_t n, int64_t k, int64_t m, int64_t h, int64_t w, int esz,
+             const FlatLay* f = nullptr) {
   g.N = (int)n;
   g.K = (int)k;
   g.M = (int)m;
@@ -497,10 +636,15 @@ void cv_geom(ConvGeom& g, int64_t n, int64_t k, int64_t m, int64_t h, int64_t w,
   g.W = (int)w;
   int sw = cv_pow2ceil(w);
   sw = sw < 32 ? 32 : (sw > kCvPix ? kCvPix : sw);
+  if (f) sw = kCvPix;
   g.sw = sw;
   g.rs = kCvPix / sw;
-  g.tiles_h = (int)((h + g.rs - 1) / g.rs);
-  g.tiles_w = (int)((w + sw - 1) / sw);
+  g.tiles_h = f ? f->ft : (int)((h + g.rs - 1) / g.rs);
+  g.tiles_w = f ? 1 : (int)((w + sw - 1) / sw);
+  g.flat = f != nullptr;
+  g.f = f ? *f : FlatLay{};
+  g.kp = (int)k;
+  g.oflat = 0;
   g.nc32 = (int)((k + 31) / 32);
   g.mb = kCvMaxMB;
   const int64_t tiles = n * g.tiles_h * g.tiles_w;
@@ -510,10 +654,14 @@ void cv_geom(ConvGeom& g, int64_t n, int64_t k, int64_t m, int64_t h, int64_t w,
   // then halve the m blocks
   g.ks = 1;
   const int64_t mg4 = (m + kCvMaxMB * 16 - 1) / (kCvMaxMB * 16);
-  while (tiles * mg4 * g.ks < kCvFillWGs && 2 * g.ks * 2 <= g.nc32) g.ks *= 2;
-  g.cc_per = (g.nc32 + g.ks - 1) / g.ks;
-  g.ks = (g.nc32 + g.cc_per - 1) / g.cc_per;
-  while (g.mb > 1 && tiles * ((m + g.mb * 16 - 1) / (g.mb * 16)) * g.ks < kCvFillWGs) g.mb /= 2;
+  if (f) {
+    cv_split_flat(g, tiles, m, esz);
+  } else {
+    while (tiles * mg4 * g.ks < kCvFillWGs && 2 * g.ks * 2 <= g.nc32) g.ks *= 2;
+    g.cc_per = (g.nc32 + g.ks - 1) / g.ks;
+    g.ks = (g.nc32 + g.cc_per - 1) / g.cc_per;
+    while (g.mb > 1 && tiles * ((m + g.mb * 16 - 1) / (g.mb * 16)) * g.ks < kCvFillWGs) g.mb /= 2;
+  }
   g.mgroups = (int)((m + g.mb * 16 - 1) / (g.mb * 16));
   // fp32: m groups per workgroup, the largest divisor of mgroups that leaves
   // at least kCvFillWGs workgroups (the input gradient at 256x256: 4 groups,
@@ -554,64 +702,117 @@ int cv_check(int64_t n, int64_t k, int64_t m, int64_t h, int64_t w, int dtype) {
 int64_t cv_align(int64_t v) { return (v + 255) / 256 * 256; }
 
 // Workspace of one direction: the packed weight, then (K split) the fp32
-// partial sums [ks][n][m][h*w].
+// partial sums [ks][n][m][h*w] (flat tiles: [ks][n][m][ft * 256]).
 int64_t cv_workspace_bytes(const ConvGeom& g, int dtype) {
   const int64_t pk = cv_pack_bytes(g, dtype);
   if (g.ks <= 1) return pk;
-  return cv_align(pk) + (int64_t)g.ks * g.N * g.M * g.H * g.W * (int64_t)sizeof(float);
+  const int64_t plane = g.flat ? (int64_t)g.f.ft * kFlatTile : (int64_t)g.H * g.W;
+  return cv_align(pk) + (int64_t)g.ks * g.N * g.M * plane * (int64_t)sizeof(float);
 }
 
-// Launch plan of one direction: the geometry, the aligned layout (256-column
-// segments on whole image rows, 16-byte rows, whole 32-plane chunks in every
-// K split) and, with 2-byte types and four m blocks, the natural slot order of
-// the transposing B reads; several m groups per workgroup only for the fp32
-// input gradient's aligned layout (plain concat layout, no bias).
+// Launch plan of one direction: the geometry, the layout of the copies
+// (kCvAl: 256-column segments on whole image rows, 16-byte rows, whole
+// 32-plane chunks in every K split; kCvFlat: flat tiles) and, with 2-byte types, aligned or
+// flat, the natural slot order of the transposing B reads; several m groups
+// per workgroup only for the fp32 input gradient's aligned and flat layouts
+// (plain concat layout, no bias).
 struct CvPlan {
   ConvGeom g;
-  bool al, nat;
+  int lay;
+  bool nat;
+  int64_t copy;  // bytes of the flat copy of `in` behind the workspace, 0: none
 };
+
+}  // namespace
+
+// Rows that are not whole 16-byte chunks are staged element by element
+// otherwise.
+bool cv_flat_rule(FlatLay& f, int64_t n, int64_t k, int64_t h, int64_t w, int esz) {
+  if (w % 8 == 0) return false;
+  return flat_lay(f, h, w, 1, flat_planes(k), esz) &&
+         flat_elems(f, n * flat_planes(k)) / 8 <= 0x7fffffffLL;
+}
+bool cv_flat_both(FlatLay& f, int64_t n, int64_t c, int64_t h, int64_t w, int esz) {
+  FlatLay fc;
+  return c % 8 == 0 && c <= 128 && cv_flat_rule(f, n, c, h, w, esz) &&
+         cv_flat_rule(fc, n, 4 * c, h, w, esz);
+}
+
+namespace {
+
+// inl: `in` is a flat tensor of that layout with kp planes per image; ol: so
+// is `out`, with m planes.
 void cv_plan(CvPlan& p, const void* in, int64_t n, int64_t k, int64_t m, int64_t h, int64_t w,
-             int dtype, bool pairs, bool bias) {
+             int dtype, bool pairs, bool bias, const FlatLay* inl = nullptr, int64_t kp = 0,
+             bool oflat = false) {
   const int esz = dtype == kF32 ? 4 : 2;
   ConvGeom& g = p.g;
-  cv_geom(g, n, k, m, h, w, esz);
+  FlatLay f;
+  p.copy = 0;
+  if (!inl && cv_flat_rule(f, n, k, h, w, esz)) {
+    inl = &f;
+    kp = flat_planes(k);
+    p.copy = cv_align(flat_elems(f, n * kp) * esz);
+  }
+  cv_geom(g, n, k, m, h, w, esz, inl);
   g.x4 = (w % 8 == 0) && ((uintptr_t)in % 16 == 0);
-  p.al = g.rs == 1 && g.sw == kCvPix && w % kCvPix == 0 && g.x4 && k % 32 == 0 &&
-         g.nc32 % g.cc_per == 0;
-  p.nat = esz == 2 && p.al && g.mb == 4;
-  if (!(esz == 4 && p.al && g.mb == 4 && !pairs && !bias)) g.mgl = 1;
+  if (inl) {
+    p.lay = kCvFlat;
+    g.kp = (int)kp;
+    g.oflat = oflat;
+  } else {
+    p.lay = g.rs == 1 && g.sw == kCvPix && w % kCvPix == 0 && g.x4 && k % 32 == 0 &&
+                    g.nc32 % g.cc_per == 0 && g.mb == 4
+                ? kCvAl
+                : kCvGeneric;
+  }
+  p.nat = esz == 2 && p.lay != kCvGeneric;
+  if (!(esz == 4 && p.lay != kCvGeneric && g.mb == 4 && !pairs && !bias)) g.mgl = 1;
+}
+
+int64_t cv_need(const CvPlan& p, int dtype) {
+  return p.copy ? cv_align(cv_workspace_bytes(p.g, dtype)) + p.copy
+                : cv_workspace_bytes(p.g, dtype);
 }
 
 // red (optional): a weight-gradient split reduction for the kernel's
 // workgroups to run.  pack false: `workspace` already holds the packed weight.
-int cv_run(const void* in, const void* wt, const void* bias, void* out, void* workspace,
-           int64_t workspace_bytes, int64_t n, int64_t k, int64_t m, int64_t h, int64_t w, int rot,
-           int dtype, hipStream_t stream, bool pairs = false, const CwReduce* red = nullptr,
-           bool pack = true) {
-  CvPlan plan;
-  cv_plan(plan, in, n, k, m, h, w, dtype, pairs, bias != nullptr);
-  ConvGeom& g = plan.g;
-  const int64_t need = cv_workspace_bytes(g, dtype);
+int cv_run(const CvPlan& plan, const void* in, const void* wt, const void* bias, void* out,
+           void* workspace, int64_t workspace_bytes, int rot, int dtype, hipStream_t stream,
+           bool pairs = false, const CwReduce* red = nullptr, bool pack = true) {
+  const ConvGeom& g = plan.g;
+  const int64_t n = g.N, m = g.M, h = g.H, w = g.W;
+  const int64_t need = cv_need(plan, dtype);
   if (!workspace || workspace_bytes < need || (uintptr_t)workspace % 16 != 0)
     return kWorkspaceTooSmall;
   float* part = g.ks > 1 ? (float*)((char*)workspace + cv_align(cv_pack_bytes(g, dtype))) : nullptr;
+  FlatCopy fc{nullptr, nullptr, 0, 0, 0};
+  if (plan.copy) {
+    void* dst = (char*)workspace + cv_align(cv_workspace_bytes(g, dtype));
+    fc = flat_copy_of(in, dst, g.f, n, g.K, g.kp);
+    in = dst;
+    if (!pack) {
+      const int e = flat_copy(&fc, 1, g.f, dtype, stream);
+      if (e != 0) return e;
+    }
+  }
   const CwReduce nored{nullptr, nullptr, nullptr, nullptr, 0, 0, 0, 0, 0};
   const CwReduce& rd = red ? *red : nored;
   return cv_with_type(dtype, [&](auto tag) {
     using T = decltype(tag);
-    const bool al = plan.al, nat = plan.nat;
+    const bool nat = plan.nat;
     const int64_t units = (int64_t)g.mgroups * g.nc32 * 9 * g.mb * 64;
-    const dim3 pgrid((unsigned)((units + 255) / 256));
+    const dim3 pgrid((unsigned)((units + 255) / 256 + (fc.chunks + 255) / 256));
     if (pack) {
       if (g.mb == 4)
         hipLaunchKernelGGL((conv3x3_pack_kernel<T, 4>), pgrid, dim3(256), 0, stream, (const T*)wt,
-                           (uint32_t*)workspace, g, rot, (int)pairs, (int)nat);
+                           (uint32_t*)workspace, g, rot, (int)pairs, (int)nat, fc);
       else if (g.mb == 2)
         hipLaunchKernelGGL((conv3x3_pack_kernel<T, 2>), pgrid, dim3(256), 0, stream, (const T*)wt,
-                           (uint32_t*)workspace, g, rot, (int)pairs, (int)nat);
+                           (uint32_t*)workspace, g, rot, (int)pairs, (int)nat, fc);
       else
         hipLaunchKernelGGL((conv3x3_pack_kernel<T, 1>), pgrid, dim3(256), 0, stream, (const T*)wt,
-                           (uint32_t*)workspace, g, rot, (int)pairs, (int)nat);
+                           (uint32_t*)workspace, g, rot, (int)pairs, (int)nat, fc);
       const int e = (int)hipGetLastError();
       if (e != 0) return e;
     }
@@ -624,6 +825,17 @@ int cv_run(const void* in, const void* wt, const void* bias, void* out, void* wo
       int e2 = (int)hipGetLastError();
       if (e2 != 0 || g.ks <= 1) return e2;
       // the K splits' partial sums (and the bias) in split order
+      if (plan.lay == kCvFlat) {
+        const uint32_t items = (uint32_t)(n * m * g.f.ft * (kFlatTile / 4));
+        const dim3 fgrid((items + 255) / 256);
+        if (bias)
+          hipLaunchKernelGGL((conv3x3_reduce_flat_kernel<T, true>), fgrid, dim3(256), 0, stream,
+                             (const float*)part, (const T*)bias, (T*)out, g, items);
+        else
+          hipLaunchKernelGGL((conv3x3_reduce_flat_kernel<T, false>), fgrid, dim3(256), 0, stream,
+                             (const float*)part, (const T*)bias, (T*)out, g, items);
+        return (int)hipGetLastError();
+      }
       const int64_t total = n * m * h * w, hw = h * w;
       const bool v4 = hw % 4 == 0 && (uintptr_t)out % (4 * sizeof(T)) == 0;
       const int64_t items = v4 ? total / 4 : total;
@@ -641,34 +853,45 @@ int cv_run(const void* in, const void* wt, const void* bias, void* out, void* wo
       return v4 ? reduce(std::false_type(), std::integral_constant<int, 4>())
                 : reduce(std::false_type(), std::integral_constant<int, 1>());
     };
+    // two chunks per stage (2-byte types): every K split's chunk count even
+    // and one workgroup per CU at most (the 122 KB of LDS leave no room for a
+    // second: with more workgroups, as the input gradient's 1024 at 256x256,
+    // measured 37 -> 50 us; forward 41.1 -> 40.2 us)
+    const bool two = g.cc_per % 2 == 0 && g.nc32 % g.cc_per == 0 && (int64_t)grid.x <= kCvFillWGs;
     auto pick = [&](auto b, auto pr) {
       constexpr bool B = decltype(b)::value;
       constexpr bool PR = decltype(pr)::value && sizeof(T) == 4;
-      // one-row segments (wide images) with the narrower staging pitch; 2-byte
-      // types take two chunks per stage where every K split's chunk count is
-      // even and the grid has one workgroup per CU at most (the 122 KB of LDS
-      // leave no room for a second: with more workgroups, as the input
-      // gradient's 1024 at 256x256, measured 37 -> 50 us; forward 41.1 ->
-      // 40.2 us)
-      if constexpr (sizeof(T) == 2) {
-        if (g.mb == 4 && g.rs == 1 && g.cc_per % 2 == 0 && g.nc32 % g.cc_per == 0 &&
-            (int64_t)grid.x <= kCvFillWGs) {
-          if (al)
-            return launch(conv3x3_kernel<T, B, 4, true, false, 2, true>,
+      auto wide = [&](auto layc) {  // aligned or flat, MB = 4
+        constexpr int LAY = decltype(layc)::value;
+        if constexpr (sizeof(T) == 2) {
+          if (two)
+            return launch(conv3x3_kernel<T, B, 4, true, false, 2, LAY>,
                           (size_t)2 * CvLds<T, 4, true, 2>::kBuf * 4);
-          return launch(conv3x3_kernel<T, B, 4, true, false, 2>,
-                        (size_t)2 * CvLds<T, 4, true, 2>::kBuf * 4);
         }
-      }
-      if (g.mb == 4 && g.rs == 1) {
         if constexpr (sizeof(T) == 4 && !B && !PR) {
           if (g.mgl > 1)
-            return launch(conv3x3_kernel<T, false, 4, true, false, 1, true, true>,
+            return launch(conv3x3_kernel<T, false, 4, true, false, 1, LAY, true>,
                           (size_t)2 * CvLds<T, 4, true>::kBuf * 4);
         }
-        if (al)
-          return launch(conv3x3_kernel<T, B, 4, true, PR, 1, true>,
-                        (size_t)2 * CvLds<T, 4, true>::kBuf * 4);
+        return launch(conv3x3_kernel<T, B, 4, true, PR, 1, LAY>,
+                      (size_t)2 * CvLds<T, 4, true>::kBuf * 4);
+      };
+      if (plan.lay == kCvFlat) {
+        if (g.mb == 4) return wide(std::integral_constant<int, kCvFlat>());
+        if (g.mb == 2)
+          return launch(conv3x3_kernel<T, B, 2, true, PR, 1, kCvFlat>,
+                        (size_t)2 * CvLds<T, 2, true>::kBuf * 4);
+        return launch(conv3x3_kernel<T, B, 1, true, PR, 1, kCvFlat>,
+                      (size_t)2 * CvLds<T, 1, true>::kBuf * 4);
+      }
+      if (plan.lay == kCvAl) return wide(std::integral_constant<int, kCvAl>());
+      // one-row segments (wide images) with the narrower staging pitch
+      if (g.mb == 4 && g.rs == 1) {
+        if constexpr (sizeof(T) == 2) {
+          if (two)
+            return launch(conv3x3_kernel<T, B, 4, true, false, 2>,
+                          (size_t)2 * CvLds<T, 4, true, 2>::kBuf * 4);
+        }
         return launch(conv3x3_kernel<T, B, 4, true, PR>, (size_t)2 * CvLds<T, 4, true>::kBuf * 4);
       }
       if (g.mb == 4)
@@ -686,6 +909,35 @@ int cv_run(const void* in, const void* wt, const void* bias, void* out, void* wo
   });
 }
 
+CvPack cv_pack_of(const CvPlan& p, const void* weight, void* workspace, int rot, bool pairs) {
+  return CvPack{weight, (uint32_t*)workspace, p.g, rot, pairs ? 1 : 0, p.nat ? 1 : 0,
+                p.g.mgroups * p.g.nc32 * 9 * p.g.mb * 64};
+}
+
+// Resolves the dtype code: kF32Pairs is fp32 with the concat in pair planes
+// (whole 32-plane chunks: C % 8 == 0).
+int cv_dtype(int& dtype, bool& pairs, int64_t c) {
+  pairs = dtype == kF32Pairs;
+  if (pairs) {
+    if (c % 8 != 0) return kUnsupported;
+    dtype = kF32;
+  }
+  return kOk;
+}
+
+// The flat layout of a concat of this shape, guard rows `guard`; kUnsupported
+// where the flat entry points do not take it.
+int cv_flat_check(FlatLay& f, int64_t n, int64_t c, int64_t h, int64_t w, int guard, int dtype) {
+  int st = cv_check(n, 4 * c, c, h, w, dtype);
+  if (st != kOk) return st;
+  if (n == 0 || c == 0 || h == 0 || w == 0) return kOk;
+  if (c % 8 != 0 || c > 128 || !flat_lay(f, h, w, guard, 4 * c, dtype == kF32 ? 4 : 2))
+    return kUnsupported;
+  // 32-bit item counts of the launches over whole tensors
+  if (flat_elems(f, n * (4 * c > 128 ? 4 * c : 128)) > 0x7fffffffLL) return kUnsupported;
+  return kOk;
+}
+
 }  // namespace
 }  // namespace ddpm
 
@@ -697,50 +949,42 @@ extern "C" int64_t ddpm_fuse_conv_workspace_bytes(int64_t n, int64_t c, int64_t 
   if (n < 0 || c <= 0 || h < 0 || w < 0 || dtype < kF32 || dtype > kF16) return 0;
   if (n == 0 || h == 0 || w == 0) return 0;
   // the larger of the two directions' needs at this shape
-  ConvGeom gf, gd;
-  cv_geom(gf, n, 4 * c, c, h, w, dtype == kF32 ? 4 : 2);  // forward: K = 4C, M = C
-  cv_geom(gd, n, c, 4 * c, h, w, dtype == kF32 ? 4 : 2);  // input gradient: K = C, M = 4C
-  const int64_t a = cv_workspace_bytes(gf, dtype), b = cv_workspace_bytes(gd, dtype);
+  CvPlan pf, pd;
+  cv_plan(pf, nullptr, n, 4 * c, c, h, w, dtype, false, true);  // forward: K = 4C, M = C
+  cv_plan(pd, nullptr, n, c, 4 * c, h, w, dtype, false, false);  // input gradient: K = C, M = 4C
+  const int64_t a = cv_need(pf, dtype), b = cv_need(pd, dtype);
   return a > b ? a : b;
 }
 
 extern "C" int ddpm_fuse_conv_fwd(const void* cat, const void* weight, const void* bias, void* out,
                                   void* workspace, int64_t workspace_bytes, int64_t n, int64_t c,
                                   int64_t h, int64_t w, int dtype, hipStream_t stream) {
-  // kF32Pairs: the concat in pair planes (whole 32-plane chunks: C % 8 == 0)
-  const bool pairs = dtype == kF32Pairs;
-  if (pairs) {
-    if (c % 8 != 0) return kUnsupported;
-    dtype = kF32;
-  }
-  int st = cv_check(n, 4 * c, c, h, w, dtype);
+  bool pairs;
+  int st = cv_dtype(dtype, pairs, c);
+  if (st == kOk) st = cv_check(n, 4 * c, c, h, w, dtype);
   if (st != kOk) return st;
   if (n == 0 || c == 0 || h == 0 || w == 0) return kOk;
   if (!cat || !weight || !out) return kBadArgument;
-  return cv_run(cat, weight, bias, out, workspace, workspace_bytes, n, 4 * c, c, h, w, 0, dtype,
-                stream, pairs);
+  CvPlan plan;
+  cv_plan(plan, cat, n, 4 * c, c, h, w, dtype, pairs, bias != nullptr);
+  return cv_run(plan, cat, weight, bias, out, workspace, workspace_bytes, 0, dtype, stream, pairs);
 }
 
 int ddpm::cv_fwd_pack(CvPack& p, const void* cat, const void* weight, void* workspace,
                       int64_t workspace_bytes, int64_t n, int64_t c, int64_t h, int64_t w,
-                      int dtype) {
+                      int dtype, const FlatLay* f) {
   p = CvPack{nullptr, nullptr, ConvGeom{}, 0, 0, 0, 0};
-  const bool pairs = dtype == kF32Pairs;
-  if (pairs) {
-    if (c % 8 != 0) return kUnsupported;
-    dtype = kF32;
-  }
-  int st = cv_check(n, 4 * c, c, h, w, dtype);
+  bool pairs;
+  int st = cv_dtype(dtype, pairs, c);
+  if (st == kOk) st = cv_check(n, 4 * c, c, h, w, dtype);
   if (st != kOk) return st;
   if (n == 0 || c == 0 || h == 0 || w == 0) return kOk;
   if (!cat || !weight) return kBadArgument;
   CvPlan plan;
-  cv_plan(plan, cat, n, 4 * c, c, h, w, dtype, pairs, false);
-  if (!workspace || workspace_bytes < cv_workspace_bytes(plan.g, dtype) ||
-      (uintptr_t)workspace % 16 != 0)
+  cv_plan(plan, cat, n, 4 * c, c, h, w, dtype, pairs, true, f, 4 * c);
+  if (!workspace || workspace_bytes < cv_need(plan, dtype) || (uintptr_t)workspace % 16 != 0)
     return kWorkspaceTooSmall;
-  p = CvPack{weight, (uint32_t*)workspace, plan.g, 0, pairs ? 1 : 0, plan.nat ? 1 : 0,
-             plan.g.mgroups * plan.g.nc32 * 9 * plan.g.mb * 64};
+  p = cv_pack_of(plan, weight, workspace, 0, pairs);
   return kOk;
 }
 
@@ -748,17 +992,16 @@ extern "C" int ddpm_fuse_conv_fwd_packed(const void* cat, const void* bias, void
                                          void* workspace, int64_t workspace_bytes, int64_t n,
                                          int64_t c, int64_t h, int64_t w, int dtype,
                                          hipStream_t stream) {
-  const bool pairs = dtype == kF32Pairs;
-  if (pairs) {
-    if (c % 8 != 0) return kUnsupported;
-    dtype = kF32;
-  }
-  int st = cv_check(n, 4 * c, c, h, w, dtype);
+  bool pairs;
+  int st = cv_dtype(dtype, pairs, c);
+  if (st == kOk) st = cv_check(n, 4 * c, c, h, w, dtype);
   if (st != kOk) return st;
   if (n == 0 || c == 0 || h == 0 || w == 0) return kOk;
   if (!cat || !out) return kBadArgument;
-  return cv_run(cat, nullptr, bias, out, workspace, workspace_bytes, n, 4 * c, c, h, w, 0, dtype,
-                stream, pairs, nullptr, false);
+  CvPlan plan;
+  cv_plan(plan, cat, n, 4 * c, c, h, w, dtype, pairs, bias != nullptr);
+  return cv_run(plan, cat, nullptr, bias, out, workspace, workspace_bytes, 0, dtype, stream, pairs,
+                nullptr, false);
 }
 
 extern "C" int ddpm_fuse_conv_bwd_data(const void* grad_out, const void* weight, void* grad_cat,
@@ -769,8 +1012,10 @@ extern "C" int ddpm_fuse_conv_bwd_data(const void* grad_out, const void* weight,
   if (st != kOk) return st;
   if (n == 0 || c == 0 || h == 0 || w == 0) return kOk;
   if (!grad_out || !weight || !grad_cat) return kBadArgument;
-  return cv_run(grad_out, weight, nullptr, grad_cat, workspace, workspace_bytes, n, c, 4 * c, h, w,
-                1, dtype, stream);
+  CvPlan plan;
+  cv_plan(plan, grad_out, n, c, 4 * c, h, w, dtype, false, false);
+  return cv_run(plan, grad_out, weight, nullptr, grad_cat, workspace, workspace_bytes, 1, dtype,
+                stream);
 }
 
 extern "C" int ddpm_fuse_conv_bwd(const void* cat, const void* weight, const void* grad_out,
@@ -794,17 +1039,146 @@ extern "C" int ddpm_fuse_conv_bwd(const void* cat, const void* weight, const voi
   if (!grad_out || !weight || !grad_cat) return kBadArgument;
   CvPlan plan;
   cv_plan(plan, grad_out, n, c, 4 * c, h, w, ddt, false, false);
-  const int64_t need = cv_workspace_bytes(plan.g, ddt);
-  if (!workspace_data || workspace_data_bytes < need || (uintptr_t)workspace_data % 16 != 0)
+  if (!workspace_data || workspace_data_bytes < cv_need(plan, ddt) ||
+      (uintptr_t)workspace_data % 16 != 0)
     return kWorkspaceTooSmall;
+  const void* go = grad_out;
+  const FlatLay f = plan.g.f;
+  FlatLay fb;
+  const bool flat = plan.copy != 0 && cv_flat_both(fb, n, c, h, w, ddt == kF32 ? 4 : 2);
+  if (flat) {
+    // grad_out flat once for both launches, the concat for the weight gradient
+    void* gof = (char*)workspace_data + cv_align(cv_workspace_bytes(plan.g, ddt));
+    void* catf = (char*)workspace_weight + cv_align(cw_flat_partial_bytes(f, n, c, ddt == kF32 ? 4 : 2));
+    const FlatCopy fc[2] = {flat_copy_of(grad_out, gof, f, n, c, plan.g.kp),
+                            flat_copy_of(cat, catf, f, n, 4 * c, 4 * c)};
+    st = flat_copy(fc, 2, f, ddt, stream);
+    if (st != kOk) return st;
+    go = gof;
+    cat = catf;
+    plan.copy = 0;
+  }
   // the weight-gradient launch packs the input gradient's weight; the input
   // gradient's launch sums the weight gradient's split partials
-  const CvPack pack{weight, (uint32_t*)workspace_data, plan.g, 1, 0, plan.nat ? 1 : 0,
-                    plan.g.mgroups * plan.g.nc32 * 9 * plan.g.mb * 64};
+  const CvPack pack = cv_pack_of(plan, weight, workspace_data, 1, false);
   CwReduce red{nullptr, nullptr, nullptr, nullptr, 0, 0, 0, 0, 0};
-  st = cw_run(cat, grad_out, grad_weight, grad_bias, workspace_weight, workspace_weight_bytes, n, c,
-              h, w, dtype, stream, false, &pack, &red);
+  st = cw_run(cat, go, grad_weight, grad_bias, workspace_weight, workspace_weight_bytes, n, c, h, w,
+              dtype, stream, false, &pack, &red, flat ? &f : nullptr, plan.g.kp);
   if (st != kOk) return st;
-  return cv_run(grad_out, weight, nullptr, grad_cat, workspace_data, workspace_data_bytes, n, c,
-                4 * c, h, w, 1, ddt, stream, false, &red, false);
+  return cv_run(plan, go, weight, nullptr, grad_cat, workspace_data, workspace_data_bytes, 1, ddt,
+                stream, false, &red, false);
+}
+
+// ---- flat concats -----------------------------------------------------------
+
+extern "C" int64_t ddpm_flat_cat_elems(int64_t n, int64_t c, int64_t h, int64_t w, int guard,
+                                       int dtype) {
+  bool pairs;
+  FlatLay f;
+  if (cv_dtype(dtype, pairs, c) != kOk) return 0;
+  if (cv_flat_check(f, n, c, h, w, guard, dtype) != kOk) return 0;
+  if (n == 0 || c == 0 || h == 0 || w == 0) return 0;
+  return flat_elems(f, n * 4 * c);
+}
+
+namespace {
+
+// Parts of ddpm_flat_fuse_conv_bwd's workspace, 256-byte aligned: grad_out
+// laid out flat, the input gradient's packed weight and partials, the weight
+// gradient's partials.
+struct CvFlatBwd {
+  CvPlan plan;
+  int64_t cp, go, data, weight;
+  int64_t bytes() const { return go + data + weight; }
+};
+void cv_flat_bwd(CvFlatBwd& b, const FlatLay& f, int64_t n, int64_t c, int64_t h, int64_t w,
+                 int dtype) {
+  const int esz = dtype == kF32 ? 4 : 2;
+  b.cp = flat_planes(c);
+  cv_plan(b.plan, nullptr, n, c, 4 * c, h, w, dtype, false, false, &f, b.cp, true);
+  b.go = cv_align(flat_elems(f, n * b.cp) * esz);
+  b.data = cv_align(cv_need(b.plan, dtype));
+  b.weight = cv_align(cw_flat_partial_bytes(f, n, c, esz));
+}
+
+}  // namespace
+
+extern "C" int64_t ddpm_flat_fuse_conv_workspace_bytes(int64_t n, int64_t c, int64_t h, int64_t w,
+                                                       int guard, int dtype) {
+  bool pairs;
+  FlatLay f;
+  if (cv_dtype(dtype, pairs, c) != kOk) return 0;
+  if (cv_flat_check(f, n, c, h, w, guard, dtype) != kOk) return 0;
+  if (n == 0 || c == 0 || h == 0 || w == 0) return 0;
+  CvPlan plan;
+  cv_plan(plan, nullptr, n, 4 * c, c, h, w, dtype, pairs, true, &f, 4 * c);
+  return cv_need(plan, dtype);
+}
+
+extern "C" int ddpm_flat_fuse_conv_fwd_packed(const void* cat, const void* bias, void* out,
+                                              void* workspace, int64_t workspace_bytes, int64_t n,
+                                              int64_t c, int64_t h, int64_t w, int guard, int dtype,
+                                              hipStream_t stream) {
+  bool pairs;
+  FlatLay f;
+  int st = cv_dtype(dtype, pairs, c);
+  if (st == kOk) st = cv_flat_check(f, n, c, h, w, guard, dtype);
+  if (st != kOk) return st;
+  if (n == 0 || c == 0 || h == 0 || w == 0) return kOk;
+  if (!cat || !out || (uintptr_t)cat % 16 != 0) return kBadArgument;
+  CvPlan plan;
+  cv_plan(plan, cat, n, 4 * c, c, h, w, dtype, pairs, bias != nullptr, &f, 4 * c);
+  return cv_run(plan, cat, nullptr, bias, out, workspace, workspace_bytes, 0, dtype, stream, pairs,
+                nullptr, false);
+}
+
+extern "C" int64_t ddpm_flat_fuse_conv_bwd_workspace_bytes(int64_t n, int64_t c, int64_t h,
+                                                           int64_t w, int guard, int dtype) {
+  bool pairs;
+  FlatLay f;
+  if (cv_dtype(dtype, pairs, c) != kOk) return 0;
+  if (cv_flat_check(f, n, c, h, w, guard, dtype) != kOk) return 0;
+  if (n == 0 || c == 0 || h == 0 || w == 0) return 0;
+  CvFlatBwd b;
+  cv_flat_bwd(b, f, n, c, h, w, dtype);
+  return b.bytes();
+}
+
+extern "C" int ddpm_flat_fuse_conv_bwd(const void* cat, const void* weight, const void* grad_out,
+                                       void* grad_cat, void* grad_weight, void* grad_bias,
+                                       void* workspace, int64_t workspace_bytes, int64_t n,
+                                       int64_t c, int64_t h, int64_t w, int guard, int dtype,
+                                       hipStream_t stream) {
+  const int code = dtype;
+  bool pairs;
+  FlatLay f;
+  int st = cv_dtype(dtype, pairs, c);
+  if (st == kOk) st = cv_flat_check(f, n, c, h, w, guard, dtype);
+  if (st != kOk) return st;
+  if (n == 0 || c == 0 || h == 0 || w == 0) return kUnsupported;
+  const bool need_w = grad_weight != nullptr;
+  if (!cat || !weight || !grad_out || (uintptr_t)cat % 16 != 0 || need_w != (grad_bias != nullptr) ||
+      (uintptr_t)grad_cat % 16 != 0)
+    return kBadArgument;
+  CvFlatBwd b;
+  cv_flat_bwd(b, f, n, c, h, w, dtype);
+  if (!workspace || workspace_bytes < b.bytes() || (uintptr_t)workspace % 16 != 0)
+    return kWorkspaceTooSmall;
+  char* ws = (char*)workspace;
+  void* go = ws;
+  void* wsd = ws + b.go;
+  void* wsw = ws + b.go + b.data;
+  const FlatCopy fc = flat_copy_of(grad_out, go, f, n, c, b.cp);
+  st = flat_copy(&fc, 1, f, dtype, stream);
+  if (st != kOk) return st;
+  const CvPack pack = cv_pack_of(b.plan, weight, wsd, 1, false);
+  CwReduce red{nullptr, nullptr, nullptr, nullptr, 0, 0, 0, 0, 0};
+  if (need_w) {
+    st = cw_run(cat, go, grad_weight, grad_bias, wsw, b.weight, n, c, h, w, code, stream, false,
+                grad_cat ? &pack : nullptr, grad_cat ? &red : nullptr, &f, b.cp);
+    if (st != kOk) return st;
+  }
+  if (!grad_cat) return kOk;
+  return cv_run(b.plan, go, weight, nullptr, grad_cat, wsd, b.data, 1, dtype, stream, false, &red,
+                !need_w);
 }

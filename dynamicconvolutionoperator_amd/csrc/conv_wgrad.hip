@@ -54,6 +54,8 @@ struct CwGeom {
   int x16;              // cat rows hold whole 16-byte chunks: one 16-byte copy per row
   int g16;              // 2-byte grad_out rows 16-byte aligned (W % 8 == 0): 16-byte copies
   int y4;               // fp32 grad_out rows 16-byte aligned (W % 4 == 0): 16-byte register loads
+  int gp;               // flat tensors (H = 1, W = f.ft * 256 positions): planes per image of grad_out
+  FlatLay f;
 };
 
 // One LDS staging buffer (dwords):
@@ -118,10 +120,12 @@ struct CwPos {
 // their lo plane.  SJ: 128-column subsegments per step (2 for 2-byte types on
 // wide images: twice the work per step and per barrier; each wave takes its
 // 32-token segment in both).
-// AL: aligned layout (16-byte cat and grad_out rows, whole steps, whole
+// LAY 1, aligned layout (16-byte cat and grad_out rows, whole steps, whole
 // 16-plane blocks of ci and co): copy offsets from per-lane parts formed once
-// and scalar parts formed per step, without per-copy tests.
-template <typename T, int MB, bool PP = false, int SJ = 1, bool AL = false>
+// and scalar parts formed per step, without per-copy tests.  LAY 2: flat
+// tensors (FlatLay) -- a step is the next TW positions of a plane, its kernel
+// rows are one row pitch apart, and nothing is outside the image.
+template <typename T, int MB, bool PP = false, int SJ = 1, int LAY = 0>
 __global__ __launch_bounds__(kCwThreads) void conv_wgrad_partial_kernel(
     const T* __restrict__ cat, const T* __restrict__ gout, float* __restrict__ pw,
     float* __restrict__ pb, T* __restrict__ dw_out, T* __restrict__ db_out, CwGeom g,
@@ -131,6 +135,7 @@ __global__ __launch_bounds__(kCwThreads) void conv_wgrad_partial_kernel(
   typedef typename M::E ME;
   typedef CwLds<T, MB, SJ> L;
   constexpr int TW = L::TW, LW = L::LW;
+  constexpr bool AL = LAY != 0, FL = LAY == 2;
   static_assert(!PP || SJ == 1, "pair planes: 128-column steps");
   constexpr int P = M::P;
   constexpr int E = (int)sizeof(T);
@@ -146,7 +151,9 @@ __global__ __launch_bounds__(kCwThreads) void conv_wgrad_partial_kernel(
   const int cb = lsc - split * g.cblocks;
   const int co0 = oh * MB * 16;  // first output plane of this workgroup
   const int C = g.C, CI = g.CI, H = g.H, W = g.W;
-  const int64_t HW = (int64_t)H * W;
+  const int64_t HW = FL ? (int64_t)g.f.S : (int64_t)H * W;  // plane stride
+  const int64_t CO = FL ? g.gp : C;                         // planes per image of grad_out
+  const uint32_t lead = FL ? g.f.lead : 0u;
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
@@ -189,8 +196,8 @@ __global__ __launch_bounds__(kCwThreads) void conv_wgrad_partial_kernel(
   auto image = [&](int n) {
     if (AL && n != rn) {
       rn = n;
-      rx = make_buf(cat + (int64_t)n * CI * HW, (uint32_t)(CI * HW * E));
-      ry = make_buf(gout + (int64_t)n * C * HW, (uint32_t)(C * HW * E));
+      rx = make_buf(cat + (int64_t)n * CI * HW, (uint32_t)((lead + CI * HW) * E));
+      ry = make_buf(gout + (int64_t)n * CO * HW, (uint32_t)((lead + CO * HW) * E));
     }
   };
 
@@ -209,14 +216,16 @@ __global__ __launch_bounds__(kCwThreads) void conv_wgrad_partial_kernel(
 #pragma unroll
       for (int rr = 0; rr < 3; ++rr) {
         const int hh = p.h + rr - 1;
-        const bool ok = (unsigned)hh < (unsigned)H;
-        roff[rr] = ok ? (uint32_t)(hh * W) * E : 0u;
+        const bool ok = FL || (unsigned)hh < (unsigned)H;
+        // flat: the window starts kCwPad elements before the step (lead >= P + 8)
+        roff[rr] = FL ? (uint32_t)((int)lead - kCwPad + p.w0 + (rr - 1) * g.f.P) * E
+                      : (ok ? (uint32_t)(hh * W) * E : 0u);
         rres[rr] = ok ? xres : xnul;
       }
       const uint32_t colb = (uint32_t)(p.w0 - kCwPad + 4 * L::kPerD * lane) * E;
       const bool left = p.w0 == 0 && lane < kCwPad / (4 * L::kPerD);  // the halo left of column 0
       const bool right = p.w0 + TW == W && 4 * L::kPerD * lane >= TW + kCwPad;
-      const uint32_t colv = left || right ? kOob : colb;
+      const uint32_t colv = FL ? 16u * lane : (left || right ? kOob : colb);
       if (lane < L::kXD / 4) {
 #pragma unroll
         for (int jc = 0; jc < (16 + kCwNW - 1) / kCwNW; ++jc) {
@@ -273,7 +282,7 @@ __global__ __launch_bounds__(kCwThreads) void conv_wgrad_partial_kernel(
     const BufRes yres = AL ? ry : make_buf(gout + (int64_t)p.n * C * HW, (uint32_t)(C * HW * E));
     const uint32_t rowel = (uint32_t)(p.h * W);
     if (AL || g.g16) {
-      const uint32_t ystep = (rowel + (uint32_t)p.w0) * 2u;
+      const uint32_t ystep = (lead + rowel + (uint32_t)p.w0) * 2u;
       const bool full = AL || p.w0 + TW <= W;
 #pragma unroll
       for (int j = 0; j < NJ; ++j) {
@@ -322,7 +331,7 @@ __global__ __launch_bounds__(kCwThreads) void conv_wgrad_partial_kernel(
   }
   auto yload = [&](const CwPos& p) {
     if constexpr (AL && kYReg) {
-      const uint32_t ys = ((uint32_t)(p.h * W) + (uint32_t)p.w0) * 4u;
+      const uint32_t ys = (lead + (uint32_t)(p.h * W) + (uint32_t)p.w0) * 4u;
 #pragma unroll
       for (int j = 0; j < YUT; ++j) {
         const int u = tid + kCwThreads * j;
@@ -616,6 +625,14 @@ void cw_geom(CwGeom& g, int64_t n, int64_t c, int64_t h, int64_t w, int tw) {
   g.x16 = 0;
   g.g16 = 0;
   g.y4 = 0;
+  g.gp = 0;
+  g.f = FlatLay{};
+}
+
+// The same for flat tensors: a plane is one row of f.ft * 256 positions.
+void cw_geom_flat(CwGeom& g, const FlatLay& f, int64_t n, int64_t c, int esz, bool pp) {
+  cw_geom(g, n, c, 1, (int64_t)f.ft * kFlatTile, esz == 2 && !pp ? 2 * kCwTW : kCwTW);
+  g.f = f;
 }
 
 int64_t cw_partial_bytes(const CwGeom& g) {
@@ -628,11 +645,37 @@ int64_t cw_partial_bytes(const CwGeom& g) {
 
 using namespace ddpm;
 
+int64_t ddpm::cw_flat_partial_bytes(const FlatLay& f, int64_t n, int64_t c, int esz) {
+  CwGeom g;
+  cw_geom_flat(g, f, n, c, esz, false);
+  return cw_partial_bytes(g);
+}
+
+namespace {
+
+int64_t cw_align(int64_t v) { return (v + 255) / 256 * 256; }
+
+// Workspace where cat and grad_out are copied flat: the split partials, the
+// concat (4C planes), grad_out.
+int64_t cw_copy_bytes(const FlatLay& f, int64_t n, int64_t c, int esz, int64_t& cat_off,
+                      int64_t& go_off) {
+  cat_off = cw_align(cw_flat_partial_bytes(f, n, c, esz));
+  go_off = cat_off + cw_align(flat_elems(f, n * 4 * c) * esz);
+  return go_off + flat_elems(f, n * flat_planes(c)) * esz;
+}
+
+}  // namespace
+
 extern "C" int64_t ddpm_fuse_conv_bwd_weight_workspace_bytes(int64_t n, int64_t c, int64_t h,
                                                              int64_t w, int dtype) {
   if (dtype == kF32Pairs) dtype = kF32;  // the same partials
   if (n <= 0 || c <= 0 || h <= 0 || w <= 0 || dtype < kF32 || dtype > kF16) return 0;
   if (n * h * ((w + kCwTW - 1) / kCwTW) > 0x7fffffffLL) return 0;
+  FlatLay f;
+  if (cv_flat_both(f, n, c, h, w, dtype == kF32 ? 4 : 2)) {
+    int64_t a, b;
+    return cw_copy_bytes(f, n, c, dtype == kF32 ? 4 : 2, a, b);
+  }
   CwGeom g;
   cw_geom(g, n, c, h, w, cw_step_cols(w, dtype == kF32 ? 4 : 2));
   return cw_partial_bytes(g);
@@ -641,7 +684,7 @@ extern "C" int64_t ddpm_fuse_conv_bwd_weight_workspace_bytes(int64_t n, int64_t 
 int ddpm::cw_run(const void* cat, const void* grad_out, void* grad_weight, void* grad_bias,
                  void* workspace, int64_t workspace_bytes, int64_t n, int64_t c, int64_t h,
                  int64_t w, int dtype, hipStream_t stream, bool check_only, const CvPack* pack,
-                 CwReduce* defer) {
+                 CwReduce* defer, const FlatLay* f, int64_t gp) {
   // kF32Pairs: `cat` in pair planes (whole 32-plane chunks: C % 8 == 0)
   const bool pp = dtype == kF32Pairs;
   if (pp) {
@@ -671,8 +714,28 @@ int ddpm::cw_run(const void* cat, const void* grad_out, void* grad_weight, void*
   if (n * h * ((w + kCwTW - 1) / kCwTW) > 0x7fffffffLL) return kUnsupported;
   // 32-bit buffer offsets inside one image's planes
   if (4 * c * h * w * esz > 0x7fffffffLL) return kUnsupported;
+  FlatLay fr;
+  if (!f && cv_flat_both(fr, n, c, h, w, esz)) {
+    int64_t cat_off, go_off;
+    const int64_t need = cw_copy_bytes(fr, n, c, esz, cat_off, go_off);
+    if (!workspace || workspace_bytes < need || (uintptr_t)workspace % 16 != 0)
+      return kWorkspaceTooSmall;
+    if (check_only) return kOk;
+    void* catf = (char*)workspace + cat_off;
+    void* gof = (char*)workspace + go_off;
+    const FlatCopy fc[2] = {flat_copy_of(cat, catf, fr, n, 4 * c, 4 * c),
+                            flat_copy_of(grad_out, gof, fr, n, c, flat_planes(c))};
+    const int e = flat_copy(fc, 2, fr, dtype, stream);
+    if (e != kOk) return e;
+    return cw_run(catf, gof, grad_weight, grad_bias, workspace, cat_off, n, c, h, w,
+                  pp ? (int)kF32Pairs : dtype, stream, false, pack, defer, &fr, flat_planes(c));
+  }
   CwGeom g;
-  cw_geom(g, n, c, h, w, pp ? kCwTW : cw_step_cols(w, esz));
+  if (f)
+    cw_geom_flat(g, *f, n, c, esz, pp);
+  else
+    cw_geom(g, n, c, h, w, pp ? kCwTW : cw_step_cols(w, esz));
+  g.gp = (int)gp;
   const int64_t need = cw_partial_bytes(g);
   if (need > 0 && (!workspace || workspace_bytes < need)) return kWorkspaceTooSmall;
   if (check_only) return kOk;
@@ -696,10 +759,13 @@ int ddpm::cw_run(const void* cat, const void* grad_out, void* grad_weight, void*
       // ci (4C) and of co (one workgroup's MB blocks, or two halves of 64)
       const bool al = g.x16 && (esz == 4 ? g.y4 : g.g16) && w % g.tw == 0 && c % 4 == 0 &&
                       (c <= 64 ? c % 16 == 0 : c == 128);
-      auto kern = pp ? (al ? conv_wgrad_partial_kernel<T, MB, sizeof(T) == 4 && SJ == 1, SJ, true>
-                           : conv_wgrad_partial_kernel<T, MB, sizeof(T) == 4 && SJ == 1, SJ>)
-                     : (al ? conv_wgrad_partial_kernel<T, MB, false, SJ, true>
-                           : conv_wgrad_partial_kernel<T, MB, false, SJ>);
+      constexpr bool PPC = sizeof(T) == 4 && SJ == 1;
+      auto kern = pp ? (f    ? conv_wgrad_partial_kernel<T, MB, PPC, SJ, 2>
+                        : al ? conv_wgrad_partial_kernel<T, MB, PPC, SJ, 1>
+                             : conv_wgrad_partial_kernel<T, MB, PPC, SJ>)
+                     : (f    ? conv_wgrad_partial_kernel<T, MB, false, SJ, 2>
+                        : al ? conv_wgrad_partial_kernel<T, MB, false, SJ, 1>
+                             : conv_wgrad_partial_kernel<T, MB, false, SJ>);
       const int ae = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds);
       if (ae != 0) return ae;
       hipLaunchKernelGGL(kern, dim3((unsigned)(g.splits * g.cblocks * g.ohalves)), dim3(kCwThreads), lds, stream,

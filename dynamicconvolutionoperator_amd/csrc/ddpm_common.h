@@ -344,6 +344,55 @@ __device__ __forceinline__ int dil_of(int b, int d0, int d1, int d2) {
   return b == 0 ? d0 : (b == 1 ? d1 : d2);
 }
 
+// ---------------------------------------------------------------------------
+// Flat layout: planes of an image whose rows are not whole 16-byte chunks or
+// whole kernel steps, stored with zeros around every row so that the staged
+// kernels can walk a plane as one run of positions.
+//
+//   * row h, column w of plane c (planes of all images in a row, `planes` per
+//     image) is element lead + c * S + h * P + w; P, S and lead are multiples
+//     of 8, so rows start on 16 bytes;
+//   * every other element a kernel reads is zero: P >= W + r columns, `lead`
+//     elements before the first plane and at least r rows plus 8 columns
+//     after the last tile of every plane.
+// A neighbour (dh, dw), |dh|, |dw| <= r, of position p is then p + dh * P +
+// dw -- zero outside the image -- for every p, and a tile is 256 consecutive
+// positions of a plane, whatever the image's width: no lane idles at row
+// ends but for the P - W pad columns.
+// ---------------------------------------------------------------------------
+constexpr int kFlatTile = 256;
+struct FlatLay {
+  int H, W, P;    // image rows and columns, row pitch
+  int ft;         // tiles of kFlatTile positions covering H * P
+  uint32_t S;     // plane stride
+  uint32_t lead;  // zeros before plane 0
+};
+
+// The flat layout of an h x w image with r guard rows and columns; false when
+// `planes` planes of elements of `esz` bytes exceed 32-bit byte offsets.
+inline bool flat_lay(FlatLay& f, int64_t h, int64_t w, int64_t r, int64_t planes, int esz) {
+  if (h < 1 || w < 1 || r < 1 || r > 64 || h > (1 << 20) || w > (1 << 20)) return false;
+  const int64_t P = (w + r + 7) / 8 * 8;
+  const int64_t ft = (h * P + kFlatTile - 1) / kFlatTile;
+  const int64_t S = (ft * kFlatTile + r * P + 8 + 7) / 8 * 8;
+  const int64_t lead = (r * P + 8 + 7) / 8 * 8;
+  if ((lead + planes * S) * esz > 0x7fffffffLL) return false;
+  f.H = (int)h;
+  f.W = (int)w;
+  f.P = (int)P;
+  f.ft = (int)ft;
+  f.S = (uint32_t)S;
+  f.lead = (uint32_t)lead;
+  return true;
+}
+
+// Channel planes of a flat copy of a c-channel tensor: whole 32-channel
+// chunks, and for 65..128 channels both halves of 64 that the weight
+// gradients' workgroups take (the extra planes are zero).
+inline int64_t flat_planes(int64_t c) { return c > 64 && c < 128 ? 128 : (c + 31) / 32 * 32; }
+
+inline int64_t flat_elems(const FlatLay& f, int64_t planes) { return f.lead + planes * (int64_t)f.S; }
+
 // Host: lets kernel `fn` launch with `bytes` of dynamic LDS (up to the 160 KB
 // of a gfx950 CU) on the current device.  hipFuncSetAttribute runs only the
 // first time a (kernel, device) pair needs more than the limit already set,

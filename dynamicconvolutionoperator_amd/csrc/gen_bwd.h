@@ -143,11 +143,12 @@ enum YtMode {
   kYtMain = 2,   // run the dY kernel only: `workspace` already holds the packed weight
 };
 // red (optional, kYtMain): a weight-gradient split reduction for the dY
-// kernel's workgroups to run.
+// kernel's workgroups to run.  f (optional): x (flat_planes(c) planes per
+// image) and grad_out (4c) are flat tensors of layout f.
 int yt_run(const void* x, const void* weight, const void* grad_out, void* grad_y, void* workspace,
            int64_t workspace_bytes, int64_t n, int64_t c, int64_t h, int64_t w, int kernel_size,
            int d0, int d1, int d2, int dtype, hipStream_t stream, int mode, YPack* pack,
-           const WReduce* red = nullptr);
+           const WReduce* red = nullptr, const FlatLay* f = nullptr);
 
 // Launches the packing `p` as its own kernel.  Defined in gen_bwd_y.hip.
 int yt_pack(const YPack& p, int kernel_size, int dtype, hipStream_t stream);

@@ -58,6 +58,8 @@ struct WGradGeom {
   int x4;              // y and gradient rows 16-byte aligned (W % 8 == 0): 16-byte copies
   int y4;              // fp32 y rows 16-byte aligned (W % 4 == 0): 16-byte register loads
   int dw_blocks;       // weight-gradient workgroups; any further ones are helpers (see below)
+  int cp;              // flat tensors (H = 1, W = f.ft * 256 positions): planes per image of x and y
+  FlatLay f;
 };
 
 // Tap groups per kernel size: the K = 3 taps are split over three waves of 3
@@ -169,7 +171,12 @@ __global__ __launch_bounds__(256) void gen_ysplit_kernel(const float* __restrict
 // SJ: 128-column subsegments per step (2 for 2-byte types on wide images:
 // twice the work per step and per barrier; each wave takes its 32-token
 // segment in both).
-template <typename T, int KS, int MB, int SJ, bool AL>
+// LAY 1: aligned layout (16-byte x, y and gradient rows, whole steps, whole
+// 16-channel blocks).  LAY 2: flat tensors (FlatLay) -- a step is the next TW
+// positions of a plane, kernel rows are d row pitches apart, and a neighbour
+// outside the image is a zero of the layout, so the copies are the aligned
+// layout's without its tests.
+template <typename T, int KS, int MB, int SJ, int LAY>
 __global__ __launch_bounds__(64 * kWgSegs * WgTaps<KS>::kGroups) void gen_bwd_w_partial_kernel(
     const T* __restrict__ x, const T* __restrict__ y, const T* __restrict__ gout,
     float* __restrict__ pw, float* __restrict__ pb, T* __restrict__ dw_out, T* __restrict__ db_out,
@@ -178,6 +185,7 @@ __global__ __launch_bounds__(64 * kWgSegs * WgTaps<KS>::kGroups) void gen_bwd_w_
   typedef typename M::V V;
   typedef typename M::E ME;
   typedef WgLds<T, KS, MB, SJ> L;
+  constexpr bool AL = LAY != 0, FL = LAY == 2;
   constexpr int TW = L::TW, LW = L::LW;
   constexpr int KK = KS * KS;
   constexpr int r = KS / 2;
@@ -225,8 +233,10 @@ __global__ __launch_bounds__(64 * kWgSegs * WgTaps<KS>::kGroups) void gen_bwd_w_
   const int i0 = ih * MB * 16;  // first input channel of this workgroup
   const int d = dil_of(b, g.d0, g.d1, g.d2);
   const int C = g.C, H = g.H, W = g.W;
-  const int64_t HW = (int64_t)H * W;
+  const int64_t HW = FL ? (int64_t)g.f.S : (int64_t)H * W;  // plane stride
   const int64_t CHW = (int64_t)C * HW;
+  const int64_t XHW = FL ? (int64_t)g.cp * HW : CHW;        // one image of x / y
+  const uint32_t lead = FL ? g.f.lead : 0u;
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
@@ -283,9 +293,9 @@ __global__ __launch_bounds__(64 * kWgSegs * WgTaps<KS>::kGroups) void gen_bwd_w_
   auto image = [&](int n) {
     if (n != rn) {
       rn = n;
-      rx = make_buf(x + (int64_t)n * CHW, (uint32_t)(CHW * E));
-      ry = make_buf(y + (int64_t)n * CHW, (uint32_t)(CHW * E));
-      rg = make_buf(gbase + (int64_t)n * 4 * CHW, (uint32_t)(CHW * E));
+      rx = make_buf(x + (int64_t)n * XHW, (uint32_t)((lead + XHW) * E));
+      ry = make_buf(y + (int64_t)n * XHW, (uint32_t)((lead + XHW) * E));
+      rg = make_buf(gbase + (int64_t)n * 4 * CHW, (uint32_t)((lead + CHW) * E));
     }
   };
 
@@ -304,14 +314,16 @@ __global__ __launch_bounds__(64 * kWgSegs * WgTaps<KS>::kGroups) void gen_bwd_w_
 #pragma unroll
       for (int rr = 0; rr < KS; ++rr) {
         const int hh = p.h + (rr - r) * d;
-        const bool ok = (unsigned)hh < (unsigned)H;
-        roff[rr] = ok ? (uint32_t)(hh * W) * E : 0u;
+        const bool ok = FL || (unsigned)hh < (unsigned)H;
+        // flat: the window starts kWgPad elements before the step (lead >= r d P + 8)
+        roff[rr] = FL ? (uint32_t)((int)lead - kWgPad + p.w0 + (rr - r) * d * g.f.P) * E
+                      : (ok ? (uint32_t)(hh * W) * E : 0u);
         rres[rr] = ok ? rx : xnul;
       }
       const uint32_t colb = (uint32_t)(p.w0 - kWgPad + 4 * L::kPerD * lane) * E;
       const bool left = p.w0 == 0 && lane < kWgPad / (4 * L::kPerD);  // the halo left of column 0
       const bool right = p.w0 + TW == W && 4 * L::kPerD * lane >= TW + kWgPad;
-      const uint32_t colv = left || right ? kOob : colb;
+      const uint32_t colv = FL ? 16u * lane : (left || right ? kOob : colb);
       if (lane < L::kXD / 4) {
 #pragma unroll
         for (int jc = 0; jc < (16 + NW - 1) / NW; ++jc) {
@@ -410,7 +422,8 @@ __global__ __launch_bounds__(64 * kWgSegs * WgTaps<KS>::kGroups) void gen_bwd_w_
       // 1 KB copies: lane l moves one 16-byte chunk; the step's byte offset
       // is the scalar offset, and lanes past the image's right edge are
       // masked only in a partial column block
-      const uint32_t ystep = (rowel + (uint32_t)p.w0) * 2u, gstep = (rowel + (uint32_t)p.w0) * E;
+      const uint32_t ystep = (lead + rowel + (uint32_t)p.w0) * 2u,
+                     gstep = (lead + rowel + (uint32_t)p.w0) * E;
       auto copies = [&](auto masked) {
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
@@ -483,7 +496,7 @@ __global__ __launch_bounds__(64 * kWgSegs * WgTaps<KS>::kGroups) void gen_bwd_w_
   }
   auto yload = [&](const WgPos& p) {
     if constexpr (AL && kYReg) {
-      const uint32_t ys = ((uint32_t)(p.h * W) + (uint32_t)p.w0) * 4u;
+      const uint32_t ys = (lead + (uint32_t)(p.h * W) + (uint32_t)p.w0) * 4u;
 #pragma unroll
       for (int j = 0; j < YUT; ++j) {
         const int u = tid + NT * j;
@@ -867,6 +880,16 @@ void wgrad_geom(WGradGeom& g, int64_t n, int64_t c, int64_t h, int64_t w, int d0
   g.x4 = 0;
   g.y4 = 0;
   g.dw_blocks = 0;
+  g.cp = 0;
+  g.f = FlatLay{};
+}
+
+// The same for flat tensors: a plane is one row of f.ft * 256 positions.
+void wgrad_geom_flat(WGradGeom& g, const FlatLay& f, int64_t n, int64_t c, int d0, int d1, int d2,
+                     int esz) {
+  wgrad_geom(g, n, c, 1, (int64_t)f.ft * kFlatTile, d0, d1, d2, esz == 2 ? 2 * kWgTW : kWgTW);
+  g.cp = (int)flat_planes(c);
+  g.f = f;
 }
 
 // Workspace: the fp32 split partials (none with one split).
@@ -890,6 +913,12 @@ extern "C" int64_t ddpm_gen_bwd_w_workspace_bytes(int64_t n, int64_t c, int64_t 
   return wg_partial_bytes(g, c, kernel_size);
 }
 
+extern "C" int64_t ddpm_flat_cat_elems(int64_t n, int64_t c, int64_t h, int64_t w, int guard,
+                                       int dtype);
+extern "C" int64_t ddpm_gen_bwd_x_workspace_bytes(int64_t n, int64_t c, int64_t h, int64_t w,
+                                                  int kernel_size, int d0, int d1, int d2);
+extern "C" int64_t ddpm_gen_bwd_y_workspace_bytes(int64_t c, int kernel_size);
+
 namespace {
 
 // Helper workgroups for a deferred halo reduction: the CUs the weight-gradient
@@ -905,12 +934,13 @@ int wg_helpers(int dw_blocks) {
 // fin (optional): a halo reduction of the input gradient to run alongside.
 // yp (optional): the dY weight packing to run alongside.  defer (optional):
 // describe the split reduction there (items 0 with one split) instead of
-// launching it.
+// launching it.  f (optional): x, y (flat_planes(c) planes per image) and
+// grad_out (4c) are flat tensors of layout f.
 int bw_run(const void* x, const void* y, const void* grad_out, void* grad_weight,
            void* grad_bias, void* workspace, int64_t workspace_bytes, int64_t n, int64_t c,
            int64_t h, int64_t w, int kernel_size, int d0, int d1, int d2, int dtype,
            hipStream_t stream, bool check_only, const BxFinish* fin, const YPack* yp = nullptr,
-           WReduce* defer = nullptr) {
+           WReduce* defer = nullptr, const FlatLay* f = nullptr) {
   if (dtype < kF32 || dtype > kF16) return kBadArgument;
   GenGeom gg;
   int st = gen_make_geom(gg, n, c, h, w, kernel_size, d0, d1, d2);
@@ -925,7 +955,10 @@ int bw_run(const void* x, const void* y, const void* grad_out, void* grad_weight
   // 32-bit indices of the split reduction
   if ((int64_t)3 * kernel_size * kernel_size * c * (c + 1) > 0x7fffffffLL) return kUnsupported;
   WGradGeom g;
-  wgrad_geom(g, n, c, h, w, gg.d0, gg.d1, gg.d2, wg_step_cols(w, esz));
+  if (f)
+    wgrad_geom_flat(g, *f, n, c, gg.d0, gg.d1, gg.d2, esz);
+  else
+    wgrad_geom(g, n, c, h, w, gg.d0, gg.d1, gg.d2, wg_step_cols(w, esz));
   const int64_t need = wg_partial_bytes(g, c, kernel_size);
   if (need > 0 && (!workspace || workspace_bytes < need)) return kWorkspaceTooSmall;
   // LDS-direct dword copies of x rows need every row to start on a dword boundary
@@ -954,7 +987,7 @@ int bw_run(const void* x, const void* y, const void* grad_out, void* grad_weight
       constexpr int KS = decltype(ks)::value;
       constexpr int MB = decltype(mbc)::value;
       constexpr int SJ = decltype(sjc)::value;
-      constexpr bool AL = decltype(alc)::value;
+      constexpr int AL = decltype(alc)::value;
       constexpr int KKc = KS * KS;
       typedef WgLds<T, KS, MB, SJ> L;
       const size_t stage = (size_t)2 * L::kBuf * 4;
@@ -1002,8 +1035,9 @@ int bw_run(const void* x, const void* y, const void* grad_out, void* grad_weight
                       (c <= 64 || c == 128);
       auto by_k = [&](auto sjc) {
         auto by_al = [&](auto ks) {
-          if (al) return launch(ks, mbc, sjc, std::true_type{});
-          return launch(ks, mbc, sjc, std::false_type{});
+          if (f) return launch(ks, mbc, sjc, std::integral_constant<int, 2>{});
+          if (al) return launch(ks, mbc, sjc, std::integral_constant<int, 1>{});
+          return launch(ks, mbc, sjc, std::integral_constant<int, 0>{});
         };
         if (kernel_size == 1) return by_al(std::integral_constant<int, 1>());
         return by_al(std::integral_constant<int, 3>());
@@ -1074,4 +1108,105 @@ extern "C" int ddpm_gen_bwd(const void* x, const void* y, const void* weight, co
   if (st != kOk) return st;
   return yt_run(x, weight, grad_out, grad_y, workspace_y, workspace_y_bytes, n, c, h, w,
                 kernel_size, d0, d1, d2, dtype, stream, kYtMain, nullptr, &red);
+}
+
+// ---- flat gradients of the concat -------------------------------------------
+
+namespace {
+
+// Parts of ddpm_flat_gen_bwd's workspace, 256-byte aligned: x and y laid out
+// flat, dX's tile partials, dY's packed weight, dW's split partials.
+struct FlatBwd {
+  FlatLay f;
+  int64_t copy, bx, by, bw;
+  int64_t bytes() const { return 2 * copy + bx + by + bw; }
+};
+
+int64_t align256(int64_t v) { return (v + 255) / 256 * 256; }
+
+int flat_bwd(FlatBwd& b, int64_t n, int64_t c, int64_t h, int64_t w, int kernel_size, int d0, int d1,
+             int d2, int guard, int dtype) {
+  if (dtype < kF32 || dtype > kF16) return kBadArgument;
+  GenGeom gg;
+  const int st = gen_make_geom(gg, n, c, h, w, kernel_size, d0, d1, d2);
+  if (st != kOk) return st;
+  if (n == 0 || c == 0 || h == 0 || w == 0) return kUnsupported;
+  const int esz = dtype == kF32 ? 4 : 2;
+  // the guard rows and columns hold every tap's neighbours
+  if (guard < gg.R || ddpm_flat_cat_elems(n, c, h, w, guard, dtype) == 0 ||
+      !flat_lay(b.f, h, w, guard, 4 * c, esz))
+    return kUnsupported;
+  WGradGeom g;
+  wgrad_geom_flat(g, b.f, n, c, gg.d0, gg.d1, gg.d2, esz);
+  b.copy = align256(flat_elems(b.f, n * flat_planes(c)) * esz);
+  b.bx = align256(ddpm_gen_bwd_x_workspace_bytes(n, c, h, w, kernel_size, d0, d1, d2));
+  b.by = align256(ddpm_gen_bwd_y_workspace_bytes(c, kernel_size));
+  b.bw = align256(wg_partial_bytes(g, c, kernel_size));
+  return kOk;
+}
+
+}  // namespace
+
+extern "C" int64_t ddpm_flat_gen_bwd_workspace_bytes(int64_t n, int64_t c, int64_t h, int64_t w,
+                                                     int kernel_size, int d0, int d1, int d2,
+                                                     int guard, int dtype) {
+  FlatBwd b;
+  return flat_bwd(b, n, c, h, w, kernel_size, d0, d1, d2, guard, dtype) == kOk ? b.bytes() : 0;
+}
+
+extern "C" int ddpm_flat_gen_bwd(const void* x, const void* y, const void* weight, const void* bias,
+                                 const void* grad_cat, void* grad_x, void* grad_y,
+                                 void* grad_weight, void* grad_bias, void* workspace,
+                                 int64_t workspace_bytes, int64_t n, int64_t c, int64_t h, int64_t w,
+                                 int kernel_size, int d0, int d1, int d2, int guard, int dtype,
+                                 hipStream_t stream) {
+  FlatBwd b;
+  int st = flat_bwd(b, n, c, h, w, kernel_size, d0, d1, d2, guard, dtype);
+  if (st != kOk) return st;
+  const bool need_w = grad_weight != nullptr;
+  if (!x || !y || !weight || !bias || !grad_cat || (uintptr_t)grad_cat % 16 != 0 ||
+      need_w != (grad_bias != nullptr))
+    return kBadArgument;
+  if (!workspace || workspace_bytes < b.bytes() || (uintptr_t)workspace % 16 != 0)
+    return kWorkspaceTooSmall;
+  char* ws = (char*)workspace;
+  void* xf = ws;
+  void* yf = ws + b.copy;
+  void* wsx = ws + 2 * b.copy;
+  void* wsy = (char*)wsx + b.bx;
+  void* wsw = (char*)wsy + b.by;
+  // every part validated before anything is launched (the x part on its launch)
+  YPack yp{nullptr, nullptr, 0, 0, 0};
+  if (need_w) {
+    st = bw_run(xf, yf, grad_cat, grad_weight, grad_bias, wsw, b.bw, n, c, h, w, kernel_size, d0, d1,
+                d2, dtype, stream, true, nullptr, nullptr, nullptr, &b.f);
+    if (st != kOk) return st;
+  }
+  if (grad_y) {
+    st = yt_run(xf, weight, grad_cat, grad_y, wsy, b.by, n, c, h, w, kernel_size, d0, d1, d2, dtype,
+                stream, kYtCheck, &yp);
+    if (st != kOk) return st;
+  }
+  BxFinish fin{nullptr, nullptr, nullptr, TileGeom{}, 0, 1};
+  if (grad_x) {
+    st = bx_run(y, weight, bias, grad_cat, grad_x, wsx, b.bx, n, c, h, w, kernel_size, d0, d1, d2,
+                dtype, stream, need_w ? &fin : nullptr, &b.f);
+    if (st != kOk) return st;
+  }
+  if (grad_y || need_w) {
+    const FlatCopy fc[2] = {flat_copy_of(x, xf, b.f, n, c, flat_planes(c)),
+                            flat_copy_of(y, yf, b.f, n, c, flat_planes(c))};
+    st = flat_copy(fc, need_w ? 2 : 1, b.f, dtype, stream);
+    if (st != kOk) return st;
+  }
+  WReduce red{nullptr, nullptr, nullptr, nullptr, 0, 0, 0, 0, 0};
+  if (need_w) {
+    st = bw_run(xf, yf, grad_cat, grad_weight, grad_bias, wsw, b.bw, n, c, h, w, kernel_size, d0, d1,
+                d2, dtype, stream, false, grad_x ? &fin : nullptr, grad_y ? &yp : nullptr,
+                grad_y ? &red : nullptr, &b.f);
+    if (st != kOk) return st;
+  }
+  if (!grad_y) return kOk;
+  return yt_run(xf, weight, grad_cat, grad_y, wsy, b.by, n, c, h, w, kernel_size, d0, d1, d2, dtype,
+                stream, need_w ? kYtMain : kYtFull, nullptr, &red, &b.f);
 }

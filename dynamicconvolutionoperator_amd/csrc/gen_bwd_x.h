@@ -8,9 +8,10 @@
 
 namespace ddpm {
 
-// One item = VEC consecutive columns of one row of dX (VEC = 4 needs W % 4 ==
-// 0: 16-byte aligned partial groups, as the tile kernel lays them out); items
-// are flattened over all rows (n, c, h) so that every lane has work.  The halo of at most one vertical and one horizontal neighbour covers a
+// One item = VEC consecutive columns of one row of dX (VEC = 4 needs 16-byte
+// partial groups, as the tile kernel lays them out, and rows of gO that start
+// on 4 elements: W % 4 == 0 or a flat gO; the last group of a row is then
+// stored in part); items are flattened over all rows (n, c, h) so that every lane has work.  The halo of at most one vertical and one horizontal neighbour covers a
 // pixel (R <= 8 is at most half a tile side), so the sum is gO_x + own +
 // vertical + horizontal + diagonal partial, in that order.
 template <typename T, int VEC>
@@ -41,10 +42,9 @@ __device__ __forceinline__ void bx_reduce_item(const float* __restrict__ part,
     return part + (wg * 16 + ch) * LHp + (lr + g.R - ddy * kGtTH) * g.LWp +
            (lc + g.R + g.pad - ddx * g.TW);
   };
-  const int64_t HW = (int64_t)g.H * g.W;
-  const int64_t pix = (int64_t)h * g.W + w;
-  const T* __restrict__ go = gout + ((int64_t)n * 4 * g.C + c) * HW + pix;
-  T* __restrict__ dst = gx + (int64_t)nc * HW + pix;
+  const T* __restrict__ go =
+      gout + g.olead + ((int64_t)n * 4 * g.C + c) * g.OS + (int64_t)h * g.OP + w;
+  T* __restrict__ dst = gx + (int64_t)nc * g.H * g.W + (int64_t)h * g.W + w;
   if constexpr (VEC == 4) {
     const TV gv = *reinterpret_cast<const TV*>(go);
     FV s = {to_f(gv[0]), to_f(gv[1]), to_f(gv[2]), to_f(gv[3])};
@@ -53,7 +53,13 @@ __device__ __forceinline__ void bx_reduce_item(const float* __restrict__ part,
     if (dx != 0) s += *reinterpret_cast<const FV*>(at(0, dx));
     if (dy != 0 && dx != 0) s += *reinterpret_cast<const FV*>(at(dy, dx));
     const TV o = {from_f<T>(s[0]), from_f<T>(s[1]), from_f<T>(s[2]), from_f<T>(s[3])};
-    *reinterpret_cast<TV*>(dst) = o;
+    if (g.vec) {
+      *reinterpret_cast<TV*>(dst) = o;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (w + e < g.W) dst[e] = o[e];
+    }
   } else {
     float s = to_f(go[0]);
     s += *at(0, 0);
@@ -72,16 +78,17 @@ struct BxFinish {
   void* gx;
   TileGeom g;
   int64_t items;
-  int vec;  // 4 (W % 4 == 0) or 1
+  int vec;  // 4 (W % 4 == 0 or a flat gO) or 1
 };
 
 // ddpm_gen_bwd_x's work: validates, launches the tile kernel and then either
 // the reduction kernel (defer == nullptr) or nothing, describing the
-// reduction in *defer instead.  Defined in gen_bwd_x.hip.
+// reduction in *defer instead.  f (optional): grad_out is a flat tensor of that
+// layout.  Defined in gen_bwd_x.hip.
 int bx_run(const void* y, const void* weight, const void* bias, const void* grad_out,
            void* grad_x, void* workspace, int64_t workspace_bytes, int64_t n, int64_t c,
            int64_t h, int64_t w, int kernel_size, int d0, int d1, int d2, int dtype,
-           hipStream_t stream, BxFinish* defer);
+           hipStream_t stream, BxFinish* defer, const FlatLay* f = nullptr);
 
 // Launches the halo reduction `f` as its own kernel.  Defined in
 // gen_bwd_x.hip.

@@ -103,7 +103,7 @@ int ddpm::bx_finish(const BxFinish& f, int dtype, hipStream_t stream) {
 int ddpm::bx_run(const void* y, const void* weight, const void* bias, const void* grad_out,
                  void* grad_x, void* workspace, int64_t workspace_bytes, int64_t n, int64_t c,
                  int64_t h, int64_t w, int kernel_size, int d0, int d1, int d2, int dtype,
-                 hipStream_t stream, BxFinish* defer) {
+                 hipStream_t stream, BxFinish* defer, const FlatLay* f) {
   if (dtype < kF32 || dtype > kF16) return kBadArgument;
   GenGeom gg;
   int st = gen_make_geom(gg, n, c, h, w, kernel_size, d0, d1, d2);
@@ -115,7 +115,7 @@ int ddpm::bx_run(const void* y, const void* weight, const void* bias, const void
   // past a channel block's first one)
   if (c * h * w * esz > 0x7fffffffLL || 16 * h * w * esz > 0x7fffffffLL) return kUnsupported;
   // reduce: one thread per group of `vec` columns of every row
-  const int vec = w % 4 == 0 ? 4 : 1;
+  const int vec = w % 4 == 0 || f ? 4 : 1;
   const int64_t ritems = n * c * h * ((w + vec - 1) / vec);
   if ((ritems + 255) / 256 > 0x7fffffffLL || n * c * h > 0x7fffffffLL) return kUnsupported;
   TileGeom g;
@@ -123,6 +123,11 @@ int ddpm::bx_run(const void* y, const void* weight, const void* bias, const void
   size_t lds;
   st = bx_geom(g, gg, cb, lds);
   if (st != kOk) return st;
+  if (f) {
+    g.OP = f->P;
+    g.OS = f->S;
+    g.olead = f->lead;
+  }
   if (!workspace || workspace_bytes < bx_part_bytes(g)) return kWorkspaceTooSmall;
   float* part = (float*)workspace;
   const int nk = gt_nk((int)c);

@@ -49,6 +49,8 @@ struct YGeom {
   int nc32;       // ceil(C / 32)
   int ihalves;    // 1, or 2 when C > 64: workgroups per segment, 16*MB output channels each
   int x4;         // x rows can be copied in 16-byte lanes (W % 8 == 0, aligned base)
+  int cp;         // flat tensors (a tile is 256 positions): planes per image of x
+  FlatLay f;
 };
 
 template <typename T, int KS, int MB>
@@ -83,8 +85,10 @@ struct YtLds {
 // AL: aligned layout (16-byte x rows, whole 32-channel chunks): the x copies
 // take the lane's column offset formed once per workgroup (kOob for the halo
 // chunks outside the image) and a scalar row offset per stage, without
-// per-copy tests.
-template <typename T, int KS, int MB, int CH, bool AL = false>
+// per-copy tests.  LAY 1.  LAY 2: flat x and grad_out (FlatLay) -- the tile is
+// 256 positions of a plane, kernel rows are d row pitches apart and nothing
+// is outside the image; dY goes to the image.
+template <typename T, int KS, int MB, int CH, int LAY = 0>
 __global__ __launch_bounds__(kYtThreads) void gen_bwd_y_kernel(const T* __restrict__ x,
                                                                const uint32_t* __restrict__ pk,
                                                                const T* __restrict__ gout,
@@ -93,6 +97,7 @@ __global__ __launch_bounds__(kYtThreads) void gen_bwd_y_kernel(const T* __restri
   typedef Mma<T> M;
   typedef typename M::V V;
   typedef YtLds<T, KS, MB, CH> L;
+  constexpr bool AL = LAY != 0, FL = LAY == 2;
   constexpr int KK = KS * KS;
   constexpr int r = KS / 2;
   constexpr int P = M::P;
@@ -102,11 +107,13 @@ __global__ __launch_bounds__(kYtThreads) void gen_bwd_y_kernel(const T* __restri
   const int logical = xcd_remap(blockIdx.x, gridDim.x);
   const int ih = logical % g.ihalves;  // output channels (ih*MB + ib)*16 + ...
   const int tile = logical / g.ihalves;
-  const int row = tile / g.col_tiles;  // image row n*H + h
+  // image row n*H + h and its column block; flat: image n, positions w0 .. w0 + 255
+  const int row = tile / g.col_tiles;
   const int w0 = (tile - row * g.col_tiles) * kYtTW;
-  const int n = row / g.H, h = row - n * g.H;
+  const int n = FL ? row : row / g.H, h = FL ? 0 : row - n * g.H;
   const int C = g.C, H = g.H, W = g.W;
-  const int64_t HW = (int64_t)H * W;
+  const int64_t HW = FL ? (int64_t)g.f.S : (int64_t)H * W;  // plane stride of x and grad_out
+  const uint32_t lead = FL ? g.f.lead : 0u;
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
@@ -116,7 +123,8 @@ __global__ __launch_bounds__(kYtThreads) void gen_bwd_y_kernel(const T* __restri
 
   // x planes of image n (per-row resources cost ~20 scalar instructions per
   // row and stage; measured bf16 44.9 -> 41.6 us)
-  const BufRes xres = make_buf(x + (int64_t)n * C * HW, (uint32_t)(C * HW * (int64_t)E));
+  const int64_t XC = FL ? g.cp : C;
+  const BufRes xres = make_buf(x + (int64_t)n * XC * HW, (uint32_t)((lead + XC * HW) * (int64_t)E));
   const BufRes xnul = make_buf(x, 0u);
   constexpr int kXP = (L::kXChunks + 63) / 64;  // copies per staged row
   uint32_t alcol[kXP];
@@ -125,7 +133,10 @@ __global__ __launch_bounds__(kYtThreads) void gen_bwd_y_kernel(const T* __restri
     for (int part = 0; part < kXP; ++part) {
       const int pc = 64 * part < L::kXChunks - 64 ? 64 * part : (L::kXChunks > 64 ? L::kXChunks - 64 : 0);
       const int gw = w0 - kYtPad + (pc + lane) * 4 * L::kPerD;
-      alcol[part] = (unsigned)gw < (unsigned)W ? (uint32_t)gw * (uint32_t)E : kOob;
+      if constexpr (FL)
+        alcol[part] = (uint32_t)((pc + lane) * 16);  // from the window's start
+      else
+        alcol[part] = (unsigned)gw < (unsigned)W ? (uint32_t)gw * (uint32_t)E : kOob;
     }
   }
   // ---- stage s = ((b * ncg) + cg) * KS + ki -> LDS buffer `buf`
@@ -139,9 +150,12 @@ __global__ __launch_bounds__(kYtThreads) void gen_bwd_y_kernel(const T* __restri
     // x rows: 32 * CH channels of row hh, columns w0 - pad .. w0 + TW + pad
     if constexpr (AL) {
       // a row outside the image copies through a resource with no records
-      const bool rok = (unsigned)hh < (unsigned)H;
+      const bool rok = FL || (unsigned)hh < (unsigned)H;
       const BufRes rs = rok ? xres : xnul;
-      const uint32_t roff = rok ? (uint32_t)(hh * W) * (uint32_t)E : 0u;
+      // flat: the window starts kYtPad elements before the tile (lead >= r d P + 8)
+      const uint32_t roff =
+          FL ? (uint32_t)((int)lead - kYtPad + w0 + (ki - r) * d * g.f.P) * (uint32_t)E
+             : (rok ? (uint32_t)(hh * W) * (uint32_t)E : 0u);
       if (L::kXChunks >= 64 || lane < L::kXChunks) {
 #pragma unroll
         for (int j = 0; j < 32 * CH / kYtWaves; ++j) {
@@ -227,12 +241,15 @@ __global__ __launch_bounds__(kYtThreads) void gen_bwd_y_kernel(const T* __restri
 #pragma unroll
   for (int blk = 0; blk < 2; ++blk) {
     const int w = w0 + px0 + 16 * blk;
-    glo[blk] = w < W ? ((uint32_t)quad * (uint32_t)HW + (uint32_t)(h * W + w)) * (uint32_t)E : kOob;
+    if constexpr (FL)
+      glo[blk] = ((uint32_t)quad * (uint32_t)HW + lead + (uint32_t)w) * (uint32_t)E;
+    else
+      glo[blk] = w < W ? ((uint32_t)quad * (uint32_t)HW + (uint32_t)(h * W + w)) * (uint32_t)E : kOob;
   }
   auto load_g = [&](int bg, float (&gd)[CH][2][8]) {
     const int cg = bg % ncg, b = bg / ncg;
     const BufRes gres = make_buf(gout + ((int64_t)n * 4 * C + (int64_t)(b + 1) * C) * HW,
-                                 (uint32_t)(C * HW * (int64_t)E));
+                                 (uint32_t)((lead + C * HW) * (int64_t)E));
 #pragma unroll
     for (int c = 0; c < CH; ++c)
 #pragma unroll
@@ -241,8 +258,12 @@ __global__ __launch_bounds__(kYtThreads) void gen_bwd_y_kernel(const T* __restri
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
           if constexpr (AL) {
-            const uint32_t so = (uint32_t)((cg * CH + c) * 32 + 4 * e) * (uint32_t)HW * (uint32_t)E;
-            gd[c][blk][e] = buf_load1<T>(gres, glo[blk], so);
+            const int c0 = (cg * CH + c) * 32 + 4 * e;
+            const uint32_t so = (uint32_t)c0 * (uint32_t)HW * (uint32_t)E;
+            // flat: channels past C (whose x planes are zero) read zero, not
+            // the next branch
+            const uint32_t vo = FL && c0 + quad >= C ? kOob : glo[blk];
+            gd[c][blk][e] = buf_load1<T>(gres, vo, so);
           } else {
             const int ch = (cg * CH + c) * 32 + 4 * e + quad;
             const uint32_t off =
@@ -337,15 +358,20 @@ __global__ __launch_bounds__(kYtThreads) void gen_bwd_y_kernel(const T* __restri
   // ---- store: lane holds dY[i = ib*16 + 4*quad + e][pixel col16 of block]
 #pragma unroll
   for (int blk = 0; blk < 2; ++blk) {
-    const int w = w0 + px0 + 16 * blk;
-    if (w < W) {
-      T* __restrict__ yo = gy + (int64_t)n * C * HW + (int64_t)h * W + w;
+    int w = w0 + px0 + 16 * blk, ho = h;
+    if constexpr (FL) {
+      ho = w / g.f.P;
+      w -= ho * g.f.P;
+    }
+    if (w < W && (!FL || ho < H)) {
+      const int64_t OHW = (int64_t)H * W;
+      T* __restrict__ yo = gy + (int64_t)n * C * OHW + (int64_t)ho * W + w;
 #pragma unroll
       for (int ib = 0; ib < MB; ++ib)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const int i = (ih * MB + ib) * 16 + 4 * quad + e;
-          if (i < C) yo[(int64_t)i * HW] = from_f<T>(acc[blk][ib][e]);
+          if (i < C) yo[(int64_t)i * OHW] = from_f<T>(acc[blk][ib][e]);
         }
     }
   }
@@ -421,7 +447,8 @@ int yt_check(const void* x, const void* weight, const void* grad_out, void* grad
 // already validated by yt_check; `packed` holds yt_pack_bytes bytes).
 int yt_launch(const void* x, const void* weight, const void* grad_out, void* grad_y, void* packed,
               int64_t n, int64_t c, int64_t h, int64_t w, int kernel_size, const GenGeom& gg,
-              int dtype, hipStream_t stream, bool pack = true, const WReduce* red = nullptr);
+              int dtype, hipStream_t stream, bool pack = true, const WReduce* red = nullptr,
+              const FlatLay* f = nullptr);
 
 }  // namespace
 
@@ -473,7 +500,7 @@ extern "C" int64_t ddpm_gen_bwd_y_workspace_bytes(int64_t c, int kernel_size) {
 int ddpm::yt_run(const void* x, const void* weight, const void* grad_out, void* grad_y,
                  void* workspace, int64_t workspace_bytes, int64_t n, int64_t c, int64_t h,
                  int64_t w, int kernel_size, int d0, int d1, int d2, int dtype, hipStream_t stream,
-                 int mode, YPack* pack, const WReduce* red) {
+                 int mode, YPack* pack, const WReduce* red, const FlatLay* f) {
   GenGeom gg;
   bool empty;
   const int st =
@@ -492,7 +519,7 @@ int ddpm::yt_run(const void* x, const void* weight, const void* grad_out, void* 
     return kOk;
   }
   return yt_launch(x, weight, grad_out, grad_y, workspace, n, c, h, w, kernel_size, gg, dtype,
-                   stream, mode != kYtMain, red);
+                   stream, mode != kYtMain, red, f);
 }
 
 int ddpm::yt_pack(const YPack& p, int kernel_size, int dtype, hipStream_t stream) {
@@ -545,7 +572,7 @@ namespace {
 
 int yt_launch(const void* x, const void* weight, const void* grad_out, void* grad_y, void* packed,
               int64_t n, int64_t c, int64_t h, int64_t w, int kernel_size, const GenGeom& gg,
-              int dtype, hipStream_t stream, bool pack, const WReduce* red) {
+              int dtype, hipStream_t stream, bool pack, const WReduce* red, const FlatLay* f) {
   void* workspace = packed;
   YGeom g;
   g.N = (int)n;
@@ -558,9 +585,12 @@ int yt_launch(const void* x, const void* weight, const void* grad_out, void* gra
   g.col_tiles = (int)((w + kYtTW - 1) / kYtTW);
   g.nc32 = (int)((c + 31) / 32);
   g.x4 = (w % 8 == 0) && ((uintptr_t)x % 16 == 0);
+  g.cp = (int)flat_planes(c);
+  g.f = f ? *f : FlatLay{};
+  if (f) g.col_tiles = f->ft;
   int mb;
   yt_split(c, g.ihalves, mb);
-  const int64_t tiles = n * h * g.col_tiles * g.ihalves;  // below 2^31 (yt_check)
+  const int64_t tiles = n * (f ? 1 : h) * g.col_tiles * g.ihalves;  // below 2^31 (yt_check)
   return yt_with_type(dtype, [&](auto tag) {
     using T = decltype(tag);
     return yt_with_mb(mb, [&](auto mbc) {
@@ -579,8 +609,9 @@ int yt_launch(const void* x, const void* weight, const void* grad_out, void* gra
         }
         const size_t lds = (size_t)2 * L::kBuf * 4;
         // aligned layout: 16-byte x rows and whole 32-channel chunks
-        auto kern = g.x4 && c % 32 == 0 ? gen_bwd_y_kernel<T, KS, MB, CH, true>
-                                        : gen_bwd_y_kernel<T, KS, MB, CH>;
+        auto kern = f                      ? gen_bwd_y_kernel<T, KS, MB, CH, 2>
+                    : g.x4 && c % 32 == 0 ? gen_bwd_y_kernel<T, KS, MB, CH, 1>
+                                          : gen_bwd_y_kernel<T, KS, MB, CH>;
         const int ae = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds);
         if (ae != 0) return ae;
         const WReduce nored{nullptr, nullptr, nullptr, nullptr, 0, 0, 0, 0, 0};

@@ -25,8 +25,8 @@ namespace ddpm {
 template <typename T, int KS, int NK, int CB, bool PP = false>
 __global__ __launch_bounds__(kGtThreads) __attribute__((amdgpu_waves_per_eu(gt_waves_per_eu<T, NK, CB>()))) void gen_fwd_kernel(
     const T* __restrict__ x, const T* __restrict__ y, const T* __restrict__ wt,
-    const T* __restrict__ bias, T* __restrict__ out, TileGeom g, CvPack fpk) {
-  gen_tile_body<T, KS, NK, CB, false, PP>(x, y, wt, bias, out, nullptr, g, fpk);
+    const T* __restrict__ bias, T* __restrict__ out, TileGeom g, CvPack fpk, FlatZero zero) {
+  gen_tile_body<T, KS, NK, CB, false, PP>(x, y, wt, bias, out, nullptr, g, fpk, zero);
 }
 
 // Two fp32 values rounded to nearest-even in T (bf16 / f16), packed low/high.
@@ -68,7 +68,7 @@ __device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float c) {
 template <typename T, int NK, int CB>
 __global__ __launch_bounds__(kGtThreads) __attribute__((amdgpu_waves_per_eu(gt_waves_per_eu<T, NK, CB>()))) void gen_fwd_pair_kernel(
     const T* __restrict__ x, const T* __restrict__ y, const T* __restrict__ wt,
-    const T* __restrict__ bias, T* __restrict__ out, TileGeom g, CvPack fpk) {
+    const T* __restrict__ bias, T* __restrict__ out, TileGeom g, CvPack fpk, FlatZero zero) {
   static_assert(sizeof(T) == 2, "2-byte types");
   typedef Mma<T> M;
   typedef typename M::V V;
@@ -94,7 +94,10 @@ __global__ __launch_bounds__(kGtThreads) __attribute__((amdgpu_waves_per_eu(gt_w
   const int ty = tile / g.tiles_w, tx = tile - ty * g.tiles_w;
   const int h0 = ty * kGtTH, w0 = tx * TW;
   const int C = g.C, H = g.H, W = g.W, R = g.R, LW = g.LW;
-  const uint32_t HWE = (uint32_t)((int64_t)H * W) * (uint32_t)E;
+  const int64_t OS = g.OS;
+  const uint32_t OSE = g.OS * (uint32_t)E;  // bytes of one concat plane
+  const int OP = g.OP;
+  out += g.olead;
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
@@ -142,6 +145,7 @@ __global__ __launch_bounds__(kGtThreads) __attribute__((amdgpu_waves_per_eu(gt_w
   // ddpm_gen_fwd_pack: this workgroup's share of the fuse convolution's
   // weight packing
   if (fpk.total > 0) cv_pack_share<T>(fpk, (int)blockIdx.x, (int)gridDim.x, tid, kGtThreads);
+  if (zero.base) flat_zero_share<T>(zero, (int)blockIdx.x, (int)gridDim.x, tid, kGtThreads);
   __builtin_amdgcn_s_waitcnt(0);  // the LDS-direct weight copies
   __syncthreads();
 
@@ -159,7 +163,7 @@ __global__ __launch_bounds__(kGtThreads) __attribute__((amdgpu_waves_per_eu(gt_w
   auto goff = [&](int blk, int mb, int e) {
     const int gh = h0 + 2 * wave + blk / CB, gw = w0 + 16 * (blk % CB) + col16;
     const int cl = 8 * mb + 2 * quad + e;
-    return (gh < H && gw < W && cl < nch) ? (uint32_t)cl * HWE + (uint32_t)(gh * W + gw) * E : kOob;
+    return (gh < H && gw < W && cl < nch) ? (uint32_t)cl * OSE + (uint32_t)(gh * OP + gw) * E : kOob;
   };
 
   float acc[NBW][2][2];  // branch output of channels (ca, cb) of each row block, per pixel block
@@ -219,8 +223,8 @@ __global__ __launch_bounds__(kGtThreads) __attribute__((amdgpu_waves_per_eu(gt_w
     }
     if (j == NPB - 1) {
       // ---- branch b: channels c0 + 8mb + 2q + e of output block b+1
-      const BufRes bres = make_buf(out + ((int64_t)n * 4 * C + (int64_t)(b + 1) * C + c0) * (H * (int64_t)W),
-                                   (uint32_t)nch * HWE);
+      const BufRes bres = make_buf(out + ((int64_t)n * 4 * C + (int64_t)(b + 1) * C + c0) * OS,
+                                   (uint32_t)nch * OSE);
 #pragma unroll
       for (int blk = 0; blk < NBW; ++blk)
 #pragma unroll
@@ -276,14 +280,19 @@ int gen_make_geom(GenGeom& g, int64_t n, int64_t c, int64_t h, int64_t w, int k,
 
 using namespace ddpm;
 
+extern "C" int64_t ddpm_flat_cat_elems(int64_t n, int64_t c, int64_t h, int64_t w, int guard,
+                                       int dtype);
+
 namespace {
 
 // ddpm_gen_fwd's work; fpk (optional): a fuse-convolution weight packing for
 // the kernel's workgroups to run.  check_only: validate and return before
-// launching.
+// launching.  f (optional): the concat is a flat tensor of that layout; the
+// kernel's workgroups zero its elements outside the images.
 int gf_run(const void* x, const void* y, const void* weight, const void* bias, void* out,
            int64_t n, int64_t c, int64_t h, int64_t w, int kernel_size, int d0, int d1, int d2,
-           int dtype, hipStream_t stream, const CvPack* fpk, bool check_only) {
+           int dtype, hipStream_t stream, const CvPack* fpk, bool check_only,
+           const FlatLay* f = nullptr) {
   // kF32Pairs: fp32 inputs, the concat written as pair planes (C % 16 == 0)
   const bool pp = dtype == kF32Pairs;
   if (pp) {
@@ -309,6 +318,13 @@ int gf_run(const void* x, const void* y, const void* weight, const void* bias, v
   int cb = 4;
   st = tile_geom_for(g, gg, 4 * esz, parts, cb, lds);
   if (st != kOk) return st;
+  FlatZero zero{nullptr, FlatLay{}, 0};
+  if (f) {
+    g.OP = f->P;
+    g.OS = f->S;
+    g.olead = f->lead;
+    zero = FlatZero{out, *f, (int)(n * 4 * c)};
+  }
   // 2-byte types at K = 3 with up to 64 channels (C % 8 == 0, aligned
   // weight): taps paired in the MFMA rows, every weight slice resident in LDS
   const size_t lds_pair = (size_t)4 * g.plane + (size_t)15 * 2 * nk * 64 * 16 + (size_t)15 * 32 * 4;
@@ -323,7 +339,7 @@ int gf_run(const void* x, const void* y, const void* weight, const void* bias, v
           if (ae != 0) return ae;
           hipLaunchKernelGGL(kern, dim3((unsigned)((int64_t)g.N * g.tiles * g.cblocks)),
                              dim3(kGtThreads), lds_pair, stream, (const T*)x, (const T*)y,
-                             (const T*)weight, (const T*)bias, (T*)out, g, pk);
+                             (const T*)weight, (const T*)bias, (T*)out, g, pk, zero);
           return (int)hipGetLastError();
         };
         if (cb == 4) return nk == 1 ? launch(gen_fwd_pair_kernel<T, 1, 4>) : launch(gen_fwd_pair_kernel<T, 2, 4>);
@@ -341,7 +357,7 @@ int gf_run(const void* x, const void* y, const void* weight, const void* bias, v
       if (ae != 0) return ae;
       hipLaunchKernelGGL(kern, dim3((unsigned)((int64_t)g.N * g.tiles * g.cblocks)),
                          dim3(kGtThreads), lds, stream, (const T*)x, (const T*)y,
-                         (const T*)weight, (const T*)bias, (T*)out, g, pk);
+                         (const T*)weight, (const T*)bias, (T*)out, g, pk, zero);
       return (int)hipGetLastError();
     };
     // 1 or 2 chunks of 32 input channels, or 4 (65..128 channels; chunks
@@ -390,4 +406,25 @@ extern "C" int ddpm_gen_fwd_pack(const void* x, const void* y, const void* weigh
   if (st != kOk) return st;
   return gf_run(x, y, weight, bias, out, n, c, h, w, kernel_size, d0, d1, d2, dtype, stream, &pk,
                 false);
+}
+
+extern "C" int ddpm_flat_gen_fwd_pack(const void* x, const void* y, const void* weight,
+                                      const void* bias, void* cat, const void* fuse_weight,
+                                      void* fuse_workspace, int64_t fuse_workspace_bytes, int64_t n,
+                                      int64_t c, int64_t h, int64_t w, int kernel_size, int d0,
+                                      int d1, int d2, int guard, int dtype, hipStream_t stream) {
+  int st = gf_run(x, y, weight, bias, cat, n, c, h, w, kernel_size, d0, d1, d2, dtype, stream,
+                  nullptr, true);
+  if (st != kOk) return st;
+  if (n == 0 || c == 0 || h == 0 || w == 0) return kOk;
+  FlatLay f;
+  if (ddpm_flat_cat_elems(n, c, h, w, guard, dtype) == 0 ||
+      !flat_lay(f, h, w, guard, 4 * c, dtype == kBF16 || dtype == kF16 ? 2 : 4))
+    return kUnsupported;
+  if ((uintptr_t)cat % 16 != 0) return kBadArgument;
+  CvPack pk;
+  st = cv_fwd_pack(pk, cat, fuse_weight, fuse_workspace, fuse_workspace_bytes, n, c, h, w, dtype, &f);
+  if (st != kOk) return st;
+  return gf_run(x, y, weight, bias, cat, n, c, h, w, kernel_size, d0, d1, d2, dtype, stream, &pk,
+                false, &f);
 }

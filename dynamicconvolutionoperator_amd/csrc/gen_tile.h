@@ -53,6 +53,10 @@ struct TileGeom {
   int pad;      // halo column j <-> position j + pad (R + pad = 0 mod 4) ...
   int LWp;      // ... of a row of LWp (multiple of 4) positions; see gen_tile_body
   int vec;      // W % 4 == 0: 4-column groups at positions 4k are whole inside or outside the image
+  // the concat (forward output, or grad_cat): row pitch, plane stride and the
+  // elements before its first plane (W, H * W and 0, or a flat layout's)
+  int OP;
+  uint32_t OS, olead;
 };
 
 // Waves per SIMD the tile kernels are compiled for: two (256 registers per
@@ -95,6 +99,9 @@ inline int tile_geom(TileGeom& f, const GenGeom& g, int entry, int parts, int cb
   f.pad = (4 - g.R % 4) % 4;
   f.LWp = (f.LW + f.pad + 3) / 4 * 4;
   f.vec = g.W % 4 == 0;
+  f.OP = g.W;
+  f.OS = (uint32_t)((int64_t)g.H * g.W);
+  f.olead = 0;
   // planes start on 256-byte boundaries: the four quads of a wave then read
   // their 4-channel entries with the fewest LDS bank conflicts (measured)
   f.plane = (f.npix * entry + 255) / 256 * 256;
@@ -184,8 +191,10 @@ __device__ __forceinline__ void gt_stage_x(const T* __restrict__ a, T* __restric
   // ---- halo tile of x (zero outside the image) -> LDS planes; the tile's
   //      own pixels also go to the identity channels of the output
   const BufRes xres = make_buf(a + ((int64_t)n * C + c0) * HW, (uint32_t)nch * HWE);
-  const BufRes ores = PP ? make_buf(out + ((int64_t)n * 4 * C + (c0 & ~31)) * HW, 32u * HWE)
-                        : make_buf(out + ((int64_t)n * 4 * C + c0) * HW, (uint32_t)nch * HWE);
+  const int64_t OS = g.OS;
+  const uint32_t OSE = g.OS * (uint32_t)E;  // bytes of one concat plane
+  const BufRes ores = PP ? make_buf(out + ((int64_t)n * 4 * C + (c0 & ~31)) * OS, 32u * OSE)
+                        : make_buf(out + ((int64_t)n * 4 * C + c0) * OS, (uint32_t)nch * OSE);
   const uint32_t pp0 = (uint32_t)((c0 & 31) >> 1);  // PP: pair index of channels (c0, c0+1)
   if (g.vec) {
     // a task = (4-channel plane, halo row, 4 image columns a multiple of 4
@@ -202,7 +211,7 @@ __device__ __forceinline__ void gt_stage_x(const T* __restrict__ a, T* __restric
     typedef uint32_t VD __attribute__((ext_vector_type(ND)));
     for (int t0 = tid; t0 < tasks; t0 += U * kGtThreads) {
       VD v[U][4];  // [task][channel]
-      uint32_t off[U];
+      uint32_t off[U], oof[U];
       int ti[U], tk[U], tg[U];
 #pragma unroll
       for (int u = 0; u < U; ++u) {
@@ -212,6 +221,7 @@ __device__ __forceinline__ void gt_stage_x(const T* __restrict__ a, T* __restric
         const int gh = h0 - R + i, gc = w0 - cpos + 4 * k;
         const bool in = task < tasks && (unsigned)gh < (unsigned)H && (unsigned)gc < (unsigned)W;
         off[u] = in ? (uint32_t)(gh * W + gc) * (uint32_t)E : kOob;
+        oof[u] = in ? (uint32_t)(gh * g.OP + gc) * (uint32_t)E : kOob;
         ti[u] = i;
         tk[u] = k;
         tg[u] = grp;
@@ -258,14 +268,14 @@ __device__ __forceinline__ void gt_stage_x(const T* __restrict__ a, T* __restric
                 hv[m] = hh;
                 lv[m] = ll;
               }
-              const uint32_t o = off[u] == kOob ? kOob : off[u] + (pp0 + 2 * grp + kp) * HWE;
+              const uint32_t o = oof[u] == kOob ? kOob : oof[u] + (pp0 + 2 * grp + kp) * OSE;
               __builtin_amdgcn_raw_buffer_store_b128(hv, ores, o, 0, 0);
-              __builtin_amdgcn_raw_buffer_store_b128(lv, ores, o == kOob ? kOob : o + 16u * HWE, 0, 0);
+              __builtin_amdgcn_raw_buffer_store_b128(lv, ores, o == kOob ? kOob : o + 16u * OSE, 0, 0);
             }
           } else {
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-              const uint32_t o = off[u] + (uint32_t)(4 * grp + e) * HWE;
+              const uint32_t o = oof[u] + (uint32_t)(4 * grp + e) * OSE;
               if constexpr (E == 4)
                 __builtin_amdgcn_raw_buffer_store_b128(v[u][e], ores, o, 0, 0);
               else
@@ -290,7 +300,7 @@ __device__ __forceinline__ void gt_stage_x(const T* __restrict__ a, T* __restric
             pix[s] < g.npix && (unsigned)gh < (unsigned)H && (unsigned)gw < (unsigned)W;
         const bool inner = i >= R && i < R + kGtTH && j >= R && j < R + TW;
         lo[s] = in ? (uint32_t)(gh * W + gw) * (uint32_t)E : kOob;
-        so[s] = (in && inner) ? lo[s] : kOob;
+        so[s] = (in && inner) ? (uint32_t)(gh * g.OP + gw) * (uint32_t)E : kOob;
       }
       uint32_t v[2][16];
 #pragma unroll
@@ -304,15 +314,15 @@ __device__ __forceinline__ void gt_stage_x(const T* __restrict__ a, T* __restric
           for (int kp = 0; kp < 8; ++kp) {
             uint32_t hh, ll;
             split_bf16x2(__uint_as_float(v[s][2 * kp]), __uint_as_float(v[s][2 * kp + 1]), hh, ll);
-            const uint32_t o = so[s] == kOob ? kOob : so[s] + (pp0 + kp) * HWE;
+            const uint32_t o = so[s] == kOob ? kOob : so[s] + (pp0 + kp) * OSE;
             __builtin_amdgcn_raw_buffer_store_b32(hh, ores, o, 0, 0);
-            __builtin_amdgcn_raw_buffer_store_b32(ll, ores, o == kOob ? kOob : o + 16u * HWE, 0, 0);
+            __builtin_amdgcn_raw_buffer_store_b32(ll, ores, o == kOob ? kOob : o + 16u * OSE, 0, 0);
           }
       } else {
 #pragma unroll
         for (int s = 0; s < 2; ++s)
 #pragma unroll
-          for (int ch = 0; ch < 16; ++ch) gf_store_raw<E>(ores, so[s] + ch * HWE, v[s][ch]);
+          for (int ch = 0; ch < 16; ++ch) gf_store_raw<E>(ores, so[s] + ch * OSE, v[s][ch]);
       }
 #pragma unroll
       for (int s = 0; s < 2; ++s) {
@@ -377,7 +387,8 @@ __device__ __forceinline__ void gen_tile_body(const T* __restrict__ a, const T* 
                                               T* __restrict__ out, float* __restrict__ part,
                                               const TileGeom& g,
                                               CvPack fpk = CvPack{nullptr, nullptr, ConvGeom{}, 0,
-                                                                  0, 0, 0}) {
+                                                                  0, 0, 0},
+                                              FlatZero zero = FlatZero{nullptr, FlatLay{}, 0}) {
   typedef Mma<T> M;
   typedef typename M::V V;
   constexpr int P = M::P;
@@ -406,7 +417,13 @@ __device__ __forceinline__ void gen_tile_body(const T* __restrict__ a, const T* 
   const int h0 = ty * kGtTH, w0 = tx * TW;
   const int C = g.C, H = g.H, W = g.W, R = g.R, LW = g.LW;
   const int64_t HW = (int64_t)H * W;
-  const uint32_t HWE = (uint32_t)HW * (uint32_t)E;  // bytes of one channel plane
+  const int64_t OS = g.OS;
+  const uint32_t OSE = g.OS * (uint32_t)E;  // bytes of one concat plane
+  const int OP = g.OP;
+  if constexpr (BX)
+    a += g.olead;
+  else
+    out += g.olead;
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
@@ -498,6 +515,7 @@ __device__ __forceinline__ void gen_tile_body(const T* __restrict__ a, const T* 
     // ddpm_gen_fwd_pack: this workgroup's share of the fuse convolution's
     // weight packing
     if (fpk.total > 0) cv_pack_share<T>(fpk, (int)blockIdx.x, (int)gridDim.x, tid, kGtThreads);
+    if (zero.base) flat_zero_share<T>(zero, (int)blockIdx.x, (int)gridDim.x, tid, kGtThreads);
   }
   __syncthreads();
 
@@ -518,12 +536,12 @@ __device__ __forceinline__ void gen_tile_body(const T* __restrict__ a, const T* 
 #pragma unroll
   for (int cp = 0; cp < CB; ++cp) {
     const int gw = w0 + 16 * cp + col16;
-    lofs[cp] = (gw < W && 4 * quad < nch) ? (uint32_t)gw * E + (uint32_t)(4 * quad) * HWE : kOob;
+    lofs[cp] = (gw < W && 4 * quad < nch) ? (uint32_t)gw * E + (uint32_t)(4 * quad) * OSE : kOob;
   }
   const int emax = nch - 4 * quad;  // channels 4*quad + e with e < emax exist
   auto goff = [&](const uint32_t (&lo)[CB], int blk, int e) {
     const int gh = h0 + 2 * wave + blk / CB;
-    return (gh < H && e < emax) ? lo[blk % CB] + (uint32_t)(gh * W) * E + (uint32_t)e * HWE : kOob;
+    return (gh < H && e < emax) ? lo[blk % CB] + (uint32_t)(gh * OP) * E + (uint32_t)e * OSE : kOob;
   };
 
   f32x4 acc[NBW];   // forward: branch output of this lane's 4 channels per block
@@ -537,8 +555,8 @@ __device__ __forceinline__ void gen_tile_body(const T* __restrict__ a, const T* 
     }
     if constexpr (BX) {
       if (t == 0) {
-        const BufRes gres = make_buf(a + ((int64_t)n * 4 * C + (int64_t)(b + 1) * C + c0) * HW,
-                                     (uint32_t)nch * HWE);
+        const BufRes gres = make_buf(a + ((int64_t)n * 4 * C + (int64_t)(b + 1) * C + c0) * OS,
+                                     (uint32_t)nch * OSE);
         uint32_t lo[CB];
 #pragma unroll
         for (int cp = 0; cp < CB; ++cp) {
@@ -617,7 +635,7 @@ __device__ __forceinline__ void gen_tile_body(const T* __restrict__ a, const T* 
         // ---- branch b as pair planes: channels (4quad + 2kp, +1) of output
         //      block b+1, split, to the hi / lo planes of their 32-plane chunk
         const int chb = (b + 1) * C + c0;
-        const BufRes pres = make_buf(out + ((int64_t)n * 4 * C + (chb & ~31)) * HW, 32u * HWE);
+        const BufRes pres = make_buf(out + ((int64_t)n * 4 * C + (chb & ~31)) * OS, 32u * OSE);
         const uint32_t pbase = (uint32_t)(((chb & 31) >> 1) + 2 * quad);
         // the lane's column offsets, formed here (kept out of registers across
         // the loop, as lofs is for the plain stores)
@@ -636,15 +654,15 @@ __device__ __forceinline__ void gen_tile_body(const T* __restrict__ a, const T* 
           for (int kp = 0; kp < 2; ++kp) {
             uint32_t hh, ll;
             split_bf16x2(acc[blk][2 * kp], acc[blk][2 * kp + 1], hh, ll);
-            const uint32_t o = ok ? pc[blk % CB] + (uint32_t)(gh * W) * 4u + (pbase + kp) * HWE : kOob;
+            const uint32_t o = ok ? pc[blk % CB] + (uint32_t)(gh * OP) * 4u + (pbase + kp) * OSE : kOob;
             __builtin_amdgcn_raw_buffer_store_b32(hh, pres, o, 0, 0);
-            __builtin_amdgcn_raw_buffer_store_b32(ll, pres, ok ? o + 16u * HWE : kOob, 0, 0);
+            __builtin_amdgcn_raw_buffer_store_b32(ll, pres, ok ? o + 16u * OSE : kOob, 0, 0);
           }
         }
       } else if (t == KK - 1) {
         // ---- branch b: channels c0 + 4*quad + e of output block b+1
-        const BufRes bres = make_buf(out + ((int64_t)n * 4 * C + (int64_t)(b + 1) * C + c0) * HW,
-                                     (uint32_t)nch * HWE);
+        const BufRes bres = make_buf(out + ((int64_t)n * 4 * C + (int64_t)(b + 1) * C + c0) * OS,
+                                     (uint32_t)nch * OSE);
         uint32_t lo[CB];
 #pragma unroll
         for (int cp = 0; cp < CB; ++cp) {

@@ -25,7 +25,9 @@ generator is the constructor's unmodified 1x1 convolution
 convolution, generator, filter, concat and fuse convolution run as one pair
 of autograd ops (``ops.fused_ddpm``) whose generator launch also packs the
 fuse weight; an fp32 concat (C % 16 == 0) is stored as bf16 pair planes,
-already split the way the fuse convolution's fp32 MFMA products need it.
+already split the way the fuse convolution's fp32 MFMA products need it.  At
+widths that are not whole steps of the kernels the concat's rows are padded to
+a pitch of their own (``ops._flat_guard``).
 """
 
 from __future__ import annotations
@@ -248,7 +250,7 @@ class DDPM(nn.Module):
                 self.kernel_size, self.dilations)
         if not supported(*args) or self._route(x, y, ops[2]) != "fused":
             return None
-        return fused_ddpm(*args)  # the arguments as checked just now
+        return fused_ddpm(*args, flat=True)  # the arguments as checked just now
 
     def forward(self, x: torch.Tensor, y: torch.Tensor) -> torch.Tensor:
         _check_inputs(x, y, self.dim)

@@ -668,35 +668,111 @@ def _cat_code(dtype: torch.dtype) -> int:
     return _PAIR_PLANES if dtype == torch.float32 else _DTYPES[dtype]
 
 
-def _concat_pack(x, y, gen_weight, gen_bias, fuse_weight, k, dil):
-    """ddpm_gen_fwd_pack: the concat (fp32 as pair planes) and, in the fuse
-    convolution's workspace, its packed weight (returned with it)."""
+def _flat_guard(x, k, dil, code, training) -> int:
+    """Guard rows and columns of the flat concat (``ddpm_flat_*``: rows padded
+    to a 16-byte pitch, tiles of 256 positions whatever the width) that this
+    shape takes between generator and fuse convolution, or 0 for the plain
+    one.  Plain rows win where they are whole steps of the kernels (fp32 /
+    bf16 C = 64: training 1x128x128 204 / 144 us plain, 230 / 158 flat;
+    inference 4x64x64 51 / 39 plain, 53 / 41 flat); every other width leaves
+    lanes idle at row ends (training 1x160x160 333 / 231 us plain, 281 / 193
+    flat, 8x64x64 390 / 262 plain, 327 / 206 flat) or, not a multiple of 8,
+    is staged element by element (bf16 training 2x135x181 1034 us plain, 251
+    flat)."""
+    n, c, h, w = x.shape
+    if w % 256 == 0 or w == 128 or (not training and w in (32, 64)):
+        return 0
+    guard = max(1, (k // 2) * max(dil)) if training else 1
+    return guard if _ws_bytes("ddpm_flat_cat_elems", n, c, h, w, guard, code) > 0 else 0
+
+
+def _concat_pack(x, y, gen_weight, gen_bias, fuse_weight, k, dil, guard):
+    """ddpm_gen_fwd_pack (or its flat form): the concat (fp32 as pair planes)
+    and, in the fuse convolution's workspace, its packed weight (returned with
+    it)."""
     n, c, h, w = x.shape
     code = _cat_code(x.dtype)
-    cat = torch.empty((n, 4 * c, h, w), dtype=x.dtype, device=x.device)
     lib = _lib.load()
     with _on(x.device):
-        ws, nbytes = _fuse_conv_workspace(n, c, h, w, code, x.device)
-        rc = lib.ddpm_gen_fwd_pack(_ptr(x), _ptr(y), _ptr(gen_weight), _ptr(gen_bias), _ptr(cat),
-                                   _ptr(fuse_weight), _ptr(ws), nbytes, n, c, h, w, k, *dil, code,
-                                   _stream(x))
+        if guard:
+            cat = torch.empty(_ws_bytes("ddpm_flat_cat_elems", n, c, h, w, guard, code), dtype=x.dtype,
+                              device=x.device)
+            nbytes = _ws_bytes("ddpm_flat_fuse_conv_workspace_bytes", n, c, h, w, guard, code)
+            ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+            rc = lib.ddpm_flat_gen_fwd_pack(
+                _ptr(x), _ptr(y), _ptr(gen_weight), _ptr(gen_bias), _ptr(cat), _ptr(fuse_weight),
+                _ptr(ws), nbytes, n, c, h, w, k, *dil, guard, code, _stream(x))
+        else:
+            cat = torch.empty((n, 4 * c, h, w), dtype=x.dtype, device=x.device)
+            ws, nbytes = _fuse_conv_workspace(n, c, h, w, code, x.device)
+            rc = lib.ddpm_gen_fwd_pack(_ptr(x), _ptr(y), _ptr(gen_weight), _ptr(gen_bias), _ptr(cat),
+                                       _ptr(fuse_weight), _ptr(ws), nbytes, n, c, h, w, k, *dil, code,
+                                       _stream(x))
     _lib.check(rc, "ddpm_gen_fwd_pack")
     return cat, ws
 
 
-def _fuse_conv_forward_packed(cat, ws, fuse_bias):
-    """ddpm_fuse_conv_fwd_packed over a concat of :func:`_concat_pack` whose
-    workspace ``ws`` holds the packed weight."""
-    n, ci, h, w = cat.shape
-    c = ci // 4
+def _fuse_conv_forward_packed(cat, ws, fuse_bias, shape, guard):
+    """ddpm_fuse_conv_fwd_packed (or its flat form) over a concat of
+    :func:`_concat_pack` whose workspace ``ws`` holds the packed weight."""
+    n, c, h, w = shape
     out = torch.empty((n, c, h, w), dtype=cat.dtype, device=cat.device)
     lib = _lib.load()
+    bias = _ptr(fuse_bias) if fuse_bias is not None else None
     with _on(cat.device):
-        rc = lib.ddpm_fuse_conv_fwd_packed(_ptr(cat), _ptr(fuse_bias) if fuse_bias is not None else None,
-                                           _ptr(out), _ptr(ws), ws.numel(), n, c, h, w,
-                                           _cat_code(cat.dtype), _stream(cat))
+        if guard:
+            rc = lib.ddpm_flat_fuse_conv_fwd_packed(_ptr(cat), bias, _ptr(out), _ptr(ws), ws.numel(), n,
+                                                    c, h, w, guard, _cat_code(cat.dtype), _stream(cat))
+        else:
+            rc = lib.ddpm_fuse_conv_fwd_packed(_ptr(cat), bias, _ptr(out), _ptr(ws), ws.numel(), n, c,
+                                               h, w, _cat_code(cat.dtype), _stream(cat))
     _lib.check(rc, "ddpm_fuse_conv_fwd_packed")
     return out
+
+
+def _flat_fuse_conv_backward(cat, weight, has_bias, grad_out, needs, shape, guard):
+    """:func:`_fuse_conv_backward` of a flat concat, the concat's gradient flat
+    too."""
+    n, c, h, w = shape
+    code = _cat_code(cat.dtype)
+    need_w = needs[1] or (has_bias and needs[2])
+    if not (needs[0] or need_w):
+        return None, None, None
+    grad_cat = torch.empty_like(cat) if needs[0] else None
+    gw = torch.empty_like(weight) if need_w else None
+    gb = torch.empty((c,), dtype=weight.dtype, device=cat.device) if need_w else None
+    nbytes = _ws_bytes("ddpm_flat_fuse_conv_bwd_workspace_bytes", n, c, h, w, guard, code)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=cat.device)
+    with _on(cat.device):
+        rc = _lib.load().ddpm_flat_fuse_conv_bwd(
+            _ptr(cat), _ptr(weight), _ptr(grad_out), _ptr(grad_cat) if needs[0] else None,
+            _ptr(gw) if need_w else None, _ptr(gb) if need_w else None, _ptr(ws), nbytes, n, c, h, w,
+            guard, code, _stream(cat))
+    _lib.check(rc, "ddpm_flat_fuse_conv_bwd")
+    return grad_cat, gw if needs[1] else None, gb if has_bias and needs[2] else None
+
+
+def _flat_generator_backward(x, y, weight, bias, grad_cat, k, dil, needs, guard):
+    """:func:`_generator_backward` from a flat gradient of the concat."""
+    n, c, h, w = x.shape
+    dt = _dt(x)
+    need_wb = needs[2] or needs[3]
+    if not (needs[0] or needs[1] or need_wb):
+        return None, None, None, None
+    gx = torch.empty_like(x) if needs[0] else None
+    gy = torch.empty_like(y) if needs[1] else None
+    gw = torch.empty_like(weight) if need_wb else None
+    gb = torch.empty_like(bias) if need_wb else None
+    nbytes = _ws_bytes("ddpm_flat_gen_bwd_workspace_bytes", n, c, h, w, k, *dil, guard, dt)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+    with _on(x.device):
+        rc = _lib.load().ddpm_flat_gen_bwd(
+            _ptr(x), _ptr(y), _ptr(weight), _ptr(bias), _ptr(grad_cat),
+            _ptr(gx) if needs[0] else None, _ptr(gy) if needs[1] else None,
+            _ptr(gw) if need_wb else None, _ptr(gb) if need_wb else None, _ptr(ws), nbytes, n, c, h, w,
+            k, *dil, guard, dt, _stream(x))
+    _lib.check(rc, "ddpm_flat_gen_bwd")
+    return gx, gy, gw if needs[2] else None, gb if needs[3] else None
 
 
 class _GeneratorConcat(torch.autograd.Function):
@@ -708,11 +784,12 @@ class _GeneratorConcat(torch.autograd.Function):
     beside the concat (no gradient)."""
 
     @staticmethod
-    def forward(ctx, x, y, gen_weight, gen_bias, fuse_weight, kernel_size, dilations):
-        cat, ws = _concat_pack(x, y, gen_weight, gen_bias, fuse_weight, kernel_size, dilations)
+    def forward(ctx, x, y, gen_weight, gen_bias, fuse_weight, kernel_size, dilations, guard):
+        cat, ws = _concat_pack(x, y, gen_weight, gen_bias, fuse_weight, kernel_size, dilations, guard)
         ctx.save_for_backward(x, y, gen_weight, gen_bias)
         ctx.kernel_size = kernel_size
         ctx.dilations = dilations
+        ctx.guard = guard
         ctx.mark_non_differentiable(ws)
         # no zero-filled gradient for the workspace output (a fill kernel per step)
         ctx.set_materialize_grads(False)
@@ -721,11 +798,12 @@ class _GeneratorConcat(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_cat, grad_ws):
         if grad_cat is None:
-            return (None,) * 7
+            return (None,) * 8
         x, y, gen_weight, gen_bias = ctx.saved_tensors
-        grads = _generator_backward(x, y, gen_weight, gen_bias, _as(grad_cat, x.dtype),
-                                    ctx.kernel_size, ctx.dilations, ctx.needs_input_grad[:4])
-        return (*grads, None, None, None)
+        args = (x, y, gen_weight, gen_bias, _as(grad_cat, x.dtype), ctx.kernel_size, ctx.dilations,
+                ctx.needs_input_grad[:4])
+        grads = _flat_generator_backward(*args, ctx.guard) if ctx.guard else _generator_backward(*args)
+        return (*grads, None, None, None, None)
 
 
 class _FuseConvOfConcat(torch.autograd.Function):
@@ -736,20 +814,27 @@ class _FuseConvOfConcat(torch.autograd.Function):
     before the generator's backward allocates its buffers."""
 
     @staticmethod
-    def forward(ctx, cat, ws, fuse_weight, fuse_bias):
+    def forward(ctx, cat, ws, fuse_weight, fuse_bias, shape, guard):
         # ws: the forward's workspace, holding the packed weight (_GeneratorConcat)
-        out = _fuse_conv_forward_packed(cat, ws, fuse_bias)
+        out = _fuse_conv_forward_packed(cat, ws, fuse_bias, shape, guard)
         ctx.save_for_backward(cat, fuse_weight)
         ctx.has_bias = fuse_bias is not None
+        ctx.shape = shape
+        ctx.guard = guard
         return out
 
     @staticmethod
     def backward(ctx, grad_out):
         cat, fuse_weight = ctx.saved_tensors
-        grads = _fuse_conv_backward(cat, fuse_weight, ctx.has_bias, _as(grad_out, cat.dtype),
-                                    (ctx.needs_input_grad[0], *ctx.needs_input_grad[2:]),
-                                    _cat_code(cat.dtype))
-        return grads[0], None, grads[1], grads[2]
+        needs = (ctx.needs_input_grad[0], *ctx.needs_input_grad[2:4])
+        grad_out = _as(grad_out, cat.dtype)
+        if ctx.guard:
+            grads = _flat_fuse_conv_backward(cat, fuse_weight, ctx.has_bias, grad_out, needs, ctx.shape,
+                                             ctx.guard)
+        else:
+            grads = _fuse_conv_backward(cat, fuse_weight, ctx.has_bias, grad_out, needs,
+                                        _cat_code(cat.dtype))
+        return grads[0], None, grads[1], grads[2], None, None
 
 
 def fused_ddpm(x, y, gen_weight, gen_bias, fuse_weight, fuse_bias, kernel_size, dilations):
@@ -766,19 +851,24 @@ def fused_ddpm(x, y, gen_weight, gen_bias, fuse_weight, fuse_bias, kernel_size, 
     return _fused_ddpm_checked(x, y, gen_weight, gen_bias, fuse_weight, fuse_bias, k, dil)
 
 
-def _fused_ddpm_checked(x, y, gen_weight, gen_bias, fuse_weight, fuse_bias, k, dil):
+def _fused_ddpm_checked(x, y, gen_weight, gen_bias, fuse_weight, fuse_bias, k, dil, flat=False):
     """:func:`fused_ddpm` for arguments :func:`fused_ddpm_supported` has
-    accepted (k an int, dil a tuple of three ints)."""
+    accepted (k an int, dil a tuple of three ints).  ``flat``: the concat may
+    be a flat one (:func:`_flat_guard`), whose tiles sum in another order
+    than the separate ops'."""
     x, y = x.contiguous(), y.contiguous()
     gen_weight, gen_bias = gen_weight.contiguous(), gen_bias.contiguous()
     fuse_weight = fuse_weight.contiguous()
     fuse_bias = fuse_bias.contiguous() if fuse_bias is not None else None
     tensors = (x, y, gen_weight, gen_bias, fuse_weight, fuse_bias)
+    shape = tuple(x.shape)
     if torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors):
-        cat, ws = _GeneratorConcat.apply(x, y, gen_weight, gen_bias, fuse_weight, k, dil)
-        return _FuseConvOfConcat.apply(cat, ws, fuse_weight, fuse_bias)
-    cat, ws = _concat_pack(x, y, gen_weight, gen_bias, fuse_weight, k, dil)
-    return _fuse_conv_forward_packed(cat, ws, fuse_bias)
+        guard = _flat_guard(x, k, dil, _cat_code(x.dtype), True) if flat else 0
+        cat, ws = _GeneratorConcat.apply(x, y, gen_weight, gen_bias, fuse_weight, k, dil, guard)
+        return _FuseConvOfConcat.apply(cat, ws, fuse_weight, fuse_bias, shape, guard)
+    guard = _flat_guard(x, k, dil, _cat_code(x.dtype), False) if flat else 0
+    cat, ws = _concat_pack(x, y, gen_weight, gen_bias, fuse_weight, k, dil, guard)
+    return _fuse_conv_forward_packed(cat, ws, fuse_bias, shape, guard)
 
 
 __all__ = [

@@ -341,6 +341,59 @@ int ddpm_fuse_conv_bwd(const void* cat, const void* weight, const void* grad_out
                        int64_t workspace_weight_bytes, int64_t n, int64_t c, int64_t h, int64_t w,
                        int dtype, hipStream_t stream);
 
+/* ---- flat concats ------------------------------------------------------
+ *
+ * The concat between the fused generator and the fuse convolution, and its
+ * gradient, in a layout whose rows start on 16 bytes whatever w is: element
+ * (n, plane, h, w) at lead + (n * 4c + plane) * S + h * P + w, P = w + guard
+ * rounded up to 8, S and lead multiples of 8, zero outside the images.  No
+ * caller reads it: the entry points below pass it to each other, in a buffer
+ * of ddpm_flat_cat_elems elements.  x, y, out and every gradient but the
+ * concat's are plain.  `guard` (1..64) is the rows and columns of zeros
+ * around an image: 1 for the forward, at least (kernel_size / 2) *
+ * max(dilation) where the backward follows; the same value in all calls. */
+
+/* Elements of a flat concat (of the concat's element size); 0 for an empty or
+ * unsupported shape (c > 128, c % 8 != 0, an image's planes beyond 2^31
+ * bytes). */
+int64_t ddpm_flat_cat_elems(int64_t n, int64_t c, int64_t h, int64_t w, int guard, int dtype);
+
+/* ddpm_gen_fwd_pack writing a flat concat; fuse_workspace as
+ * ddpm_flat_fuse_conv_workspace_bytes.  dtype 3: pair planes. */
+int ddpm_flat_gen_fwd_pack(const void* x, const void* y, const void* weight, const void* bias,
+                           void* cat, const void* fuse_weight, void* fuse_workspace,
+                           int64_t fuse_workspace_bytes, int64_t n, int64_t c, int64_t h, int64_t w,
+                           int kernel_size, int d0, int d1, int d2, int guard, int dtype,
+                           hipStream_t stream);
+
+/* ddpm_fuse_conv_fwd_packed of a flat concat. */
+int64_t ddpm_flat_fuse_conv_workspace_bytes(int64_t n, int64_t c, int64_t h, int64_t w, int guard,
+                                            int dtype);
+int ddpm_flat_fuse_conv_fwd_packed(const void* cat, const void* bias, void* out, void* workspace,
+                                   int64_t workspace_bytes, int64_t n, int64_t c, int64_t h,
+                                   int64_t w, int guard, int dtype, hipStream_t stream);
+
+/* ddpm_fuse_conv_bwd of a flat concat; grad_cat is flat (plain fp32 for dtype
+ * 3), its elements outside the images unspecified beyond the rows' pads.
+ * grad_cat, or grad_weight and grad_bias together, may be NULL: not computed. */
+int64_t ddpm_flat_fuse_conv_bwd_workspace_bytes(int64_t n, int64_t c, int64_t h, int64_t w,
+                                                int guard, int dtype);
+int ddpm_flat_fuse_conv_bwd(const void* cat, const void* weight, const void* grad_out,
+                            void* grad_cat, void* grad_weight, void* grad_bias, void* workspace,
+                            int64_t workspace_bytes, int64_t n, int64_t c, int64_t h, int64_t w,
+                            int guard, int dtype, hipStream_t stream);
+
+/* ddpm_gen_bwd from a flat grad_cat.  grad_x, grad_y, or grad_weight and
+ * grad_bias together, may be NULL: not computed. */
+int64_t ddpm_flat_gen_bwd_workspace_bytes(int64_t n, int64_t c, int64_t h, int64_t w,
+                                          int kernel_size, int d0, int d1, int d2, int guard,
+                                          int dtype);
+int ddpm_flat_gen_bwd(const void* x, const void* y, const void* weight, const void* bias,
+                      const void* grad_cat, void* grad_x, void* grad_y, void* grad_weight,
+                      void* grad_bias, void* workspace, int64_t workspace_bytes, int64_t n,
+                      int64_t c, int64_t h, int64_t w, int kernel_size, int d0, int d1, int d2,
+                      int guard, int dtype, hipStream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

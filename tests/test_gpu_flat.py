@@ -1,0 +1,95 @@
+"""The flat concat route (rows padded to a 16-byte pitch, tiles of 256
+positions) between the fused generator and the fuse convolution, and the flat
+copies of the stand-alone fuse convolution, against the fp64 oracle."""
+
+import pytest
+import torch
+
+from dynamicconvolutionoperator_amd import DDPM, ops
+from oracle.unfold_ref import UnfoldDDPM
+from tests.gpu_helpers import DEV, DIL, TOL, assert_close, randn, say
+
+pytestmark = pytest.mark.gpu
+
+# (n, c, h, w): one position over and under a tile of 256, rows shorter than
+# the halo, a single row, a padded pitch of exactly one tile, several images,
+# channel counts below and between the 16-, 32- and 64-channel blocks
+SHAPES = [
+    (1, 16, 1, 5), (2, 16, 15, 17), (1, 32, 3, 251), (1, 48, 9, 249), (3, 64, 20, 30),
+    (1, 64, 31, 257), (2, 96, 11, 35), (1, 128, 24, 40),
+]
+
+
+def _modules(c, k, dtype):
+    torch.manual_seed(7)
+    ref = UnfoldDDPM(c, k)
+    mod = DDPM(c, k, fused_generator_training=True)
+    mod.load_state_dict(ref.state_dict())
+    mod = mod.to(DEV, dtype)
+    with torch.no_grad():
+        for p, q in zip(ref.parameters(), mod.parameters()):
+            p.copy_(q.float().cpu())
+    return ref.double(), mod
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_flat_training_matches_oracle(shape, dtype):
+    n, c, h, w = shape
+    say(f"flat training {shape} {dtype}")
+    ref, mod = _modules(c, 3, dtype)
+    x, y, g = (randn(shape, s, dtype=dtype) for s in (1, 2, 3))
+    assert ops._flat_guard(x, 3, DIL, ops._cat_code(dtype), True) == 5
+    xg, yg = (t.to(DEV).requires_grad_() for t in (x, y))
+    xr, yr = (t.double().requires_grad_() for t in (x, y))
+    # memory that no kernel writes holds NaN
+    junk = torch.full((1 << 24,), float("nan"), device=DEV)
+    del junk
+    out = mod(xg, yg)
+    out_ref = ref(xr, yr)
+    grads = torch.autograd.grad(out, (xg, yg, *mod.parameters()), g.to(DEV))
+    grads_ref = torch.autograd.grad(out_ref, (xr, yr, *ref.parameters()), g.double())
+    assert_close(out, out_ref, *TOL["module_fwd"][dtype], "out")
+    atol, rtol = TOL["module_bwd"][dtype]
+    for name, a, e in zip(("dx", "dy", "dgw", "dgb", "dfw", "dfb"), grads, grads_ref):
+        assert_close(a, e, atol * max(e.abs().max().item(), 1e-6), rtol, name)
+
+
+def test_flat_partial_gradients_match_all():
+    """Each subset of the gradients is bit for bit the full backward's."""
+    shape, dtype = (2, 32, 13, 21), torch.bfloat16
+    _, mod = _modules(32, 3, dtype)
+    x, y, g = (randn(shape, s, dtype=dtype).to(DEV) for s in (1, 2, 3))
+    tensors = (x, y, *(p.detach() for p in mod.parameters()))
+
+    def grads(needs):
+        t = [v.clone().requires_grad_(f) for v, f in zip(tensors, needs)]
+        out = ops._fused_ddpm_checked(*t, 3, DIL, flat=True)
+        it = iter(torch.autograd.grad(out, [v for v, f in zip(t, needs) if f], g))
+        return [next(it) if f else None for f in needs]
+
+    full = grads((True,) * 6)
+    for needs in [(1, 0, 0, 0, 0, 0), (0, 1, 0, 0, 0, 0), (0, 0, 1, 1, 0, 0), (0, 0, 0, 0, 1, 1),
+                  (1, 1, 0, 0, 0, 0), (1, 0, 0, 1, 0, 0), (0, 1, 1, 0, 1, 0)]:
+        for a, e in zip(grads([bool(f) for f in needs]), full):
+            assert a is None or torch.equal(a, e), needs
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("shape", [(2, 24, 15, 17), (1, 20, 9, 33), (1, 64, 7, 255)])
+def test_stand_alone_fuse_conv_copies_flat(shape, dtype):
+    """Odd widths: the public NCHW fuse convolution lays its operands out flat
+    (C % 8 != 0: the weight gradient does not)."""
+    n, c, h, w = shape
+    cat, g = randn((n, 4 * c, h, w), 1, dtype=dtype), randn(shape, 2, dtype=dtype)
+    wt, b = randn((c, 4 * c, 3, 3), 3, dtype=dtype, scale=0.05), randn((c,), 4, dtype=dtype)
+    dev = [t.to(DEV).requires_grad_() for t in (cat, wt, b)]
+    ref = [t.double().requires_grad_() for t in (cat, wt, b)]
+    out = ops.fuse_conv3x3(*dev)
+    out_ref = torch.nn.functional.conv2d(ref[0], ref[1], ref[2], padding=1)
+    got = torch.autograd.grad(out, dev, g.to(DEV))
+    want = torch.autograd.grad(out_ref, ref, g.double())
+    assert_close(out, out_ref, *TOL["module_fwd"][dtype], "out")
+    atol, rtol = TOL["module_bwd"][dtype]
+    for name, a, e in zip(("dcat", "dw", "db"), got, want):
+        assert_close(a, e, atol * e.abs().max().item(), rtol, name)
