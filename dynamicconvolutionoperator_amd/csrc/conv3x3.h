@@ -26,6 +26,7 @@ struct ConvGeom {
   int flat;           // the input is a flat tensor (FlatLay) of `kp` planes per image: tiles of
                       // 256 positions (tiles_h = f.ft, tiles_w = 1), H and W the image's
   int kp;
+  int pairs;          // channels-last: m-group pairs per workgroup (0: one group)
   int oflat;          // the output is flat too (layout f, M planes per image)
   FlatLay f;
 };

@@ -40,6 +40,7 @@
 //   * v_mfma_f32_16x16x32_{bf16,f16}; fp32 operands run as three bf16
 //     products (hi*hi + hi*lo + lo*hi), accumulation in fp32.
 
+#include "cl_conv.h"
 #include "conv3x3.h"
 
 #include <type_traits>
@@ -135,7 +136,7 @@ __device__ __forceinline__ void cv_store_flat(const f32x4 (&acc)[2][MB], int mg,
                                               const T* __restrict__ bias, T* __restrict__ out,
                                               float* __restrict__ part, int ksplit, int n, int pos,
                                               int quad) {
-  const uint32_t FS = (uint32_t)g.f.ft * kFlatTile;
+  const uint32_t FS = flat_span(g.f);
 #pragma unroll
   for (int blk = 0; blk < 2; ++blk) {
     const int p = pos + 16 * blk;
@@ -545,7 +546,7 @@ __global__ __launch_bounds__(256) void conv3x3_reduce_flat_kernel(const float* _
                                                                   uint32_t items) {
   const uint32_t i = blockIdx.x * 256u + threadIdx.x;
   if (i >= items) return;
-  const uint32_t FS = (uint32_t)g.f.ft * kFlatTile;
+  const uint32_t FS = flat_span(g.f);
   const uint32_t plane = i / (FS / 4);
   const int p = (int)(i - plane * (FS / 4)) * 4;
   const int row = p / g.f.P, col = p - row * g.f.P;
@@ -594,7 +595,42 @@ int cv_pow2ceil(int64_t v) {
   return p;
 }
 
-// Input-plane splits and m blocks of flat tiles.  A flat grid is any number of
+// The channels-last kernel's (2-byte types) geometry: m blocks, input-plane
+// splits in groups of 64, or the m groups in pairs per workgroup (mgl pairs,
+// one group to each half of its waves).  One workgroup fits a CU, so the grid
+// costs rounds of workgroups; a stage measured 0.55 + 0.17 us per m block, a
+// workgroup's start and end together about 6 us, a pair's stores 1 us, the
+// partials' second pass 3.5 us and its bytes.
+void cv_split_cl(ConvGeom& g, int64_t tiles, int64_t m, bool split) {
+  const int gs = (g.nc32 + 1) / 2;
+  double best = 1e30;
+  auto take = [&](double t, int mb, int ks, int per, int pairs) {
+    if (t >= best) return;
+    best = t;
+    g.mb = mb;
+    g.ks = ks;
+    g.cc_per = per;
+    g.pairs = pairs;
+  };
+  auto rounds = [](int64_t wgs) { return (double)((wgs + kCvFillWGs - 1) / kCvFillWGs); };
+  for (int mb = kCvMaxMB; mb >= 1; mb /= 2) {
+    const int64_t groups = (m + mb * 16 - 1) / (mb * 16);
+    const double stage = 0.55 + 0.17 * mb;
+    for (int ks = 1; ks <= (split ? gs : 1); ++ks) {
+      const int per = (gs + ks - 1) / ks;
+      if ((gs + per - 1) / per != ks) continue;
+      double t = rounds(tiles * groups * ks) * (6.0 + 3 * per * stage);
+      if (ks > 1) t += 3.5 + 4e-6 * (double)tiles * kFlatTile * (double)m * (ks + 1) / 4.0;
+      take(t, mb, ks, per, 0);
+    }
+    const int64_t pairs = (groups + 1) / 2;
+    for (int p = 1; groups > 1 && p <= pairs; ++p)
+      if (pairs % p == 0)
+        take(rounds(tiles * (pairs / p)) * (6.0 + p * (3 * g.nc32 * stage + 1.0)), mb, 1, gs, p);
+  }
+}
+
+// Input-plane splits and m blocks of flat tiles (fp32).  A flat grid is any number of
 // workgroups, and one past a multiple of the CUs costs a whole round of them
 // (fp32 forward at 1x64x128x128: 68 tiles x 4 splits = 272 workgroups 30.0 us,
 // x 3 = 204 workgroups of half again the stages 24 us): the choice minimizes
@@ -628,7 +664,7 @@ void cv_split_flat(ConvGeom& g, int64_t tiles, int64_t m, int esz) {
 // fewer than kCvFillWGs workgroups.  `esz` sizes the LDS staging buffers.
 // f: flat tiles of layout f instead of segments.
 void cv_geom(ConvGeom& g, int64_t n, int64_t k, int64_t m, int64_t h, int64_t w, int esz,
-             const FlatLay* f = nullptr) {
+             const FlatLay* f = nullptr, bool split = true) {
   g.N = (int)n;
   g.K = (int)k;
   g.M = (int)m;
@@ -645,6 +681,7 @@ void cv_geom(ConvGeom& g, int64_t n, int64_t k, int64_t m, int64_t h, int64_t w,
   g.f = f ? *f : FlatLay{};
   g.kp = (int)k;
   g.oflat = 0;
+  g.pairs = 0;
   g.nc32 = (int)((k + 31) / 32);
   g.mb = kCvMaxMB;
   const int64_t tiles = n * g.tiles_h * g.tiles_w;
@@ -654,7 +691,9 @@ void cv_geom(ConvGeom& g, int64_t n, int64_t k, int64_t m, int64_t h, int64_t w,
   // then halve the m blocks
   g.ks = 1;
   const int64_t mg4 = (m + kCvMaxMB * 16 - 1) / (kCvMaxMB * 16);
-  if (f) {
+  if (f && esz == 2) {
+    cv_split_cl(g, tiles, m, split);
+  } else if (f) {
     cv_split_flat(g, tiles, m, esz);
   } else {
     while (tiles * mg4 * g.ks < kCvFillWGs && 2 * g.ks * 2 <= g.nc32) g.ks *= 2;
@@ -706,7 +745,7 @@ int64_t cv_align(int64_t v) { return (v + 255) / 256 * 256; }
 int64_t cv_workspace_bytes(const ConvGeom& g, int dtype) {
   const int64_t pk = cv_pack_bytes(g, dtype);
   if (g.ks <= 1) return pk;
-  const int64_t plane = g.flat ? (int64_t)g.f.ft * kFlatTile : (int64_t)g.H * g.W;
+  const int64_t plane = g.flat ? (int64_t)flat_span(g.f) : (int64_t)g.H * g.W;
   return cv_align(pk) + (int64_t)g.ks * g.N * g.M * plane * (int64_t)sizeof(float);
 }
 
@@ -729,8 +768,8 @@ struct CvPlan {
 // otherwise.
 bool cv_flat_rule(FlatLay& f, int64_t n, int64_t k, int64_t h, int64_t w, int esz) {
   if (w % 8 == 0) return false;
-  return flat_lay(f, h, w, 1, flat_planes(k), esz) &&
-         flat_elems(f, n * flat_planes(k)) / 8 <= 0x7fffffffLL;
+  return flat_lay(f, h, w, 1, flat_planes(k) + 16, esz) &&
+         flat_elems(f, n * flat_planes(k), esz) / 8 <= 0x7fffffffLL;
 }
 bool cv_flat_both(FlatLay& f, int64_t n, int64_t c, int64_t h, int64_t w, int esz) {
   FlatLay fc;
@@ -752,9 +791,9 @@ void cv_plan(CvPlan& p, const void* in, int64_t n, int64_t k, int64_t m, int64_t
   if (!inl && cv_flat_rule(f, n, k, h, w, esz)) {
     inl = &f;
     kp = flat_planes(k);
-    p.copy = cv_align(flat_elems(f, n * kp) * esz);
+    p.copy = cv_align(flat_elems(f, n * kp, esz) * esz);
   }
-  cv_geom(g, n, k, m, h, w, esz, inl);
+  cv_geom(g, n, k, m, h, w, esz, inl, !oflat);
   g.x4 = (w % 8 == 0) && ((uintptr_t)in % 16 == 0);
   if (inl) {
     p.lay = kCvFlat;
@@ -789,7 +828,7 @@ int cv_run(const CvPlan& plan, const void* in, const void* wt, const void* bias,
   FlatCopy fc{nullptr, nullptr, 0, 0, 0};
   if (plan.copy) {
     void* dst = (char*)workspace + cv_align(cv_workspace_bytes(g, dtype));
-    fc = flat_copy_of(in, dst, g.f, n, g.K, g.kp);
+    fc = flat_copy_of(in, dst, g.f, n, g.K, g.kp, dtype == kF32 ? 4 : 2);
     in = dst;
     if (!pack) {
       const int e = flat_copy(&fc, 1, g.f, dtype, stream);
@@ -816,6 +855,46 @@ int cv_run(const CvPlan& plan, const void* in, const void* wt, const void* bias,
       const int e = (int)hipGetLastError();
       if (e != 0) return e;
     }
+    auto reduce_flat = [&]() {
+      // the K splits' partial sums (and the bias) in split order
+      const uint32_t items = (uint32_t)(n * m * (flat_span(g.f) / 4));
+      const dim3 fgrid((items + 255) / 256);
+      if (bias)
+        hipLaunchKernelGGL((conv3x3_reduce_flat_kernel<T, true>), fgrid, dim3(256), 0, stream,
+                           (const float*)part, (const T*)bias, (T*)out, g, items);
+      else
+        hipLaunchKernelGGL((conv3x3_reduce_flat_kernel<T, false>), fgrid, dim3(256), 0, stream,
+                           (const float*)part, (const T*)bias, (T*)out, g, items);
+      return (int)hipGetLastError();
+    };
+    if constexpr (sizeof(T) == 2) {
+      if (plan.lay == kCvFlat) {
+        const int64_t c = rot ? g.K : g.M;  // channels of the module
+        ClConvGeom cg{};
+        cg.N = g.N;
+        cg.M = g.M;
+        cg.H = g.H;
+        cg.W = g.W;
+        cg.f = g.f;
+        cg.q = g.kp / 16;
+        cg.in_img = rot || plan.copy ? (int64_t)g.kp * g.f.S : 4 * c * (int64_t)g.f.S;
+        cg.nc32 = g.nc32;
+        cg.nb = 1;
+        cg.d0 = cg.d1 = cg.d2 = 1;
+        cg.mgroups = g.mgroups;
+        cg.gs = (g.nc32 + 1) / 2;
+        cg.ks = g.ks;
+        cg.gs_per = g.cc_per;
+        cg.pairs = g.pairs;
+        cg.out = g.oflat ? kClOutGrad : kClOutImage;
+        cg.C = (int)c;
+        cg.out_img = cl_cat_planes(c) * g.f.S;
+        const int e2 = cl_conv_launch(dtype, 0, 3, g.mb, cg, in, nullptr, workspace, bias, out, part,
+                                      rd, WReduce{nullptr, nullptr, nullptr, nullptr, 0, 0, 0, 0, 0},
+                                      stream);
+        return e2 != 0 || g.ks <= 1 ? e2 : reduce_flat();
+      }
+    }
     const dim3 grid((unsigned)((int64_t)n * g.tiles_h * g.tiles_w * (g.mgroups / g.mgl) * g.ks));
     auto launch = [&](auto kern, size_t lds) {
       const int ae = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds);
@@ -825,17 +904,7 @@ int cv_run(const CvPlan& plan, const void* in, const void* wt, const void* bias,
       int e2 = (int)hipGetLastError();
       if (e2 != 0 || g.ks <= 1) return e2;
       // the K splits' partial sums (and the bias) in split order
-      if (plan.lay == kCvFlat) {
-        const uint32_t items = (uint32_t)(n * m * g.f.ft * (kFlatTile / 4));
-        const dim3 fgrid((items + 255) / 256);
-        if (bias)
-          hipLaunchKernelGGL((conv3x3_reduce_flat_kernel<T, true>), fgrid, dim3(256), 0, stream,
-                             (const float*)part, (const T*)bias, (T*)out, g, items);
-        else
-          hipLaunchKernelGGL((conv3x3_reduce_flat_kernel<T, false>), fgrid, dim3(256), 0, stream,
-                             (const float*)part, (const T*)bias, (T*)out, g, items);
-        return (int)hipGetLastError();
-      }
+      if (plan.lay == kCvFlat) return reduce_flat();
       const int64_t total = n * m * h * w, hw = h * w;
       const bool v4 = hw % 4 == 0 && (uintptr_t)out % (4 * sizeof(T)) == 0;
       const int64_t items = v4 ? total / 4 : total;
@@ -876,13 +945,15 @@ int cv_run(const CvPlan& plan, const void* in, const void* wt, const void* bias,
         return launch(conv3x3_kernel<T, B, 4, true, PR, 1, LAY>,
                       (size_t)2 * CvLds<T, 4, true>::kBuf * 4);
       };
-      if (plan.lay == kCvFlat) {
-        if (g.mb == 4) return wide(std::integral_constant<int, kCvFlat>());
-        if (g.mb == 2)
-          return launch(conv3x3_kernel<T, B, 2, true, PR, 1, kCvFlat>,
-                        (size_t)2 * CvLds<T, 2, true>::kBuf * 4);
-        return launch(conv3x3_kernel<T, B, 1, true, PR, 1, kCvFlat>,
-                      (size_t)2 * CvLds<T, 1, true>::kBuf * 4);
+      if constexpr (sizeof(T) == 4) {
+        if (plan.lay == kCvFlat) {
+          if (g.mb == 4) return wide(std::integral_constant<int, kCvFlat>());
+          if (g.mb == 2)
+            return launch(conv3x3_kernel<T, B, 2, true, PR, 1, kCvFlat>,
+                          (size_t)2 * CvLds<T, 2, true>::kBuf * 4);
+          return launch(conv3x3_kernel<T, B, 1, true, PR, 1, kCvFlat>,
+                        (size_t)2 * CvLds<T, 1, true>::kBuf * 4);
+        }
       }
       if (plan.lay == kCvAl) return wide(std::integral_constant<int, kCvAl>());
       // one-row segments (wide images) with the narrower staging pitch
@@ -931,10 +1002,10 @@ int cv_flat_check(FlatLay& f, int64_t n, int64_t c, int64_t h, int64_t w, int gu
   int st = cv_check(n, 4 * c, c, h, w, dtype);
   if (st != kOk) return st;
   if (n == 0 || c == 0 || h == 0 || w == 0) return kOk;
-  if (c % 8 != 0 || c > 128 || !flat_lay(f, h, w, guard, 4 * c, dtype == kF32 ? 4 : 2))
+  if (c % 8 != 0 || c > 128 || !flat_lay(f, h, w, guard, 4 * c + 64, dtype == kF32 ? 4 : 2))
     return kUnsupported;
   // 32-bit item counts of the launches over whole tensors
-  if (flat_elems(f, n * (4 * c > 128 ? 4 * c : 128)) > 0x7fffffffLL) return kUnsupported;
+  if (flat_elems(f, n * (4 * c > 128 ? 4 * c + 16 : 128), 2) > 0x7fffffffLL) return kUnsupported;
   return kOk;
 }
 
@@ -1043,6 +1114,10 @@ extern "C" int ddpm_fuse_conv_bwd(const void* cat, const void* weight, const voi
       (uintptr_t)workspace_data % 16 != 0)
     return kWorkspaceTooSmall;
   const void* go = grad_out;
+  // the weight-gradient launch (or the flat copies') packs the input
+  // gradient's weight; the input gradient's launch sums the weight gradient's
+  // split partials
+  const CvPack pack = cv_pack_of(plan, weight, workspace_data, 1, false);
   const FlatLay f = plan.g.f;
   FlatLay fb;
   const bool flat = plan.copy != 0 && cv_flat_both(fb, n, c, h, w, ddt == kF32 ? 4 : 2);
@@ -1050,20 +1125,18 @@ extern "C" int ddpm_fuse_conv_bwd(const void* cat, const void* weight, const voi
     // grad_out flat once for both launches, the concat for the weight gradient
     void* gof = (char*)workspace_data + cv_align(cv_workspace_bytes(plan.g, ddt));
     void* catf = (char*)workspace_weight + cv_align(cw_flat_partial_bytes(f, n, c, ddt == kF32 ? 4 : 2));
-    const FlatCopy fc[2] = {flat_copy_of(grad_out, gof, f, n, c, plan.g.kp),
-                            flat_copy_of(cat, catf, f, n, 4 * c, 4 * c)};
-    st = flat_copy(fc, 2, f, ddt, stream);
+    const int esz = ddt == kF32 ? 4 : 2;
+    const FlatCopy fc[2] = {flat_copy_of(grad_out, gof, f, n, c, plan.g.kp, esz),
+                            flat_copy_of(cat, catf, f, n, 4 * c, 4 * c, esz)};
+    st = flat_copy(fc, 2, f, ddt, stream, &pack);
     if (st != kOk) return st;
     go = gof;
     cat = catf;
     plan.copy = 0;
   }
-  // the weight-gradient launch packs the input gradient's weight; the input
-  // gradient's launch sums the weight gradient's split partials
-  const CvPack pack = cv_pack_of(plan, weight, workspace_data, 1, false);
   CwReduce red{nullptr, nullptr, nullptr, nullptr, 0, 0, 0, 0, 0};
   st = cw_run(cat, go, grad_weight, grad_bias, workspace_weight, workspace_weight_bytes, n, c, h, w,
-              dtype, stream, false, &pack, &red, flat ? &f : nullptr, plan.g.kp);
+              dtype, stream, false, flat ? nullptr : &pack, &red, flat ? &f : nullptr, plan.g.kp);
   if (st != kOk) return st;
   return cv_run(plan, go, weight, nullptr, grad_cat, workspace_data, workspace_data_bytes, 1, ddt,
                 stream, false, &red, false);
@@ -1078,7 +1151,7 @@ extern "C" int64_t ddpm_flat_cat_elems(int64_t n, int64_t c, int64_t h, int64_t 
   if (cv_dtype(dtype, pairs, c) != kOk) return 0;
   if (cv_flat_check(f, n, c, h, w, guard, dtype) != kOk) return 0;
   if (n == 0 || c == 0 || h == 0 || w == 0) return 0;
-  return flat_elems(f, n * 4 * c);
+  return dtype == kF32 ? flat_elems(f, n * 4 * c, 4) : flat_elems(f, n * cl_cat_planes(c), 2);
 }
 
 namespace {
@@ -1096,7 +1169,7 @@ void cv_flat_bwd(CvFlatBwd& b, const FlatLay& f, int64_t n, int64_t c, int64_t h
   const int esz = dtype == kF32 ? 4 : 2;
   b.cp = flat_planes(c);
   cv_plan(b.plan, nullptr, n, c, 4 * c, h, w, dtype, false, false, &f, b.cp, true);
-  b.go = cv_align(flat_elems(f, n * b.cp) * esz);
+  b.go = cv_align(flat_elems(f, n * b.cp, esz) * esz);
   b.data = cv_align(cv_need(b.plan, dtype));
   b.weight = cv_align(cw_flat_partial_bytes(f, n, c, esz));
 }
@@ -1168,17 +1241,17 @@ extern "C" int ddpm_flat_fuse_conv_bwd(const void* cat, const void* weight, cons
   void* go = ws;
   void* wsd = ws + b.go;
   void* wsw = ws + b.go + b.data;
-  const FlatCopy fc = flat_copy_of(grad_out, go, f, n, c, b.cp);
-  st = flat_copy(&fc, 1, f, dtype, stream);
-  if (st != kOk) return st;
+  const FlatCopy fc = flat_copy_of(grad_out, go, f, n, c, b.cp, dtype == kF32 ? 4 : 2);
   const CvPack pack = cv_pack_of(b.plan, weight, wsd, 1, false);
+  st = flat_copy(&fc, 1, f, dtype, stream, grad_cat ? &pack : nullptr);
+  if (st != kOk) return st;
   CwReduce red{nullptr, nullptr, nullptr, nullptr, 0, 0, 0, 0, 0};
   if (need_w) {
     st = cw_run(cat, go, grad_weight, grad_bias, wsw, b.weight, n, c, h, w, code, stream, false,
-                grad_cat ? &pack : nullptr, grad_cat ? &red : nullptr, &f, b.cp);
+                nullptr, grad_cat ? &red : nullptr, &f, b.cp);
     if (st != kOk) return st;
   }
   if (!grad_cat) return kOk;
   return cv_run(b.plan, go, weight, nullptr, grad_cat, wsd, b.data, 1, dtype, stream, false, &red,
-                !need_w);
+                false);
 }

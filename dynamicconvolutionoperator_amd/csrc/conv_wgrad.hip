@@ -30,7 +30,7 @@
 //     16-plane block of grad_out with one more MFMA per step and part (a
 //     fragment of ones times grad_out).
 
-#include "conv3x3.h"
+#include "cl_wgrad.h"
 
 #include <type_traits>
 
@@ -646,6 +646,11 @@ int64_t cw_partial_bytes(const CwGeom& g) {
 using namespace ddpm;
 
 int64_t ddpm::cw_flat_partial_bytes(const FlatLay& f, int64_t n, int64_t c, int esz) {
+  if (esz == 2) {
+    ClWGeom cg;
+    clw_geom(cg, f, n, c, false);
+    return clw_partial_bytes(cg, 9, false);
+  }
   CwGeom g;
   cw_geom_flat(g, f, n, c, esz, false);
   return cw_partial_bytes(g);
@@ -660,8 +665,8 @@ int64_t cw_align(int64_t v) { return (v + 255) / 256 * 256; }
 int64_t cw_copy_bytes(const FlatLay& f, int64_t n, int64_t c, int esz, int64_t& cat_off,
                       int64_t& go_off) {
   cat_off = cw_align(cw_flat_partial_bytes(f, n, c, esz));
-  go_off = cat_off + cw_align(flat_elems(f, n * 4 * c) * esz);
-  return go_off + flat_elems(f, n * flat_planes(c)) * esz;
+  go_off = cat_off + cw_align(flat_elems(f, n * 4 * c, esz) * esz);
+  return go_off + flat_elems(f, n * flat_planes(c), esz) * esz;
 }
 
 }  // namespace
@@ -723,20 +728,28 @@ int ddpm::cw_run(const void* cat, const void* grad_out, void* grad_weight, void*
     if (check_only) return kOk;
     void* catf = (char*)workspace + cat_off;
     void* gof = (char*)workspace + go_off;
-    const FlatCopy fc[2] = {flat_copy_of(cat, catf, fr, n, 4 * c, 4 * c),
-                            flat_copy_of(grad_out, gof, fr, n, c, flat_planes(c))};
+    const FlatCopy fc[2] = {flat_copy_of(cat, catf, fr, n, 4 * c, 4 * c, esz),
+                            flat_copy_of(grad_out, gof, fr, n, c, flat_planes(c), esz)};
     const int e = flat_copy(fc, 2, fr, dtype, stream);
     if (e != kOk) return e;
     return cw_run(catf, gof, grad_weight, grad_bias, workspace, cat_off, n, c, h, w,
                   pp ? (int)kF32Pairs : dtype, stream, false, pack, defer, &fr, flat_planes(c));
   }
   CwGeom g;
-  if (f)
+  ClWGeom cg{};
+  if (f && esz == 2) {
+    // channels-last tensors: the splits are that kernel's
+    clw_geom(cg, *f, n, c, false);
+    g.splits = cg.splits;
+    g.direct = cg.direct;
+    g.CI = (int)(4 * c);
+    g.C = (int)c;
+  } else if (f)
     cw_geom_flat(g, *f, n, c, esz, pp);
   else
     cw_geom(g, n, c, h, w, pp ? kCwTW : cw_step_cols(w, esz));
   g.gp = (int)gp;
-  const int64_t need = cw_partial_bytes(g);
+  const int64_t need = f && esz == 2 ? clw_partial_bytes(cg, 9, false) : cw_partial_bytes(g);
   if (need > 0 && (!workspace || workspace_bytes < need)) return kWorkspaceTooSmall;
   if (check_only) return kOk;
   g.x16 = (w % (16 / esz) == 0) && ((uintptr_t)cat % 16 == 0);
@@ -748,31 +761,8 @@ int ddpm::cw_run(const void* cat, const void* grad_out, void* grad_weight, void*
   const CvPack nopack{nullptr, nullptr, ConvGeom{}, 0, 0, 0, 0};
   return cw_with_type(dtype, [&](auto tag) {
     using T = decltype(tag);
-    auto launch = [&](auto mbc, auto sjc) {
-      constexpr int MB = decltype(mbc)::value;
-      constexpr int SJ = decltype(sjc)::value;
-      typedef CwLds<T, MB, SJ> L;
-      const size_t stage = (size_t)2 * L::kBuf * 4;
-      const size_t red = (size_t)(kCwSegs * 9 * 16 * (MB * 16 + 1) + kCwSegs * 16) * sizeof(float);
-      const size_t lds = stage > red ? stage : red;
-      // aligned layout: 16-byte rows, whole steps, whole 16-plane blocks of
-      // ci (4C) and of co (one workgroup's MB blocks, or two halves of 64)
-      const bool al = g.x16 && (esz == 4 ? g.y4 : g.g16) && w % g.tw == 0 && c % 4 == 0 &&
-                      (c <= 64 ? c % 16 == 0 : c == 128);
-      constexpr bool PPC = sizeof(T) == 4 && SJ == 1;
-      auto kern = pp ? (f    ? conv_wgrad_partial_kernel<T, MB, PPC, SJ, 2>
-                        : al ? conv_wgrad_partial_kernel<T, MB, PPC, SJ, 1>
-                             : conv_wgrad_partial_kernel<T, MB, PPC, SJ>)
-                     : (f    ? conv_wgrad_partial_kernel<T, MB, false, SJ, 2>
-                        : al ? conv_wgrad_partial_kernel<T, MB, false, SJ, 1>
-                             : conv_wgrad_partial_kernel<T, MB, false, SJ>);
-      const int ae = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds);
-      if (ae != 0) return ae;
-      hipLaunchKernelGGL(kern, dim3((unsigned)(g.splits * g.cblocks * g.ohalves)), dim3(kCwThreads), lds, stream,
-                         (const T*)cat, (const T*)grad_out, pw, pb, (T*)grad_weight, (T*)grad_bias, g,
-                         pack ? *pack : nopack);
-      int e = (int)hipGetLastError();
-      if (e != 0 || g.direct) return e;
+    // the split reduction: launched here, or described in *defer
+    auto reduce = [&]() {
       // four elements per item where the partials and grad_weight allow
       // 16-byte loads and 4-element stores (36 C^2 is a multiple of 4)
       const uint32_t nw = (uint32_t)(36 * c * c);
@@ -793,6 +783,39 @@ int ddpm::cw_run(const void* cat, const void* grad_out, void* grad_weight, void*
                            (const float*)pw, (const float*)pb, (T*)grad_weight, (T*)grad_bias, nw,
                            (uint32_t)c, g.splits);
       return (int)hipGetLastError();
+    };
+    if (f && esz == 2) {
+      // (its callers pack in the copies' launch)
+      const int e = clw_launch_conv(dtype, cg, cat, grad_out, pw, pb, grad_weight, grad_bias, stream);
+      return e != 0 || g.direct ? e : reduce();
+    }
+    auto launch = [&](auto mbc, auto sjc) {
+      constexpr int MB = decltype(mbc)::value;
+      constexpr int SJ = decltype(sjc)::value;
+      typedef CwLds<T, MB, SJ> L;
+      const size_t stage = (size_t)2 * L::kBuf * 4;
+      const size_t red = (size_t)(kCwSegs * 9 * 16 * (MB * 16 + 1) + kCwSegs * 16) * sizeof(float);
+      const size_t lds = stage > red ? stage : red;
+      // aligned layout: 16-byte rows, whole steps, whole 16-plane blocks of
+      // ci (4C) and of co (one workgroup's MB blocks, or two halves of 64)
+      const bool al = g.x16 && (esz == 4 ? g.y4 : g.g16) && w % g.tw == 0 && c % 4 == 0 &&
+                      (c <= 64 ? c % 16 == 0 : c == 128);
+      constexpr bool PPC = sizeof(T) == 4 && SJ == 1;
+      constexpr int FLC = sizeof(T) == 4 ? 2 : 0;  // (2-byte flat tensors: cl_wgrad.hip)
+      auto kern = pp ? (f    ? conv_wgrad_partial_kernel<T, MB, PPC, SJ, FLC>
+                        : al ? conv_wgrad_partial_kernel<T, MB, PPC, SJ, 1>
+                             : conv_wgrad_partial_kernel<T, MB, PPC, SJ>)
+                     : (f    ? conv_wgrad_partial_kernel<T, MB, false, SJ, FLC>
+                        : al ? conv_wgrad_partial_kernel<T, MB, false, SJ, 1>
+                             : conv_wgrad_partial_kernel<T, MB, false, SJ>);
+      const int ae = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds);
+      if (ae != 0) return ae;
+      hipLaunchKernelGGL(kern, dim3((unsigned)(g.splits * g.cblocks * g.ohalves)), dim3(kCwThreads), lds, stream,
+                         (const T*)cat, (const T*)grad_out, pw, pb, (T*)grad_weight, (T*)grad_bias, g,
+                         pack ? *pack : nopack);
+      int e = (int)hipGetLastError();
+      if (e != 0 || g.direct) return e;
+      return reduce();
     };
     return cw_with_mb(mb, [&](auto mbc) {
       if constexpr (sizeof(T) == 2) {

@@ -71,6 +71,17 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float a, float b) {
   return __builtin_bit_cast(uint32_t, r);
 }
 
+// Two fp32 values rounded to nearest-even in T (bf16 / f16), packed low/high.
+template <typename T>
+__device__ __forceinline__ uint32_t pack2(float a, float b) {
+  if constexpr (!__is_same(T, f16)) {
+    return pack_bf16x2(a, b);
+  } else {
+    typedef f16 f16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){a, b}, f16x2));
+  }
+}
+
 template <typename T>
 __device__ __forceinline__ void quant4(const f32x4& v, float (&q)[4]) {
   if constexpr (__is_same(T, bf16)) {
@@ -363,10 +374,15 @@ __device__ __forceinline__ int dil_of(int b, int d0, int d1, int d2) {
 constexpr int kFlatTile = 256;
 struct FlatLay {
   int H, W, P;    // image rows and columns, row pitch
-  int ft;         // tiles of kFlatTile positions covering H * P
+  int ft;         // tiles of kFlatTile positions covering the image
   uint32_t S;     // plane stride
   uint32_t lead;  // zeros before plane 0
 };
+
+// Positions of a plane's split partial sums.
+__host__ __device__ inline uint32_t flat_span(const FlatLay& f) {
+  return (uint32_t)f.ft * kFlatTile;
+}
 
 // The flat layout of an h x w image with r guard rows and columns; false when
 // `planes` planes of elements of `esz` bytes exceed 32-bit byte offsets.
@@ -391,7 +407,12 @@ inline bool flat_lay(FlatLay& f, int64_t h, int64_t w, int64_t r, int64_t planes
 // gradients' workgroups take (the extra planes are zero).
 inline int64_t flat_planes(int64_t c) { return c > 64 && c < 128 ? 128 : (c + 31) / 32 * 32; }
 
-inline int64_t flat_elems(const FlatLay& f, int64_t planes) { return f.lead + planes * (int64_t)f.S; }
+// Elements of a flat tensor of `planes` planes (a multiple of 16 for 2-byte
+// elements, which are held channels-last: cl.h; their lead is `lead`
+// positions of 16 channels).
+inline int64_t flat_elems(const FlatLay& f, int64_t planes, int esz) {
+  return (esz == 2 ? 16 : 1) * (int64_t)f.lead + planes * (int64_t)f.S;
+}
 
 // Host: lets kernel `fn` launch with `bytes` of dynamic LDS (up to the 160 KB
 // of a gfx950 CU) on the current device.  hipFuncSetAttribute runs only the

@@ -6,53 +6,98 @@
 
 namespace ddpm {
 
+// Planes that one image of a flat concat of 2-byte elements takes (either
+// form): its gradient keeps the C x-planes plane-major, since only
+// element-wise code reads them, and the 3C branch planes channels-last in
+// whole 16-channel blocks.
+inline int64_t cl_cat_planes(int64_t c) { return c + (3 * c + 15) / 16 * 16; }
+
 // One tensor to lay out flat: src [n][c][H][W] -> dst (flat, cp planes per
 // image; planes c .. cp-1 and everything outside the images zero).
 struct FlatCopy {
   const void* src;
   void* dst;
   uint32_t c, cp;
-  uint32_t chunks;  // 8-element chunks of dst (0: no copy)
+  uint32_t chunks;  // work items (0: no copy): 8 elements, or a position's 16 channels
 };
 
 inline FlatCopy flat_copy_of(const void* src, void* dst, const FlatLay& f, int64_t n, int64_t c,
-                             int64_t cp) {
-  return FlatCopy{src, dst, (uint32_t)c, (uint32_t)cp, (uint32_t)(flat_elems(f, n * cp) / 8)};
+                             int64_t cp, int esz) {
+  return FlatCopy{src, dst, (uint32_t)c, (uint32_t)cp,
+                  (uint32_t)(flat_elems(f, n * cp, esz) / (esz == 2 ? 16 : 8))};
 }
 
-// One 8-element chunk of a destination: it lies in one row (P, S and lead are
-// multiples of 8), and its source elements are read by two vector loads of
-// any alignment, or one by one in the last chunk of a row.
+// One item of a copy.  4-byte elements: 8 elements of one row (P, S and lead
+// are multiples of 8), read by two vector loads of any alignment, or one by
+// one at the end of a row.  2-byte elements: a position of a 16-channel block
+// (channels-last), read from 16 planes; neighbouring lanes take neighbouring
+// positions of each plane.
 template <typename T>
 __device__ __forceinline__ void flat_copy_chunk(const FlatCopy& t, const FlatLay& f, uint32_t idx) {
   const T* __restrict__ src = static_cast<const T*>(t.src);
-  T* __restrict__ dst = static_cast<T*>(t.dst) + (size_t)idx * 8;
-  typedef T V8 __attribute__((ext_vector_type(8)));
-  V8 v = {(T)0.f, (T)0.f, (T)0.f, (T)0.f, (T)0.f, (T)0.f, (T)0.f, (T)0.f};
-  const uint32_t lead8 = f.lead / 8;
-  if (idx >= lead8) {
-    const uint32_t s8 = f.S / 8, p8 = (uint32_t)f.P / 8;
-    const uint32_t i = idx - lead8;
-    const uint32_t plane = i / s8, k = i - plane * s8;
-    const uint32_t n = plane / t.cp, c = plane - n * t.cp;
-    const uint32_t h = k / p8, w = (k - h * p8) * 8;
-    if (c < t.c && h < (uint32_t)f.H && w < (uint32_t)f.W) {
-      const T* __restrict__ s = src + (((size_t)n * t.c + c) * f.H + h) * f.W + w;
-      if (w + 8 <= (uint32_t)f.W) {
-        __builtin_memcpy(&v, s, sizeof(v));
-      } else {
+  if constexpr (sizeof(T) == 2) {
+    T* __restrict__ dst = static_cast<T*>(t.dst) + (size_t)idx * 16;
+    uint32_t v[8] = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};
+    if (idx >= f.lead) {
+      const uint32_t i = idx - f.lead;
+      const uint32_t blk = i / f.S, p = i - blk * f.S;
+      const uint32_t n = blk / (t.cp / 16), c0 = (blk - n * (t.cp / 16)) * 16;
+      const uint32_t h = p / (uint32_t)f.P, w = p - h * (uint32_t)f.P;
+      if (c0 < t.c && h < (uint32_t)f.H && w < (uint32_t)f.W) {
+        const size_t hw = (size_t)f.H * f.W;
+        const uint16_t* __restrict__ s = reinterpret_cast<const uint16_t*>(src) +
+                                         ((size_t)n * t.c + c0) * hw + (size_t)h * f.W + w;
+        if (c0 + 16 <= t.c) {
+          uint16_t e[16];
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
-          if (w + e < (uint32_t)f.W) v[e] = s[e];
+          for (int k = 0; k < 16; ++k) e[k] = s[k * hw];
+#pragma unroll
+          for (int k = 0; k < 8; ++k) v[k] = (uint32_t)e[2 * k] | ((uint32_t)e[2 * k + 1] << 16);
+        } else {
+#pragma unroll
+          for (int k = 0; k < 16; ++k)
+            if (c0 + k < t.c) v[k >> 1] |= (uint32_t)s[k * hw] << (16 * (k & 1));
+        }
       }
     }
+    u32x4* __restrict__ o = reinterpret_cast<u32x4*>(dst);
+    o[0] = (u32x4){v[0], v[1], v[2], v[3]};
+    o[1] = (u32x4){v[4], v[5], v[6], v[7]};
+    return;
+  } else {
+    T* __restrict__ dst = static_cast<T*>(t.dst) + (size_t)idx * 8;
+    typedef T V8 __attribute__((ext_vector_type(8)));
+    V8 v = {(T)0.f, (T)0.f, (T)0.f, (T)0.f, (T)0.f, (T)0.f, (T)0.f, (T)0.f};
+    const uint32_t lead8 = f.lead / 8;
+    if (idx >= lead8) {
+      const uint32_t s8 = f.S / 8, p8 = (uint32_t)f.P / 8;
+      const uint32_t i = idx - lead8;
+      const uint32_t plane = i / s8, k = i - plane * s8;
+      const uint32_t n = plane / t.cp, c = plane - n * t.cp;
+      const uint32_t h = k / p8, w = (k - h * p8) * 8;
+      if (c < t.c && h < (uint32_t)f.H && w < (uint32_t)f.W) {
+        const T* __restrict__ s = src + (((size_t)n * t.c + c) * f.H + h) * f.W + w;
+        if (w + 8 <= (uint32_t)f.W) {
+          __builtin_memcpy(&v, s, sizeof(v));
+        } else {
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            if (w + e < (uint32_t)f.W) v[e] = s[e];
+        }
+      }
+    }
+    *reinterpret_cast<V8*>(dst) = v;
   }
-  *reinterpret_cast<V8*>(dst) = v;
 }
 
+struct CvPack;
+struct YPack;
+
 // Lays out `count` (1 or 2) tensors of `dtype` and the same n, H, W flat in one
-// launch.  Defined in flat.hip.
-int flat_copy(const FlatCopy* t, int count, const FlatLay& f, int dtype, hipStream_t stream);
+// launch, whose first workgroups run a weight packing of the launches that
+// follow (optional; ypack: kernel size `ks`).  Defined in flat.hip.
+int flat_copy(const FlatCopy* t, int count, const FlatLay& f, int dtype, hipStream_t stream,
+              const CvPack* cpack = nullptr, const YPack* ypack = nullptr, int ks = 0);
 
 // Zeroing of the elements of a flat tensor (`planes` planes in all) that lie
 // outside the images, shared out over the workgroups of the launch that
@@ -68,25 +113,33 @@ __device__ __forceinline__ void flat_zero_share(const FlatZero& z, int wg, int w
                                                 int nthreads) {
   T* __restrict__ base = static_cast<T*>(z.base);
   const FlatLay& f = z.f;
+  // runs of memory per plane (2-byte elements: per 16-channel block, each
+  // position 16 elements)
+  constexpr uint32_t EP = sizeof(T) == 2 ? 16 : 1;
+  const uint32_t units = (uint32_t)z.planes / EP;
   const int stride = wgs * nthreads, first = wg * nthreads + tid;
   const uint32_t tail = f.S - (uint32_t)(f.H * f.P);  // a multiple of 8
   typedef uint32_t V4 __attribute__((ext_vector_type(4)));
   constexpr int VE = 16 / (int)sizeof(T);
   const V4 zero = {0u, 0u, 0u, 0u};
-  // the lead and the tail of every plane, 16 bytes at a time
-  const uint32_t lv = f.lead / VE, tv = tail / VE;
+  // the lead and the tail of every run, 16 bytes at a time
+  const uint32_t lv = f.lead * EP / VE, tv = tail * EP / VE;
   for (uint32_t i = first; i < lv; i += stride) reinterpret_cast<V4*>(base)[i] = zero;
-  const uint32_t tot = tv * (uint32_t)z.planes;
+  const uint32_t tot = tv * units;
   for (uint32_t i = first; i < tot; i += stride) {
     const uint32_t pl = i / tv, k = i - pl * tv;
-    reinterpret_cast<V4*>(base + f.lead + (size_t)pl * f.S + (size_t)f.H * f.P)[k] = zero;
+    reinterpret_cast<V4*>(base + (f.lead + (size_t)pl * f.S + (size_t)f.H * f.P) * EP)[k] = zero;
   }
   // the pad columns of every row
-  const uint32_t pad = (uint32_t)(f.P - f.W), rows = (uint32_t)z.planes * (uint32_t)f.H;
+  const uint32_t pad = (uint32_t)(f.P - f.W), rows = units * (uint32_t)f.H;
   for (uint32_t i = first; i < rows; i += stride) {
     const uint32_t pl = i / (uint32_t)f.H, h = i - pl * (uint32_t)f.H;
-    T* __restrict__ d = base + f.lead + (size_t)pl * f.S + (size_t)h * f.P + f.W;
-    for (uint32_t e = 0; e < pad; ++e) d[e] = (T)0.f;
+    T* __restrict__ d = base + (f.lead + (size_t)pl * f.S + (size_t)h * f.P + f.W) * EP;
+    if constexpr (EP == 16) {
+      for (uint32_t e = 0; e < 2 * pad; ++e) reinterpret_cast<V4*>(d)[e] = zero;
+    } else {
+      for (uint32_t e = 0; e < pad; ++e) d[e] = (T)0.f;
+    }
   }
 }
 

@@ -20,9 +20,11 @@ __host__ __device__ constexpr int yt_parts() {
 
 // One thread's share of the packing: 64-lane unit `idx` of
 // ihalves * 3 * nc32 * KS*KS * MB * 64.
+// nat: K slot 8q + e holds channel 8q + e (the channels-last kernel) instead
+// of 4e + q.
 template <typename T, int KS, int MB>
 __device__ __forceinline__ void yt_pack_item(const T* __restrict__ wt, uint32_t* __restrict__ pk,
-                                             int C, int nc32, int idx) {
+                                             int C, int nc32, int idx, int nat = 0) {
   constexpr int KK = KS * KS;
   constexpr int P = yt_parts<T>();
   const int lane = idx & 63;
@@ -39,7 +41,7 @@ __device__ __forceinline__ void yt_pack_item(const T* __restrict__ wt, uint32_t*
   float v[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
-    const int c = cc * 32 + 4 * e + q;
+    const int c = cc * 32 + (nat ? 8 * q + e : 4 * e + q);
     v[e] = (i < C && c < C) ? to_f(wt[((int64_t)(b * C + c) * KK + t) * C + i]) : 0.f;
   }
   typename Mma<T>::V o[P];
@@ -134,7 +136,21 @@ struct YPack {
   uint32_t* pk;
   int C, nc32;
   int total;
+  int mb = 0, nat = 0;  // 16-channel blocks per half; natural slot order (channels-last)
 };
+
+template <typename T, int KS>
+__device__ __forceinline__ void yt_pack_any(const YPack& p, int idx) {
+  const T* __restrict__ wt = static_cast<const T*>(p.wt);
+  if (p.mb == 4)
+    yt_pack_item<T, KS, 4>(wt, p.pk, p.C, p.nc32, idx, p.nat);
+  else if (p.mb == 3)
+    yt_pack_item<T, KS, 3>(wt, p.pk, p.C, p.nc32, idx, p.nat);
+  else if (p.mb == 2)
+    yt_pack_item<T, KS, 2>(wt, p.pk, p.C, p.nc32, idx, p.nat);
+  else
+    yt_pack_item<T, KS, 1>(wt, p.pk, p.C, p.nc32, idx, p.nat);
+}
 
 // ddpm_gen_bwd_y's work by mode.  Defined in gen_bwd_y.hip.
 enum YtMode {

@@ -31,7 +31,7 @@
 // writes their split to LDS after the step's MFMAs (no pre-pass over y, no
 // workspace planes), so every B fragment is a plain 16-byte LDS read.
 
-#include "gen_bwd.h"
+#include "cl_wgrad.h"
 #include <type_traits>
 
 namespace ddpm {
@@ -172,7 +172,7 @@ __global__ __launch_bounds__(256) void gen_ysplit_kernel(const float* __restrict
 // twice the work per step and per barrier; each wave takes its 32-token
 // segment in both).
 // LAY 1: aligned layout (16-byte x, y and gradient rows, whole steps, whole
-// 16-channel blocks).  LAY 2: flat tensors (FlatLay) -- a step is the next TW
+// 16-channel blocks).  LAY 2 (fp32): flat tensors (FlatLay) -- a step is the next TW
 // positions of a plane, kernel rows are d row pitches apart, and a neighbour
 // outside the image is a zero of the layout, so the copies are the aligned
 // layout's without its tests.
@@ -216,7 +216,7 @@ __global__ __launch_bounds__(64 * kWgSegs * WgTaps<KS>::kGroups) void gen_bwd_w_
     const T* __restrict__ fgo = static_cast<const T*>(fin.gout);
     T* __restrict__ fgx = static_cast<T*>(fin.gx);
     if (fin.vec == 4) {
-      for (int64_t it = first; it < fin.items; it += stride) bx_reduce_item<T, 4>(fin.part, fgo, fgx, fin.g, it);
+      for (int64_t it = first; it < fin.items; it += stride) bx_reduce_item<T, 4, FL>(fin.part, fgo, fgx, fin.g, it);
     } else {
       for (int64_t it = first; it < fin.items; it += stride) bx_reduce_item<T, 1>(fin.part, fgo, fgx, fin.g, it);
     }
@@ -955,11 +955,22 @@ int bw_run(const void* x, const void* y, const void* grad_out, void* grad_weight
   // 32-bit indices of the split reduction
   if ((int64_t)3 * kernel_size * kernel_size * c * (c + 1) > 0x7fffffffLL) return kUnsupported;
   WGradGeom g;
-  if (f)
+  ClWGeom cg{};
+  if (f && esz == 2) {
+    // channels-last tensors: the splits are that kernel's
+    clw_geom(cg, *f, n, c, true);
+    cg.d0 = gg.d0;
+    cg.d1 = gg.d1;
+    cg.d2 = gg.d2;
+    g.C = (int)c;
+    g.splits = cg.splits;
+    g.direct = cg.direct;
+  } else if (f)
     wgrad_geom_flat(g, *f, n, c, gg.d0, gg.d1, gg.d2, esz);
   else
     wgrad_geom(g, n, c, h, w, gg.d0, gg.d1, gg.d2, wg_step_cols(w, esz));
-  const int64_t need = wg_partial_bytes(g, c, kernel_size);
+  const int64_t need =
+      f && esz == 2 ? clw_partial_bytes(cg, kernel_size * kernel_size, true) : wg_partial_bytes(g, c, kernel_size);
   if (need > 0 && (!workspace || workspace_bytes < need)) return kWorkspaceTooSmall;
   // LDS-direct dword copies of x rows need every row to start on a dword boundary
   g.xdma = (esz == 4) || ((w % 2 == 0) && ((uintptr_t)x % 4 == 0));
@@ -971,7 +982,7 @@ int bw_run(const void* x, const void* y, const void* grad_out, void* grad_weight
   const int kk = kernel_size * kernel_size;
   if (kernel_size != 1 && kernel_size != 3) return kUnsupported;
   if (check_only) return kOk;
-  g.dw_blocks = g.splits * 3 * g.cblocks * g.ihalves;
+  g.dw_blocks = f && esz == 2 ? cg.dw_blocks : g.splits * 3 * g.cblocks * g.ihalves;
   const int helpers = (fin || yp) ? wg_helpers(g.dw_blocks) : 0;
   const BxFinish none{nullptr, nullptr, nullptr, TileGeom{}, 0, 1};
   const YPack nopack{nullptr, nullptr, 0, 0, 0};
@@ -983,6 +994,36 @@ int bw_run(const void* x, const void* y, const void* grad_out, void* grad_weight
   float* pb = g.direct ? nullptr : pw + (int64_t)g.splits * 3 * kk * c * c;
   return wg_with_type(dtype, [&](auto tag) {
     using T = decltype(tag);
+    // after the partial kernel: the halo reduction where it had no helpers,
+    // then the split reduction (launched, or described in *defer)
+    auto finish = [&](int e) {
+      if (e == 0 && fin && helpers == 0) e = bx_finish(*fin, dtype, stream);
+      if (e != 0 || g.direct) return e;
+      const int64_t total_w = (int64_t)3 * kk * c * c;
+      // four input channels per thread when the rows allow 16-byte partial
+      // loads and 4-element stores
+      const bool v4 = c % 4 == 0 && reinterpret_cast<uintptr_t>(pw) % 16 == 0 &&
+                      reinterpret_cast<uintptr_t>(grad_weight) % (4 * sizeof(T)) == 0;
+      const int64_t items = (v4 ? total_w / 4 : total_w) + 3 * kk * c;
+      if (defer) {
+        *defer = WReduce{pw, pb, grad_weight, grad_bias, (uint32_t)c, (uint32_t)kk, g.splits,
+                         v4 ? 1 : 0, (int)items};
+        return 0;
+      }
+      const dim3 rgrid((unsigned)((items + kWgRedThreads - 1) / kWgRedThreads));
+      if (v4)
+        hipLaunchKernelGGL((gen_bwd_w_reduce_kernel<T, 4>), rgrid, dim3(kWgRedThreads), 0, stream, pw,
+                           pb, (T*)grad_weight, (T*)grad_bias, (uint32_t)c, (uint32_t)kk, g.splits);
+      else
+        hipLaunchKernelGGL((gen_bwd_w_reduce_kernel<T, 1>), rgrid, dim3(kWgRedThreads), 0, stream, pw,
+                           pb, (T*)grad_weight, (T*)grad_bias, (uint32_t)c, (uint32_t)kk, g.splits);
+      return (int)hipGetLastError();
+    };
+    const BxFinish& hfin = helpers > 0 && fin ? *fin : none;
+    const YPack& hyp = helpers > 0 && yp ? *yp : nopack;
+    if (f && esz == 2)
+      return finish(clw_launch_gen(dtype, kernel_size, cg, x, y, grad_out, pw, pb, grad_weight,
+                                   grad_bias, helpers, hfin, stream));
     auto launch = [&](auto ks, auto mbc, auto sjc, auto alc) {
       constexpr int KS = decltype(ks)::value;
       constexpr int MB = decltype(mbc)::value;
@@ -1000,32 +1041,8 @@ int bw_run(const void* x, const void* y, const void* grad_out, void* grad_weight
       hipLaunchKernelGGL((gen_bwd_w_partial_kernel<T, KS, MB, SJ, AL>), grid,
                          dim3(64 * kWgSegs * WgTaps<KS>::kGroups), lds, stream, (const T*)x,
                          (const T*)y, (const T*)grad_out, pw, pb, (T*)grad_weight, (T*)grad_bias, g,
-                         helpers > 0 && fin ? *fin : none, helpers > 0 && yp ? *yp : nopack);
-      int e = (int)hipGetLastError();
-      if (e == 0 && fin && helpers == 0) e = bx_finish(*fin, dtype, stream);
-      if (e != 0 || g.direct) return e;
-      const int64_t total_w = (int64_t)3 * KKc * c * c;
-      // four input channels per thread when the rows allow 16-byte partial
-      // loads and 4-element stores
-      const bool v4 = c % 4 == 0 && reinterpret_cast<uintptr_t>(pw) % 16 == 0 &&
-                      reinterpret_cast<uintptr_t>(grad_weight) % (4 * sizeof(T)) == 0;
-      const int64_t items = (v4 ? total_w / 4 : total_w) + 3 * KKc * c;
-      if (defer) {
-        *defer = WReduce{pw, pb, grad_weight, grad_bias, (uint32_t)c, (uint32_t)KKc, g.splits,
-                         v4 ? 1 : 0, (int)items};
-        return 0;
-      }
-      if (v4)
-        hipLaunchKernelGGL((gen_bwd_w_reduce_kernel<T, 4>),
-                           dim3((unsigned)((items + kWgRedThreads - 1) / kWgRedThreads)),
-                           dim3(kWgRedThreads), 0, stream, pw, pb, (T*)grad_weight, (T*)grad_bias,
-                           (uint32_t)c, (uint32_t)KKc, g.splits);
-      else
-        hipLaunchKernelGGL((gen_bwd_w_reduce_kernel<T, 1>),
-                           dim3((unsigned)((items + kWgRedThreads - 1) / kWgRedThreads)),
-                           dim3(kWgRedThreads), 0, stream, pw, pb, (T*)grad_weight, (T*)grad_bias,
-                           (uint32_t)c, (uint32_t)KKc, g.splits);
-      return (int)hipGetLastError();
+                         hfin, hyp);
+      return finish((int)hipGetLastError());
     };
     return wg_with_mb(mb, [&](auto mbc) {
       // aligned layout (16-byte x, y and gradient rows, whole steps, whole
@@ -1035,7 +1052,9 @@ int bw_run(const void* x, const void* y, const void* grad_out, void* grad_weight
                       (c <= 64 || c == 128);
       auto by_k = [&](auto sjc) {
         auto by_al = [&](auto ks) {
-          if (f) return launch(ks, mbc, sjc, std::integral_constant<int, 2>{});
+          if constexpr (sizeof(T) == 4) {
+            if (f) return launch(ks, mbc, sjc, std::integral_constant<int, 2>{});
+          }
           if (al) return launch(ks, mbc, sjc, std::integral_constant<int, 1>{});
           return launch(ks, mbc, sjc, std::integral_constant<int, 0>{});
         };
@@ -1138,10 +1157,13 @@ int flat_bwd(FlatBwd& b, int64_t n, int64_t c, int64_t h, int64_t w, int kernel_
     return kUnsupported;
   WGradGeom g;
   wgrad_geom_flat(g, b.f, n, c, gg.d0, gg.d1, gg.d2, esz);
-  b.copy = align256(flat_elems(b.f, n * flat_planes(c)) * esz);
+  ClWGeom cg;
+  clw_geom(cg, b.f, n, c, true);
+  b.copy = align256(flat_elems(b.f, n * flat_planes(c), esz) * esz);
   b.bx = align256(ddpm_gen_bwd_x_workspace_bytes(n, c, h, w, kernel_size, d0, d1, d2));
   b.by = align256(ddpm_gen_bwd_y_workspace_bytes(c, kernel_size));
-  b.bw = align256(wg_partial_bytes(g, c, kernel_size));
+  b.bw = align256(esz == 2 ? clw_partial_bytes(cg, kernel_size * kernel_size, true)
+                           : wg_partial_bytes(g, c, kernel_size));
   return kOk;
 }
 
@@ -1184,7 +1206,7 @@ extern "C" int ddpm_flat_gen_bwd(const void* x, const void* y, const void* weigh
   }
   if (grad_y) {
     st = yt_run(xf, weight, grad_cat, grad_y, wsy, b.by, n, c, h, w, kernel_size, d0, d1, d2, dtype,
-                stream, kYtCheck, &yp);
+                stream, kYtCheck, &yp, nullptr, &b.f);
     if (st != kOk) return st;
   }
   BxFinish fin{nullptr, nullptr, nullptr, TileGeom{}, 0, 1};
@@ -1194,19 +1216,21 @@ extern "C" int ddpm_flat_gen_bwd(const void* x, const void* y, const void* weigh
     if (st != kOk) return st;
   }
   if (grad_y || need_w) {
-    const FlatCopy fc[2] = {flat_copy_of(x, xf, b.f, n, c, flat_planes(c)),
-                            flat_copy_of(y, yf, b.f, n, c, flat_planes(c))};
-    st = flat_copy(fc, need_w ? 2 : 1, b.f, dtype, stream);
+    const int esz = dtype == kF32 ? 4 : 2;
+    const FlatCopy fc[2] = {flat_copy_of(x, xf, b.f, n, c, flat_planes(c), esz),
+                            flat_copy_of(y, yf, b.f, n, c, flat_planes(c), esz)};
+    st = flat_copy(fc, need_w ? 2 : 1, b.f, dtype, stream, nullptr, grad_y ? &yp : nullptr,
+                   kernel_size);
     if (st != kOk) return st;
   }
   WReduce red{nullptr, nullptr, nullptr, nullptr, 0, 0, 0, 0, 0};
   if (need_w) {
     st = bw_run(xf, yf, grad_cat, grad_weight, grad_bias, wsw, b.bw, n, c, h, w, kernel_size, d0, d1,
-                d2, dtype, stream, false, grad_x ? &fin : nullptr, grad_y ? &yp : nullptr,
+                d2, dtype, stream, false, grad_x ? &fin : nullptr, nullptr,
                 grad_y ? &red : nullptr, &b.f);
     if (st != kOk) return st;
   }
   if (!grad_y) return kOk;
   return yt_run(xf, weight, grad_cat, grad_y, wsy, b.by, n, c, h, w, kernel_size, d0, d1, d2, dtype,
-                stream, need_w ? kYtMain : kYtFull, nullptr, &red, &b.f);
+                stream, kYtMain, nullptr, &red, &b.f);
 }

@@ -27,19 +27,19 @@
 
 namespace ddpm {
 
-template <typename T, int KS, int NK, int CB>
+template <typename T, int KS, int NK, int CB, bool CL>
 __global__ __launch_bounds__(kGtThreads) __attribute__((amdgpu_waves_per_eu(gt_waves_per_eu<T, NK, CB>()))) void gen_bwd_x_tile_kernel(
     const T* __restrict__ gout, const T* __restrict__ y, const T* __restrict__ wt,
     const T* __restrict__ bias, float* __restrict__ part, TileGeom g) {
-  gen_tile_body<T, KS, NK, CB, true>(gout, y, wt, bias, nullptr, part, g);
+  gen_tile_body<T, KS, NK, CB, true, false, CL>(gout, y, wt, bias, nullptr, part, g);
 }
 
 // One thread per item (bx_reduce_item: VEC columns of one row of dX).
-template <typename T, int VEC>
+template <typename T, int VEC, bool FL>
 __global__ __launch_bounds__(256) void gen_bwd_x_reduce_kernel(const float* __restrict__ part,
                                                                const T* __restrict__ gout,
                                                                T* __restrict__ gx, TileGeom g) {
-  bx_reduce_item<T, VEC>(part, gout, gx, g, (int64_t)blockIdx.x * 256 + threadIdx.x);
+  bx_reduce_item<T, VEC, FL>(part, gout, gx, g, (int64_t)blockIdx.x * 256 + threadIdx.x);
 }
 
 namespace {
@@ -90,12 +90,15 @@ int ddpm::bx_finish(const BxFinish& f, int dtype, hipStream_t stream) {
   return xt_with_type(dtype, [&](auto tag) {
     using T = decltype(tag);
     const dim3 rgrid((unsigned)((f.items + 255) / 256));
-    if (f.vec == 4)
-      hipLaunchKernelGGL((gen_bwd_x_reduce_kernel<T, 4>), rgrid, dim3(256), 0, stream, f.part,
-                         (const T*)f.gout, (T*)f.gx, f.g);
+    auto launch = [&](auto kern) {
+      hipLaunchKernelGGL(kern, rgrid, dim3(256), 0, stream, f.part, (const T*)f.gout, (T*)f.gx, f.g);
+    };
+    if (f.g.olead != 0)  // flat tensors start with a guard
+      launch(gen_bwd_x_reduce_kernel<T, 4, true>);
+    else if (f.vec == 4)
+      launch(gen_bwd_x_reduce_kernel<T, 4, false>);
     else
-      hipLaunchKernelGGL((gen_bwd_x_reduce_kernel<T, 1>), rgrid, dim3(256), 0, stream, f.part,
-                         (const T*)f.gout, (T*)f.gx, f.g);
+      launch(gen_bwd_x_reduce_kernel<T, 1, false>);
     return (int)hipGetLastError();
   });
 }
@@ -127,6 +130,7 @@ int ddpm::bx_run(const void* y, const void* weight, const void* bias, const void
     g.OP = f->P;
     g.OS = f->S;
     g.olead = f->lead;
+    g.oimg = (esz == 2 ? cl_cat_planes(c) : 4 * c) * (int64_t)f->S;
   }
   if (!workspace || workspace_bytes < bx_part_bytes(g)) return kWorkspaceTooSmall;
   float* part = (float*)workspace;
@@ -150,20 +154,24 @@ int ddpm::bx_run(const void* y, const void* weight, const void* bias, const void
     };
     // 1 or 2 chunks of 32 input channels, or 4 (65..128 channels, always
     // 32-column tiles; chunks past C read zeros)
-    auto pick = [&](auto ks) {
+    auto pick = [&](auto ks, auto clc) {
       constexpr int KS = decltype(ks)::value;
-      if (nk > 2) return launch(gen_bwd_x_tile_kernel<T, KS, 4, 2>);
+      constexpr bool CL = decltype(clc)::value && sizeof(T) == 2;
+      if (nk > 2) return launch(gen_bwd_x_tile_kernel<T, KS, 4, 2, CL>);
       if (cb == 4)
-        return nk == 1 ? launch(gen_bwd_x_tile_kernel<T, KS, 1, 4>)
-                       : launch(gen_bwd_x_tile_kernel<T, KS, 2, 4>);
+        return nk == 1 ? launch(gen_bwd_x_tile_kernel<T, KS, 1, 4, CL>)
+                       : launch(gen_bwd_x_tile_kernel<T, KS, 2, 4, CL>);
       if (cb == 1)
-        return nk == 1 ? launch(gen_bwd_x_tile_kernel<T, KS, 1, 1>)
-                       : launch(gen_bwd_x_tile_kernel<T, KS, 2, 1>);
-      return nk == 1 ? launch(gen_bwd_x_tile_kernel<T, KS, 1, 2>)
-                     : launch(gen_bwd_x_tile_kernel<T, KS, 2, 2>);
+        return nk == 1 ? launch(gen_bwd_x_tile_kernel<T, KS, 1, 1, CL>)
+                       : launch(gen_bwd_x_tile_kernel<T, KS, 2, 1, CL>);
+      return nk == 1 ? launch(gen_bwd_x_tile_kernel<T, KS, 1, 2, CL>)
+                     : launch(gen_bwd_x_tile_kernel<T, KS, 2, 2, CL>);
     };
-    if (kernel_size == 1) return pick(std::integral_constant<int, 1>());
-    return pick(std::integral_constant<int, 3>());
+    auto by_k = [&](auto clc) {
+      if (kernel_size == 1) return pick(std::integral_constant<int, 1>(), clc);
+      return pick(std::integral_constant<int, 3>(), clc);
+    };
+    return f ? by_k(std::true_type()) : by_k(std::false_type());
   });
 }
 

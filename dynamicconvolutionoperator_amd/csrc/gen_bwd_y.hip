@@ -27,7 +27,7 @@
 //   * v_mfma_f32_16x16x32_{bf16,f16}; fp32 operands run as three bf16
 //     products (hi*hi + hi*lo + lo*hi).
 
-#include "gen_bwd.h"
+#include "cl_conv.h"
 
 #include <atomic>
 #include <mutex>
@@ -56,9 +56,9 @@ struct YGeom {
 template <typename T, int KS, int MB>
 __global__ __launch_bounds__(256) void gen_pack_wt_kernel(const T* __restrict__ wt,
                                                           uint32_t* __restrict__ pk, int C,
-                                                          int nc32, int total) {
+                                                          int nc32, int total, int nat) {
   const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx < total) yt_pack_item<T, KS, MB>(wt, pk, C, nc32, idx);
+  if (idx < total) yt_pack_item<T, KS, MB>(wt, pk, C, nc32, idx, nat);
 }
 
 // One LDS staging buffer (dwords): x rows [CH * 32 channels][kXS] then the
@@ -415,9 +415,15 @@ void yt_split(int64_t c, int& ihalves, int& mb) {
   mb = c > 64 ? 4 : (int)((c + 15) / 16);
 }
 
+// The same for the channels-last kernel (1, 2 or 4 blocks).
+void yt_split_cl(int64_t c, int& ihalves, int& mb) {
+  yt_split(c, ihalves, mb);
+  if (mb == 3) mb = 4;
+}
+
 int64_t yt_pack_bytes(int64_t c, int k, int dtype) {
   int ih, mb;
-  yt_split(c, ih, mb);
+  yt_split_cl(c, ih, mb);  // (at least as large as the plane-major kernel's)
   const int64_t nc32 = (c + 31) / 32;
   return (int64_t)ih * 3 * nc32 * k * k * mb * (dtype == kF32 ? 2 : 1) * 64 * 16;
 }
@@ -510,10 +516,17 @@ int ddpm::yt_run(const void* x, const void* weight, const void* grad_out, void* 
   const int64_t need = yt_pack_bytes(c, kernel_size, dtype);
   if (!workspace || workspace_bytes < need) return kWorkspaceTooSmall;
   if (kernel_size != 1 && kernel_size != 3) return kUnsupported;
+  const bool cl = f && dtype != kF32;
   if (mode == kYtCheck) {
     if (pack) {
       int ih, mb;
-      yt_split(c, ih, mb);
+      if (cl) {
+        yt_split_cl(c, ih, mb);
+        pack->nat = 1;
+      } else {
+        yt_split(c, ih, mb);
+      }
+      pack->mb = mb;
       pack->total = ih * 3 * pack->nc32 * kernel_size * kernel_size * mb * 64;
     }
     return kOk;
@@ -523,8 +536,7 @@ int ddpm::yt_run(const void* x, const void* weight, const void* grad_out, void* 
 }
 
 int ddpm::yt_pack(const YPack& p, int kernel_size, int dtype, hipStream_t stream) {
-  int ih, mb;
-  yt_split(p.C, ih, mb);
+  const int mb = p.mb;
   return yt_with_type(dtype, [&](auto tag) {
     using T = decltype(tag);
     return yt_with_mb(mb, [&](auto mbc) {
@@ -532,10 +544,10 @@ int ddpm::yt_pack(const YPack& p, int kernel_size, int dtype, hipStream_t stream
       const dim3 grid((unsigned)((p.total + 255) / 256));
       if (kernel_size == 1)
         hipLaunchKernelGGL((gen_pack_wt_kernel<T, 1, MB>), grid, dim3(256), 0, stream,
-                           (const T*)p.wt, p.pk, p.C, p.nc32, p.total);
+                           (const T*)p.wt, p.pk, p.C, p.nc32, p.total, p.nat);
       else
         hipLaunchKernelGGL((gen_pack_wt_kernel<T, 3, MB>), grid, dim3(256), 0, stream,
-                           (const T*)p.wt, p.pk, p.C, p.nc32, p.total);
+                           (const T*)p.wt, p.pk, p.C, p.nc32, p.total, p.nat);
       return (int)hipGetLastError();
     });
   });
@@ -589,6 +601,40 @@ int yt_launch(const void* x, const void* weight, const void* grad_out, void* gra
   g.f = f ? *f : FlatLay{};
   if (f) g.col_tiles = f->ft;
   int mb;
+  if (f && dtype != kF32) {
+    yt_split_cl(c, g.ihalves, mb);
+    const int k2 = kernel_size * kernel_size;
+    if (pack) {
+      YPack yp{weight, (uint32_t*)workspace, (int)c, g.nc32, g.ihalves * 3 * g.nc32 * k2 * mb * 64};
+      yp.mb = mb;
+      yp.nat = 1;
+      const int e = yt_pack(yp, kernel_size, dtype, stream);
+      if (e != 0) return e;
+    }
+    ClConvGeom cg{};
+    cg.N = g.N;
+    cg.M = g.C;
+    cg.H = g.H;
+    cg.W = g.W;
+    cg.f = *f;
+    cg.q = g.cp / 16;
+    cg.in_img = (int64_t)g.cp * f->S;
+    cg.nc32 = g.nc32;
+    cg.nb = 3;
+    cg.d0 = g.d0;
+    cg.d1 = g.d1;
+    cg.d2 = g.d2;
+    cg.mgroups = g.ihalves;
+    cg.gs = cg.gs_per = (g.nc32 + 1) / 2;
+    cg.ks = 1;
+    cg.out = kClOutImage;
+    cg.C = g.C;
+    cg.out_img = cl_cat_planes(c) * f->S;
+    const WReduce none{nullptr, nullptr, nullptr, nullptr, 0, 0, 0, 0, 0};
+    return cl_conv_launch(dtype, 1, kernel_size, mb, cg, x, grad_out, workspace, nullptr, grad_y,
+                          nullptr, CwReduce{nullptr, nullptr, nullptr, nullptr, 0, 0, 0, 0, 0},
+                          red ? *red : none, stream);
+  }
   yt_split(c, g.ihalves, mb);
   const int64_t tiles = n * (f ? 1 : h) * g.col_tiles * g.ihalves;  // below 2^31 (yt_check)
   return yt_with_type(dtype, [&](auto tag) {
@@ -603,13 +649,14 @@ int yt_launch(const void* x, const void* weight, const void* grad_out, void* gra
           const int units = g.ihalves * 3 * g.nc32 * KS * KS * MB * 64;
           hipLaunchKernelGGL((gen_pack_wt_kernel<T, KS, MB>), dim3((units + 255) / 256), dim3(256),
                              0, stream, (const T*)weight, (uint32_t*)workspace, (int)c, g.nc32,
-                             units);
+                             units, 0);
           int e = (int)hipGetLastError();
           if (e != 0) return e;
         }
         const size_t lds = (size_t)2 * L::kBuf * 4;
         // aligned layout: 16-byte x rows and whole 32-channel chunks
-        auto kern = f                      ? gen_bwd_y_kernel<T, KS, MB, CH, 2>
+        constexpr int FLC = sizeof(T) == 4 ? 2 : 0;  // (2-byte flat tensors: above)
+        auto kern = f                      ? gen_bwd_y_kernel<T, KS, MB, CH, FLC>
                     : g.x4 && c % 32 == 0 ? gen_bwd_y_kernel<T, KS, MB, CH, 1>
                                           : gen_bwd_y_kernel<T, KS, MB, CH>;
         const int ae = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds);

@@ -21,23 +21,13 @@ namespace ddpm {
 // CB = 4: 256 registers per lane (one 8-wave workgroup per CU, whose 133 KB
 // halo tile fills the LDS anyway); CB = 2: 128 registers, two workgroups per
 // CU, unless the y operand needs more (gt_waves_per_eu).
-// PP: the concat as pair planes (kF32Pairs, fp32 only).
-template <typename T, int KS, int NK, int CB, bool PP = false>
+// PP: the concat as pair planes (kF32Pairs, fp32 only); CL: channels-last in
+// a flat layout (2-byte types).
+template <typename T, int KS, int NK, int CB, bool PP = false, bool CL = false>
 __global__ __launch_bounds__(kGtThreads) __attribute__((amdgpu_waves_per_eu(gt_waves_per_eu<T, NK, CB>()))) void gen_fwd_kernel(
     const T* __restrict__ x, const T* __restrict__ y, const T* __restrict__ wt,
     const T* __restrict__ bias, T* __restrict__ out, TileGeom g, CvPack fpk, FlatZero zero) {
-  gen_tile_body<T, KS, NK, CB, false, PP>(x, y, wt, bias, out, nullptr, g, fpk, zero);
-}
-
-// Two fp32 values rounded to nearest-even in T (bf16 / f16), packed low/high.
-template <typename T>
-__device__ __forceinline__ uint32_t pack2(float a, float b) {
-  if constexpr (sizeof(T) == 2 && __is_same(T, bf16)) {
-    return pack_bf16x2(a, b);
-  } else {
-    typedef f16 f16x2 __attribute__((ext_vector_type(2)));
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){a, b}, f16x2));
-  }
+  gen_tile_body<T, KS, NK, CB, false, PP, CL>(x, y, wt, bias, out, nullptr, g, fpk, zero);
 }
 
 // a.lo * b.lo + a.hi * b.hi + c on packed T pairs (v_dot2_f32_bf16 / _f16).
@@ -65,7 +55,7 @@ __device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float c) {
 // straight from the weight rows; C % 8 == 0) stays in LDS, so the loop has no
 // barrier.  The x halo tile, the identity channels and the y operand are
 // the tile kernels' (gen_tile.h).
-template <typename T, int NK, int CB>
+template <typename T, int NK, int CB, bool CL>
 __global__ __launch_bounds__(kGtThreads) __attribute__((amdgpu_waves_per_eu(gt_waves_per_eu<T, NK, CB>()))) void gen_fwd_pair_kernel(
     const T* __restrict__ x, const T* __restrict__ y, const T* __restrict__ wt,
     const T* __restrict__ bias, T* __restrict__ out, TileGeom g, CvPack fpk, FlatZero zero) {
@@ -107,7 +97,7 @@ __global__ __launch_bounds__(kGtThreads) __attribute__((amdgpu_waves_per_eu(gt_w
 
   // x halo tile first (its loads are consumed here); then the bias rows, the
   // weight slices and the y operand, all in flight together
-  gt_stage_x<T, XB, CB>(x, out, xs, g, n, c0, nch, h0, w0, TW, tid);
+  gt_stage_x<T, XB, CB, false, CL>(x, out, xs, g, n, c0, nch, h0, w0, TW, tid);
   // ---- bias rows [ps][mb*16 + m], written to LDS at the end of the prologue
   static_assert(NPS * 32 <= kGtThreads, "one bias value per thread");
   uint32_t bv;
@@ -145,7 +135,7 @@ __global__ __launch_bounds__(kGtThreads) __attribute__((amdgpu_waves_per_eu(gt_w
   // ddpm_gen_fwd_pack: this workgroup's share of the fuse convolution's
   // weight packing
   if (fpk.total > 0) cv_pack_share<T>(fpk, (int)blockIdx.x, (int)gridDim.x, tid, kGtThreads);
-  if (zero.base) flat_zero_share<T>(zero, (int)blockIdx.x, (int)gridDim.x, tid, kGtThreads);
+  if constexpr (CL) flat_zero_share<T>(zero, (int)blockIdx.x, (int)gridDim.x, tid, kGtThreads);
   __builtin_amdgcn_s_waitcnt(0);  // the LDS-direct weight copies
   __syncthreads();
 
@@ -223,14 +213,32 @@ __global__ __launch_bounds__(kGtThreads) __attribute__((amdgpu_waves_per_eu(gt_w
     }
     if (j == NPB - 1) {
       // ---- branch b: channels c0 + 8mb + 2q + e of output block b+1
-      const BufRes bres = make_buf(out + ((int64_t)n * 4 * C + (int64_t)(b + 1) * C + c0) * OS,
-                                   (uint32_t)nch * OSE);
+      if constexpr (CL) {
+        // channels-last: two channels per store
+        const BufRes cres = make_buf(out + n * g.oimg, (uint32_t)(4 * C) * OSE);
 #pragma unroll
-      for (int blk = 0; blk < NBW; ++blk)
+        for (int blk = 0; blk < NBW; ++blk) {
+          const int gh = h0 + 2 * wave + blk / CB, gw = w0 + 16 * (blk % CB) + col16;
+          const uint32_t pos = (uint32_t)(gh * OP + gw);
 #pragma unroll
-        for (int mb = 0; mb < 2; ++mb)
+          for (int mb = 0; mb < 2; ++mb) {
+            const int cl = 8 * mb + 2 * quad, pl = (b + 1) * C + c0 + cl;
+            const uint32_t o = gh < H && gw < W && cl < nch
+                                   ? (((uint32_t)(pl >> 4) * g.OS + pos) * 16u + (uint32_t)(pl & 15)) * 2u
+                                   : kOob;
+            __builtin_amdgcn_raw_buffer_store_b32(pack2<T>(acc[blk][mb][0], acc[blk][mb][1]), cres, o, 0, 0);
+          }
+        }
+      } else {
+        const BufRes bres = make_buf(out + n * g.oimg + ((int64_t)(b + 1) * C + c0) * OS,
+                                     (uint32_t)nch * OSE);
 #pragma unroll
-          for (int e = 0; e < 2; ++e) buf_store1<T>(bres, goff(blk, mb, e), acc[blk][mb][e]);
+        for (int blk = 0; blk < NBW; ++blk)
+#pragma unroll
+          for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+            for (int e = 0; e < 2; ++e) buf_store1<T>(bres, goff(blk, mb, e), acc[blk][mb][e]);
+      }
     }
   }
 }
@@ -322,7 +330,8 @@ int gf_run(const void* x, const void* y, const void* weight, const void* bias, v
   if (f) {
     g.OP = f->P;
     g.OS = f->S;
-    g.olead = f->lead;
+    g.olead = (esz == 2 ? 16 : 1) * f->lead;
+    g.oimg = 4 * c * (int64_t)f->S;
     zero = FlatZero{out, *f, (int)(n * 4 * c)};
   }
   // 2-byte types at K = 3 with up to 64 channels (C % 8 == 0, aligned
@@ -342,9 +351,15 @@ int gf_run(const void* x, const void* y, const void* weight, const void* bias, v
                              (const T*)weight, (const T*)bias, (T*)out, g, pk, zero);
           return (int)hipGetLastError();
         };
-        if (cb == 4) return nk == 1 ? launch(gen_fwd_pair_kernel<T, 1, 4>) : launch(gen_fwd_pair_kernel<T, 2, 4>);
-        if (cb == 2) return nk == 1 ? launch(gen_fwd_pair_kernel<T, 1, 2>) : launch(gen_fwd_pair_kernel<T, 2, 2>);
-        return nk == 1 ? launch(gen_fwd_pair_kernel<T, 1, 1>) : launch(gen_fwd_pair_kernel<T, 2, 1>);
+        auto pick = [&](auto clc) {
+          constexpr bool CL = decltype(clc)::value;
+          if (cb == 4)
+            return nk == 1 ? launch(gen_fwd_pair_kernel<T, 1, 4, CL>) : launch(gen_fwd_pair_kernel<T, 2, 4, CL>);
+          if (cb == 2)
+            return nk == 1 ? launch(gen_fwd_pair_kernel<T, 1, 2, CL>) : launch(gen_fwd_pair_kernel<T, 2, 2, CL>);
+          return nk == 1 ? launch(gen_fwd_pair_kernel<T, 1, 1, CL>) : launch(gen_fwd_pair_kernel<T, 2, 1, CL>);
+        };
+        return f ? pick(std::true_type()) : pick(std::false_type());
       } else {
         return (int)kBadArgument;
       }
@@ -362,24 +377,26 @@ int gf_run(const void* x, const void* y, const void* weight, const void* bias, v
     };
     // 1 or 2 chunks of 32 input channels, or 4 (65..128 channels; chunks
     // past C read zeros)
-    auto pick = [&](auto ks, auto ppc) {
+    auto pick = [&](auto ks, auto ppc, auto clc) {
       constexpr int KS = decltype(ks)::value;
       constexpr bool PP = decltype(ppc)::value && sizeof(T) == 4;
+      constexpr bool CL = decltype(clc)::value && sizeof(T) == 2;
       if (nk > 2) {
-        return launch(gen_fwd_kernel<T, KS, 4, 2, PP>);  // 32-column tiles
+        return launch(gen_fwd_kernel<T, KS, 4, 2, PP, CL>);  // 32-column tiles
       }
       if (cb == 4)
-        return nk == 1 ? launch(gen_fwd_kernel<T, KS, 1, 4, PP>) : launch(gen_fwd_kernel<T, KS, 2, 4, PP>);
+        return nk == 1 ? launch(gen_fwd_kernel<T, KS, 1, 4, PP, CL>) : launch(gen_fwd_kernel<T, KS, 2, 4, PP, CL>);
       if (cb == 1)
-        return nk == 1 ? launch(gen_fwd_kernel<T, KS, 1, 1, PP>) : launch(gen_fwd_kernel<T, KS, 2, 1, PP>);
-      return nk == 1 ? launch(gen_fwd_kernel<T, KS, 1, 2, PP>) : launch(gen_fwd_kernel<T, KS, 2, 2, PP>);
+        return nk == 1 ? launch(gen_fwd_kernel<T, KS, 1, 1, PP, CL>) : launch(gen_fwd_kernel<T, KS, 2, 1, PP, CL>);
+      return nk == 1 ? launch(gen_fwd_kernel<T, KS, 1, 2, PP, CL>) : launch(gen_fwd_kernel<T, KS, 2, 2, PP, CL>);
     };
-    auto by_k = [&](auto ppc) {
-      if (kernel_size == 1) return pick(std::integral_constant<int, 1>(), ppc);
-      if (kernel_size == 3) return pick(std::integral_constant<int, 3>(), ppc);
-      return pick(std::integral_constant<int, 5>(), ppc);
+    auto by_k = [&](auto ppc, auto clc) {
+      if (kernel_size == 1) return pick(std::integral_constant<int, 1>(), ppc, clc);
+      if (kernel_size == 3) return pick(std::integral_constant<int, 3>(), ppc, clc);
+      return pick(std::integral_constant<int, 5>(), ppc, clc);
     };
-    return pp ? by_k(std::true_type()) : by_k(std::false_type());
+    if (pp) return by_k(std::true_type(), std::false_type());
+    return f ? by_k(std::false_type(), std::true_type()) : by_k(std::false_type(), std::false_type());
   });
 }
 

@@ -33,6 +33,8 @@
 
 #include "conv3x3.h"
 
+#include <type_traits>
+
 namespace ddpm {
 
 constexpr int kGtWaves = 8;
@@ -57,6 +59,7 @@ struct TileGeom {
   // elements before its first plane (W, H * W and 0, or a flat layout's)
   int OP;
   uint32_t OS, olead;
+  int64_t oimg;  // elements from one image of it to the next
 };
 
 // Waves per SIMD the tile kernels are compiled for: two (256 registers per
@@ -102,6 +105,7 @@ inline int tile_geom(TileGeom& f, const GenGeom& g, int entry, int parts, int cb
   f.OP = g.W;
   f.OS = (uint32_t)((int64_t)g.H * g.W);
   f.olead = 0;
+  f.oimg = (int64_t)4 * g.C * f.OS;
   // planes start on 256-byte boundaries: the four quads of a wave then read
   // their 4-channel entries with the fewest LDS bank conflicts (measured)
   f.plane = (f.npix * entry + 255) / 256 * 256;
@@ -178,7 +182,8 @@ __device__ __forceinline__ void gf_store_raw(BufRes r, uint32_t off, uint32_t v)
 // PP (fp32 only): the identity channels go to `out` as pair planes
 // (kF32Pairs): channels (c, c+1) of a 32-plane chunk as one hi and one lo
 // plane, 16 planes apart; C % 16 == 0.
-template <typename T, int XB, int CB, bool PP = false>
+// CL (2-byte types): they go out channels-last.
+template <typename T, int XB, int CB, bool PP = false, bool CL = false>
 __device__ __forceinline__ void gt_stage_x(const T* __restrict__ a, T* __restrict__ out,
                                            unsigned char* __restrict__ xs, const TileGeom& g,
                                            int n, int c0, int nch, int h0, int w0, int TW,
@@ -193,8 +198,8 @@ __device__ __forceinline__ void gt_stage_x(const T* __restrict__ a, T* __restric
   const BufRes xres = make_buf(a + ((int64_t)n * C + c0) * HW, (uint32_t)nch * HWE);
   const int64_t OS = g.OS;
   const uint32_t OSE = g.OS * (uint32_t)E;  // bytes of one concat plane
-  const BufRes ores = PP ? make_buf(out + ((int64_t)n * 4 * C + (c0 & ~31)) * OS, 32u * OSE)
-                        : make_buf(out + ((int64_t)n * 4 * C + c0) * OS, (uint32_t)nch * OSE);
+  const BufRes ores = PP ? make_buf(out + n * g.oimg + (c0 & ~31) * OS, 32u * OSE)
+                        : make_buf(out + n * g.oimg + c0 * OS, (uint32_t)(CL ? 16 : nch) * OSE);
   const uint32_t pp0 = (uint32_t)((c0 & 31) >> 1);  // PP: pair index of channels (c0, c0+1)
   if (g.vec) {
     // a task = (4-channel plane, halo row, 4 image columns a multiple of 4
@@ -253,8 +258,13 @@ __device__ __forceinline__ void gt_stage_x(const T* __restrict__ a, T* __restric
             q[1] = __builtin_amdgcn_perm(v[u][3][m >> 1], v[u][2][m >> 1], sel);
           }
           *reinterpret_cast<XQ*>(xs + grp * g.plane + (i * LW + j) * XB) = q;
+          if constexpr (CL) {
+            // the identity channels are 16-channel block c0 / 16
+            if (i >= R && i < R + kGtTH && j >= R && j < R + TW && oof[u] != kOob && 4 * grp < nch)
+              __builtin_amdgcn_raw_buffer_store_b64(q, ores, 16u * (oof[u] + 2u * m) + 8u * grp, 0, 0);
+          }
         }
-        if (i >= R && i < R + kGtTH && 4 * k >= cpos && 4 * k < cpos + TW) {
+        if (!CL && i >= R && i < R + kGtTH && 4 * k >= cpos && 4 * k < cpos + TW) {
           if constexpr (PP) {
             // channels (4grp + 2kp, +1): their 4 columns split into a hi and a lo vector
 #pragma unroll
@@ -317,6 +327,18 @@ __device__ __forceinline__ void gt_stage_x(const T* __restrict__ a, T* __restric
             const uint32_t o = so[s] == kOob ? kOob : so[s] + (pp0 + kp) * OSE;
             __builtin_amdgcn_raw_buffer_store_b32(hh, ores, o, 0, 0);
             __builtin_amdgcn_raw_buffer_store_b32(ll, ores, o == kOob ? kOob : o + 16u * OSE, 0, 0);
+          }
+      } else if constexpr (CL) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+          for (int h8 = 0; h8 < 2; ++h8) {
+            u32x4 o;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              o[e] = v[s][8 * h8 + 2 * e] | (v[s][8 * h8 + 2 * e + 1] << 16);
+            const uint32_t ob = so[s] != kOob && 8 * h8 < nch ? 16u * so[s] + 16u * h8 : kOob;
+            __builtin_amdgcn_raw_buffer_store_b128(o, ores, ob, 0, 0);
           }
       } else {
 #pragma unroll
@@ -381,7 +403,9 @@ __device__ __forceinline__ void gt_load_y(const T* __restrict__ y,
 // own partial (c + R + pad) and in its left / right neighbour's (c + R + pad
 // -/+ TW), and the 4-column groups that a neighbour's halo only partly covers
 // read zeros for the rest.
-template <typename T, int KS, int NK, int CB, bool BX, bool PP = false>
+// CL (2-byte types): the concat is channels-last (cl.h) in a flat layout.  A
+// template argument: as a branch it slowed the plain layouts' kernels by 2%.
+template <typename T, int KS, int NK, int CB, bool BX, bool PP = false, bool CL = false>
 __device__ __forceinline__ void gen_tile_body(const T* __restrict__ a, const T* __restrict__ y,
                                               const T* __restrict__ wt, const T* __restrict__ bias,
                                               T* __restrict__ out, float* __restrict__ part,
@@ -505,7 +529,7 @@ __device__ __forceinline__ void gen_tile_body(const T* __restrict__ a, const T* 
     // the x halo tile first (its loads are consumed there), then the bias
     // rows, the first weight slice and the y operand with their loads in
     // flight together
-    gt_stage_x<T, XB, CB, PP>(a, out, xs, g, n, c0, nch, h0, w0, TW, tid);
+    gt_stage_x<T, XB, CB, PP, CL>(a, out, xs, g, n, c0, nch, h0, w0, TW, tid);
     bias_load();
     wload(0);
     gt_load_y<T, NK, CB>(y, bfr, g, n, h0, w0, wave, col16, quad);
@@ -515,7 +539,9 @@ __device__ __forceinline__ void gen_tile_body(const T* __restrict__ a, const T* 
     // ddpm_gen_fwd_pack: this workgroup's share of the fuse convolution's
     // weight packing
     if (fpk.total > 0) cv_pack_share<T>(fpk, (int)blockIdx.x, (int)gridDim.x, tid, kGtThreads);
-    if (zero.base) flat_zero_share<T>(zero, (int)blockIdx.x, (int)gridDim.x, tid, kGtThreads);
+    if constexpr (E == 4 || CL) {
+      if (zero.base) flat_zero_share<T>(zero, (int)blockIdx.x, (int)gridDim.x, tid, kGtThreads);
+    }
   }
   __syncthreads();
 
@@ -554,8 +580,29 @@ __device__ __forceinline__ void gen_tile_body(const T* __restrict__ a, const T* 
       if (bt + 2 < NBT) wload(bt + 2);
     }
     if constexpr (BX) {
-      if (t == 0) {
-        const BufRes gres = make_buf(a + ((int64_t)n * 4 * C + (int64_t)(b + 1) * C + c0) * OS,
+      if (CL && t == 0) {
+        // channels-last branch gradients (behind the x-planes): this lane's 4
+        // channels in one load
+        const BufRes gres =
+            make_buf(a + n * g.oimg + C * OS, (uint32_t)((3 * C + 15) / 16) * 16u * OSE);
+        const int j = b * C + c0 + 4 * quad;
+#pragma unroll
+        for (int blk = 0; blk < NBW; ++blk) {
+          const int gh = h0 + 2 * wave + blk / CB, gw = w0 + 16 * (blk % CB) + col16;
+          const uint32_t o =
+              gh < H && gw < W && 4 * quad < nch
+                  ? (((uint32_t)(j >> 4) * g.OS + (uint32_t)(gh * OP + gw)) * 16u + (uint32_t)(j & 15)) * 2u
+                  : kOob;
+          typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+          const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(gres, o, 0, 0);
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            go[blk][e] = to_f(__builtin_bit_cast(
+                typename std::conditional<E == 2, T, uint16_t>::type,
+                (unsigned short)(v[e >> 1] >> (16 * (e & 1)))));
+        }
+      } else if (t == 0) {
+        const BufRes gres = make_buf(a + n * g.oimg + ((int64_t)(b + 1) * C + c0) * OS,
                                      (uint32_t)nch * OSE);
         uint32_t lo[CB];
 #pragma unroll
@@ -635,7 +682,7 @@ __device__ __forceinline__ void gen_tile_body(const T* __restrict__ a, const T* 
         // ---- branch b as pair planes: channels (4quad + 2kp, +1) of output
         //      block b+1, split, to the hi / lo planes of their 32-plane chunk
         const int chb = (b + 1) * C + c0;
-        const BufRes pres = make_buf(out + ((int64_t)n * 4 * C + (chb & ~31)) * OS, 32u * OSE);
+        const BufRes pres = make_buf(out + n * g.oimg + (chb & ~31) * OS, 32u * OSE);
         const uint32_t pbase = (uint32_t)(((chb & 31) >> 1) + 2 * quad);
         // the lane's column offsets, formed here (kept out of registers across
         // the loop, as lofs is for the plain stores)
@@ -659,9 +706,25 @@ __device__ __forceinline__ void gen_tile_body(const T* __restrict__ a, const T* 
             __builtin_amdgcn_raw_buffer_store_b32(ll, pres, ok ? o + 16u * OSE : kOob, 0, 0);
           }
         }
+      } else if (CL && t == KK - 1) {
+        // ---- branch b, channels-last: this lane's 4 channels in one store
+        const BufRes bres = make_buf(out + n * g.oimg, (uint32_t)(4 * C) * OSE);
+        const int pl = (b + 1) * C + c0 + 4 * quad;
+#pragma unroll
+        for (int blk = 0; blk < NBW; ++blk) {
+          const int gh = h0 + 2 * wave + blk / CB, gw = w0 + 16 * (blk % CB) + col16;
+          const uint32_t o =
+              gh < H && gw < W && 4 * quad < nch
+                  ? (((uint32_t)(pl >> 4) * g.OS + (uint32_t)(gh * OP + gw)) * 16u + (uint32_t)(pl & 15)) * 2u
+                  : kOob;
+          typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+          __builtin_amdgcn_raw_buffer_store_b64((u32x2){pack2<T>(acc[blk][0], acc[blk][1]),
+                                                        pack2<T>(acc[blk][2], acc[blk][3])},
+                                                bres, o, 0, 0);
+        }
       } else if (t == KK - 1) {
         // ---- branch b: channels c0 + 4*quad + e of output block b+1
-        const BufRes bres = make_buf(out + ((int64_t)n * 4 * C + (int64_t)(b + 1) * C + c0) * OS,
+        const BufRes bres = make_buf(out + n * g.oimg + ((int64_t)(b + 1) * C + c0) * OS,
                                      (uint32_t)nch * OSE);
         uint32_t lo[CB];
 #pragma unroll

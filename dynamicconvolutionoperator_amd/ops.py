@@ -670,17 +670,20 @@ def _cat_code(dtype: torch.dtype) -> int:
 
 def _flat_guard(x, k, dil, code, training) -> int:
     """Guard rows and columns of the flat concat (``ddpm_flat_*``: rows padded
-    to a 16-byte pitch, tiles of 256 positions whatever the width) that this
-    shape takes between generator and fuse convolution, or 0 for the plain
-    one.  Plain rows win where they are whole steps of the kernels (fp32 /
-    bf16 C = 64: training 1x128x128 204 / 144 us plain, 230 / 158 flat;
-    inference 4x64x64 51 / 39 plain, 53 / 41 flat); every other width leaves
-    lanes idle at row ends (training 1x160x160 333 / 231 us plain, 281 / 193
-    flat, 8x64x64 390 / 262 plain, 327 / 206 flat) or, not a multiple of 8,
-    is staged element by element (bf16 training 2x135x181 1034 us plain, 251
-    flat)."""
+    with zeros, tiles of 256 positions whatever the width; 2-byte types
+    channels-last) that this shape takes between generator and fuse
+    convolution, or 0 for the plain one.  Plain rows win where they are whole
+    steps of the kernels (C = 64 training: fp32 1x128x128 204 us plain, 230
+    flat, bf16 4x128x128 317 / 335, 8x256x256 1971 / 2015); every other width
+    leaves lanes idle at row ends (8x64x64 fp32 390 plain, 327 flat, bf16 272 /
+    200) or, not a multiple of 8, is staged element by element (bf16
+    2x135x181 1034 us plain).  Inference has no copies to pay for: 2-byte types
+    take the flat concat at 32, 64 and 128 columns too (1x128x128 39.9 us
+    plain, 35.9 flat), fp32 does not (51 / 53)."""
     n, c, h, w = x.shape
-    if w % 256 == 0 or w == 128 or (not training and w in (32, 64)):
+    if w % 256 == 0 or (w == 128 and (training or x.dtype == torch.float32)):
+        return 0
+    if not training and x.dtype == torch.float32 and w in (32, 64):
         return 0
     guard = max(1, (k // 2) * max(dil)) if training else 1
     return guard if _ws_bytes("ddpm_flat_cat_elems", n, c, h, w, guard, code) > 0 else 0

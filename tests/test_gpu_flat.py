@@ -16,7 +16,8 @@ pytestmark = pytest.mark.gpu
 # channel counts below and between the 16-, 32- and 64-channel blocks
 SHAPES = [
     (1, 16, 1, 5), (2, 16, 15, 17), (1, 32, 3, 251), (1, 48, 9, 249), (3, 64, 20, 30),
-    (1, 64, 31, 257), (2, 96, 11, 35), (1, 128, 24, 40),
+    (1, 64, 31, 257), (2, 96, 11, 35), (1, 128, 24, 40), (1, 24, 30, 50), (2, 40, 17, 8),
+    (1, 64, 70, 300),
 ]
 
 
@@ -50,6 +51,8 @@ def test_flat_training_matches_oracle(shape, dtype):
     grads = torch.autograd.grad(out, (xg, yg, *mod.parameters()), g.to(DEV))
     grads_ref = torch.autograd.grad(out_ref, (xr, yr, *ref.parameters()), g.double())
     assert_close(out, out_ref, *TOL["module_fwd"][dtype], "out")
+    with torch.no_grad():  # (its layout has one guard row, the training one five)
+        assert_close(mod(xg, yg), out_ref, *TOL["module_fwd"][dtype], "inference")
     atol, rtol = TOL["module_bwd"][dtype]
     for name, a, e in zip(("dx", "dy", "dgw", "dgb", "dfw", "dfb"), grads, grads_ref):
         assert_close(a, e, atol * max(e.abs().max().item(), 1e-6), rtol, name)
