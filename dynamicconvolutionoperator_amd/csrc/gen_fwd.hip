@@ -43,6 +43,19 @@ __device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float c) {
   }
 }
 
+// Exchanges between the wave's rows of 16 lanes: rows 2, 3 of a with rows 0, 1
+// of b; rows 1, 3 of a with rows 0, 2 of b.
+__device__ __forceinline__ void swap_rows32(uint32_t& a, uint32_t& b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+  a = r[0];
+  b = r[1];
+}
+__device__ __forceinline__ void swap_rows16(uint32_t& a, uint32_t& b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+  a = r[0];
+  b = r[1];
+}
+
 // Forward for 2-byte types at K = 3 with the taps paired in the MFMA rows.
 // The generator rows of a step are 8 channels x 2 taps (row m: channel
 // c0 + 8*mb + m/2, tap 2j + m%2; the fifth pair of a branch holds tap 8 and a
@@ -138,6 +151,7 @@ __global__ __launch_bounds__(kGtThreads) __attribute__((amdgpu_waves_per_eu(gt_w
   if constexpr (CL) flat_zero_share<T>(zero, (int)blockIdx.x, (int)gridDim.x, tid, kGtThreads);
   __builtin_amdgcn_s_waitcnt(0);  // the LDS-direct weight copies
   __syncthreads();
+  if constexpr (CL) gt_store_identity<T, CB>(out, xs, g, n, c0, nch, h0, w0, tid);
 
   // x entry of this lane's two channels (8mb + 2q, +1) at its block-0 pixel:
   // plane 2mb + q/2, bytes 4*(q%2) .. +3 of the 4-channel entry
@@ -214,19 +228,37 @@ __global__ __launch_bounds__(kGtThreads) __attribute__((amdgpu_waves_per_eu(gt_w
     if (j == NPB - 1) {
       // ---- branch b: channels c0 + 8mb + 2q + e of output block b+1
       if constexpr (CL) {
-        // channels-last: two channels per store
+        // channels-last.  A lane holds 2 of a pixel's 8 channels per row block;
+        // swapping rows of 16 lanes between four pixel blocks gives lane row
+        // q the 8 channels of block q's pixels, one 16-byte store (two blocks:
+        // lane rows q and q + 2 hold 4 channels each of block q % 2, 8 bytes)
         const BufRes cres = make_buf(out + n * g.oimg, (uint32_t)(4 * C) * OSE);
 #pragma unroll
-        for (int blk = 0; blk < NBW; ++blk) {
-          const int gh = h0 + 2 * wave + blk / CB, gw = w0 + 16 * (blk % CB) + col16;
-          const uint32_t pos = (uint32_t)(gh * OP + gw);
+        for (int mb = 0; mb < 2; ++mb) {
+          const int cl = 8 * mb, pl = (b + 1) * C + c0 + cl;
+          const uint32_t base = (uint32_t)(pl >> 4) * g.OS * 32u + (uint32_t)(pl & 15) * 2u;
+          constexpr int Q = NBW < 4 ? 2 : 4;  // pixel blocks per exchange
 #pragma unroll
-          for (int mb = 0; mb < 2; ++mb) {
-            const int cl = 8 * mb + 2 * quad, pl = (b + 1) * C + c0 + cl;
+          for (int b0 = 0; b0 < NBW; b0 += Q) {
+            const int blk = b0 + (quad & (Q - 1));
+            const int gh = h0 + 2 * wave + blk / CB, gw = w0 + 16 * (blk % CB) + col16;
             const uint32_t o = gh < H && gw < W && cl < nch
-                                   ? (((uint32_t)(pl >> 4) * g.OS + pos) * 16u + (uint32_t)(pl & 15)) * 2u
+                                   ? base + (uint32_t)(gh * OP + gw) * 32u + (Q == 4 ? 0u : 8u * (quad >> 1))
                                    : kOob;
-            __builtin_amdgcn_raw_buffer_store_b32(pack2<T>(acc[blk][mb][0], acc[blk][mb][1]), cres, o, 0, 0);
+            uint32_t d[Q];
+#pragma unroll
+            for (int i = 0; i < Q; ++i) d[i] = pack2<T>(acc[b0 + i][mb][0], acc[b0 + i][mb][1]);
+            if constexpr (Q == 4) {
+              swap_rows32(d[0], d[2]);
+              swap_rows32(d[1], d[3]);
+              swap_rows16(d[0], d[1]);
+              swap_rows16(d[2], d[3]);
+              __builtin_amdgcn_raw_buffer_store_b128((u32x4){d[0], d[1], d[2], d[3]}, cres, o, 0, 0);
+            } else {
+              swap_rows16(d[0], d[1]);
+              typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+              __builtin_amdgcn_raw_buffer_store_b64((u32x2){d[0], d[1]}, cres, o, 0, 0);
+            }
           }
         }
       } else {

@@ -182,7 +182,7 @@ __device__ __forceinline__ void gf_store_raw(BufRes r, uint32_t off, uint32_t v)
 // PP (fp32 only): the identity channels go to `out` as pair planes
 // (kF32Pairs): channels (c, c+1) of a 32-plane chunk as one hi and one lo
 // plane, 16 planes apart; C % 16 == 0.
-// CL (2-byte types): they go out channels-last.
+// CL (2-byte types): the identity channels are left to gt_store_identity.
 template <typename T, int XB, int CB, bool PP = false, bool CL = false>
 __device__ __forceinline__ void gt_stage_x(const T* __restrict__ a, T* __restrict__ out,
                                            unsigned char* __restrict__ xs, const TileGeom& g,
@@ -199,7 +199,7 @@ __device__ __forceinline__ void gt_stage_x(const T* __restrict__ a, T* __restric
   const int64_t OS = g.OS;
   const uint32_t OSE = g.OS * (uint32_t)E;  // bytes of one concat plane
   const BufRes ores = PP ? make_buf(out + n * g.oimg + (c0 & ~31) * OS, 32u * OSE)
-                        : make_buf(out + n * g.oimg + c0 * OS, (uint32_t)(CL ? 16 : nch) * OSE);
+                        : make_buf(out + n * g.oimg + c0 * OS, (uint32_t)nch * OSE);
   const uint32_t pp0 = (uint32_t)((c0 & 31) >> 1);  // PP: pair index of channels (c0, c0+1)
   if (g.vec) {
     // a task = (4-channel plane, halo row, 4 image columns a multiple of 4
@@ -258,11 +258,6 @@ __device__ __forceinline__ void gt_stage_x(const T* __restrict__ a, T* __restric
             q[1] = __builtin_amdgcn_perm(v[u][3][m >> 1], v[u][2][m >> 1], sel);
           }
           *reinterpret_cast<XQ*>(xs + grp * g.plane + (i * LW + j) * XB) = q;
-          if constexpr (CL) {
-            // the identity channels are 16-channel block c0 / 16
-            if (i >= R && i < R + kGtTH && j >= R && j < R + TW && oof[u] != kOob && 4 * grp < nch)
-              __builtin_amdgcn_raw_buffer_store_b64(q, ores, 16u * (oof[u] + 2u * m) + 8u * grp, 0, 0);
-          }
         }
         if (!CL && i >= R && i < R + kGtTH && 4 * k >= cpos && 4 * k < cpos + TW) {
           if constexpr (PP) {
@@ -328,19 +323,7 @@ __device__ __forceinline__ void gt_stage_x(const T* __restrict__ a, T* __restric
             __builtin_amdgcn_raw_buffer_store_b32(hh, ores, o, 0, 0);
             __builtin_amdgcn_raw_buffer_store_b32(ll, ores, o == kOob ? kOob : o + 16u * OSE, 0, 0);
           }
-      } else if constexpr (CL) {
-#pragma unroll
-        for (int s = 0; s < 2; ++s)
-#pragma unroll
-          for (int h8 = 0; h8 < 2; ++h8) {
-            u32x4 o;
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-              o[e] = v[s][8 * h8 + 2 * e] | (v[s][8 * h8 + 2 * e + 1] << 16);
-            const uint32_t ob = so[s] != kOob && 8 * h8 < nch ? 16u * so[s] + 16u * h8 : kOob;
-            __builtin_amdgcn_raw_buffer_store_b128(o, ores, ob, 0, 0);
-          }
-      } else {
+      } else if constexpr (!CL) {
 #pragma unroll
         for (int s = 0; s < 2; ++s)
 #pragma unroll
@@ -363,6 +346,33 @@ __device__ __forceinline__ void gt_stage_x(const T* __restrict__ a, T* __restric
         }
       }
     }
+  }
+}
+
+// The tile's own pixels of the staged x (2-byte types) -> the identity
+// channels of a channels-last concat, 16-channel block c0 / 16: a task = (pixel,
+// 8 channels), one 16-byte store, so that a wave's store is 1 KB in a run
+// (from the staging registers it was 8-byte pieces 128 bytes apart).  After the
+// barrier that ends the staging.
+template <typename T, int CB>
+__device__ __forceinline__ void gt_store_identity(T* __restrict__ out,
+                                                  const unsigned char* __restrict__ xs,
+                                                  const TileGeom& g, int n, int c0, int nch, int h0,
+                                                  int w0, int tid) {
+  constexpr int TW = 16 * CB;
+  typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+  const BufRes ores = make_buf(out + n * g.oimg + c0 * (int64_t)g.OS, g.OS * 32u);
+#pragma unroll
+  for (int u = tid; u < kGtTH * TW * 2; u += kGtThreads) {
+    const int h8 = u & 1, c = (u >> 1) % TW, rr = (u >> 1) / TW;
+    const unsigned char* __restrict__ src =
+        xs + 2 * h8 * g.plane + ((rr + g.R) * g.LW + c + g.R) * 8;
+    const u32x2 a = *reinterpret_cast<const u32x2*>(src);
+    const u32x2 b = *reinterpret_cast<const u32x2*>(src + g.plane);
+    const uint32_t o = h0 + rr < g.H && w0 + c < g.W && 8 * h8 < nch
+                           ? (uint32_t)((h0 + rr) * g.OP + w0 + c) * 32u + 16u * h8
+                           : kOob;
+    __builtin_amdgcn_raw_buffer_store_b128((u32x4){a[0], a[1], b[0], b[1]}, ores, o, 0, 0);
   }
 }
 
@@ -544,6 +554,7 @@ __device__ __forceinline__ void gen_tile_body(const T* __restrict__ a, const T* 
     }
   }
   __syncthreads();
+  if constexpr (CL && !BX) gt_store_identity<T, CB>(out, xs, g, n, c0, nch, h0, w0, tid);
 
   // Addresses inside the loop are a lane part, kept in a few registers, plus
   // a part uniform over the wave; the asm barriers below keep the compiler
