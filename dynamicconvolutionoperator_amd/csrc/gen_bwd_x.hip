@@ -152,12 +152,14 @@ int ddpm::bx_run(const void* y, const void* weight, const void* bias, const void
       }
       return bx_finish(fin, dtype, stream);
     };
-    // 1 or 2 chunks of 32 input channels, or 4 (65..128 channels, always
-    // 32-column tiles; chunks past C read zeros)
+    // 1 to 4 chunks of 32 input channels (more than 64 channels: always
+    // 32-column tiles)
     auto pick = [&](auto ks, auto clc) {
       constexpr int KS = decltype(ks)::value;
       constexpr bool CL = decltype(clc)::value && sizeof(T) == 2;
-      if (nk > 2) return launch(gen_bwd_x_tile_kernel<T, KS, 4, 2, CL>);
+      if (nk > 2)
+        return nk == 3 ? launch(gen_bwd_x_tile_kernel<T, KS, 3, 2, CL>)
+                       : launch(gen_bwd_x_tile_kernel<T, KS, 4, 2, CL>);
       if (cb == 4)
         return nk == 1 ? launch(gen_bwd_x_tile_kernel<T, KS, 1, 4, CL>)
                        : launch(gen_bwd_x_tile_kernel<T, KS, 2, 4, CL>);

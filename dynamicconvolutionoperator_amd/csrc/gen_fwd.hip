@@ -366,11 +366,42 @@ int gf_run(const void* x, const void* y, const void* weight, const void* bias, v
     g.oimg = 4 * c * (int64_t)f->S;
     zero = FlatZero{out, *f, (int)(n * 4 * c)};
   }
-  // 2-byte types at K = 3 with up to 64 channels (C % 8 == 0, aligned
-  // weight): taps paired in the MFMA rows, every weight slice resident in LDS
-  const size_t lds_pair = (size_t)4 * g.plane + (size_t)15 * 2 * nk * 64 * 16 + (size_t)15 * 32 * 4;
-  const bool pair = esz == 2 && kernel_size == 3 && nk <= 2 && c % 8 == 0 &&
-                    (uintptr_t)weight % 16 == 0 && lds_pair <= (size_t)kGtMaxLds;
+  // 2-byte types at K = 3 (C % 8 == 0, aligned weight): taps paired in the
+  // MFMA rows, every weight slice resident in LDS, where that leaves room for
+  // the halo tile
+  auto pair_lds = [&](const TileGeom& t) {
+    return (size_t)4 * t.plane + (size_t)15 * 2 * nk * 64 * 16 + (size_t)15 * 32 * 4;
+  };
+  size_t lds_pair = pair_lds(g);
+  bool pair = esz == 2 && kernel_size == 3 && c % 8 == 0 && (uintptr_t)weight % 16 == 0;
+  if (pair && nk > 2) {
+    // one workgroup per CU (the weights take 92 or 123 KB): the tile width
+    // with the shortest run of rounds, a workgroup taking about 1 + cb.  f16
+    // at three chunks and 64 columns spills (184 us, 32 columns 152 us at
+    // 4x96x150x211; bf16's 256 registers just hold it, 151 us).  The kernel
+    // with one tap per step and 128 channels' padding took 219 us there
+    // (bf16), and 158 us against 117 us at 1x128x256x256.
+    pair = false;
+    int64_t best = 0;
+    for (int tcb = dtype == kF16 ? 2 : 4; tcb >= 1; tcb /= 2) {
+      TileGeom t;
+      size_t tl;
+      if (tile_geom(t, gg, 4 * esz, parts, tcb, tl) != kOk || pair_lds(t) > (size_t)kGtMaxLds) continue;
+      const int64_t cost =
+          ((int64_t)t.N * t.tiles * t.cblocks + kGtFillWGs - 1) / kGtFillWGs * (1 + tcb);
+      if (pair && cost >= best) continue;
+      pair = true;
+      best = cost;
+      cb = tcb;
+      t.OP = g.OP;
+      t.OS = g.OS;
+      t.olead = g.olead;
+      t.oimg = g.oimg;
+      lds_pair = pair_lds(t);
+      g = t;
+    }
+  }
+  pair = pair && lds_pair <= (size_t)kGtMaxLds;
   if (pair) {
     return with_type(dtype, [&](auto tag) {
       using T = decltype(tag);
@@ -385,11 +416,18 @@ int gf_run(const void* x, const void* y, const void* weight, const void* bias, v
         };
         auto pick = [&](auto clc) {
           constexpr bool CL = decltype(clc)::value;
-          if (cb == 4)
-            return nk == 1 ? launch(gen_fwd_pair_kernel<T, 1, 4, CL>) : launch(gen_fwd_pair_kernel<T, 2, 4, CL>);
-          if (cb == 2)
-            return nk == 1 ? launch(gen_fwd_pair_kernel<T, 1, 2, CL>) : launch(gen_fwd_pair_kernel<T, 2, 2, CL>);
-          return nk == 1 ? launch(gen_fwd_pair_kernel<T, 1, 1, CL>) : launch(gen_fwd_pair_kernel<T, 2, 1, CL>);
+          auto by_nk = [&](auto cbc) {
+            constexpr int CB = decltype(cbc)::value;
+            if (nk == 1) return launch(gen_fwd_pair_kernel<T, 1, CB, CL>);
+            if (nk == 2) return launch(gen_fwd_pair_kernel<T, 2, CB, CL>);
+            if (nk == 3)  // (f16: at most 32 columns)
+              return launch(gen_fwd_pair_kernel<T, 3, CB == 4 && __is_same(T, f16) ? 2 : CB, CL>);
+            // (64-column tiles do not fit the LDS beside four chunks' weights)
+            return launch(gen_fwd_pair_kernel<T, 4, CB == 4 ? 2 : CB, CL>);
+          };
+          if (cb == 4) return by_nk(std::integral_constant<int, 4>());
+          if (cb == 2) return by_nk(std::integral_constant<int, 2>());
+          return by_nk(std::integral_constant<int, 1>());
         };
         return f ? pick(std::true_type()) : pick(std::false_type());
       } else {
@@ -407,15 +445,13 @@ int gf_run(const void* x, const void* y, const void* weight, const void* bias, v
                          (const T*)weight, (const T*)bias, (T*)out, g, pk, zero);
       return (int)hipGetLastError();
     };
-    // 1 or 2 chunks of 32 input channels, or 4 (65..128 channels; chunks
-    // past C read zeros)
+    // 1 to 4 chunks of 32 input channels
     auto pick = [&](auto ks, auto ppc, auto clc) {
       constexpr int KS = decltype(ks)::value;
       constexpr bool PP = decltype(ppc)::value && sizeof(T) == 4;
       constexpr bool CL = decltype(clc)::value && sizeof(T) == 2;
-      if (nk > 2) {
-        return launch(gen_fwd_kernel<T, KS, 4, 2, PP, CL>);  // 32-column tiles
-      }
+      if (nk > 2)  // 32-column tiles
+        return nk == 3 ? launch(gen_fwd_kernel<T, KS, 3, 2, PP, CL>) : launch(gen_fwd_kernel<T, KS, 4, 2, PP, CL>);
       if (cb == 4)
         return nk == 1 ? launch(gen_fwd_kernel<T, KS, 1, 4, PP, CL>) : launch(gen_fwd_kernel<T, KS, 2, 4, PP, CL>);
       if (cb == 1)

@@ -63,22 +63,23 @@ struct TileGeom {
 };
 
 // Waves per SIMD the tile kernels are compiled for: two (256 registers per
-// lane) for the 64-column tile and for 65..128 input channels (NK = 4: the y
-// operand alone takes 64 registers per 2-byte column block pair, 128 for
-// fp32), else four.
+// lane) for the 64-column tile and for more than 64 input channels (NK > 2:
+// the y operand alone takes 16 registers per chunk, 32 for fp32; forced into
+// 128 registers, two workgroups per CU, the input gradient of 128 channels
+// went from 69 to 115 us at fp16 2x128x96x96), else four.
 template <typename T, int NK, int CB>
 constexpr int gt_waves_per_eu() {
-  return (CB == 4 || NK == 4) ? 2 : 4;
+  return (CB == 4 || NK > 2) ? 2 : 4;
 }
 
 // Column blocks of 16 pixels per tile row the tile kernels try first: the y
-// operand of the 64-column tile with more than 64 input channels (NK = 4)
+// operand of the 64-column tile with more than 64 input channels (NK > 2)
 // would not fit the registers, so those use 32 columns.
 inline int gt_first_cb(int nk) { return nk > 2 ? 2 : 4; }
 
-// Chunks of 32 input channels the tile kernels are instantiated for: 1, 2,
-// or 4 for 65..128 channels (chunks past C hold zeros).
-inline int gt_nk(int c) { return c <= 32 ? 1 : (c <= 64 ? 2 : 4); }
+// Chunks of 32 input channels the tile kernels are instantiated for (the last
+// one's channels past C hold zeros).
+inline int gt_nk(int c) { return (c + 31) / 32; }
 
 // Tiling and LDS bytes for a tile of 16 x 16*cb pixels whose LDS tile holds
 // `entry` bytes per 4-channel pixel and whose weight slices have `parts`

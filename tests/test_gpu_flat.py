@@ -96,3 +96,25 @@ def test_stand_alone_fuse_conv_copies_flat(shape, dtype):
     atol, rtol = TOL["module_bwd"][dtype]
     for name, a, e in zip(("dcat", "dw", "db"), got, want):
         assert_close(a, e, atol * e.abs().max().item(), rtol, name)
+
+
+# more than 64 channels: (c, h, w) whose grids take each tile width of the
+# paired forward (16, 32 and 64 columns beside three chunks' weights, 16 and
+# 32 beside four's) with a ragged last chunk, tile row and tile column, and a
+# channel count the paired forward does not take
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("shape", [
+    (72, 33, 40), (72, 45, 397), (72, 99, 397), (104, 20, 37), (120, 30, 395), (72, 97, 384), (76, 20, 37),
+])
+def test_wide_modules_match_oracle(shape, dtype):
+    c, h, w = shape
+    say(f"wide inference {shape} {dtype}")
+    ref, mod = _modules(c, 3, dtype)
+    x, y = (randn((1, c, h, w), s, dtype=dtype) for s in (1, 2))
+    with torch.no_grad():
+        out_ref = ref(x.double(), y.double())
+        assert_close(mod(x.to(DEV), y.to(DEV)), out_ref, *TOL["module_fwd"][dtype], "module")
+        cat = ops.fused_generator_dynamic_cat(x.to(DEV), y.to(DEV), mod.generator.weight,
+                                              mod.generator.bias, 3, DIL)
+        out = torch.nn.functional.conv2d(cat.double().cpu(), ref.fuse.weight, ref.fuse.bias, padding=1)
+        assert_close(out, out_ref, *TOL["module_fwd"][dtype], "plain concat")
