@@ -342,6 +342,7 @@ void clw_geom(ClWGeom& g, const FlatLay& f, int64_t n, int64_t c, bool generator
   const int64_t steps = n * f.ft;
   int64_t splits = 16;
   if (splits > (steps + kClwMinSteps - 1) / kClwMinSteps) splits = (steps + kClwMinSteps - 1) / kClwMinSteps;
+  splits = wgrad_splits(splits, steps, (int64_t)g.blocks * g.halves);
   g.steps = (int)steps;
   g.steps_per_split = (int)((steps + splits - 1) / splits);
   g.splits = (int)((steps + g.steps_per_split - 1) / g.steps_per_split);

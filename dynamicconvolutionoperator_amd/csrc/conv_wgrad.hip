@@ -10,7 +10,7 @@
 // place of y.  Work decomposition (CDNA4):
 //   * one workgroup per (pixel split, 16-plane block of ci, and above 64
 //     output planes half of the co planes): at most 16
-//     splits of at least 4 steps -- a step is one image-row segment of 128
+//     splits (wgrad_splits) of at least 4 steps -- a step is one image-row segment of 128
 //     columns -- (16 splits x 16 blocks = 256 workgroups at C = 64, 256x256);
 //     their fp32 partials are summed in split order by a second kernel
 //     (deterministic, no atomics); a single split writes the gradients
@@ -617,7 +617,7 @@ void cw_geom(CwGeom& g, int64_t n, int64_t c, int64_t h, int64_t w, int tw) {
   const int64_t steps = n * h * g.col_blocks;
   int64_t splits = kCwMaxSplits;
   if (splits > (steps + kCwMinSteps - 1) / kCwMinSteps) splits = (steps + kCwMinSteps - 1) / kCwMinSteps;
-  if (splits < 1) splits = 1;
+  splits = wgrad_splits(splits < 1 ? 1 : splits, steps, (int64_t)g.cblocks * g.ohalves);
   g.steps = (int)steps;
   g.steps_per_split = (int)((steps + splits - 1) / splits);
   g.splits = (int)((steps + g.steps_per_split - 1) / g.steps_per_split);

@@ -420,4 +420,23 @@ inline int64_t flat_elems(const FlatLay& f, int64_t planes, int esz) {
 // not on every launch.  Returns 0 or the hipError_t of the attribute call.
 int allow_dynamic_lds(const void* fn, size_t bytes);
 
+// Splits (at most `most`) of a weight gradient's `steps`, `blocks` workgroups
+// each and one workgroup per CU: the number with the shortest run of rounds
+// over 256 CUs, a workgroup's start and end taking about four steps.  Up to 64
+// channels all 16 splits fit one round; 36 blocks (96 channels) x 16 would be
+// 2.25 rounds, 14 are two (generator's / convolution's weight gradient, us,
+// 16 splits -> these: bf16 1x96x200x256 109 -> 76 / 86 -> 71, fp16
+// 2x128x96x96 46 -> 33 / 37 -> 31, fp32 1x128x192x256 172 -> 170 / 199 -> 187).
+inline int64_t wgrad_splits(int64_t most, int64_t steps, int64_t blocks) {
+  int64_t best = most, cost = 0;
+  for (int64_t s = most; s >= 1; --s) {
+    const int64_t per = (steps + s - 1) / s, used = (steps + per - 1) / per;
+    const int64_t c = (used * blocks + 255) / 256 * (per + 4);
+    if (cost != 0 && c >= cost) continue;
+    best = s;
+    cost = c;
+  }
+  return best;
+}
+
 }  // namespace ddpm

@@ -11,7 +11,8 @@
 // Work decomposition (CDNA4): one workgroup per (token split, branch b,
 // 16-channel block of c, and above 64 channels half of the input channels i).  Splits are equal ranges of steps -- one step is
 // one row segment of 128 columns -- at most 16 of them (the reference's
-// bound, :1001-1005) and at least 4 steps each (16 splits x 3 branches x 4
+// bound, :1001-1005; above 64 channels those that fill whole rounds of CUs,
+// wgrad_splits) and at least 4 steps each (16 splits x 3 branches x 4
 // channel blocks = 192 workgroups at C = 64, 256x256); they write fp32
 // partials that a second kernel sums in a fixed order (deterministic, no
 // atomics), and a single split writes grad_weight / grad_bias directly.  Everything a step reads -- the K rows
@@ -870,7 +871,7 @@ void wgrad_geom(WGradGeom& g, int64_t n, int64_t c, int64_t h, int64_t w, int d0
   const int64_t steps = n * h * g.col_blocks;
   int64_t splits = kWgMaxSplits;
   if (splits > (steps + kWgMinSteps - 1) / kWgMinSteps) splits = (steps + kWgMinSteps - 1) / kWgMinSteps;
-  if (splits < 1) splits = 1;
+  splits = wgrad_splits(splits < 1 ? 1 : splits, steps, (int64_t)3 * g.cblocks * g.ihalves);
   g.steps = (int)steps;
   g.steps_per_split = (int)((steps + splits - 1) / splits);
   g.splits = (int)((steps + g.steps_per_split - 1) / g.steps_per_split);

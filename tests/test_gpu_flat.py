@@ -36,11 +36,24 @@ def _modules(c, k, dtype):
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("shape", SHAPES)
 def test_flat_training_matches_oracle(shape, dtype):
+    _check_training(shape, dtype, 5)
+
+
+# wide modules whose weight gradients take fewer splits than their steps allow
+# (two rounds of workgroups instead of a third partly filled one): flat, and
+# plain rows
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("shape,guard", [((2, 96, 60, 66), 5), ((1, 96, 34, 256), 0), ((1, 128, 25, 256), 0)])
+def test_wide_training_matches_oracle(shape, guard, dtype):
+    _check_training(shape, dtype, guard)
+
+
+def _check_training(shape, dtype, guard):
     n, c, h, w = shape
-    say(f"flat training {shape} {dtype}")
+    say(f"training {shape} {dtype}")
     ref, mod = _modules(c, 3, dtype)
     x, y, g = (randn(shape, s, dtype=dtype) for s in (1, 2, 3))
-    assert ops._flat_guard(x, 3, DIL, ops._cat_code(dtype), True) == 5
+    assert ops._flat_guard(x, 3, DIL, ops._cat_code(dtype), True) == guard
     xg, yg = (t.to(DEV).requires_grad_() for t in (x, y))
     xr, yr = (t.double().requires_grad_() for t in (x, y))
     # memory that no kernel writes holds NaN
