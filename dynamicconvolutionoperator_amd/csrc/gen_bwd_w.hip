@@ -51,6 +51,7 @@ struct WGradGeom {
   int tw;              // columns per step: kWgTW, or 2 * kWgTW (wg_step_cols)
   int col_blocks;      // ceil(W / tw)
   int splits;
+  int ws_splits;  // splits the workspace is sized for (at least `splits`)
   int steps;           // N * H * col_blocks
   int steps_per_split;
   int direct;          // one split: write grad_weight / grad_bias directly
@@ -871,7 +872,10 @@ void wgrad_geom(WGradGeom& g, int64_t n, int64_t c, int64_t h, int64_t w, int d0
   const int64_t steps = n * h * g.col_blocks;
   int64_t splits = kWgMaxSplits;
   if (splits > (steps + kWgMinSteps - 1) / kWgMinSteps) splits = (steps + kWgMinSteps - 1) / kWgMinSteps;
-  splits = wgrad_splits(splits < 1 ? 1 : splits, steps, (int64_t)3 * g.cblocks * g.ihalves);
+  if (splits < 1) splits = 1;
+  // (the most the steps allow: what callers reserve does not depend on the rule)
+  g.ws_splits = (int)((steps + (steps + splits - 1) / splits - 1) / ((steps + splits - 1) / splits));
+  splits = wgrad_splits(splits, steps, (int64_t)3 * g.cblocks * g.ihalves);
   g.steps = (int)steps;
   g.steps_per_split = (int)((steps + splits - 1) / splits);
   g.splits = (int)((steps + g.steps_per_split - 1) / g.steps_per_split);
@@ -895,8 +899,8 @@ void wgrad_geom_flat(WGradGeom& g, const FlatLay& f, int64_t n, int64_t c, int d
 
 // Workspace: the fp32 split partials (none with one split).
 int64_t wg_partial_bytes(const WGradGeom& g, int64_t c, int k) {
-  if (g.direct) return 0;
-  return (int64_t)g.splits * 3 * k * k * c * (c + 1) * (int64_t)sizeof(float);
+  if (g.ws_splits == 1) return 0;
+  return (int64_t)g.ws_splits * 3 * k * k * c * (c + 1) * (int64_t)sizeof(float);
 }
 
 }  // namespace
