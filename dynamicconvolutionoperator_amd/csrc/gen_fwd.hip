@@ -380,10 +380,12 @@ int gf_run(const void* x, const void* y, const void* weight, const void* bias, v
     // at three chunks and 64 columns spills (184 us, 32 columns 152 us at
     // 4x96x150x211; bf16's 256 registers just hold it, 151 us).  The kernel
     // with one tap per step and 128 channels' padding took 219 us there
-    // (bf16), and 158 us against 117 us at 1x128x256x256.
+    // (bf16), and 158 us against 117 us at 1x128x256x256.  At four chunks 64
+    // columns fit the LDS with dilations (1, 1, 1) only: no kernel is built
+    // for them.
     pair = false;
     int64_t best = 0;
-    for (int tcb = dtype == kF16 ? 2 : 4; tcb >= 1; tcb /= 2) {
+    for (int tcb = nk == 4 || dtype == kF16 ? 2 : 4; tcb >= 1; tcb /= 2) {
       TileGeom t;
       size_t tl;
       if (tile_geom(t, gg, 4 * esz, parts, tcb, tl) != kOk || pair_lds(t) > (size_t)kGtMaxLds) continue;
@@ -420,10 +422,14 @@ int gf_run(const void* x, const void* y, const void* weight, const void* bias, v
             constexpr int CB = decltype(cbc)::value;
             if (nk == 1) return launch(gen_fwd_pair_kernel<T, 1, CB, CL>);
             if (nk == 2) return launch(gen_fwd_pair_kernel<T, 2, CB, CL>);
-            if (nk == 3)  // (f16: at most 32 columns)
-              return launch(gen_fwd_pair_kernel<T, 3, CB == 4 && __is_same(T, f16) ? 2 : CB, CL>);
-            // (64-column tiles do not fit the LDS beside four chunks' weights)
-            return launch(gen_fwd_pair_kernel<T, 4, CB == 4 ? 2 : CB, CL>);
+            // (the tile is the geometry's: one that has no kernel is refused)
+            if constexpr (CB < 4 || !__is_same(T, f16)) {
+              if (nk == 3) return launch(gen_fwd_pair_kernel<T, 3, CB, CL>);
+            }
+            if constexpr (CB < 4) {
+              if (nk == 4) return launch(gen_fwd_pair_kernel<T, 4, CB, CL>);
+            }
+            return (int)kUnsupported;
           };
           if (cb == 4) return by_nk(std::integral_constant<int, 4>());
           if (cb == 2) return by_nk(std::integral_constant<int, 2>());

@@ -6,8 +6,9 @@ import pytest
 import torch
 
 from dynamicconvolutionoperator_amd import DDPM, ops
+from oracle import unfold_ref
 from oracle.unfold_ref import UnfoldDDPM
-from tests.gpu_helpers import DEV, DIL, TOL, assert_close, randn, say
+from tests.gpu_helpers import DEV, DIL, TOL, assert_close, default_generator_params, randn, say
 
 pytestmark = pytest.mark.gpu
 
@@ -131,3 +132,27 @@ def test_wide_modules_match_oracle(shape, dtype):
                                               mod.generator.bias, 3, DIL)
         out = torch.nn.functional.conv2d(cat.double().cpu(), ref.fuse.weight, ref.fuse.bias, padding=1)
         assert_close(out, out_ref, *TOL["module_fwd"][dtype], "plain concat")
+
+
+def _nan_memory():
+    """Leaves NaN in the memory that the allocator hands out next, in its
+    large and its small blocks."""
+    junk = [torch.full((1 << 24,), float("nan"), device=DEV)]
+    junk += [torch.full((1 << 17,), float("nan"), device=DEV) for _ in range(64)]
+    del junk
+
+
+# 104 to 128 channels at a halo of one pixel, where a 64-column tile fits the
+# LDS and takes the fewest rounds of workgroups, but no kernel has that tile
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("c,w", [(104, 256), (128, 256), (120, 250)])
+def test_wide_forward_at_unit_dilations(c, w, dtype):
+    shape, dil = (1, c, 128, w), (1, 1, 1)
+    say(f"unit dilations {shape} {dtype}")
+    x, y = randn(shape, 1, dtype), randn(shape, 2, dtype)
+    wt, b = default_generator_params(c, 3, 3, dtype)
+    _nan_memory()
+    out = ops.fused_generator_dynamic_cat(x.to(DEV), y.to(DEV), wt.to(DEV), b.to(DEV), 3, dil)
+    kernels = unfold_ref.generated_kernels(y.double(), wt.double(), b.double(), 3).to(dtype).double()
+    atol, rtol = TOL["gen_fwd"][dtype]
+    assert_close(out, unfold_ref.dynamic_cat(x.double(), kernels, 3, dil), atol, rtol, "concat")
