@@ -1243,7 +1243,9 @@ extern "C" int ddpm_flat_fuse_conv_bwd(const void* cat, const void* weight, cons
   void* wsw = ws + b.go + b.data;
   const FlatCopy fc = flat_copy_of(grad_out, go, f, n, c, b.cp, dtype == kF32 ? 4 : 2);
   const CvPack pack = cv_pack_of(b.plan, weight, wsd, 1, false);
-  st = flat_copy(&fc, 1, f, dtype, stream, grad_cat ? &pack : nullptr);
+  const FlatGradZero zero = flat_grad_zero(grad_cat, f, n, c, dtype == kF32 ? 4 : 2);
+  st = flat_copy(&fc, 1, f, dtype, stream, grad_cat ? &pack : nullptr, nullptr, 0,
+                 grad_cat ? &zero : nullptr);
   if (st != kOk) return st;
   CwReduce red{nullptr, nullptr, nullptr, nullptr, 0, 0, 0, 0, 0};
   if (need_w) {

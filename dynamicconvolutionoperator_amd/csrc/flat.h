@@ -90,14 +90,81 @@ __device__ __forceinline__ void flat_copy_chunk(const FlatCopy& t, const FlatLay
   }
 }
 
+// Zeroing of the elements of a concat's flat gradient that the input gradient's
+// tiles do not cover: the lead, the guard rows after each plane's last tile
+// and, for 2-byte elements, the channels past 3C of the last 16-channel block
+// and what the buffer holds past the last image.  No kernel reads them, but
+// the gradient is a tensor that autograd hands on, and its checks (NaN
+// detection, hooks) read all of it.  One item = 16 bytes.
+struct FlatGradZero {
+  void* base;       // null: nothing to do
+  uint32_t n, c;    // images, channels
+  uint32_t runs;    // tails per image, in planes: C (or 4C) plane-major ones, then the blocks' 16 each
+  uint32_t tail;    // items of one plane's tail
+  uint32_t lead;    // items of the lead
+  uint32_t spare;   // items per image of the last block's spare channels
+  uint32_t end;     // items past the last image
+  uint32_t items;   // in all
+};
+
+inline FlatGradZero flat_grad_zero(void* grad, const FlatLay& f, int64_t n, int64_t c, int esz) {
+  const uint32_t ve = 16 / (uint32_t)esz;  // (lead, S and the tiles are multiples of 8 elements)
+  const bool cl = esz == 2;
+  FlatGradZero z{grad, (uint32_t)n, (uint32_t)c, 0, 0, 0, 0, 0, 0};
+  z.runs = (uint32_t)(cl ? cl_cat_planes(c) : 4 * c);
+  z.tail = (f.S - flat_span(f)) / ve;
+  z.lead = f.lead / ve;
+  z.spare = cl && 3 * c % 16 != 0 ? flat_span(f) : 0;
+  z.end = cl ? 15 * f.lead / ve : 0;
+  z.items = z.lead + z.end + z.n * (z.runs * z.tail + z.spare);
+  return z;
+}
+
+template <typename T>
+__device__ __forceinline__ void flat_grad_zero_item(const FlatGradZero& z, const FlatLay& f,
+                                                    uint32_t i) {
+  constexpr uint32_t VE = 16 / (uint32_t)sizeof(T);
+  T* __restrict__ base = static_cast<T*>(z.base);
+  const uint32_t FS = flat_span(f);
+  const size_t img = (size_t)z.runs * f.S;
+  size_t o;  // element
+  if (i < z.lead) {
+    o = (size_t)i * VE;
+  } else if ((i -= z.lead) < z.end) {
+    o = f.lead + z.n * img + (size_t)i * VE;
+  } else {
+    i -= z.end;
+    const uint32_t per = z.runs * z.tail + z.spare;
+    const uint32_t n = i / per, k = i - n * per;
+    o = f.lead + n * img;
+    if (k < z.runs * z.tail) {
+      const uint32_t pl = k / z.tail;
+      uint32_t e = k - pl * z.tail;
+      if (sizeof(T) == 2 && pl >= z.c) {
+        // a block's tail is one run of 16 planes' tails
+        const uint32_t blk = (pl - z.c) / 16;
+        e += (pl - z.c - 16 * blk) * z.tail;
+        o += (size_t)(z.c + 16 * blk) * f.S + (size_t)FS * 16 + (size_t)e * VE;
+      } else {
+        o += (size_t)pl * f.S + FS + (size_t)e * VE;
+      }
+    } else {
+      o += (size_t)(z.runs - 16) * f.S + (size_t)(k - z.runs * z.tail) * 16 + 8;
+    }
+  }
+  *reinterpret_cast<u32x4*>(base + o) = (u32x4){0u, 0u, 0u, 0u};
+}
+
 struct CvPack;
 struct YPack;
 
 // Lays out `count` (1 or 2) tensors of `dtype` and the same n, H, W flat in one
 // launch, whose first workgroups run a weight packing of the launches that
-// follow (optional; ypack: kernel size `ks`).  Defined in flat.hip.
+// follow (optional; ypack: kernel size `ks`) and whose last ones zero the rest
+// of the gradient that those write (optional).  Defined in flat.hip.
 int flat_copy(const FlatCopy* t, int count, const FlatLay& f, int dtype, hipStream_t stream,
-              const CvPack* cpack = nullptr, const YPack* ypack = nullptr, int ks = 0);
+              const CvPack* cpack = nullptr, const YPack* ypack = nullptr, int ks = 0,
+              const FlatGradZero* zero = nullptr);
 
 // Zeroing of the elements of a flat tensor (`planes` planes in all) that lie
 // outside the images, shared out over the workgroups of the launch that

@@ -374,7 +374,8 @@ int ddpm_flat_fuse_conv_fwd_packed(const void* cat, const void* bias, void* out,
                                    int64_t w, int guard, int dtype, hipStream_t stream);
 
 /* ddpm_fuse_conv_bwd of a flat concat; grad_cat is flat (plain fp32 for dtype
- * 3), its elements outside the images unspecified beyond the rows' pads.
+ * 3; all ddpm_flat_cat_elems elements are written, those outside the images
+ * with zero).
  * grad_cat, or grad_weight and grad_bias together, may be NULL: not computed. */
 int64_t ddpm_flat_fuse_conv_bwd_workspace_bytes(int64_t n, int64_t c, int64_t h, int64_t w,
                                                 int guard, int dtype);

@@ -156,3 +156,23 @@ def test_wide_forward_at_unit_dilations(c, w, dtype):
     kernels = unfold_ref.generated_kernels(y.double(), wt.double(), b.double(), 3).to(dtype).double()
     atol, rtol = TOL["gen_fwd"][dtype]
     assert_close(out, unfold_ref.dynamic_cat(x.double(), kernels, 3, dil), atol, rtol, "concat")
+
+
+@pytest.mark.parametrize("dtype,c", [(torch.float32, 16), (torch.float32, 48), (torch.bfloat16, 24), (torch.float16, 64)])
+def test_flat_gradient_is_written_whole(dtype, c):
+    """The concat's flat gradient passes through autograd: every element of it
+    is a number, whatever its memory held (3C a multiple of 16 and not), so
+    that NaN detection accepts a step."""
+    say(f"anomaly detection C={c} {dtype}")
+    _, mod = _modules(c, 3, dtype)
+    x, y, g = (randn((2, c, 45, 51), s, dtype=dtype).to(DEV).requires_grad_() for s in (1, 2, 3))
+    seen = []
+    out = mod(x, y)
+    out.grad_fn.register_hook(lambda grads_in, grads_out: seen.append(grads_in[0]))
+    _nan_memory()
+    out.backward(g)
+    assert seen[0].ndim == 1 and bool(torch.isfinite(seen[0]).all())
+    with torch.autograd.detect_anomaly():
+        out = mod(x, y)
+        _nan_memory()
+        out.backward(g)
