@@ -124,8 +124,7 @@ __global__ __launch_bounds__(64 * kClwSegs * KS) void cl_wgrad_kernel(
     }
   };
   // step q: tile q % ft of image q / ft
-  int sn = step_beg / g.f.ft, sp = step_beg - sn * g.f.ft;
-  int spos = sp * kFlatTile;
+  int sn, sp, spos;
   auto stage = [&](int buf) {
     image(sn);
     char* __restrict__ dst = cwsm + buf * L::kBuf;
@@ -173,68 +172,99 @@ __global__ __launch_bounds__(64 * kClwSegs * KS) void cl_wgrad_kernel(
     for (int e = 0; e < 8; ++e) ones[e] = one;
   }
   f32x4 acc[KS][MB], accb[PROD ? KS : 1];
-#pragma unroll
-  for (int kj = 0; kj < KS; ++kj) {
-    accb[PROD ? kj : 0] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int ib = 0; ib < MB; ++ib) acc[kj][ib] = f32x4{0.f, 0.f, 0.f, 0.f};
-  }
-
-  if (steps > 0) stage(0);
-  __builtin_amdgcn_s_waitcnt(0);
-  __syncthreads();
-
   // this lane's row of a transposing read: position 4 * quad + e of 16, bytes
   // 8a .. 8a + 7 of its 32
   const int trl = (4 * quad + ((lane >> 2) & 3)) * 32 + (lane & 3) * 8 + 32 * 32 * sg;
-  int xl[KS];
+  // The sums over this split's steps.  MASK: positions outside the image left
+  // out (flat_any).
+  auto run = [&](auto maskc) {
+    constexpr bool MASK = decltype(maskc)::value;
+    int xl[KS];
 #pragma unroll
-  for (int kj = 0; kj < KS; ++kj) xl[kj] = ki * L::kX1 + trl + (kClPad + (kj - r) * d) * 32;
-  for (int s = 0; s < steps; ++s) {
-    const int buf = s & 1;
-    const bool more = s + 1 < steps;
-    if (more) stage(buf ^ 1);
-    const char* __restrict__ bb = cwsm + buf * L::kBuf;
-    auto read8 = [&](int off) {
-      u32x4 v;
-      uint32_t a0, a1, b0, b1;
-      cl_read_tr(bb + off, a0, a1);
-      cl_read_tr(bb + off + 512, b0, b1);
-      v[0] = a0;
-      v[1] = a1;
-      v[2] = b0;
-      v[3] = b1;
-      return v;
-    };
+    for (int kj = 0; kj < KS; ++kj) xl[kj] = ki * L::kX1 + trl + (kClPad + (kj - r) * d) * 32;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int jo = 4096 * j;  // 128 positions of 32 bytes
-      V bfr[MB];
+    for (int kj = 0; kj < KS; ++kj) {
+      accb[PROD ? kj : 0] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int ib = 0; ib < MB; ++ib)
-        bfr[ib] = __builtin_bit_cast(V, read8(L::kYOff + ib * L::kY1 + trl + jo));
-      ClProd<T> gp;
-      if constexpr (PROD) gp.set(read8(L::kGOff + trl + jo));
-      if (!PROD && do_bias) {
-#pragma unroll
-        for (int ib = 0; ib < MB; ++ib)
-          if (ib == bib) accb[0] = M::mac1(ones, bfr[ib], accb[0]);
-      }
-      u32x4 xv[KS];
-#pragma unroll
-      for (int kj = 0; kj < KS; ++kj) xv[kj] = read8(xl[kj] + jo);
-#pragma unroll
-      for (int kj = 0; kj < KS; ++kj) {
-        u32x4 av = xv[kj];
-        if constexpr (PROD) av = gp.mul(av);
-        const V afr = __builtin_bit_cast(V, av);
-#pragma unroll
-        for (int ib = 0; ib < MB; ++ib) acc[kj][ib] = M::mac1(afr, bfr[ib], acc[kj][ib]);
-        if constexpr (PROD) accb[kj] = M::mac1(afr, ones, accb[kj]);
-      }
+      for (int ib = 0; ib < MB; ++ib) acc[kj][ib] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
+    sn = step_beg / g.f.ft;
+    sp = step_beg - sn * g.f.ft;
+    spos = sp * kFlatTile;
+    if (steps > 0) stage(0);
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
+    for (int s = 0; s < steps; ++s) {
+      const int buf = s & 1;
+      const bool more = s + 1 < steps;
+      if (more) stage(buf ^ 1);
+      const char* __restrict__ bb = cwsm + buf * L::kBuf;
+      auto read8 = [&](int off) {
+        u32x4 v;
+        uint32_t a0, a1, b0, b1;
+        cl_read_tr(bb + off, a0, a1);
+        cl_read_tr(bb + off + 512, b0, b1);
+        v[0] = a0;
+        v[1] = a1;
+        v[2] = b0;
+        v[3] = b1;
+        return v;
+      };
+      // (the masked form stays rolled: unrolled, it cost the other one's
+      // schedule, bf16 4x32x135x181 42.1 -> 46.8 us)
+#pragma unroll(MASK ? 1 : 2)
+      for (int j = 0; j < 2; ++j) {
+        const int jo = 4096 * j;  // 128 positions of 32 bytes
+        V bfr[MB];
+#pragma unroll
+        for (int ib = 0; ib < MB; ++ib)
+          bfr[ib] = __builtin_bit_cast(V, read8(L::kYOff + ib * L::kY1 + trl + jo));
+        ClProd<T> gp;
+        if constexpr (PROD) gp.set(read8(L::kGOff + trl + jo));
+        if (!PROD && do_bias) {
+#pragma unroll
+          for (int ib = 0; ib < MB; ++ib)
+            if (ib == bib) accb[0] = M::mac1(ones, bfr[ib], accb[0]);
+        }
+        u32x4 xv[KS];
+#pragma unroll
+        for (int kj = 0; kj < KS; ++kj) xv[kj] = read8(xl[kj] + jo);
+        int in0 = 8, in1 = 8;
+        if constexpr (MASK) {
+          const int pos = (step_beg + s) % g.f.ft * kFlatTile + 128 * j + 32 * sg + 4 * quad;
+          in0 = flat_inside(g.f, pos);
+          in1 = flat_inside(g.f, pos + 16);
+        }
+#pragma unroll
+        for (int kj = 0; kj < KS; ++kj) {
+          u32x4 av = xv[kj];
+          if constexpr (PROD) av = gp.mul(av);
+          if constexpr (MASK)
+            av = (u32x4){flat_keep2(av[0], in0, 0), flat_keep2(av[1], in0, 2),
+                         flat_keep2(av[2], in1, 0), flat_keep2(av[3], in1, 2)};
+          const V afr = __builtin_bit_cast(V, av);
+#pragma unroll
+          for (int ib = 0; ib < MB; ++ib) acc[kj][ib] = M::mac1(afr, bfr[ib], acc[kj][ib]);
+          if constexpr (PROD) accb[kj] = M::mac1(afr, ones, accb[kj]);
+        }
+      }
+      __builtin_amdgcn_s_waitcnt(0);
+      __syncthreads();
+    }
+  };
+  run(std::false_type());
+  {
+    bool nan = false;
+#pragma unroll
+    for (int kj = 0; kj < KS; ++kj) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (PROD) nan = nan || accb[kj][e] != accb[kj][e];
+#pragma unroll
+        for (int ib = 0; ib < MB; ++ib) nan = nan || acc[kj][ib][e] != acc[kj][ib][e];
+      }
+    }
+    if (__builtin_expect(flat_any<NW>(nan, reinterpret_cast<uint32_t*>(cwsm), wave), 0)) run(std::true_type());
   }
 
   // ---- fixed-order sum over the segments through LDS

@@ -382,121 +382,154 @@ __global__ __launch_bounds__(kCwThreads) void conv_wgrad_partial_kernel(
   V ones;
 #pragma unroll
   for (int e = 0; e < 8; ++e) ones[e] = (ME)1.0f;
-  f32x4 acc[3][MB], accb = f32x4{0.f, 0.f, 0.f, 0.f};
+  f32x4 acc[3][MB], accb;
+  // The sums over this split's steps.  MASK (flat tensors): positions outside
+  // the image left out (flat_any).
+  auto run = [&](auto maskc) {
+    constexpr bool MASK = decltype(maskc)::value;
+    accb = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int kj = 0; kj < 3; ++kj)
+    for (int kj = 0; kj < 3; ++kj)
 #pragma unroll
-    for (int ib = 0; ib < MB; ++ib) acc[kj][ib] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int ib = 0; ib < MB; ++ib) acc[kj][ib] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  CwPos nxt;
-  {
-    const int row = step_beg / g.col_blocks;
-    nxt.cbk = step_beg - row * g.col_blocks;
-    nxt.w0 = nxt.cbk * TW;
-    nxt.n = row / H;
-    nxt.h = row - nxt.n * H;
-  }
-  if (steps > 0) {
-    image(nxt.n);
-    yload(nxt);
-    stage(nxt, 0);
-    nxt.advance(g);
-    ystore(0);
-  }
-  // ddpm_fuse_conv_bwd: this workgroup's share of the input gradient's
-  // weight packing, before the first step's copies are waited for
-  if (pack.total > 0) cv_pack_share<T>(pack, (int)blockIdx.x, (int)gridDim.x, tid, kCwThreads);
-  __builtin_amdgcn_s_waitcnt(0);
-  __syncthreads();
-  const int wl = 32 * sg + 8 * quad;  // this lane's first token within a 128-column subsegment
-  // element index of the lane's first cat value per tap kj (row ki, plane col16)
-  int xel[3];
-#pragma unroll
-  for (int kj = 0; kj < 3; ++kj) xel[kj] = (ki * 16 + col16) * L::kXSD * L::kPerD + kCwPad + wl + kj - 1;
-  // PP: this lane's channel is half (col16 & 1) of the pair in rows col16/2 (hi)
-  // and 8 + col16/2 (lo)
-  const int ppel = (ki * 16 + (col16 >> 1)) * L::kXSD + kCwPad + wl - 1;
-  const uint32_t ppsel = (col16 & 1) ? 0x07060302u : 0x05040100u;
-  const int bib = cb - oh * MB;  // the staged gO block this workgroup sums for the bias
-  for (int s = 0; s < steps; ++s) {
-    const int buf = s & 1;
-    const bool more = s + 1 < steps;
-    if (more) {
+    CwPos nxt;
+    {
+      const int row = step_beg / g.col_blocks;
+      nxt.cbk = step_beg - row * g.col_blocks;
+      nxt.w0 = nxt.cbk * TW;
+      nxt.n = row / H;
+      nxt.h = row - nxt.n * H;
+    }
+    int pos = nxt.w0;  // flat: the step's first position
+    if (steps > 0) {
       image(nxt.n);
       yload(nxt);
-      stage(nxt, buf ^ 1);
+      stage(nxt, 0);
       nxt.advance(g);
+      ystore(0);
     }
-    const uint32_t* __restrict__ bb = csm + buf * L::kBuf;
-#pragma unroll
-    for (int j = 0; j < SJ; ++j) {
-      // subsegment j: this lane's tokens wl + 128 j
-      const int kyj = ((wl + kCwTW * j) >> 3) ^ col16;
-      V bfr[MB][P];
-#pragma unroll
-      for (int ib = 0; ib < MB; ++ib)
-#pragma unroll
-        for (int pp = 0; pp < P; ++pp)
-          bfr[ib][pp] = __builtin_bit_cast(
-              V, *reinterpret_cast<const u32x4*>(bb + L::kYOff + ((pp * MB + ib) * 16 + col16) * L::kYD +
-                                                 4 * kyj));
-      if (do_bias) {
-        // grad_bias partials: ones x gO block bib (every row of D gets the sum)
-#pragma unroll
-        for (int ib = 0; ib < MB; ++ib)
-          if (ib == bib)
-#pragma unroll
-            for (int pp = 0; pp < P; ++pp) accb = M::mac1(ones, bfr[ib][pp], accb);
-      }
-#pragma unroll
-      for (int kj = 0; kj < 3; ++kj) {
-        V afr[P];
-        if constexpr (PP) {
-          uint32_t dh[8], dl[8];
-#pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            dh[e] = bb[ppel + kCwTW * j + kj + e];
-            dl[e] = bb[ppel + 8 * L::kXSD + kCwTW * j + kj + e];
-          }
-          u32x4 h4, l4;
-#pragma unroll
-          for (int jj = 0; jj < 4; ++jj) {
-            h4[jj] = __builtin_amdgcn_perm(dh[2 * jj + 1], dh[2 * jj], ppsel);
-            l4[jj] = __builtin_amdgcn_perm(dl[2 * jj + 1], dl[2 * jj], ppsel);
-          }
-          afr[0] = __builtin_bit_cast(V, h4);
-          afr[1] = __builtin_bit_cast(V, l4);
-        } else if constexpr (sizeof(T) == 4) {
-          float xv[8];
-#pragma unroll
-          for (int e = 0; e < 8; ++e) xv[e] = cw_lds_elem<T>(bb, xel[kj] + kCwTW * j + e);
-          M::pack(xv, afr);
-        } else {
-          // the 8 two-byte values as staged, already the fragment's element
-          // pairs: 4 dword reads where the window starts on a dword (kj = 1),
-          // else 5 realigned by one element (the shift kj - 1 is odd; the row
-          // pitch, the pad and the lane's token offset are even)
-          const uint32_t* __restrict__ xp = bb + ((xel[kj] + kCwTW * j) >> 1);
-          u32x4 wv;
-          if (kj != 1) {
-            uint32_t d5[5];
-#pragma unroll
-            for (int k = 0; k < 5; ++k) d5[k] = xp[k];
-#pragma unroll
-            for (int k = 0; k < 4; ++k) wv[k] = __builtin_amdgcn_alignbyte(d5[k + 1], d5[k], 2);
-          } else {
-#pragma unroll
-            for (int k = 0; k < 4; ++k) wv[k] = xp[k];
-          }
-          afr[0] = __builtin_bit_cast(V, wv);
-        }
-#pragma unroll
-        for (int ib = 0; ib < MB; ++ib) acc[kj][ib] = M::mac(afr, bfr[ib], acc[kj][ib]);
-      }
-    }
-    if (more) ystore(buf ^ 1);
+    // ddpm_fuse_conv_bwd: this workgroup's share of the input gradient's
+    // weight packing, before the first step's copies are waited for
+    if (!MASK && pack.total > 0) cv_pack_share<T>(pack, (int)blockIdx.x, (int)gridDim.x, tid, kCwThreads);
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
+    const int wl = 32 * sg + 8 * quad;  // this lane's first token within a 128-column subsegment
+    // element index of the lane's first cat value per tap kj (row ki, plane col16)
+    int xel[3];
+#pragma unroll
+    for (int kj = 0; kj < 3; ++kj) xel[kj] = (ki * 16 + col16) * L::kXSD * L::kPerD + kCwPad + wl + kj - 1;
+    // PP: this lane's channel is half (col16 & 1) of the pair in rows col16/2 (hi)
+    // and 8 + col16/2 (lo)
+    const int ppel = (ki * 16 + (col16 >> 1)) * L::kXSD + kCwPad + wl - 1;
+    const uint32_t ppsel = (col16 & 1) ? 0x07060302u : 0x05040100u;
+    const int bib = cb - oh * MB;  // the staged gO block this workgroup sums for the bias
+    for (int s = 0; s < steps; ++s) {
+      const int buf = s & 1;
+      const bool more = s + 1 < steps;
+      const int pos1 = nxt.w0;
+      if (more) {
+        image(nxt.n);
+        yload(nxt);
+        stage(nxt, buf ^ 1);
+        nxt.advance(g);
+      }
+      const uint32_t* __restrict__ bb = csm + buf * L::kBuf;
+#pragma unroll
+      for (int j = 0; j < SJ; ++j) {
+        // subsegment j: this lane's tokens wl + 128 j
+        const int kyj = ((wl + kCwTW * j) >> 3) ^ col16;
+        // the lane's tokens inside the image
+        const int in = MASK ? flat_inside(g.f, pos + wl + kCwTW * j) : 8;
+        V bfr[MB][P];
+#pragma unroll
+        for (int ib = 0; ib < MB; ++ib)
+#pragma unroll
+          for (int pp = 0; pp < P; ++pp)
+            bfr[ib][pp] = __builtin_bit_cast(
+                V, *reinterpret_cast<const u32x4*>(bb + L::kYOff + ((pp * MB + ib) * 16 + col16) * L::kYD +
+                                                   4 * kyj));
+        if (do_bias) {
+          // grad_bias partials: ones x gO block bib (every row of D gets the sum)
+#pragma unroll
+          for (int ib = 0; ib < MB; ++ib)
+            if (ib == bib)
+#pragma unroll
+              for (int pp = 0; pp < P; ++pp) accb = M::mac1(ones, bfr[ib][pp], accb);
+        }
+#pragma unroll
+        for (int kj = 0; kj < 3; ++kj) {
+          V afr[P];
+          if constexpr (PP) {
+            uint32_t dh[8], dl[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+              dh[e] = bb[ppel + kCwTW * j + kj + e];
+              dl[e] = bb[ppel + 8 * L::kXSD + kCwTW * j + kj + e];
+            }
+            u32x4 h4, l4;
+#pragma unroll
+            for (int jj = 0; jj < 4; ++jj) {
+              h4[jj] = __builtin_amdgcn_perm(dh[2 * jj + 1], dh[2 * jj], ppsel);
+              l4[jj] = __builtin_amdgcn_perm(dl[2 * jj + 1], dl[2 * jj], ppsel);
+            }
+            if constexpr (MASK) {
+#pragma unroll
+              for (int jj = 0; jj < 4; ++jj) {
+                h4[jj] = flat_keep2(h4[jj], in, 2 * jj);
+                l4[jj] = flat_keep2(l4[jj], in, 2 * jj);
+              }
+            }
+            afr[0] = __builtin_bit_cast(V, h4);
+            afr[1] = __builtin_bit_cast(V, l4);
+          } else if constexpr (sizeof(T) == 4) {
+            float xv[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) xv[e] = cw_lds_elem<T>(bb, xel[kj] + kCwTW * j + e);
+            if constexpr (MASK) {
+#pragma unroll
+              for (int e = 0; e < 8; ++e) xv[e] = e < in ? xv[e] : 0.f;
+            }
+            M::pack(xv, afr);
+          } else {
+            // the 8 two-byte values as staged, already the fragment's element
+            // pairs: 4 dword reads where the window starts on a dword (kj = 1),
+            // else 5 realigned by one element (the shift kj - 1 is odd; the row
+            // pitch, the pad and the lane's token offset are even)
+            const uint32_t* __restrict__ xp = bb + ((xel[kj] + kCwTW * j) >> 1);
+            u32x4 wv;
+            if (kj != 1) {
+              uint32_t d5[5];
+#pragma unroll
+              for (int k = 0; k < 5; ++k) d5[k] = xp[k];
+#pragma unroll
+              for (int k = 0; k < 4; ++k) wv[k] = __builtin_amdgcn_alignbyte(d5[k + 1], d5[k], 2);
+            } else {
+#pragma unroll
+              for (int k = 0; k < 4; ++k) wv[k] = xp[k];
+            }
+            afr[0] = __builtin_bit_cast(V, wv);
+          }
+#pragma unroll
+          for (int ib = 0; ib < MB; ++ib) acc[kj][ib] = M::mac(afr, bfr[ib], acc[kj][ib]);
+        }
+      }
+      if (more) ystore(buf ^ 1);
+      pos = pos1;
+      __builtin_amdgcn_s_waitcnt(0);
+      __syncthreads();
+    }
+  };
+  run(std::false_type());
+  if constexpr (FL) {
+    bool nan = false;
+#pragma unroll
+    for (int kj = 0; kj < 3; ++kj)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int ib = 0; ib < MB; ++ib) nan = nan || acc[kj][ib][e] != acc[kj][ib][e];
+    if (flat_any<kCwNW>(nan, csm, wave)) run(std::true_type());
   }
 
   // ---- fixed-order reduction over the segments through LDS: each segment's

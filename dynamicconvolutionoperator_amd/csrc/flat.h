@@ -90,6 +90,43 @@ __device__ __forceinline__ void flat_copy_chunk(const FlatCopy& t, const FlatLay
   }
 }
 
+// The weight gradients of flat tensors sum over whole tiles of positions, so
+// those outside the images take part with a gradient of zero; an infinite or
+// NaN x (or concat value) beside them makes that product NaN, in the sums of
+// taps that meet the value nowhere inside the image.  Masking every fragment
+// would cost the vector instructions that bound these kernels, so a workgroup
+// whose sums hold a NaN forms them a second time with such positions' products
+// replaced by zero: finite inputs pay one vote of a workgroup's waves
+// (generator / convolution, us, without -> with: bf16 4x64x135x181 74.0 ->
+// 74.0 / 42.5 -> 42.8, fp16 2x128x96x96 31.2 -> 33.1 / 33.5 -> 34.3, fp32
+// 4x64x135x181 122.4 -> 123.3 / 100.8 -> 103.4).
+
+// Positions of one row from `pos` (rows start on multiples of 8) that lie
+// inside the image, at most 8: none above the last column or row.
+__device__ __forceinline__ int flat_inside(const FlatLay& f, int pos) {
+  const int row = pos / f.P, n = f.W - (pos - row * f.P);
+  return row < f.H && n > 0 ? (n < 8 ? n : 8) : 0;
+}
+
+// The first n (from `first` on) of two 2-byte values in a dword, the others zero.
+__device__ __forceinline__ uint32_t flat_keep2(uint32_t v, int n, int first) {
+  return n >= first + 2 ? v : (n > first ? v & 0xffffu : 0u);
+}
+
+// Whether `mine` holds in any lane of the workgroup's NW waves.  votes: NW
+// words of LDS that nothing else uses until the call returns.
+template <int NW>
+__device__ __forceinline__ bool flat_any(bool mine, uint32_t* __restrict__ votes, int wave) {
+  const uint32_t any = __builtin_amdgcn_ballot_w64(mine) != 0 ? 1u : 0u;
+  if ((threadIdx.x & 63) == 0) votes[wave] = any;
+  __syncthreads();
+  uint32_t all = 0;
+#pragma unroll
+  for (int i = 0; i < NW; ++i) all |= votes[i];
+  __syncthreads();
+  return __builtin_amdgcn_readfirstlane(all) != 0;
+}
+
 // Zeroing of the elements of a concat's flat gradient that the input gradient's
 // tiles do not cover: the lead, the guard rows after each plane's last tile
 // and, for 2-byte elements, the channels past 3C of the last 16-channel block

@@ -555,152 +555,178 @@ __global__ __launch_bounds__(64 * kWgSegs * WgTaps<KS>::kGroups) void gen_bwd_w_
   }
   f32x4 acc[TPH][MB], accb[TPH];
   float dbs[TPH];  // kVBias: sum of the lane's products per tap
+  // The sums over this split's steps.  MASK (flat tensors): positions outside
+  // the image left out (flat_any).
+  auto run = [&](auto maskc) {
+    constexpr bool MASK = decltype(maskc)::value;
 #pragma unroll
-  for (int tt = 0; tt < TPH; ++tt) {
-    accb[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    dbs[tt] = 0.f;
+    for (int tt = 0; tt < TPH; ++tt) {
+      accb[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
+      dbs[tt] = 0.f;
 #pragma unroll
-    for (int ib = 0; ib < MB; ++ib) acc[tt][ib] = f32x4{0.f, 0.f, 0.f, 0.f};
-  }
+      for (int ib = 0; ib < MB; ++ib) acc[tt][ib] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
 
-  WgPos nxt;
-  {
-    const int row = step_beg / g.col_blocks;
-    nxt.cbk = step_beg - row * g.col_blocks;
-    nxt.w0 = nxt.cbk * TW;
-    nxt.n = row / H;
-    nxt.h = row - nxt.n * H;
-  }
-  if (steps > 0) {
-    image(nxt.n);
-    yload(nxt);
-    stage(nxt, 0);
-    nxt.advance(g);
-    ystore(0);
-  }
-  __builtin_amdgcn_s_waitcnt(0);
-  __syncthreads();
-  const int wl = 32 * sg + 8 * quad;  // this lane's first token within a 128-column subsegment
-  // element index (from the buffer start) of the lane's first x value per tap
-  int xel[TPH];
-#pragma unroll
-  for (int tt = 0; tt < TPH; ++tt) {
-    const int t = th * TPH + tt;
-    const int ki = t / KS, kj = t - ki * KS;
-    xel[tt] = (ki * 16 + col16) * L::kXSD * L::kPerD + kWgPad + wl + (kj - r) * d;
-  }
-  for (int s = 0; s < steps; ++s) {
-    const int buf = s & 1;
-    const bool more = s + 1 < steps;
-    if (more) {
+    WgPos nxt;
+    {
+      const int row = step_beg / g.col_blocks;
+      nxt.cbk = step_beg - row * g.col_blocks;
+      nxt.w0 = nxt.cbk * TW;
+      nxt.n = row / H;
+      nxt.h = row - nxt.n * H;
+    }
+    int pos = nxt.w0;  // flat: the step's first position
+    if (steps > 0) {
       image(nxt.n);
       yload(nxt);
-      stage(nxt, buf ^ 1);
+      stage(nxt, 0);
       nxt.advance(g);
+      ystore(0);
     }
-    const uint32_t* __restrict__ bb = wsm + buf * L::kBuf;
-#pragma unroll
-    for (int j = 0; j < SJ; ++j) {
-      // subsegment j: this lane's tokens wl + 128 j
-      const int wlj = wl + kWgTW * j;
-      const int kyj = (wlj >> 3) ^ col16;
-      V bfr[MB][P];
-#pragma unroll
-      for (int ib = 0; ib < MB; ++ib)
-#pragma unroll
-        for (int pp = 0; pp < P; ++pp)
-          bfr[ib][pp] = __builtin_bit_cast(
-              V, *reinterpret_cast<const u32x4*>(bb + L::kYOff + ((pp * MB + ib) * 16 + col16) * L::kYD +
-                                                 4 * kyj));
-      // branch gradient of channel col16 at the lane's 8 tokens
-      float gv[8];
-      {
-        const uint32_t* __restrict__ gr = bb + L::kGOff + col16 * L::kGD;
-        if constexpr (E == 4) {
-          const int kg = wlj >> 2;
-          const u32x4 a0 = *reinterpret_cast<const u32x4*>(gr + 4 * (kg ^ col16));
-          const u32x4 a1 = *reinterpret_cast<const u32x4*>(gr + 4 * ((kg + 1) ^ col16));
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            gv[e] = __uint_as_float(a0[e]);
-            gv[4 + e] = __uint_as_float(a1[e]);
-          }
-        } else {
-          typedef T T8 __attribute__((ext_vector_type(8)));
-          const T8 t8 = __builtin_bit_cast(T8, *reinterpret_cast<const u32x4*>(gr + 4 * kyj));
-#pragma unroll
-          for (int e = 0; e < 8; ++e) gv[e] = to_f(t8[e]);
-        }
-      }
-      // The A fragment of tap tt+1 (x reads, products, bf16 split) is formed
-      // while tap tt's MFMAs run: the scheduling groups below put its LDS reads
-      // first and then interleave each MFMA with 3 VALU instructions (measured
-      // 3-5% faster than the compiler's clustering, which left the MFMA pipe
-      // idle during each tap's VALU stretch)
-      auto make_afr = [&](int tt, V (&af)[P]) {
-        float dk[8];
-        if constexpr (E == 2) {
-          // the lane's 8 consecutive 2-byte x values by dword reads: 4 dwords
-          // when the window starts on a dword, else 5 realigned by one element.
-          // The parity is the tap shift's, (kj - r) * d: the row pitch, the pad
-          // and the lane's token offset are even (wave-uniform branch)
-          const int t = th * TPH + tt;
-          const int kj = t - (t / KS) * KS;
-          const int el = xel[tt] + kWgTW * j;
-          const uint32_t* __restrict__ xp = bb + (el >> 1);
-          uint32_t w[4];
-          if (((kj - r) * d) & 1) {
-            uint32_t d5[5];
-#pragma unroll
-            for (int k = 0; k < 5; ++k) d5[k] = xp[k];
-#pragma unroll
-            for (int k = 0; k < 4; ++k) w[k] = __builtin_amdgcn_alignbyte(d5[k + 1], d5[k], 2);
-          } else {
-#pragma unroll
-            for (int k = 0; k < 4; ++k) w[k] = xp[k];
-          }
-#pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            dk[2 * k] = gv[2 * k] * to_f(__builtin_bit_cast(T, (unsigned short)(w[k] & 0xffffu)));
-            dk[2 * k + 1] = gv[2 * k + 1] * to_f(__builtin_bit_cast(T, (unsigned short)(w[k] >> 16)));
-          }
-        } else {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) dk[e] = gv[e] * lds_elem<T>(bb, xel[tt] + kWgTW * j + e);
-        }
-        M::pack(dk, af);
-        if constexpr (kVBias)
-          dbs[tt] += ((dk[0] + dk[1]) + (dk[2] + dk[3])) + ((dk[4] + dk[5]) + (dk[6] + dk[7]));
-      };
-      V afc[P];
-      make_afr(0, afc);
-#pragma unroll
-      for (int tt = 0; tt < TPH; ++tt) {
-        const int t = th * TPH + tt;  // wave-uniform
-        if (KK % NH != 0 && t >= KK) break;
-        V afn[P];
-        if (tt + 1 < TPH) make_afr(tt + 1, afn);
-#pragma unroll
-        for (int ib = 0; ib < MB; ++ib) acc[tt][ib] = M::mac(afc, bfr[ib], acc[tt][ib]);
-        if constexpr (!kVBias) {
-#pragma unroll
-          for (int pp = 0; pp < P; ++pp) accb[tt] = M::mac1(afc[pp], ones, accb[tt]);
-        }
-        if (tt + 1 < TPH) {
-          __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);  // LDS reads
-#pragma unroll
-          for (int i = 0; i < MB * (P == 2 ? 3 : 1) + (kVBias ? 0 : P); ++i) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
-            __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);  // three VALU
-          }
-        }
-#pragma unroll
-        for (int pp = 0; pp < P; ++pp) afc[pp] = afn[pp];
-      }
-    }
-    if (more) ystore(buf ^ 1);
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
+    const int wl = 32 * sg + 8 * quad;  // this lane's first token within a 128-column subsegment
+    // element index (from the buffer start) of the lane's first x value per tap
+    int xel[TPH];
+#pragma unroll
+    for (int tt = 0; tt < TPH; ++tt) {
+      const int t = th * TPH + tt;
+      const int ki = t / KS, kj = t - ki * KS;
+      xel[tt] = (ki * 16 + col16) * L::kXSD * L::kPerD + kWgPad + wl + (kj - r) * d;
+    }
+    for (int s = 0; s < steps; ++s) {
+      const int buf = s & 1;
+      const bool more = s + 1 < steps;
+      const int pos1 = nxt.w0;
+      if (more) {
+        image(nxt.n);
+        yload(nxt);
+        stage(nxt, buf ^ 1);
+        nxt.advance(g);
+      }
+      const uint32_t* __restrict__ bb = wsm + buf * L::kBuf;
+#pragma unroll
+      for (int j = 0; j < SJ; ++j) {
+        // subsegment j: this lane's tokens wl + 128 j
+        const int wlj = wl + kWgTW * j;
+        const int kyj = (wlj >> 3) ^ col16;
+        const int in = MASK ? flat_inside(g.f, pos + wlj) : 8;  // the lane's tokens inside the image
+        V bfr[MB][P];
+#pragma unroll
+        for (int ib = 0; ib < MB; ++ib)
+#pragma unroll
+          for (int pp = 0; pp < P; ++pp)
+            bfr[ib][pp] = __builtin_bit_cast(
+                V, *reinterpret_cast<const u32x4*>(bb + L::kYOff + ((pp * MB + ib) * 16 + col16) * L::kYD +
+                                                   4 * kyj));
+        // branch gradient of channel col16 at the lane's 8 tokens
+        float gv[8];
+        {
+          const uint32_t* __restrict__ gr = bb + L::kGOff + col16 * L::kGD;
+          if constexpr (E == 4) {
+            const int kg = wlj >> 2;
+            const u32x4 a0 = *reinterpret_cast<const u32x4*>(gr + 4 * (kg ^ col16));
+            const u32x4 a1 = *reinterpret_cast<const u32x4*>(gr + 4 * ((kg + 1) ^ col16));
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              gv[e] = __uint_as_float(a0[e]);
+              gv[4 + e] = __uint_as_float(a1[e]);
+            }
+          } else {
+            typedef T T8 __attribute__((ext_vector_type(8)));
+            const T8 t8 = __builtin_bit_cast(T8, *reinterpret_cast<const u32x4*>(gr + 4 * kyj));
+#pragma unroll
+            for (int e = 0; e < 8; ++e) gv[e] = to_f(t8[e]);
+          }
+        }
+        // The A fragment of tap tt+1 (x reads, products, bf16 split) is formed
+        // while tap tt's MFMAs run: the scheduling groups below put its LDS reads
+        // first and then interleave each MFMA with 3 VALU instructions (measured
+        // 3-5% faster than the compiler's clustering, which left the MFMA pipe
+        // idle during each tap's VALU stretch)
+        auto make_afr = [&](int tt, V (&af)[P]) {
+          float dk[8];
+          if constexpr (E == 2) {
+            // the lane's 8 consecutive 2-byte x values by dword reads: 4 dwords
+            // when the window starts on a dword, else 5 realigned by one element.
+            // The parity is the tap shift's, (kj - r) * d: the row pitch, the pad
+            // and the lane's token offset are even (wave-uniform branch)
+            const int t = th * TPH + tt;
+            const int kj = t - (t / KS) * KS;
+            const int el = xel[tt] + kWgTW * j;
+            const uint32_t* __restrict__ xp = bb + (el >> 1);
+            uint32_t w[4];
+            if (((kj - r) * d) & 1) {
+              uint32_t d5[5];
+#pragma unroll
+              for (int k = 0; k < 5; ++k) d5[k] = xp[k];
+#pragma unroll
+              for (int k = 0; k < 4; ++k) w[k] = __builtin_amdgcn_alignbyte(d5[k + 1], d5[k], 2);
+            } else {
+#pragma unroll
+              for (int k = 0; k < 4; ++k) w[k] = xp[k];
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+              dk[2 * k] = gv[2 * k] * to_f(__builtin_bit_cast(T, (unsigned short)(w[k] & 0xffffu)));
+              dk[2 * k + 1] = gv[2 * k + 1] * to_f(__builtin_bit_cast(T, (unsigned short)(w[k] >> 16)));
+            }
+          } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) dk[e] = gv[e] * lds_elem<T>(bb, xel[tt] + kWgTW * j + e);
+          }
+          if constexpr (MASK) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) dk[e] = e < in ? dk[e] : 0.f;
+          }
+          M::pack(dk, af);
+          if constexpr (kVBias)
+            dbs[tt] += ((dk[0] + dk[1]) + (dk[2] + dk[3])) + ((dk[4] + dk[5]) + (dk[6] + dk[7]));
+        };
+        V afc[P];
+        make_afr(0, afc);
+#pragma unroll
+        for (int tt = 0; tt < TPH; ++tt) {
+          const int t = th * TPH + tt;  // wave-uniform
+          if (KK % NH != 0 && t >= KK) break;
+          V afn[P];
+          if (tt + 1 < TPH) make_afr(tt + 1, afn);
+#pragma unroll
+          for (int ib = 0; ib < MB; ++ib) acc[tt][ib] = M::mac(afc, bfr[ib], acc[tt][ib]);
+          if constexpr (!kVBias) {
+#pragma unroll
+            for (int pp = 0; pp < P; ++pp) accb[tt] = M::mac1(afc[pp], ones, accb[tt]);
+          }
+          if (tt + 1 < TPH) {
+            __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);  // LDS reads
+#pragma unroll
+            for (int i = 0; i < MB * (P == 2 ? 3 : 1) + (kVBias ? 0 : P); ++i) {
+              __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
+              __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);  // three VALU
+            }
+          }
+#pragma unroll
+          for (int pp = 0; pp < P; ++pp) afc[pp] = afn[pp];
+        }
+      }
+      if (more) ystore(buf ^ 1);
+      pos = pos1;
+      __builtin_amdgcn_s_waitcnt(0);
+      __syncthreads();
+    }
+  };
+  run(std::false_type{});
+  if constexpr (FL) {
+    bool nan = false;
+#pragma unroll
+    for (int tt = 0; tt < TPH; ++tt) {
+      nan = nan || dbs[tt] != dbs[tt];
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int ib = 0; ib < MB; ++ib) nan = nan || acc[tt][ib][e] != acc[tt][ib][e];
+    }
+    if (flat_any<NW>(nan, wsm, wave)) run(std::true_type{});
   }
 
   // ---- deterministic reduction over the segments (fixed order) through LDS:

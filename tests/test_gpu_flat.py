@@ -176,3 +176,38 @@ def test_flat_gradient_is_written_whole(dtype, c):
         out = mod(x, y)
         _nan_memory()
         out.backward(g)
+
+
+# an infinite x reaches the weight gradients of the taps that meet it inside
+# the image and no others (dilated taps from the first and last columns and
+# rows lie outside): finite where the oracle is, and equal there
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("c,k", [(32, 3), (96, 3), (64, 1)])
+def test_flat_infinities_stay_in_their_taps(c, k, dtype):
+    say(f"infinities C={c} K={k} {dtype}")
+    shape = (2, c, 20, 30)
+    oracle, mod = _modules(c, k, dtype)
+    x, y, g = (randn(shape, s, dtype=dtype) for s in (1, 2, 3))
+    x[0, 1, 7, 0] = x[1, 5, 19, 12] = x[1, 9, 3, 29] = float("inf")
+    x[0, 20, 0, 0] = -float("inf")
+    xg, yg = (t.to(DEV).requires_grad_() for t in (x, y))
+    xr, yr = (t.double().requires_grad_() for t in (x, y))
+    got = torch.autograd.grad(mod(xg, yg), (xg, yg, *mod.parameters()), g.to(DEV))
+    want = torch.autograd.grad(oracle(xr, yr), (xr, yr, *oracle.parameters()), g.double())
+    atol, rtol = TOL["module_bwd"][dtype]
+    for name, a, e in zip(("dx", "dy", "dgw", "dgb", "dfw", "dfb"), got, want):
+        a, finite = a.detach().double().cpu(), torch.isfinite(e)
+        assert torch.equal(torch.isfinite(a), finite), name
+        assert_close(a[finite], e[finite], atol * e[finite].abs().max().item(), rtol, name)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_stand_alone_fuse_conv_infinities_stay_in_their_taps(dtype):
+    n, c, h, w = 2, 32, 61, 125
+    cat, g = randn((n, 4 * c, h, w), 1, dtype=dtype), randn((n, c, h, w), 2, dtype=dtype)
+    cat[0, 3, 7, 0] = cat[1, 50, h - 1, 12] = cat[1, 9, 3, w - 1] = float("inf")
+    wt = randn((c, 4 * c, 3, 3), 3, dtype=dtype, scale=0.05)
+    wd, wr = wt.to(DEV).requires_grad_(), wt.double().requires_grad_()
+    (got,) = torch.autograd.grad(ops.fuse_conv3x3(cat.to(DEV), wd, None), wd, g.to(DEV))
+    (want,) = torch.autograd.grad(torch.nn.functional.conv2d(cat.double(), wr, padding=1), wr, g.double())
+    assert torch.equal(torch.isfinite(got.cpu()), torch.isfinite(want))
