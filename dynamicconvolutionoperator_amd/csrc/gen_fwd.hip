@@ -58,8 +58,9 @@ __device__ __forceinline__ void swap_rows16(uint32_t& a, uint32_t& b) {
 
 // Forward for 2-byte types at K = 3 with the taps paired in the MFMA rows.
 // The generator rows of a step are 8 channels x 2 taps (row m: channel
-// c0 + 8*mb + m/2, tap 2j + m%2; the fifth pair of a branch holds tap 8 and a
-// zero row), so a lane's 4 results are (ca, t0), (ca, t1), (cb, t0), (cb, t1)
+// c0 + 8*mb + m/2, tap 2j + m%2; the fifth step of a branch holds tap 8 and a
+// zero row, a step of its own without the partner's reads: 8x64x256x256 bf16
+// 280 -> 262 us, 4x96x150x211 159 -> 140 us), so a lane's 4 results are (ca, t0), (ca, t1), (cb, t0), (cb, t1)
 // for two channels ca, cb: one cvt_pk rounds a channel's two taps to T
 // together and one v_dot2_f32 multiplies them by x at the two shifted pixels
 // and accumulates -- 1.5 VALU instructions per (channel, tap, pixel) where the
@@ -155,40 +156,35 @@ __global__ __launch_bounds__(kGtThreads) __attribute__((amdgpu_waves_per_eu(gt_w
 
   // x entry of this lane's two channels (8mb + 2q, +1) at its block-0 pixel:
   // plane 2mb + q/2, bytes 4*(q%2) .. +3 of the 4-channel entry
-  uint32_t lb[2];
-#pragma unroll
-  for (int mb = 0; mb < 2; ++mb)
-    lb[mb] = (uint32_t)((2 * mb + (quad >> 1)) * g.plane + col16 * XB + 4 * (quad & 1));
-  // byte offset of row rr (0, 1) of this wave's blocks at zero shift; block
-  // blk sits at row blk / CB, 16 * (blk % CB) entries to the right
-  auto rbase = [&](int rr) { return (uint32_t)(((2 * wave + rr + R) * LW + R) * XB); };
-  // global byte offset of channel c0 + 8mb + 2q + e at this lane's pixel of
+  const uint32_t lb = (uint32_t)((quad >> 1) * g.plane + col16 * XB + 4 * (quad & 1));
+  // byte offset of row rr (0, 1) of this wave's blocks at zero shift in row
+  // block mb's planes; block blk sits at row blk / CB, 16 * (blk % CB) entries
+  // to the right
+  auto rbase = [&](int rr, int mb) {
+    return (uint32_t)(((2 * wave + rr + R) * LW + R) * XB + 2 * mb * g.plane);
+  };
+  // global byte offset of channel c0 + 8mb + 2q + e at pixel column `col` of
   // block blk (kOob outside the image or the channel block)
-  auto goff = [&](int blk, int mb, int e) {
-    const int gh = h0 + 2 * wave + blk / CB, gw = w0 + 16 * (blk % CB) + col16;
+  auto goff = [&](int col, int blk, int mb, int e) {
+    const int gh = h0 + 2 * wave + blk / CB, gw = w0 + 16 * (blk % CB) + col;
     const int cl = 8 * mb + 2 * quad + e;
     return (gh < H && gw < W && cl < nch) ? (uint32_t)cl * OSE + (uint32_t)(gh * OP + gw) * E : kOob;
   };
 
   float acc[NBW][2][2];  // branch output of channels (ca, cb) of each row block, per pixel block
-#pragma unroll 1
-  for (int ps = 0; ps < NPS; ++ps) {
-    const int b = ps / NPB, j = ps - b * NPB;
+  // Pair step j of branch b.  TWO: taps 2j and 2j + 1; else the lone tap 8,
+  // whose partner -- a zero row, NaN where y is infinite -- is left out on
+  // both sides.
+  auto step = [&](int b, int j, auto twoc) {
+    constexpr bool TWO = decltype(twoc)::value;
+    const int ps = b * NPB + j;
     const int d = dil_of(b, g.d0, g.d1, g.d2);
     const int t0 = 2 * j, t1 = t0 + 1;
     const int sh0 = ((t0 / 3 - 1) * d * LW + (t0 % 3 - 1) * d) * XB;
-    const bool pair = t1 < KK;  // wave-uniform
-    const int sh1 = pair ? ((t1 / 3 - 1) * d * LW + (t1 % 3 - 1) * d) * XB : sh0;
-    // x pairs (channel a: t0, t1) and (channel b: t0, t1) from the two reads;
-    // the lone tap 8 pairs with zero
-    const uint32_t sela = pair ? 0x05040100u : 0x0c0c0100u;
-    const uint32_t selb = pair ? 0x07060302u : 0x0c0c0302u;
-    if (j == 0) {
-#pragma unroll
-      for (int blk = 0; blk < NBW; ++blk)
-#pragma unroll
-        for (int mb = 0; mb < 2; ++mb) acc[blk][mb][0] = acc[blk][mb][1] = 0.f;
-    }
+    const int sh1 = TWO ? ((t1 / 3 - 1) * d * LW + (t1 % 3 - 1) * d) * XB : sh0;
+    // x pairs (channel a: t0, t1) and (channel b: t0, t1) from the two reads
+    constexpr uint32_t sela = TWO ? 0x05040100u : 0x0c0c0100u;
+    constexpr uint32_t selb = TWO ? 0x07060302u : 0x0c0c0302u;
     const unsigned char* __restrict__ ab = abuf + ps * SU * 64 * 16;
     // both row blocks' MFMAs first, then both epilogues: the second block's
     // MFMAs run while the first block's epilogue issues
@@ -209,68 +205,78 @@ __global__ __launch_bounds__(kGtThreads) __attribute__((amdgpu_waves_per_eu(gt_w
     }
 #pragma unroll
     for (int mb = 0; mb < 2; ++mb) {
-      uint32_t l = lb[mb];
+      uint32_t l = lb;
       asm volatile("" : "+v"(l));
       // one base per (row, shift); the block's column is the reads' immediate offset
-      const unsigned char* __restrict__ p0[2] = {xs + l + (rbase(0) + sh0), xs + l + (rbase(1) + sh0)};
-      const unsigned char* __restrict__ p1[2] = {xs + l + (rbase(0) + sh1), xs + l + (rbase(1) + sh1)};
+      const unsigned char* __restrict__ p0[2] = {xs + l + (rbase(0, mb) + sh0), xs + l + (rbase(1, mb) + sh0)};
+      const unsigned char* __restrict__ p1[2] = {xs + l + (rbase(0, mb) + sh1), xs + l + (rbase(1, mb) + sh1)};
 #pragma unroll
       for (int blk = 0; blk < NBW; ++blk) {
         const int co = 16 * (blk % CB) * XB;
         const uint32_t x0 = *reinterpret_cast<const uint32_t*>(p0[blk / CB] + co);
-        const uint32_t x1 = *reinterpret_cast<const uint32_t*>(p1[blk / CB] + co);
-        const uint32_t qa = pack2<T>(dacc[mb][blk][0], dacc[mb][blk][1]);
-        const uint32_t qb = pack2<T>(dacc[mb][blk][2], dacc[mb][blk][3]);
+        const uint32_t x1 = TWO ? *reinterpret_cast<const uint32_t*>(p1[blk / CB] + co) : x0;
+        const uint32_t qa = pack2<T>(dacc[mb][blk][0], TWO ? dacc[mb][blk][1] : 0.f);
+        const uint32_t qb = pack2<T>(dacc[mb][blk][2], TWO ? dacc[mb][blk][3] : 0.f);
         acc[blk][mb][0] = dot2<T>(qa, __builtin_amdgcn_perm(x1, x0, sela), acc[blk][mb][0]);
         acc[blk][mb][1] = dot2<T>(qb, __builtin_amdgcn_perm(x1, x0, selb), acc[blk][mb][1]);
       }
     }
-    if (j == NPB - 1) {
-      // ---- branch b: channels c0 + 8mb + 2q + e of output block b+1
-      if constexpr (CL) {
-        // channels-last.  A lane holds 2 of a pixel's 8 channels per row block;
-        // swapping rows of 16 lanes between four pixel blocks gives lane row
-        // q the 8 channels of block q's pixels, one 16-byte store (two blocks:
-        // lane rows q and q + 2 hold 4 channels each of block q % 2, 8 bytes)
-        const BufRes cres = make_buf(out + n * g.oimg, (uint32_t)(4 * C) * OSE);
+  };
+#pragma unroll 1
+  for (int b = 0; b < 3; ++b) {
 #pragma unroll
-        for (int mb = 0; mb < 2; ++mb) {
-          const int cl = 8 * mb, pl = (b + 1) * C + c0 + cl;
-          const uint32_t base = (uint32_t)(pl >> 4) * g.OS * 32u + (uint32_t)(pl & 15) * 2u;
-          constexpr int Q = NBW < 4 ? 2 : 4;  // pixel blocks per exchange
+    for (int blk = 0; blk < NBW; ++blk)
 #pragma unroll
-          for (int b0 = 0; b0 < NBW; b0 += Q) {
-            const int blk = b0 + (quad & (Q - 1));
-            const int gh = h0 + 2 * wave + blk / CB, gw = w0 + 16 * (blk % CB) + col16;
-            const uint32_t o = gh < H && gw < W && cl < nch
-                                   ? base + (uint32_t)(gh * OP + gw) * 32u + (Q == 4 ? 0u : 8u * (quad >> 1))
-                                   : kOob;
-            uint32_t d[Q];
+      for (int mb = 0; mb < 2; ++mb) acc[blk][mb][0] = acc[blk][mb][1] = 0.f;
+#pragma unroll 1
+    for (int j = 0; j < NPB - 1; ++j) step(b, j, std::true_type());
+    step(b, NPB - 1, std::false_type());
+    // ---- branch b: channels c0 + 8mb + 2q + e of output block b+1
+    if constexpr (CL) {
+      // channels-last.  A lane holds 2 of a pixel's 8 channels per row block;
+      // swapping rows of 16 lanes between four pixel blocks gives lane row
+      // q the 8 channels of block q's pixels, one 16-byte store (two blocks:
+      // lane rows q and q + 2 hold 4 channels each of block q % 2, 8 bytes)
+      const BufRes cres = make_buf(out + n * g.oimg, (uint32_t)(4 * C) * OSE);
 #pragma unroll
-            for (int i = 0; i < Q; ++i) d[i] = pack2<T>(acc[b0 + i][mb][0], acc[b0 + i][mb][1]);
-            if constexpr (Q == 4) {
-              swap_rows32(d[0], d[2]);
-              swap_rows32(d[1], d[3]);
-              swap_rows16(d[0], d[1]);
-              swap_rows16(d[2], d[3]);
-              __builtin_amdgcn_raw_buffer_store_b128((u32x4){d[0], d[1], d[2], d[3]}, cres, o, 0, 0);
-            } else {
-              swap_rows16(d[0], d[1]);
-              typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-              __builtin_amdgcn_raw_buffer_store_b64((u32x2){d[0], d[1]}, cres, o, 0, 0);
-            }
+      for (int mb = 0; mb < 2; ++mb) {
+        const int cl = 8 * mb, pl = (b + 1) * C + c0 + cl;
+        const uint32_t base = (uint32_t)(pl >> 4) * g.OS * 32u + (uint32_t)(pl & 15) * 2u;
+        constexpr int Q = NBW < 4 ? 2 : 4;  // pixel blocks per exchange
+#pragma unroll
+        for (int b0 = 0; b0 < NBW; b0 += Q) {
+          const int blk = b0 + (quad & (Q - 1));
+          const int gh = h0 + 2 * wave + blk / CB, gw = w0 + 16 * (blk % CB) + col16;
+          const uint32_t o = gh < H && gw < W && cl < nch
+                                 ? base + (uint32_t)(gh * OP + gw) * 32u + (Q == 4 ? 0u : 8u * (quad >> 1))
+                                 : kOob;
+          uint32_t d[Q];
+#pragma unroll
+          for (int i = 0; i < Q; ++i) d[i] = pack2<T>(acc[b0 + i][mb][0], acc[b0 + i][mb][1]);
+          if constexpr (Q == 4) {
+            swap_rows32(d[0], d[2]);
+            swap_rows32(d[1], d[3]);
+            swap_rows16(d[0], d[1]);
+            swap_rows16(d[2], d[3]);
+            __builtin_amdgcn_raw_buffer_store_b128((u32x4){d[0], d[1], d[2], d[3]}, cres, o, 0, 0);
+          } else {
+            swap_rows16(d[0], d[1]);
+            typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+            __builtin_amdgcn_raw_buffer_store_b64((u32x2){d[0], d[1]}, cres, o, 0, 0);
           }
         }
-      } else {
-        const BufRes bres = make_buf(out + n * g.oimg + ((int64_t)(b + 1) * C + c0) * OS,
-                                     (uint32_t)nch * OSE);
-#pragma unroll
-        for (int blk = 0; blk < NBW; ++blk)
-#pragma unroll
-          for (int mb = 0; mb < 2; ++mb)
-#pragma unroll
-            for (int e = 0; e < 2; ++e) buf_store1<T>(bres, goff(blk, mb, e), acc[blk][mb][e]);
       }
+    } else {
+      const BufRes bres = make_buf(out + n * g.oimg + ((int64_t)(b + 1) * C + c0) * OS,
+                                   (uint32_t)nch * OSE);
+      int col = col16;  // (opaque: the offsets stay out of the steps' registers)
+      asm volatile("" : "+v"(col));
+#pragma unroll
+      for (int blk = 0; blk < NBW; ++blk)
+#pragma unroll
+        for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+          for (int e = 0; e < 2; ++e) buf_store1<T>(bres, goff(col, blk, mb, e), acc[blk][mb][e]);
     }
   }
 }

@@ -211,3 +211,18 @@ def test_stand_alone_fuse_conv_infinities_stay_in_their_taps(dtype):
     (got,) = torch.autograd.grad(ops.fuse_conv3x3(cat.to(DEV), wd, None), wd, g.to(DEV))
     (want,) = torch.autograd.grad(torch.nn.functional.conv2d(cat.double(), wr, padding=1), wr, g.double())
     assert torch.equal(torch.isfinite(got.cpu()), torch.isfinite(want))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("c", [64, 72, 128])
+def test_paired_forward_of_infinite_kernels(c, dtype):
+    """An infinite y makes the generated kernels infinite, and the branches
+    with them, not NaN: the last tap of a branch has no partner to pair with."""
+    shape = (1, c, 20, 40)
+    x, y = randn(shape, 1, dtype).abs() + 0.5, randn(shape, 2, dtype)
+    wt, b = default_generator_params(c, 3, 3, dtype)
+    wt = wt.abs() + 2.0**-6  # (no zero weight, no cancelling signs)
+    y[0, 5, 9, 11] = float("inf")
+    out = ops.fused_generator_dynamic_cat(x.to(DEV), y.to(DEV), wt.to(DEV), b.to(DEV), 3, DIL).cpu()
+    want = unfold_ref.generator_dynamic_cat(x.double(), y.double(), wt.double(), b.double(), 3)
+    assert torch.equal(torch.isinf(out), torch.isinf(want)) and not bool(torch.isnan(out).any())
