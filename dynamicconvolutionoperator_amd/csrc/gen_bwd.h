@@ -166,6 +166,9 @@ int yt_run(const void* x, const void* weight, const void* grad_out, void* grad_y
            int d0, int d1, int d2, int dtype, hipStream_t stream, int mode, YPack* pack,
            const WReduce* red = nullptr, const FlatLay* f = nullptr);
 
+// Workspace bytes of yt_run on flat tensors.
+int64_t yt_flat_workspace_bytes(int64_t c, int kernel_size, int dtype);
+
 // Launches the packing `p` as its own kernel.  Defined in gen_bwd_y.hip.
 int yt_pack(const YPack& p, int kernel_size, int dtype, hipStream_t stream);
 

@@ -948,7 +948,6 @@ extern "C" int64_t ddpm_flat_cat_elems(int64_t n, int64_t c, int64_t h, int64_t 
                                        int dtype);
 extern "C" int64_t ddpm_gen_bwd_x_workspace_bytes(int64_t n, int64_t c, int64_t h, int64_t w,
                                                   int kernel_size, int d0, int d1, int d2);
-extern "C" int64_t ddpm_gen_bwd_y_workspace_bytes(int64_t c, int kernel_size);
 
 namespace {
 
@@ -1192,7 +1191,7 @@ int flat_bwd(FlatBwd& b, int64_t n, int64_t c, int64_t h, int64_t w, int kernel_
   clw_geom(cg, b.f, n, c, true);
   b.copy = align256(flat_elems(b.f, n * flat_planes(c), esz) * esz);
   b.bx = align256(ddpm_gen_bwd_x_workspace_bytes(n, c, h, w, kernel_size, d0, d1, d2));
-  b.by = align256(ddpm_gen_bwd_y_workspace_bytes(c, kernel_size));
+  b.by = align256(yt_flat_workspace_bytes(c, kernel_size, dtype));
   b.bw = align256(esz == 2 ? clw_partial_bytes(cg, kernel_size * kernel_size, true)
                            : wg_partial_bytes(g, c, kernel_size));
   return kOk;

@@ -421,9 +421,13 @@ void yt_split_cl(int64_t c, int& ihalves, int& mb) {
   if (mb == 3) mb = 4;
 }
 
-int64_t yt_pack_bytes(int64_t c, int k, int dtype) {
+// cl: the channels-last kernel's packing.
+int64_t yt_pack_bytes(int64_t c, int k, int dtype, bool cl) {
   int ih, mb;
-  yt_split_cl(c, ih, mb);  // (at least as large as the plane-major kernel's)
+  if (cl)
+    yt_split_cl(c, ih, mb);
+  else
+    yt_split(c, ih, mb);
   const int64_t nc32 = (c + 31) / 32;
   return (int64_t)ih * 3 * nc32 * k * k * mb * (dtype == kF32 ? 2 : 1) * 64 * 16;
 }
@@ -500,7 +504,11 @@ using namespace ddpm;
 
 extern "C" int64_t ddpm_gen_bwd_y_workspace_bytes(int64_t c, int kernel_size) {
   if (c <= 0 || c > 128 || kernel_size < 1) return 0;
-  return yt_pack_bytes(c, kernel_size, kF32);
+  return yt_pack_bytes(c, kernel_size, kF32, false);
+}
+
+int64_t ddpm::yt_flat_workspace_bytes(int64_t c, int kernel_size, int dtype) {
+  return yt_pack_bytes(c, kernel_size, dtype, dtype != kF32);
 }
 
 int ddpm::yt_run(const void* x, const void* weight, const void* grad_out, void* grad_y,
@@ -513,10 +521,10 @@ int ddpm::yt_run(const void* x, const void* weight, const void* grad_out, void* 
       yt_check(x, weight, grad_out, grad_y, n, c, h, w, kernel_size, d0, d1, d2, dtype, gg, empty);
   if (pack) *pack = YPack{weight, (uint32_t*)workspace, (int)c, (int)((c + 31) / 32), 0};
   if (st != kOk || empty) return st;
-  const int64_t need = yt_pack_bytes(c, kernel_size, dtype);
+  const bool cl = f && dtype != kF32;
+  const int64_t need = yt_pack_bytes(c, kernel_size, dtype, cl);
   if (!workspace || workspace_bytes < need) return kWorkspaceTooSmall;
   if (kernel_size != 1 && kernel_size != 3) return kUnsupported;
-  const bool cl = f && dtype != kF32;
   if (mode == kYtCheck) {
     if (pack) {
       int ih, mb;
@@ -570,7 +578,7 @@ extern "C" int ddpm_gen_bwd_y_noalloc(const void* x, const void* weight, const v
   int st =
       yt_check(x, weight, grad_out, grad_y, n, c, h, w, kernel_size, d0, d1, d2, dtype, gg, empty);
   if (st != kOk || empty) return st;
-  if (yt_pack_bytes(c, kernel_size, dtype) > kYtScratchBytes) return kScratchTooSmall;
+  if (yt_pack_bytes(c, kernel_size, dtype, false) > kYtScratchBytes) return kScratchTooSmall;
   void* packed = nullptr;
   st = scratch_address(&packed);
   if (st != kOk) return st;

@@ -86,6 +86,7 @@ def test_host_only_queries():
     # dY's packed weight: [output-channel halves][3 branches][32-channel chunks][K*K]
     # [16-channel blocks per half][hi, lo][64 lanes] x 16 bytes
     assert lib.ddpm_gen_bwd_y_workspace_bytes(64, 3) == 1 * 3 * 2 * 9 * 4 * 2 * 64 * 16
+    assert lib.ddpm_gen_bwd_y_workspace_bytes(48, 3) == 1 * 3 * 2 * 9 * 3 * 2 * 64 * 16
     assert lib.ddpm_gen_bwd_y_workspace_bytes(96, 3) == 2 * 3 * 3 * 9 * 4 * 2 * 64 * 16
     assert lib.ddpm_gen_bwd_y_workspace_bytes(128, 3) == 2 * 3 * 4 * 9 * 4 * 2 * 64 * 16
     assert lib.ddpm_gen_bwd_y_workspace_bytes(129, 3) == 0
