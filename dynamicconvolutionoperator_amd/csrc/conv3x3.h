@@ -207,6 +207,17 @@ bool cv_flat_rule(FlatLay& f, int64_t n, int64_t k, int64_t h, int64_t w, int es
 bool cv_flat_both(FlatLay& f, int64_t n, int64_t c, int64_t h, int64_t w, int esz);
 // Bytes of its split partials on flat tensors (c <= 128).
 int64_t cw_flat_partial_bytes(const FlatLay& f, int64_t n, int64_t c, int esz);
+// Where the weight gradient's flat copies go in its workspace (byte offsets
+// behind the split partials).
+struct CwCopies {
+  FlatLay f;
+  int64_t cat, go, bytes;
+};
+// Whether it copies its operands flat: cv_flat_both, and a workspace that
+// starts on 16 bytes and holds the copies (else the operands are staged as
+// they lie, which needs the plain split partials alone).
+bool cw_copies(CwCopies& cc, const void* workspace, int64_t workspace_bytes, int64_t n, int64_t c,
+               int64_t h, int64_t w, int esz);
 
 // The fuse convolution's forward weight packing as a descriptor for another
 // launch (defined in conv3x3.hip): validates the forward's shape (n, 4c -> c,

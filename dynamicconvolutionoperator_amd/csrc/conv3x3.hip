@@ -779,11 +779,19 @@ bool cv_flat_both(FlatLay& f, int64_t n, int64_t c, int64_t h, int64_t w, int es
 
 namespace {
 
-// inl: `in` is a flat tensor of that layout with kp planes per image; ol: so
-// is `out`, with m planes.
+int64_t cv_need(const CvPlan& p, int dtype) {
+  return p.copy ? cv_align(cv_workspace_bytes(p.g, dtype)) + p.copy
+                : cv_workspace_bytes(p.g, dtype);
+}
+
+// room: the workspace's bytes.  `in` is copied flat where that pays and the
+// workspace holds the copy, else staged as it lies: a workspace of the packed
+// weight and the partial sums alone is enough for every call.  inl: `in` is a
+// flat tensor of that layout with kp planes per image; oflat: so is `out`,
+// with m planes.
 void cv_plan(CvPlan& p, const void* in, int64_t n, int64_t k, int64_t m, int64_t h, int64_t w,
-             int dtype, bool pairs, bool bias, const FlatLay* inl = nullptr, int64_t kp = 0,
-             bool oflat = false) {
+             int dtype, bool pairs, bool bias, int64_t room, const FlatLay* inl = nullptr,
+             int64_t kp = 0, bool oflat = false) {
   const int esz = dtype == kF32 ? 4 : 2;
   ConvGeom& g = p.g;
   FlatLay f;
@@ -792,8 +800,13 @@ void cv_plan(CvPlan& p, const void* in, int64_t n, int64_t k, int64_t m, int64_t
     inl = &f;
     kp = flat_planes(k);
     p.copy = cv_align(flat_elems(f, n * kp, esz) * esz);
+    cv_geom(g, n, k, m, h, w, esz, inl);
+    if (cv_need(p, dtype) > room) {
+      inl = nullptr;
+      p.copy = 0;
+    }
   }
-  cv_geom(g, n, k, m, h, w, esz, inl, !oflat);
+  if (!p.copy) cv_geom(g, n, k, m, h, w, esz, inl, !oflat);
   g.x4 = (w % 8 == 0) && ((uintptr_t)in % 16 == 0);
   if (inl) {
     p.lay = kCvFlat;
@@ -807,11 +820,6 @@ void cv_plan(CvPlan& p, const void* in, int64_t n, int64_t k, int64_t m, int64_t
   }
   p.nat = esz == 2 && p.lay != kCvGeneric;
   if (!(esz == 4 && p.lay != kCvGeneric && g.mb == 4 && !pairs && !bias)) g.mgl = 1;
-}
-
-int64_t cv_need(const CvPlan& p, int dtype) {
-  return p.copy ? cv_align(cv_workspace_bytes(p.g, dtype)) + p.copy
-                : cv_workspace_bytes(p.g, dtype);
 }
 
 // red (optional): a weight-gradient split reduction for the kernel's
@@ -1019,10 +1027,10 @@ extern "C" int64_t ddpm_fuse_conv_workspace_bytes(int64_t n, int64_t c, int64_t 
   if (dtype == kF32Pairs) dtype = kF32;  // the same packed weight and partials
   if (n < 0 || c <= 0 || h < 0 || w < 0 || dtype < kF32 || dtype > kF16) return 0;
   if (n == 0 || h == 0 || w == 0) return 0;
-  // the larger of the two directions' needs at this shape
+  // the larger of the two directions' needs at this shape, copies included
   CvPlan pf, pd;
-  cv_plan(pf, nullptr, n, 4 * c, c, h, w, dtype, false, true);  // forward: K = 4C, M = C
-  cv_plan(pd, nullptr, n, c, 4 * c, h, w, dtype, false, false);  // input gradient: K = C, M = 4C
+  cv_plan(pf, nullptr, n, 4 * c, c, h, w, dtype, false, true, INT64_MAX);  // forward: K = 4C, M = C
+  cv_plan(pd, nullptr, n, c, 4 * c, h, w, dtype, false, false, INT64_MAX);  // input gradient: K = C, M = 4C
   const int64_t a = cv_need(pf, dtype), b = cv_need(pd, dtype);
   return a > b ? a : b;
 }
@@ -1037,7 +1045,7 @@ extern "C" int ddpm_fuse_conv_fwd(const void* cat, const void* weight, const voi
   if (n == 0 || c == 0 || h == 0 || w == 0) return kOk;
   if (!cat || !weight || !out) return kBadArgument;
   CvPlan plan;
-  cv_plan(plan, cat, n, 4 * c, c, h, w, dtype, pairs, bias != nullptr);
+  cv_plan(plan, cat, n, 4 * c, c, h, w, dtype, pairs, bias != nullptr, workspace_bytes);
   return cv_run(plan, cat, weight, bias, out, workspace, workspace_bytes, 0, dtype, stream, pairs);
 }
 
@@ -1052,7 +1060,7 @@ int ddpm::cv_fwd_pack(CvPack& p, const void* cat, const void* weight, void* work
   if (n == 0 || c == 0 || h == 0 || w == 0) return kOk;
   if (!cat || !weight) return kBadArgument;
   CvPlan plan;
-  cv_plan(plan, cat, n, 4 * c, c, h, w, dtype, pairs, true, f, 4 * c);
+  cv_plan(plan, cat, n, 4 * c, c, h, w, dtype, pairs, true, workspace_bytes, f, 4 * c);
   if (!workspace || workspace_bytes < cv_need(plan, dtype) || (uintptr_t)workspace % 16 != 0)
     return kWorkspaceTooSmall;
   p = cv_pack_of(plan, weight, workspace, 0, pairs);
@@ -1070,7 +1078,7 @@ extern "C" int ddpm_fuse_conv_fwd_packed(const void* cat, const void* bias, void
   if (n == 0 || c == 0 || h == 0 || w == 0) return kOk;
   if (!cat || !out) return kBadArgument;
   CvPlan plan;
-  cv_plan(plan, cat, n, 4 * c, c, h, w, dtype, pairs, bias != nullptr);
+  cv_plan(plan, cat, n, 4 * c, c, h, w, dtype, pairs, bias != nullptr, workspace_bytes);
   return cv_run(plan, cat, nullptr, bias, out, workspace, workspace_bytes, 0, dtype, stream, pairs,
                 nullptr, false);
 }
@@ -1084,7 +1092,7 @@ extern "C" int ddpm_fuse_conv_bwd_data(const void* grad_out, const void* weight,
   if (n == 0 || c == 0 || h == 0 || w == 0) return kOk;
   if (!grad_out || !weight || !grad_cat) return kBadArgument;
   CvPlan plan;
-  cv_plan(plan, grad_out, n, c, 4 * c, h, w, dtype, false, false);
+  cv_plan(plan, grad_out, n, c, 4 * c, h, w, dtype, false, false, workspace_bytes);
   return cv_run(plan, grad_out, weight, nullptr, grad_cat, workspace, workspace_bytes, 1, dtype,
                 stream);
 }
@@ -1109,7 +1117,7 @@ extern "C" int ddpm_fuse_conv_bwd(const void* cat, const void* weight, const voi
                   n, c, h, w, dtype, stream, false, nullptr, nullptr);
   if (!grad_out || !weight || !grad_cat) return kBadArgument;
   CvPlan plan;
-  cv_plan(plan, grad_out, n, c, 4 * c, h, w, ddt, false, false);
+  cv_plan(plan, grad_out, n, c, 4 * c, h, w, ddt, false, false, workspace_data_bytes);
   if (!workspace_data || workspace_data_bytes < cv_need(plan, ddt) ||
       (uintptr_t)workspace_data % 16 != 0)
     return kWorkspaceTooSmall;
@@ -1119,13 +1127,13 @@ extern "C" int ddpm_fuse_conv_bwd(const void* cat, const void* weight, const voi
   // split partials
   const CvPack pack = cv_pack_of(plan, weight, workspace_data, 1, false);
   const FlatLay f = plan.g.f;
-  FlatLay fb;
-  const bool flat = plan.copy != 0 && cv_flat_both(fb, n, c, h, w, ddt == kF32 ? 4 : 2);
+  const int esz = ddt == kF32 ? 4 : 2;
+  CwCopies cc;
+  const bool flat = plan.copy != 0 && cw_copies(cc, workspace_weight, workspace_weight_bytes, n, c, h, w, esz);
   if (flat) {
     // grad_out flat once for both launches, the concat for the weight gradient
     void* gof = (char*)workspace_data + cv_align(cv_workspace_bytes(plan.g, ddt));
-    void* catf = (char*)workspace_weight + cv_align(cw_flat_partial_bytes(f, n, c, ddt == kF32 ? 4 : 2));
-    const int esz = ddt == kF32 ? 4 : 2;
+    void* catf = (char*)workspace_weight + cc.cat;
     const FlatCopy fc[2] = {flat_copy_of(grad_out, gof, f, n, c, plan.g.kp, esz),
                             flat_copy_of(cat, catf, f, n, 4 * c, 4 * c, esz)};
     st = flat_copy(fc, 2, f, ddt, stream, &pack);
@@ -1168,7 +1176,7 @@ void cv_flat_bwd(CvFlatBwd& b, const FlatLay& f, int64_t n, int64_t c, int64_t h
                  int dtype) {
   const int esz = dtype == kF32 ? 4 : 2;
   b.cp = flat_planes(c);
-  cv_plan(b.plan, nullptr, n, c, 4 * c, h, w, dtype, false, false, &f, b.cp, true);
+  cv_plan(b.plan, nullptr, n, c, 4 * c, h, w, dtype, false, false, INT64_MAX, &f, b.cp, true);
   b.go = cv_align(flat_elems(f, n * b.cp, esz) * esz);
   b.data = cv_align(cv_need(b.plan, dtype));
   b.weight = cv_align(cw_flat_partial_bytes(f, n, c, esz));
@@ -1184,7 +1192,7 @@ extern "C" int64_t ddpm_flat_fuse_conv_workspace_bytes(int64_t n, int64_t c, int
   if (cv_flat_check(f, n, c, h, w, guard, dtype) != kOk) return 0;
   if (n == 0 || c == 0 || h == 0 || w == 0) return 0;
   CvPlan plan;
-  cv_plan(plan, nullptr, n, 4 * c, c, h, w, dtype, pairs, true, &f, 4 * c);
+  cv_plan(plan, nullptr, n, 4 * c, c, h, w, dtype, pairs, true, INT64_MAX, &f, 4 * c);
   return cv_need(plan, dtype);
 }
 
@@ -1200,7 +1208,7 @@ extern "C" int ddpm_flat_fuse_conv_fwd_packed(const void* cat, const void* bias,
   if (n == 0 || c == 0 || h == 0 || w == 0) return kOk;
   if (!cat || !out || (uintptr_t)cat % 16 != 0) return kBadArgument;
   CvPlan plan;
-  cv_plan(plan, cat, n, 4 * c, c, h, w, dtype, pairs, bias != nullptr, &f, 4 * c);
+  cv_plan(plan, cat, n, 4 * c, c, h, w, dtype, pairs, bias != nullptr, workspace_bytes, &f, 4 * c);
   return cv_run(plan, cat, nullptr, bias, out, workspace, workspace_bytes, 0, dtype, stream, pairs,
                 nullptr, false);
 }

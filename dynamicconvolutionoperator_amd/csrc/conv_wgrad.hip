@@ -693,30 +693,29 @@ namespace {
 
 int64_t cw_align(int64_t v) { return (v + 255) / 256 * 256; }
 
-// Workspace where cat and grad_out are copied flat: the split partials, the
-// concat (4C planes), grad_out.
-int64_t cw_copy_bytes(const FlatLay& f, int64_t n, int64_t c, int esz, int64_t& cat_off,
-                      int64_t& go_off) {
-  cat_off = cw_align(cw_flat_partial_bytes(f, n, c, esz));
-  go_off = cat_off + cw_align(flat_elems(f, n * 4 * c, esz) * esz);
-  return go_off + flat_elems(f, n * flat_planes(c), esz) * esz;
-}
-
 }  // namespace
+
+bool ddpm::cw_copies(CwCopies& cc, const void* workspace, int64_t workspace_bytes, int64_t n,
+                     int64_t c, int64_t h, int64_t w, int esz) {
+  if (!cv_flat_both(cc.f, n, c, h, w, esz)) return false;
+  cc.cat = cw_align(cw_flat_partial_bytes(cc.f, n, c, esz));
+  cc.go = cc.cat + cw_align(flat_elems(cc.f, n * 4 * c, esz) * esz);
+  cc.bytes = cc.go + flat_elems(cc.f, n * flat_planes(c), esz) * esz;
+  return workspace && workspace_bytes >= cc.bytes && (uintptr_t)workspace % 16 == 0;
+}
 
 extern "C" int64_t ddpm_fuse_conv_bwd_weight_workspace_bytes(int64_t n, int64_t c, int64_t h,
                                                              int64_t w, int dtype) {
   if (dtype == kF32Pairs) dtype = kF32;  // the same partials
   if (n <= 0 || c <= 0 || h <= 0 || w <= 0 || dtype < kF32 || dtype > kF16) return 0;
   if (n * h * ((w + kCwTW - 1) / kCwTW) > 0x7fffffffLL) return 0;
-  FlatLay f;
-  if (cv_flat_both(f, n, c, h, w, dtype == kF32 ? 4 : 2)) {
-    int64_t a, b;
-    return cw_copy_bytes(f, n, c, dtype == kF32 ? 4 : 2, a, b);
-  }
   CwGeom g;
   cw_geom(g, n, c, h, w, cw_step_cols(w, dtype == kF32 ? 4 : 2));
-  return cw_partial_bytes(g);
+  const int64_t plain = cw_partial_bytes(g);
+  CwCopies cc;
+  cc.bytes = 0;
+  cw_copies(cc, nullptr, 0, n, c, h, w, dtype == kF32 ? 4 : 2);
+  return cc.bytes > plain ? cc.bytes : plain;
 }
 
 int ddpm::cw_run(const void* cat, const void* grad_out, void* grad_weight, void* grad_bias,
@@ -752,21 +751,17 @@ int ddpm::cw_run(const void* cat, const void* grad_out, void* grad_weight, void*
   if (n * h * ((w + kCwTW - 1) / kCwTW) > 0x7fffffffLL) return kUnsupported;
   // 32-bit buffer offsets inside one image's planes
   if (4 * c * h * w * esz > 0x7fffffffLL) return kUnsupported;
-  FlatLay fr;
-  if (!f && cv_flat_both(fr, n, c, h, w, esz)) {
-    int64_t cat_off, go_off;
-    const int64_t need = cw_copy_bytes(fr, n, c, esz, cat_off, go_off);
-    if (!workspace || workspace_bytes < need || (uintptr_t)workspace % 16 != 0)
-      return kWorkspaceTooSmall;
+  CwCopies cc;
+  if (!f && cw_copies(cc, workspace, workspace_bytes, n, c, h, w, esz)) {
     if (check_only) return kOk;
-    void* catf = (char*)workspace + cat_off;
-    void* gof = (char*)workspace + go_off;
-    const FlatCopy fc[2] = {flat_copy_of(cat, catf, fr, n, 4 * c, 4 * c, esz),
-                            flat_copy_of(grad_out, gof, fr, n, c, flat_planes(c), esz)};
-    const int e = flat_copy(fc, 2, fr, dtype, stream);
+    void* catf = (char*)workspace + cc.cat;
+    void* gof = (char*)workspace + cc.go;
+    const FlatCopy fc[2] = {flat_copy_of(cat, catf, cc.f, n, 4 * c, 4 * c, esz),
+                            flat_copy_of(grad_out, gof, cc.f, n, c, flat_planes(c), esz)};
+    const int e = flat_copy(fc, 2, cc.f, dtype, stream, pack);
     if (e != kOk) return e;
-    return cw_run(catf, gof, grad_weight, grad_bias, workspace, cat_off, n, c, h, w,
-                  pp ? (int)kF32Pairs : dtype, stream, false, pack, defer, &fr, flat_planes(c));
+    return cw_run(catf, gof, grad_weight, grad_bias, workspace, cc.cat, n, c, h, w,
+                  pp ? (int)kF32Pairs : dtype, stream, false, nullptr, defer, &cc.f, flat_planes(c));
   }
   CwGeom g;
   ClWGeom cg{};

@@ -256,12 +256,15 @@ int ddpm_gen_bwd(const void* x, const void* y, const void* weight, const void* b
 
 /* ---- the 3x3 fuse convolution (Conv2d(4C -> C, 3, padding 1)) -------- */
 
-/* Bytes of workspace ddpm_fuse_conv_fwd / _bwd_data need at this shape: the
- * packed weight (MFMA fragment order; fp32 as bf16 hi / lo) and, where the
+/* Bytes of workspace for ddpm_fuse_conv_fwd / _bwd_data at this shape: the
+ * packed weight (MFMA fragment order; fp32 as bf16 hi / lo), where the
  * image is too small to fill the GPU with whole input-plane loops (e.g.
- * 128x128 C=64 forward), the fp32 partial sums of the input-plane splits,
- * summed by a second kernel in split order.  The larger of the two
- * directions, so one buffer serves both. */
+ * 128x128 C=64 forward) the fp32 partial sums of the input-plane splits,
+ * summed by a second kernel in split order, and at widths that are not
+ * multiples of 8 a copy of the input with rows padded to 16 bytes.  The larger
+ * of the two directions, so one buffer serves both.  A workspace without room
+ * for the copy is accepted too: the rows are then staged element by element
+ * (at bf16 1x64x135x181 129 instead of 30 us), the sums in another order. */
 int64_t ddpm_fuse_conv_workspace_bytes(int64_t n, int64_t c, int64_t h, int64_t w, int dtype);
 
 /* out[n][co][h][w] = bias[co] + sum_{ci,ki,kj} weight[co][ci][ki][kj] *
@@ -290,7 +293,8 @@ int ddpm_gen_fwd_pack(const void* x, const void* y, const void* weight, const vo
                       int d2, int dtype, hipStream_t stream);
 
 /* ddpm_fuse_conv_fwd whose workspace already holds the packed weight that
- * ddpm_gen_fwd_pack wrote for this concat (same shape, dtype and buffer). */
+ * ddpm_gen_fwd_pack wrote for this concat (same shape, dtype and buffer, and
+ * the same workspace_bytes in both calls). */
 int ddpm_fuse_conv_fwd_packed(const void* cat, const void* bias, void* out, void* workspace,
                               int64_t workspace_bytes, int64_t n, int64_t c, int64_t h, int64_t w,
                               int dtype, hipStream_t stream);
@@ -303,9 +307,12 @@ int ddpm_fuse_conv_bwd_data(const void* grad_out, const void* weight, void* grad
                             void* workspace, int64_t workspace_bytes, int64_t n, int64_t c,
                             int64_t h, int64_t w, int dtype, hipStream_t stream);
 
-/* Bytes of workspace ddpm_fuse_conv_bwd_weight needs for `dtype`: fp32
- * split partials of the weight and bias gradients (none with one split; the
- * same for every dtype). */
+/* Bytes of workspace for ddpm_fuse_conv_bwd_weight with `dtype`: fp32 split
+ * partials of the weight and bias gradients (none with one split) and, at
+ * widths that are not multiples of 8 with c % 8 == 0, copies of the concat and of
+ * grad_out with rows padded to 16 bytes.  The partials alone (the same for
+ * every dtype), or a workspace that does not start on 16 bytes, are accepted
+ * too: the rows are then staged element by element, the sums in another order. */
 int64_t ddpm_fuse_conv_bwd_weight_workspace_bytes(int64_t n, int64_t c, int64_t h, int64_t w,
                                                   int dtype);
 
@@ -324,9 +331,11 @@ int ddpm_fuse_conv_bwd_weight(const void* cat, const void* grad_out, void* grad_
 
 /* Input, weight and bias gradients of the fuse convolution in one call
  * (ddpm_fuse_conv_bwd_weight, then ddpm_fuse_conv_bwd_data), bit-identical to
- * the two calls in two launches instead of four: the weight-gradient launch's
- * workgroups also pack the input gradient's weight, and the input-gradient
- * launch's workgroups also sum the weight gradient's split partials.
+ * the two calls with the same workspaces in two launches instead of four: the
+ * weight-gradient launch's workgroups also pack the input gradient's weight,
+ * and the input-gradient launch's workgroups also sum the weight gradient's
+ * split partials.  Where the operands are copied, one launch before the two
+ * copies both and packs the weight.
  * `dtype` is the concat's code (3: pair planes; grad_out, weight and grad_cat
  * are then plain fp32).  workspace_data as for ddpm_fuse_conv_bwd_data
  * (ddpm_fuse_conv_workspace_bytes), workspace_weight as for

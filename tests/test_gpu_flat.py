@@ -5,7 +5,7 @@ copies of the stand-alone fuse convolution, against the fp64 oracle."""
 import pytest
 import torch
 
-from dynamicconvolutionoperator_amd import DDPM, ops
+from dynamicconvolutionoperator_amd import DDPM, _lib, ops
 from oracle import unfold_ref
 from oracle.unfold_ref import UnfoldDDPM
 from tests.gpu_helpers import DEV, DIL, TOL, assert_close, default_generator_params, randn, say
@@ -226,3 +226,60 @@ def test_paired_forward_of_infinite_kernels(c, dtype):
     out = ops.fused_generator_dynamic_cat(x.to(DEV), y.to(DEV), wt.to(DEV), b.to(DEV), 3, DIL).cpu()
     want = unfold_ref.generator_dynamic_cat(x.double(), y.double(), wt.double(), b.double(), 3)
     assert torch.equal(torch.isinf(out), torch.isinf(want)) and not bool(torch.isnan(out).any())
+
+
+@pytest.mark.parametrize("code,dtype", [(0, torch.float32), (1, torch.bfloat16)])
+def test_stand_alone_fuse_conv_workspaces(code, dtype):
+    """At an odd width the fuse convolution copies its operands flat; a
+    workspace without room for the copies (the packed weight and the partial
+    sums alone), one off a 16-byte boundary for the weight gradient, and none
+    where a single split needs none, give the same gradients without them."""
+    lib = _lib.load()
+    n, c, h, w = 1, 64, 135, 181
+    stream = torch.cuda.current_stream().cuda_stream
+    cat, g = randn((n, 4 * c, h, w), 1).to(dtype).to(DEV), randn((n, c, h, w), 2).to(dtype).to(DEV)
+    wt, b = randn((c, 4 * c, 3, 3), 3, scale=0.05).to(dtype).to(DEV), randn((c,), 4).to(dtype).to(DEV)
+
+    def buffers():
+        shapes = (g.shape, cat.shape, wt.shape, b.shape)
+        return [torch.full(s, float("nan"), dtype=dtype, device=DEV) for s in shapes]
+
+    def memory(nbytes, off=0):
+        return torch.empty(nbytes + 16, dtype=torch.uint8, device=DEV)[off:]
+
+    query = lib.ddpm_fuse_conv_workspace_bytes(n, c, h, w, code)
+    query_w = lib.ddpm_fuse_conv_bwd_weight_workspace_bytes(n, c, h, w, code)
+    # forward: 8 chunks of 32 planes x 9 taps x 4 blocks x 1 KB (fp32: hi and lo),
+    # two plane splits; weight gradient: 16 splits of 36 C^2 + C
+    plain = 8 * 9 * 4 * 1024 * (2 if code == 0 else 1) + 2 * n * c * h * w * 4
+    plain_w = 16 * (36 * c * c + c) * 4
+    assert plain < query and plain_w < query_w
+    results = []
+    for size, size_w, off in ((query, query_w, 0), (plain, plain_w, 0), (query, plain_w, 0),
+                              (plain, query_w, 0), (query, query_w, 4)):
+        out, gc, gw, gb = buffers()
+        ws, wsw = memory(size), memory(size_w, off)
+        rc = lib.ddpm_fuse_conv_fwd(cat.data_ptr(), wt.data_ptr(), b.data_ptr(), out.data_ptr(), ws.data_ptr(),
+                                    size, n, c, h, w, code, stream)
+        assert rc == 0, rc
+        rc = lib.ddpm_fuse_conv_bwd(cat.data_ptr(), wt.data_ptr(), g.data_ptr(), gc.data_ptr(), gw.data_ptr(),
+                                    gb.data_ptr(), ws.data_ptr(), size, wsw.data_ptr(), size_w, n, c, h, w,
+                                    code, stream)
+        assert rc == 0, rc
+        results.append((out, gc, gw, gb))
+        _, _, gw, gb = buffers()
+        rc = lib.ddpm_fuse_conv_bwd_weight(cat.data_ptr(), g.data_ptr(), gw.data_ptr(), gb.data_ptr(),
+                                           wsw.data_ptr(), size_w, n, c, h, w, code, stream)
+        assert rc == 0, rc
+        assert torch.equal(gw, results[-1][2]) and torch.equal(gb, results[-1][3])
+    for got in results[1:]:
+        for name, a, e in zip(("out", "dcat", "dw", "db"), got, results[0]):
+            # the same products in another order: fp32 sums, then one rounding
+            tol = 2e-5 if dtype == torch.float32 else 1e-2
+            assert_close(a, e.double().cpu(), tol * e.abs().max().item(), tol, name)
+    _, _, gw, gb = buffers()
+    few = cat[:, :, :1, :17].contiguous(), g[:, :, :1, :17].contiguous()
+    rc = lib.ddpm_fuse_conv_bwd_weight(few[0].data_ptr(), few[1].data_ptr(), gw.data_ptr(), gb.data_ptr(), None,
+                                       0, n, c, 1, 17, code, stream)
+    torch.cuda.synchronize()
+    assert rc == 0 and not bool(torch.isnan(gw).any()), rc
