@@ -733,6 +733,13 @@ def _fuse_conv_forward_packed(cat, ws, fuse_bias, shape, guard):
     return out
 
 
+def _on_16_bytes(t):
+    """t, or a copy where it does not start on 16 bytes: a flat tensor that came
+    back through autograd may be another one (saved-tensor hooks, hooks on the
+    gradient)."""
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
 def _flat_fuse_conv_backward(cat, weight, has_bias, grad_out, needs, shape, guard):
     """:func:`_fuse_conv_backward` of a flat concat, the concat's gradient flat
     too."""
@@ -741,6 +748,7 @@ def _flat_fuse_conv_backward(cat, weight, has_bias, grad_out, needs, shape, guar
     need_w = needs[1] or (has_bias and needs[2])
     if not (needs[0] or need_w):
         return None, None, None
+    cat = _on_16_bytes(cat)
     grad_cat = torch.empty_like(cat) if needs[0] else None
     gw = torch.empty_like(weight) if need_w else None
     gb = torch.empty((c,), dtype=weight.dtype, device=cat.device) if need_w else None
@@ -762,6 +770,7 @@ def _flat_generator_backward(x, y, weight, bias, grad_cat, k, dil, needs, guard)
     need_wb = needs[2] or needs[3]
     if not (needs[0] or needs[1] or need_wb):
         return None, None, None, None
+    grad_cat = _on_16_bytes(grad_cat)
     gx = torch.empty_like(x) if needs[0] else None
     gy = torch.empty_like(y) if needs[1] else None
     gw = torch.empty_like(weight) if need_wb else None

@@ -283,3 +283,24 @@ def test_stand_alone_fuse_conv_workspaces(code, dtype):
                                        0, n, c, 1, 17, code, stream)
     torch.cuda.synchronize()
     assert rc == 0 and not bool(torch.isnan(gw).any()), rc
+
+
+def test_flat_backward_of_tensors_off_16_bytes():
+    """Saved-tensor and gradient hooks may hand back tensors that start anywhere."""
+    _, mod = _modules(32, 3, torch.bfloat16)
+    x, y, g = (randn((1, 32, 45, 51), s, dtype=torch.bfloat16).to(DEV).requires_grad_() for s in (1, 2, 3))
+    leaves = (x, y, *mod.parameters())
+
+    def unaligned(t):
+        if t is None or t.dtype != torch.bfloat16:
+            return t
+        buf = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
+        return buf[1:].view(t.shape).copy_(t)
+
+    want = torch.autograd.grad(mod(x, y), leaves, g)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unaligned):
+        out = mod(x, y)
+        out.grad_fn.register_hook(lambda grads_in, grads_out: tuple(unaligned(t) for t in grads_in))
+        got = torch.autograd.grad(out, leaves, g)
+    for a, e in zip(got, want):
+        assert torch.equal(a, e)
