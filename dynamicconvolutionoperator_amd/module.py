@@ -27,7 +27,7 @@ of autograd ops (``ops.fused_ddpm``) whose generator launch also packs the
 fuse weight; an fp32 concat (C % 16 == 0) is stored as bf16 pair planes,
 already split the way the fuse convolution's fp32 MFMA products need it.  At
 widths that are not whole steps of the kernels the concat's rows are padded to
-a pitch of their own (``ops._flat_guard``).
+a pitch of their own (``ops._flat_pays``).
 """
 
 from __future__ import annotations

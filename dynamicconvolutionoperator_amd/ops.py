@@ -668,46 +668,70 @@ def _cat_code(dtype: torch.dtype) -> int:
     return _PAIR_PLANES if dtype == torch.float32 else _DTYPES[dtype]
 
 
+def _flat_pays(n, c, h, w, code, training) -> bool:
+    """Whether rows of w columns are better held flat.  Plain rows win where they
+    are whole steps of the kernels: multiples of 256 columns, and 128 in
+    training (C = 64, us a pass, plain / flat: fp32 1x128x128 201 / 229, bf16
+    4x128x128 300 / 305); every other width leaves lanes idle at row ends (8x48x48
+    fp32 342 / 259, bf16 241 / 167) or, not a multiple of 8, is staged element by
+    element (bf16 2x135x181 1034 plain).
+
+    Inference at 32, 64 and 128 columns: fp32 stays plain (16x64x64 112 / 146).
+    2-byte types gain from channels-last (1x128x128 43 / 37, 5x128x128 108 / 94)
+    unless, at up to 64 channels, the padded columns take one more round of
+    256-position tiles over 256 CUs (4x128x128, 256 / 272 tiles, 72 / 78; from
+    96 channels on the same (144 / 144), or the call is a few tiles above 64
+    channels (C = 128, 1x32x32 43 / 45, 4x32x32 44 / 46, 4x64x64 79 / 76)."""
+    if w % 256 == 0 or (training and w == 128):
+        return False
+    if training or w not in (32, 64, 128):
+        return True
+    if code == _PAIR_PLANES:
+        return False
+    if c > 64:
+        return n * h * w > 4096
+    plain, flat = n * -(-h * w // 256), n * -(-h * (w + 8) // 256)
+    return -(-plain // 256) == -(-flat // 256)
+
+
+@functools.lru_cache(maxsize=512)
+def _concat_plan(n, c, h, w, k, max_dil, code, training, flat) -> tuple[int, int, int]:
+    """How the concat between generator and fuse convolution is held, for one
+    shape (a pure function of it): guard rows and columns of the flat layout
+    (``ddpm_flat_*``: rows padded with zeros, tiles of 256 positions whatever the
+    width; 2-byte types channels-last) or 0 for the plain one, the flat concat's
+    elements, and the bytes of the fuse convolution's forward workspace.  One
+    lookup per call: the flat queries each had cost the host 0.4 us."""
+    if flat and _flat_pays(n, c, h, w, code, training):
+        guard = max(1, (k // 2) * max_dil) if training else 1
+        elems = _ws_bytes("ddpm_flat_cat_elems", n, c, h, w, guard, code)
+        if elems > 0:
+            return guard, elems, _ws_bytes("ddpm_flat_fuse_conv_workspace_bytes", n, c, h, w, guard, code)
+    return 0, 0, _ws_bytes("ddpm_fuse_conv_workspace_bytes", n, c, h, w, code)
+
+
 def _flat_guard(x, k, dil, code, training) -> int:
-    """Guard rows and columns of the flat concat (``ddpm_flat_*``: rows padded
-    with zeros, tiles of 256 positions whatever the width; 2-byte types
-    channels-last) that this shape takes between generator and fuse
-    convolution, or 0 for the plain one.  Plain rows win where they are whole
-    steps of the kernels (C = 64 training: fp32 1x128x128 204 us plain, 230
-    flat, bf16 4x128x128 317 / 335, 8x256x256 1971 / 2015); every other width
-    leaves lanes idle at row ends (8x64x64 fp32 390 plain, 327 flat, bf16 272 /
-    200) or, not a multiple of 8, is staged element by element (bf16
-    2x135x181 1034 us plain).  Inference has no copies to pay for: 2-byte types
-    take the flat concat at 32, 64 and 128 columns too (1x128x128 39.9 us
-    plain, 35.9 flat), fp32 does not (51 / 53)."""
-    n, c, h, w = x.shape
-    if w % 256 == 0 or (w == 128 and (training or x.dtype == torch.float32)):
-        return 0
-    if not training and x.dtype == torch.float32 and w in (32, 64):
-        return 0
-    guard = max(1, (k // 2) * max(dil)) if training else 1
-    return guard if _ws_bytes("ddpm_flat_cat_elems", n, c, h, w, guard, code) > 0 else 0
+    """The guard of x's flat concat on the module's route, or 0 (:func:`_concat_plan`)."""
+    return _concat_plan(*x.shape, k, max(dil), code, training, True)[0]
 
 
-def _concat_pack(x, y, gen_weight, gen_bias, fuse_weight, k, dil, guard):
+def _concat_pack(x, y, gen_weight, gen_bias, fuse_weight, k, dil, plan):
     """ddpm_gen_fwd_pack (or its flat form): the concat (fp32 as pair planes)
     and, in the fuse convolution's workspace, its packed weight (returned with
-    it)."""
+    it).  ``plan``: :func:`_concat_plan`'s."""
     n, c, h, w = x.shape
     code = _cat_code(x.dtype)
+    guard, elems, nbytes = plan
     lib = _lib.load()
     with _on(x.device):
+        ws = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=x.device)
         if guard:
-            cat = torch.empty(_ws_bytes("ddpm_flat_cat_elems", n, c, h, w, guard, code), dtype=x.dtype,
-                              device=x.device)
-            nbytes = _ws_bytes("ddpm_flat_fuse_conv_workspace_bytes", n, c, h, w, guard, code)
-            ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
+            cat = torch.empty(elems, dtype=x.dtype, device=x.device)
             rc = lib.ddpm_flat_gen_fwd_pack(
                 _ptr(x), _ptr(y), _ptr(gen_weight), _ptr(gen_bias), _ptr(cat), _ptr(fuse_weight),
                 _ptr(ws), nbytes, n, c, h, w, k, *dil, guard, code, _stream(x))
         else:
             cat = torch.empty((n, 4 * c, h, w), dtype=x.dtype, device=x.device)
-            ws, nbytes = _fuse_conv_workspace(n, c, h, w, code, x.device)
             rc = lib.ddpm_gen_fwd_pack(_ptr(x), _ptr(y), _ptr(gen_weight), _ptr(gen_bias), _ptr(cat),
                                        _ptr(fuse_weight), _ptr(ws), nbytes, n, c, h, w, k, *dil, code,
                                        _stream(x))
@@ -796,12 +820,12 @@ class _GeneratorConcat(torch.autograd.Function):
     beside the concat (no gradient)."""
 
     @staticmethod
-    def forward(ctx, x, y, gen_weight, gen_bias, fuse_weight, kernel_size, dilations, guard):
-        cat, ws = _concat_pack(x, y, gen_weight, gen_bias, fuse_weight, kernel_size, dilations, guard)
+    def forward(ctx, x, y, gen_weight, gen_bias, fuse_weight, kernel_size, dilations, plan):
+        cat, ws = _concat_pack(x, y, gen_weight, gen_bias, fuse_weight, kernel_size, dilations, plan)
         ctx.save_for_backward(x, y, gen_weight, gen_bias)
         ctx.kernel_size = kernel_size
         ctx.dilations = dilations
-        ctx.guard = guard
+        ctx.guard = plan[0]
         ctx.mark_non_differentiable(ws)
         # no zero-filled gradient for the workspace output (a fill kernel per step)
         ctx.set_materialize_grads(False)
@@ -866,7 +890,7 @@ def fused_ddpm(x, y, gen_weight, gen_bias, fuse_weight, fuse_bias, kernel_size, 
 def _fused_ddpm_checked(x, y, gen_weight, gen_bias, fuse_weight, fuse_bias, k, dil, flat=False):
     """:func:`fused_ddpm` for arguments :func:`fused_ddpm_supported` has
     accepted (k an int, dil a tuple of three ints).  ``flat``: the concat may
-    be a flat one (:func:`_flat_guard`), whose tiles sum in another order
+    be a flat one (:func:`_flat_pays`), whose tiles sum in another order
     than the separate ops'."""
     x, y = x.contiguous(), y.contiguous()
     gen_weight, gen_bias = gen_weight.contiguous(), gen_bias.contiguous()
@@ -874,13 +898,13 @@ def _fused_ddpm_checked(x, y, gen_weight, gen_bias, fuse_weight, fuse_bias, k, d
     fuse_bias = fuse_bias.contiguous() if fuse_bias is not None else None
     tensors = (x, y, gen_weight, gen_bias, fuse_weight, fuse_bias)
     shape = tuple(x.shape)
-    if torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors):
-        guard = _flat_guard(x, k, dil, _cat_code(x.dtype), True) if flat else 0
-        cat, ws = _GeneratorConcat.apply(x, y, gen_weight, gen_bias, fuse_weight, k, dil, guard)
-        return _FuseConvOfConcat.apply(cat, ws, fuse_weight, fuse_bias, shape, guard)
-    guard = _flat_guard(x, k, dil, _cat_code(x.dtype), False) if flat else 0
-    cat, ws = _concat_pack(x, y, gen_weight, gen_bias, fuse_weight, k, dil, guard)
-    return _fuse_conv_forward_packed(cat, ws, fuse_bias, shape, guard)
+    training = torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors)
+    plan = _concat_plan(*shape, k, max(dil), _cat_code(x.dtype), training, flat)
+    if training:
+        cat, ws = _GeneratorConcat.apply(x, y, gen_weight, gen_bias, fuse_weight, k, dil, plan)
+        return _FuseConvOfConcat.apply(cat, ws, fuse_weight, fuse_bias, shape, plan[0])
+    cat, ws = _concat_pack(x, y, gen_weight, gen_bias, fuse_weight, k, dil, plan)
+    return _fuse_conv_forward_packed(cat, ws, fuse_bias, shape, plan[0])
 
 
 __all__ = [

@@ -346,3 +346,24 @@ def test_bench_prices_every_step_entry_point():
     for name in step:
         nbytes, flops = bench.work_per_launch(name, 4)
         assert nbytes > 0, name
+
+
+@pytest.mark.parametrize("shape,code,training,expect", [
+    # (whole kernel steps: plain rows)
+    ((1, 64, 256, 256), 1, True, 0), ((4, 64, 128, 128), 1, True, 0), ((1, 64, 9, 512), 3, False, 0),
+    # other widths, multiples of 8 and odd ones; the guard holds the halo only where a backward follows
+    ((2, 64, 96, 96), 3, True, 5), ((2, 64, 135, 181), 1, True, 5), ((1, 32, 48, 48), 3, False, 1),
+    # inference at 32, 64 and 128 columns: fp32 plain; 2-byte types flat ...
+    ((4, 64, 64, 64), 3, False, 0), ((1, 64, 128, 128), 1, False, 1), ((5, 64, 128, 128), 2, False, 1),
+    # ... unless the padding takes one more round of tiles (256 / 272, 512 / 544),
+    # which more than 64 channels hide, or those have only a few tiles
+    ((4, 64, 128, 128), 1, False, 0), ((8, 32, 128, 128), 2, False, 0), ((16, 64, 64, 64), 1, False, 0),
+    ((4, 96, 128, 128), 1, False, 1), ((4, 128, 32, 32), 1, False, 0), ((4, 128, 64, 64), 1, False, 1),
+    # shapes the flat entry points do not take, and empty ones
+    ((1, 136, 20, 30), 1, False, 0), ((0, 64, 20, 30), 1, False, 0),
+])
+def test_flat_concat_rule(shape, code, training, expect):
+    from dynamicconvolutionoperator_amd import ops
+
+    assert ops._concat_plan(*shape, 3, 5, code, training, True)[0] == expect
+    assert ops._concat_plan(*shape, 3, 5, code, training, False)[:2] == (0, 0)
