@@ -226,8 +226,9 @@ __global__ __launch_bounds__(kClcThreads) __attribute__((amdgpu_waves_per_eu(2))
   __syncthreads();
 
   // One block of 16 positions and 16 output planes from m, straight from the
-  // accumulators.  Whether a block's
-  // position lies inside the image (flat outputs hold zero elsewhere):
+  // accumulators (input planes unsplit: the pairs of m groups, and the concat
+  // gradient).  Whether a block's position lies inside the image (flat outputs
+  // hold zero elsewhere):
   bool inside[NB4];
 #pragma unroll
   for (int blk = 0; blk < NB4; ++blk) {
@@ -237,14 +238,6 @@ __global__ __launch_bounds__(kClcThreads) __attribute__((amdgpu_waves_per_eu(2))
   auto store = [&](f32x4 v, int m, int blk) {
     const int pos = p0 + pw + 16 * blk + col16;
     if (m >= g.M) return;
-    if (g.ks > 1) {
-      const uint32_t FS = flat_span(g.f);
-      float* __restrict__ po = part + (((size_t)ksplit * g.N + n) * g.M + m) * FS + pos;
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (m + e < g.M) po[(size_t)e * FS] = v[e];
-      return;
-    }
     if (g.out == kClOutImage) {
       if (!inside[blk]) return;
       const int row = pos / g.f.P, col = pos - row * g.f.P;
@@ -295,7 +288,7 @@ __global__ __launch_bounds__(kClcThreads) __attribute__((amdgpu_waves_per_eu(2))
       __builtin_amdgcn_raw_buffer_store_b64((u32x2){d0, d1}, ores, vo, so, 0);
     }
   };
-  const bool grad16 = g.out == kClOutGrad && g.C % 16 == 0 && g.ks == 1;
+  const bool grad16 = g.out == kClOutGrad && g.C % 16 == 0;
   // sums of 8 positions of plane m into the image (cols: of one row, P % 8 == 0)
   auto store8 = [&](const float (&v)[8], int m, int pos) {
     const int row = pos / g.f.P, col = pos - row * g.f.P;

@@ -636,8 +636,8 @@ void cv_split_cl(ConvGeom& g, int64_t tiles, int64_t m, bool split) {
 // x 3 = 204 workgroups of half again the stages 24 us): the choice minimizes
 // rounds x stages by the measured cost of a stage (us, of one or more m
 // blocks) and of the partials' second pass.
-void cv_split_flat(ConvGeom& g, int64_t tiles, int64_t m, int esz) {
-  const double base = esz == 4 ? 0.65 : 0.45, per = esz == 4 ? 0.36 : 0.14;
+void cv_split_flat(ConvGeom& g, int64_t tiles, int64_t m) {
+  const double base = 0.65, per = 0.36;
   double best = 1e30;
   for (int mb = kCvMaxMB; mb >= 1; mb /= 2) {
     const int64_t groups = (m + mb * 16 - 1) / (mb * 16);
@@ -694,7 +694,7 @@ void cv_geom(ConvGeom& g, int64_t n, int64_t k, int64_t m, int64_t h, int64_t w,
   if (f && esz == 2) {
     cv_split_cl(g, tiles, m, split);
   } else if (f) {
-    cv_split_flat(g, tiles, m, esz);
+    cv_split_flat(g, tiles, m);
   } else {
     while (tiles * mg4 * g.ks < kCvFillWGs && 2 * g.ks * 2 <= g.nc32) g.ks *= 2;
     g.cc_per = (g.nc32 + g.ks - 1) / g.ks;

@@ -662,9 +662,9 @@ void cw_geom(CwGeom& g, int64_t n, int64_t c, int64_t h, int64_t w, int tw) {
   g.f = FlatLay{};
 }
 
-// The same for flat tensors: a plane is one row of f.ft * 256 positions.
-void cw_geom_flat(CwGeom& g, const FlatLay& f, int64_t n, int64_t c, int esz, bool pp) {
-  cw_geom(g, n, c, 1, (int64_t)f.ft * kFlatTile, esz == 2 && !pp ? 2 * kCwTW : kCwTW);
+// The same for flat fp32 tensors: a plane is one row of f.ft * 256 positions.
+void cw_geom_flat(CwGeom& g, const FlatLay& f, int64_t n, int64_t c) {
+  cw_geom(g, n, c, 1, (int64_t)f.ft * kFlatTile, kCwTW);
   g.f = f;
 }
 
@@ -685,7 +685,7 @@ int64_t ddpm::cw_flat_partial_bytes(const FlatLay& f, int64_t n, int64_t c, int 
     return clw_partial_bytes(cg, 9, false);
   }
   CwGeom g;
-  cw_geom_flat(g, f, n, c, esz, false);
+  cw_geom_flat(g, f, n, c);
   return cw_partial_bytes(g);
 }
 
@@ -773,7 +773,7 @@ int ddpm::cw_run(const void* cat, const void* grad_out, void* grad_weight, void*
     g.CI = (int)(4 * c);
     g.C = (int)c;
   } else if (f)
-    cw_geom_flat(g, *f, n, c, esz, pp);
+    cw_geom_flat(g, *f, n, c);
   else
     cw_geom(g, n, c, h, w, pp ? kCwTW : cw_step_cols(w, esz));
   g.gp = (int)gp;

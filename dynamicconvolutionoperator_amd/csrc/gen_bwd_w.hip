@@ -915,10 +915,9 @@ void wgrad_geom(WGradGeom& g, int64_t n, int64_t c, int64_t h, int64_t w, int d0
   g.f = FlatLay{};
 }
 
-// The same for flat tensors: a plane is one row of f.ft * 256 positions.
-void wgrad_geom_flat(WGradGeom& g, const FlatLay& f, int64_t n, int64_t c, int d0, int d1, int d2,
-                     int esz) {
-  wgrad_geom(g, n, c, 1, (int64_t)f.ft * kFlatTile, d0, d1, d2, esz == 2 ? 2 * kWgTW : kWgTW);
+// The same for flat fp32 tensors: a plane is one row of f.ft * 256 positions.
+void wgrad_geom_flat(WGradGeom& g, const FlatLay& f, int64_t n, int64_t c, int d0, int d1, int d2) {
+  wgrad_geom(g, n, c, 1, (int64_t)f.ft * kFlatTile, d0, d1, d2, kWgTW);
   g.cp = (int)flat_planes(c);
   g.f = f;
 }
@@ -996,7 +995,7 @@ int bw_run(const void* x, const void* y, const void* grad_out, void* grad_weight
     g.splits = cg.splits;
     g.direct = cg.direct;
   } else if (f)
-    wgrad_geom_flat(g, *f, n, c, gg.d0, gg.d1, gg.d2, esz);
+    wgrad_geom_flat(g, *f, n, c, gg.d0, gg.d1, gg.d2);
   else
     wgrad_geom(g, n, c, h, w, gg.d0, gg.d1, gg.d2, wg_step_cols(w, esz));
   const int64_t need =
@@ -1185,15 +1184,18 @@ int flat_bwd(FlatBwd& b, int64_t n, int64_t c, int64_t h, int64_t w, int kernel_
   if (guard < gg.R || ddpm_flat_cat_elems(n, c, h, w, guard, dtype) == 0 ||
       !flat_lay(b.f, h, w, guard, 4 * c, esz))
     return kUnsupported;
-  WGradGeom g;
-  wgrad_geom_flat(g, b.f, n, c, gg.d0, gg.d1, gg.d2, esz);
-  ClWGeom cg;
-  clw_geom(cg, b.f, n, c, true);
   b.copy = align256(flat_elems(b.f, n * flat_planes(c), esz) * esz);
   b.bx = align256(ddpm_gen_bwd_x_workspace_bytes(n, c, h, w, kernel_size, d0, d1, d2));
   b.by = align256(yt_flat_workspace_bytes(c, kernel_size, dtype));
-  b.bw = align256(esz == 2 ? clw_partial_bytes(cg, kernel_size * kernel_size, true)
-                           : wg_partial_bytes(g, c, kernel_size));
+  if (esz == 2) {
+    ClWGeom cg;
+    clw_geom(cg, b.f, n, c, true);
+    b.bw = align256(clw_partial_bytes(cg, kernel_size * kernel_size, true));
+  } else {
+    WGradGeom g;
+    wgrad_geom_flat(g, b.f, n, c, gg.d0, gg.d1, gg.d2);
+    b.bw = align256(wg_partial_bytes(g, c, kernel_size));
+  }
   return kOk;
 }
 
