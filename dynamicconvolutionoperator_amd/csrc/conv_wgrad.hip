@@ -529,7 +529,7 @@ __global__ __launch_bounds__(kCwThreads) void conv_wgrad_partial_kernel(
       for (int e = 0; e < 4; ++e)
 #pragma unroll
         for (int ib = 0; ib < MB; ++ib) nan = nan || acc[kj][ib][e] != acc[kj][ib][e];
-    if (flat_any<kCwNW>(nan, csm, wave)) run(std::true_type());
+    if (__builtin_expect(flat_any<kCwNW>(nan, csm, wave), 0)) run(std::true_type());
   }
 
   // ---- fixed-order reduction over the segments through LDS: each segment's

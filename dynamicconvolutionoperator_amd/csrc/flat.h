@@ -99,7 +99,7 @@ __device__ __forceinline__ void flat_copy_chunk(const FlatCopy& t, const FlatLay
 // replaced by zero: finite inputs pay one vote of a workgroup's waves
 // (generator / convolution, us, without -> with: bf16 4x64x135x181 74.0 ->
 // 74.0 / 42.5 -> 42.8, fp16 2x128x96x96 31.2 -> 33.1 / 33.5 -> 34.3, fp32
-// 4x64x135x181 122.4 -> 123.3 / 100.8 -> 103.4).
+// 4x64x135x181 122.4 -> 123.3 / 100.8 -> 102.3).
 
 // Positions of one row from `pos` (rows start on multiples of 8) that lie
 // inside the image, at most 8: none above the last column or row.
