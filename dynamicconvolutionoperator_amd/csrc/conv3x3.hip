@@ -635,10 +635,14 @@ void cv_split_cl(ConvGeom& g, int64_t tiles, int64_t m, bool split) {
 // (fp32 forward at 1x64x128x128: 68 tiles x 4 splits = 272 workgroups 30.0 us,
 // x 3 = 204 workgroups of half again the stages 24 us): the choice minimizes
 // rounds x stages by the measured cost of a stage (us, of one or more m
-// blocks) and of the partials' second pass.
+// blocks) and of the partials' second pass.  That pass is one more launch, 3.5
+// us of the host, which bounds passes of such kernels: splits that save less of
+// an unsplit kernel under 12 us are not worth it (C = 24 at 2x15x17, three
+// chunks: kernel estimated at 11.6 us unsplit, 9.0 split).
 void cv_split_flat(ConvGeom& g, int64_t tiles, int64_t m) {
   const double base = 0.65, per = 0.36;
-  double best = 1e30;
+  double best = 1e30, unsplit = 1e30;
+  int unsplit_mb = 1;
   for (int mb = kCvMaxMB; mb >= 1; mb /= 2) {
     const int64_t groups = (m + mb * 16 - 1) / (mb * 16);
     if (mb > 1 && groups * mb * 16 - m >= mb * 8 && m < mb * 16) continue;  // idle m blocks
@@ -649,6 +653,10 @@ void cv_split_flat(ConvGeom& g, int64_t tiles, int64_t m) {
       const double rounds = (double)((wgs + kCvFillWGs - 1) / kCvFillWGs);
       double t = rounds * (2.5 + 3 * cc * (base + per * mb));
       if (ks > 1) t += 3.5 + 4e-6 * (double)tiles * kFlatTile * (double)m * (ks + 1) / 4.0;
+      if (ks == 1 && t < unsplit) {
+        unsplit = t;
+        unsplit_mb = mb;
+      }
       if (t < best) {
         best = t;
         g.mb = mb;
@@ -656,6 +664,11 @@ void cv_split_flat(ConvGeom& g, int64_t tiles, int64_t m) {
         g.cc_per = cc;
       }
     }
+  }
+  if (g.ks > 1 && unsplit < 12.0 && unsplit - best < 3.5) {
+    g.mb = unsplit_mb;
+    g.ks = 1;
+    g.cc_per = g.nc32;
   }
 }
 

@@ -367,3 +367,16 @@ def test_flat_concat_rule(shape, code, training, expect):
 
     assert ops._concat_plan(*shape, 3, 5, code, training, True)[0] == expect
     assert ops._concat_plan(*shape, 3, 5, code, training, False)[:2] == (0, 0)
+
+
+def test_small_fuse_convolution_is_not_split():
+    """fp32, C = 24 at 2x15x17: three 32-plane chunks in one workgroup each -- the
+    packed weight (3 chunks x 9 taps x 2 blocks of 16 output planes, hi and lo
+    of 1 KB) and the flat copy of the concat (96 planes held as 128), no partial sums and so
+    no second launch."""
+    lib = _lib.load()
+    pitch, tile = 24, 256  # 17 + 1 columns to whole 8, positions of a tile
+    plane = 2 * tile + pitch + 8  # (15 rows are two tiles, one guard row, 8 columns)
+    copy = (pitch + 8 + 2 * 128 * plane) * 4
+    want = 3 * 9 * 2 * 2 * 1024
+    assert lib.ddpm_fuse_conv_workspace_bytes(2, 24, 15, 17, 0) == want + (copy + 255) // 256 * 256
