@@ -383,10 +383,11 @@ int gf_run(const void* x, const void* y, const void* weight, const void* bias, v
   if (pair && nk > 2) {
     // one workgroup per CU (the weights take 92 or 123 KB): the tile width
     // with the shortest run of rounds, a workgroup taking about 1 + cb.  f16
-    // at three chunks and 64 columns spills (184 us, 32 columns 152 us at
-    // 4x96x150x211; bf16's 256 registers just hold it, 151 us).  The kernel
-    // with one tap per step and 128 channels' padding took 219 us there
-    // (bf16), and 158 us against 117 us at 1x128x256x256.  At four chunks 64
+    // at three chunks and 64 columns spills (184 us against 32 columns' 152 us
+    // at 4x96x150x211 when it was built, 149 us now; bf16's 256 registers just
+    // hold it in its loops, 144 us).  The kernel with one tap per step and 128
+    // channels' padding took 219 us there (bf16), and 158 us against 115 us at
+    // 1x128x256x256.  At four chunks 64
     // columns fit the LDS with dilations (1, 1, 1) only: no kernel is built
     // for them.
     pair = false;

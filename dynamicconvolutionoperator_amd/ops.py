@@ -679,9 +679,9 @@ def _flat_pays(n, c, h, w, code, training) -> bool:
     Inference at 32, 64 and 128 columns: fp32 stays plain (16x64x64 112 / 146).
     2-byte types gain from channels-last (1x128x128 43 / 37, 5x128x128 108 / 94)
     unless, at up to 64 channels, the padded columns take one more round of
-    256-position tiles over 256 CUs (4x128x128, 256 / 272 tiles, 72 / 78; from
-    96 channels on the same (144 / 144), or the call is a few tiles above 64
-    channels (C = 128, 1x32x32 43 / 45, 4x32x32 44 / 46, 4x64x64 79 / 76)."""
+    256-position tiles over 256 CUs (4x128x128, 256 / 272 tiles, 72 / 78; C = 96
+    144 / 144), or the call is a few tiles of more channels (C = 128, 1x32x32
+    43 / 45, 4x32x32 44 / 46, 4x64x64 79 / 76)."""
     if w % 256 == 0 or (training and w == 128):
         return False
     if training or w not in (32, 64, 128):
@@ -708,11 +708,6 @@ def _concat_plan(n, c, h, w, k, max_dil, code, training, flat) -> tuple[int, int
         if elems > 0:
             return guard, elems, _ws_bytes("ddpm_flat_fuse_conv_workspace_bytes", n, c, h, w, guard, code)
     return 0, 0, _ws_bytes("ddpm_fuse_conv_workspace_bytes", n, c, h, w, code)
-
-
-def _flat_guard(x, k, dil, code, training) -> int:
-    """The guard of x's flat concat on the module's route, or 0 (:func:`_concat_plan`)."""
-    return _concat_plan(*x.shape, k, max(dil), code, training, True)[0]
 
 
 def _concat_pack(x, y, gen_weight, gen_bias, fuse_weight, k, dil, plan):
