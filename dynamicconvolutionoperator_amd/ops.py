@@ -674,7 +674,9 @@ def _flat_pays(n, c, h, w, code, training) -> bool:
     training (C = 64, us a pass, plain / flat: fp32 1x128x128 201 / 229, bf16
     4x128x128 300 / 305); every other width leaves lanes idle at row ends (8x48x48
     fp32 342 / 259, bf16 241 / 167) or, not a multiple of 8, is staged element by
-    element (bf16 2x135x181 1034 plain).
+    element (bf16 2x135x181 1034 plain).  Training a few fp32 tiles of whole 16-byte
+    rows gains nothing and takes two launches more (1x64x64 170 / 179, 1x48x48
+    171 / 181, 2x64x64 188 / 194, 2x80x80 233 / 200; C = 96 at 1x48x48 272 / 241).
 
     Inference at 32, 64 and 128 columns: fp32 stays plain (16x64x64 112 / 146).
     2-byte types gain from channels-last (1x128x128 43 / 37, 5x128x128 108 / 94)
@@ -683,6 +685,8 @@ def _flat_pays(n, c, h, w, code, training) -> bool:
     144 / 144), or the call is a few tiles of more channels (C = 128, 1x32x32
     43 / 45, 4x32x32 44 / 46, 4x64x64 79 / 76)."""
     if w % 256 == 0 or (training and w == 128):
+        return False
+    if training and code == _PAIR_PLANES and c <= 64 and w % 8 == 0 and n * h * w <= 4096:
         return False
     if training or w not in (32, 64, 128):
         return True

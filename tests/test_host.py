@@ -353,6 +353,9 @@ def test_bench_prices_every_step_entry_point():
     ((1, 64, 256, 256), 1, True, 0), ((4, 64, 128, 128), 1, True, 0), ((1, 64, 9, 512), 3, False, 0),
     # other widths, multiples of 8 and odd ones; the guard holds the halo only where a backward follows
     ((2, 64, 96, 96), 3, True, 5), ((2, 64, 135, 181), 1, True, 5), ((1, 32, 48, 48), 3, False, 1),
+    # a few fp32 tiles of whole 16-byte rows trained: plain (2-byte types, more channels, odd widths: flat)
+    ((1, 64, 48, 48), 3, True, 0), ((1, 64, 64, 64), 3, True, 0), ((1, 64, 48, 48), 1, True, 5),
+    ((1, 96, 48, 48), 3, True, 5), ((1, 64, 41, 45), 3, True, 5), ((1, 64, 80, 80), 3, True, 5),
     # inference at 32, 64 and 128 columns: fp32 plain; 2-byte types flat ...
     ((4, 64, 64, 64), 3, False, 0), ((1, 64, 128, 128), 1, False, 1), ((5, 64, 128, 128), 2, False, 1),
     # ... unless the padding takes one more round of tiles (256 / 272, 512 / 544),
